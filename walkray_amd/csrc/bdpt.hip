@@ -18,7 +18,7 @@
 // The visibility tests of the connections are not traced by the lane that
 // forms them: each connection that passes every other test appends its
 // visibility ray (and its contribution and target pixel) to a queue, traced
-// afterwards one ray per lane by the batch NoSelf query (k_closest_hit_path:
+// afterwards one ray per lane by the batch NoSelf query (k_closest_hit:
 // the same traversal, so the same answers) and folded in by k_bdpt_accum; a
 // lane whose queue is full traces in place.
 // The sub-paths live in device memory (one block of records per lane).  A
@@ -1134,7 +1134,7 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     if (nq > q.cap) nq = q.cap;
     if (nq) {
-        if ((e = launch_closest_hit_path(S, H, q.rays, nq, q.hits, st)) != hipSuccess)
+        if ((e = launch_closest_hit_path(S, H, q.rays, nq, q.hits, q.work, st)) != hipSuccess)
             return hip_fail(ctx, e, "wr_render_vcm: visibility");
         wrd::k_bdpt_accum<<<(nq + 255) / 256, 256, 0, st>>>(nq, q.pay, q.dst, (const uint4*)q.hits, pix);
     }
@@ -1203,7 +1203,7 @@ hipError_t launch_bdpt_passes(const SceneDev& S, const wr_tree_hdr& H, const Cam
     if (e != hipSuccess) return e;
     if (nq > q.cap) nq = q.cap;
     if (nq) {
-        e = launch_closest_hit_path(S, H, q.rays, nq, q.hits, st);
+        e = launch_closest_hit_path(S, H, q.rays, nq, q.hits, q.work, st);
         if (e != hipSuccess) return e;
         wrd::k_bdpt_accum<<<(nq + 255) / 256, 256, 0, st>>>(nq, q.pay, q.dst, (const uint4*)q.hits, pix);
     }

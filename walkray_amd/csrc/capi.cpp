@@ -981,7 +981,7 @@ int wr_autotune_closest_hit(wr_ctx* ctx, wr_scene* s, const wr_ray* d_rays, uint
     const uint32_t refills[] = {4, 8, 16, 24, 32};
     const uint32_t blocks[] = {0, 7, 6, 5};
     const uint32_t levels[] = {4, 8, 16};
-    const uint32_t batches[] = {128, 256, 512, 1024};
+    const uint32_t batches[] = {64, 128, 256, 512};
     for (int pass = 0; pass < 2 && e == hipSuccess; pass++) {
         for (uint32_t v : nodes) {
             ChTune t = cur;
@@ -1041,15 +1041,15 @@ int wr_scene_set_closest_hit_tuning(wr_scene* s, const wr_closest_hit_tuning* t)
     s->ch_tune.refill_min = t->refill_min;
     s->ch_tune.node_phase_min = t->node_phase_min;
     s->ch_tune.blocks_per_cu = t->blocks_per_cu;
-    s->ch_tune.batch = t->batch ? t->batch : 256u;
+    s->ch_tune.batch = t->batch ? t->batch : 128u;
     return WR_OK;
 }
 
 int wr_closest_hit_noself(wr_ctx* ctx, const wr_scene* s, const wr_path_ray* d_rays, uint64_t n, wr_hit* d_hits) {
     if (!ctx || !s || (n && (!d_rays || !d_hits))) return fail(ctx, WR_EINVAL, "wr_closest_hit_noself: bad argument");
     if (!s->built) return fail(ctx, WR_ESTATE, "wr_closest_hit_noself: scene not built");
-    hipError_t e = launch_closest_hit_path(s->dev, s->hdrs[0], (const uint32_t*)d_rays, n, d_hits, ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, e, "k_closest_hit_path launch");
+    hipError_t e = launch_closest_hit_path(s->dev, s->hdrs[0], (const uint32_t*)d_rays, n, d_hits, ctx->d_work, ctx->stream);
+    if (e != hipSuccess) return hip_fail(ctx, e, "wr_closest_hit_noself launch");
     return WR_OK;
 }
 

@@ -274,6 +274,7 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     // the visibility queue: 32 entries per lane, at most 24M (1.6 GB); a full queue
     // makes the remaining connections trace in place
     BdptQueue q{};
+    q.work = ctx->d_work;
     q.cap = prm->wave_slots ? prm->wave_slots : (uint32_t)std::min<uint64_t>(32ull * npix * batch, 24ull << 20);
     void* qbuf = nullptr;
     hipError_t e = hipMalloc(&verts, per_pass * batch);
@@ -347,6 +348,7 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     batch = std::min<uint64_t>(batch, std::max<uint64_t>(1, ((1ull << 31) - 1) / (npix * maxv)));
     const uint64_t lanes = batch * npix;
     BdptQueue q{};
+    q.work = ctx->d_work;
     q.cap = prm->wave_slots ? prm->wave_slots : (uint32_t)std::min<uint64_t>(32ull * lanes, 24ull << 20);
     VcmBufs vb{};
     vb.cap = lanes * maxv;

@@ -2,14 +2,17 @@
 //
 //  k_closest_hit        KDTree::intersect without Condition (kdtree.cpp:349-353),
 //                       as used by Scene::intersect for camera rays (camera.cpp:52)
-//  k_closest_hit_path   the same query with NoSelfCondition (mcRenderer.cpp:42-44,
-//                       noself.cpp:13-20)
+//                       and, as its NOSELF instance, with NoSelfCondition
+//                       (mcRenderer.cpp:42-44, noself.cpp:13-20)
 //  k_inside_object      Scene::findInsideObject (scene.cpp:115-144)
 //
 // One lane per ray, wave64, 256-lane workgroups; per-lane node stack in LDS;
-// workgroup ids are remapped so each XCD walks a contiguous range of rays
-// (neighbouring rays share tree nodes, and each XCD has its own L2).
+// the finishing kernel's workgroup ids are remapped so each XCD walks a
+// contiguous range of rays (neighbouring rays share chain records, and each
+// XCD has its own L2).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "trace_dev.h"
 #include "wr_kernels.h"
@@ -18,7 +21,6 @@
 
 namespace wrd {
 
-using wr::kWorkDone;
 using wr::kWorkStride;
 using wr::kXcds;
 
@@ -57,42 +59,83 @@ __device__ __forceinline__ void add_counters(unsigned long long* out, const Coun
     }
 }
 
-// Fast pass of the batch closest-hit query as a persistent kernel: each wave
-// takes rays in batches of `batch` from a work counter and refills a lane with
-// the next ray as soon as its traversal ends, so a wave never waits for its
-// slowest ray.  The result of the fast pass (record, t, first record of the
-// leaf, overflow flag) goes to hits[ray]; k_closest_hit_finish completes it.
-// Work queues: the rays are cut into kXcds contiguous ranges, range q handed
-// out by the counter work[q * kWorkStride] to the workgroups of XCD q
-// (workgroups are dispatched to the XCDs round-robin), so neighbouring rays
-// share one XCD's L2 and each counter takes an eighth of the atomics.  A wave
-// whose range is used up moves on to the next range (and so on round the
-// ranges); once it has found all of them used up it is done.  work[kWorkDone]
-// counts finished waves; the last wave out zeroes every counter for the next
-// launch.  Compiled for 8 waves per SIMD (64
-// VGPRs): more waves in flight hide more of the node-fetch latency.
+// One ray of a batch: closest-hit rays are 6 floats (origin, direction), NoSelf
+// rays 8 words (origin, direction, inside, contact).
+template <bool NOSELF>
+__device__ __forceinline__ void load_ray(const uint32_t* __restrict__ rays, uint64_t i, f3& o, f3& d, uint32_t& inside,
+                                         uint32_t& contact) {
+    const uint32_t* rp = rays + (NOSELF ? 8 : 6) * i;
+    o = mk(__uint_as_float(rp[0]), __uint_as_float(rp[1]), __uint_as_float(rp[2]));
+    d = mk(__uint_as_float(rp[3]), __uint_as_float(rp[4]), __uint_as_float(rp[5]));
+    inside = NOSELF ? rp[6] : WR_NONE;
+    contact = NOSELF ? rp[7] : WR_NONE;
+}
+
+template <bool NOSELF>
+__device__ __forceinline__ NoSelf make_noself(const SceneDev& S, const wr_tree_hdr& H, uint32_t inside,
+                                              uint32_t contact) {
+    if (!NOSELF) return NoSelf{};
+    return NoSelf{inside, contact, S.rec_nrm + 9 * (size_t)H.rec_base, S.obj_has_normals};
+}
+
+// Fast pass of the batch closest-hit query as a persistent kernel, for batches
+// of more rays than the device holds lanes: a wave takes one unit of 64 rays
+// at a time and refills a lane with the next ray as soon as its traversal
+// ends, so a wave never waits for its slowest ray.  The result of the fast
+// pass (record, t, first record of the leaf, overflow flag) goes to hits[ray];
+// k_closest_hit_finish completes it.
+// Work distribution: every XCD has a range of the units (workgroups are
+// dispatched to the XCDs round-robin), made of stripes of `stripe` units that
+// the XCDs take in turn: neighbouring rays share one XCD's L2, and every range
+// sees the whole ray array, so the ranges end together and none needs another
+// XCD's help.  What bounds the distribution is the shared counters: an atomic
+// on one address takes about 65 ns here whatever the number of waves, and so
+// does a load that other XCDs' atomics keep out of L2.  So a workgroup's first
+// `first` units need no counter, later ones come `batch` at a time from the
+// range's counter into a pool in LDS that its four waves share, and a wave
+// that finds the range used up is done: no probing of other ranges, no count
+// of finished waves (k_closest_hit_finish zeroes the counters).  With one
+// counter atomic per wave and 256 rays, probing of the other seven ranges and
+// the count, 400,009 incoherent rays on the 512-object field took 242 us and
+// 8M camera rays 0.93 ms; now 142 us and 0.80 ms (with the finishing kernel; 16.8M rays on the 2.1M-triangle heightfield, where
+// the traversal itself is all, stay at 2.6 ms coherent, 3.2 ms incoherent).  Compiled for 8 waves per SIMD (64
+// VGPRs): more waves in flight hide more of the node-fetch latency; with the
+// NoSelf test for the 5 that its registers allow.
 // Scheduling knobs (ChTune, chosen by the autotuner): idle lanes are refilled
 // once at least refill_min are idle; a wave runs node-only steps while at
 // least node_phase_min lanes sit at wide nodes (a mixed step pays for both the
 // node code and the triangle code).
 // D: stack levels in LDS (the autotuner's stack-depth knob).
-template <bool COUNT, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_closest_hit(
-    SceneDev S, wr_tree_hdr H, const float* __restrict__ rays, uint64_t n, uint4* __restrict__ hits,
+template <bool NOSELF, bool COUNT, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NOSELF ? 5 : 8))) void k_closest_hit(
+    SceneDev S, wr_tree_hdr H, const uint32_t* __restrict__ rays, uint64_t n, uint4* __restrict__ hits,
     unsigned long long* counters, unsigned long long* work, uint32_t refill_min, uint32_t node_phase_min,
-    uint32_t batch) {
+    uint32_t batch, uint32_t first, uint32_t stripe) {
     const Tree tr = make_tree(H, S);
     StackSpillT<D> spill;
     LaneStackT<D> st(&spill);
     Counters cnt{0, 0, 0};
-    const NoSelf ns{};
+    NoSelf ns{};
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = (1ull << lane) - 1ull;
-    uint64_t bnext = 0, bend = 0;  // the wave's current batch [bnext, bend)
+    // the workgroup's units of its range: next | end << 32
+    __shared__ unsigned long long pool;
+    const uint32_t ranges = gridDim.x < kXcds ? gridDim.x : kXcds;
+    const uint32_t q = blockIdx.x % ranges;
+    const uint32_t units = (uint32_t)((n + 63) / 64), row = stripe * ranges;
+    // units of range q: whole rows of stripes, and its part of the last one
+    const uint32_t rest = units % row;
+    const uint32_t len = units / row * stripe + (rest > q * stripe ? min(rest - q * stripe, stripe) : 0u);
+    const uint32_t firsts = (gridDim.x - q + ranges - 1) / ranges * first;  // taken without the counter
+    if (threadIdx.x == 0) {
+        const uint32_t a = blockIdx.x / ranges * first;
+        pool = a < len ? (a | (unsigned long long)min(a + first, len) << 32) : 0ull;
+    }
+    __syncthreads();
+    uint32_t kept = 0, kept_end = 0;  // units of the range that this wave keeps to itself
+    uint64_t bnext = 0, bend = 0;     // the rays of its current unit [bnext, bend)
     bool exhausted = false;
     bool active = false, overflow = false;
-    uint32_t q = blockIdx.x % kXcds;  // the work range of this workgroup's XCD
-    uint32_t used_up = 0;             // ranges this wave has found used up (each once: they stay so)
     uint64_t rid = 0;
     uint32_t ref = 0;
     RayPre r{};
@@ -102,33 +145,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         if (!exhausted && (uint32_t)__popcll(idle) >= refill_min) {
             while (idle != 0) {
                 if (bnext == bend) {
-                    // next batch: from range q, or the next range once q is used up
-                    bool got = false;
-                    while (used_up < kXcds) {
-                        const uint64_t lo = n * q / kXcds, hi = n * (q + 1) / kXcds;
-                        unsigned long long base = 0;
-                        if (lane == 0) base = atomicAdd(work + kWorkStride * q, (unsigned long long)batch);
-                        base = __shfl(base, 0);
-                        if (lo + base < hi) {
-                            bnext = lo + base;
-                            bend = lo + base + batch < hi ? lo + base + batch : hi;
-                            got = true;
-                            break;
-                        }
-                        q = q + 1 < kXcds ? q + 1 : 0;
-                        used_up++;
+                    uint32_t a = kept < kept_end ? kept++ : len;
+                    if (a == len) {
+                        unsigned long long p = 0;
+                        if (lane == 0) p = atomicAdd(&pool, 1ull);
+                        p = __shfl(p, 0);
+                        if ((uint32_t)p < (uint32_t)(p >> 32)) a = (uint32_t)p;
                     }
-                    if (!got) {
+                    if (a == len && firsts < len) {  // the pool is empty: the next units of the range
+                        unsigned long long c = 0, pub = 0;
+                        if (lane == 0) {
+                            c = firsts + atomicAdd(work + kWorkStride * q, (unsigned long long)batch);
+                            if (c + 1 < len) {  // all but the first go to the pool, if no other wave has filled it
+                                const unsigned long long next = (c + 1) | min(c + batch, (unsigned long long)len) << 32;
+                                unsigned long long cur = atomicAdd(&pool, 0ull);
+                                while (!pub && (uint32_t)cur >= (uint32_t)(cur >> 32)) {
+                                    const unsigned long long old = atomicCAS(&pool, cur, next);
+                                    pub = old == cur;
+                                    cur = old;
+                                }
+                            }
+                        }
+                        c = __shfl(c, 0);
+                        if (c < len) {
+                            a = (uint32_t)c;
+                            if (!__shfl(pub, 0)) {  // another wave filled it: this one keeps its units
+                                kept = a + 1;
+                                kept_end = (uint32_t)min(c + batch, (unsigned long long)len);
+                            }
+                        }
+                    }
+                    if (a == len) {
                         exhausted = true;
                         break;
                     }
+                    const uint32_t u = a / stripe * row + q * stripe + a % stripe;
+                    bnext = 64ull * u;
+                    bend = bnext + 64 < n ? bnext + 64 : n;
                 }
                 const uint64_t avail = bend - bnext;
                 const uint64_t rank = (uint64_t)__popcll(idle & below);
                 if (!active && rank < avail) {
                     rid = bnext + rank;
-                    const float* rp = rays + 6 * rid;
-                    r = make_ray(mk(rp[0], rp[1], rp[2]), mk(rp[3], rp[4], rp[5]), tr.scale);
+                    f3 o, d;
+                    uint32_t inside, contact;
+                    load_ray<NOSELF>(rays, rid, o, d, inside, contact);
+                    r = make_ray(o, d, tr.scale);
+                    ns = make_noself<NOSELF>(S, H, inside, contact);
                     overflow = false;
                     if (wide_begin(tr, r, st, h, ref)) active = true;
                     else hits[rid] = make_uint4(WR_NONE, 0u, 0u, 0u);  // misses the root box
@@ -144,33 +207,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         for (;;) {
             const bool at_node = active && !(ref & WR_LEAF_BIT);
             if ((uint32_t)__popcll(__ballot(at_node)) < node_phase_min) break;
-            if (at_node && !wide_step<false, COUNT>(tr, r, ns, st, h, ref, overflow, cnt)) {
+            if (at_node && !wide_step<NOSELF, COUNT>(tr, r, ns, st, h, ref, overflow, cnt)) {
                 hits[rid] = make_uint4(h.rec, __float_as_uint(h.t), h.leaf, overflow ? 1u : 0u);
                 active = false;
             }
         }
-        if (active && !wide_step<false, COUNT>(tr, r, ns, st, h, ref, overflow, cnt)) {
+        if (active && !wide_step<NOSELF, COUNT>(tr, r, ns, st, h, ref, overflow, cnt)) {
             hits[rid] = make_uint4(h.rec, __float_as_uint(h.t), h.leaf, overflow ? 1u : 0u);
             active = false;
         }
     }
     if (COUNT) add_counters(counters, cnt);
-    if (lane == 0) {
-        const unsigned long long waves = (unsigned long long)gridDim.x * (blockDim.x / 64);
-        if (atomicAdd(work + kWorkDone, 1ull) == waves - 1) {
-            for (uint32_t k = 0; k < kXcds; k++) atomicExch(work + kWorkStride * k, 0ull);
-            atomicExch(work + kWorkDone, 0ull);
-        }
-    }
 }
 
-// Completion of k_closest_hit's records: binary fast pass after a wide-stack
-// overflow, chain verification, exact fallback, barycentrics, output.  One
-// lane per ray, so the verification walks of a wave run together.
-template <bool COUNT, int D>
+// Completion of one ray's fast pass (binary fast pass after a wide-stack
+// overflow, chain verification, exact fallback) and its output record.
+template <bool NOSELF, bool COUNT, class Stack>
+__device__ __forceinline__ uint4 complete_hit(const Tree& tr, const RayPre& r, const NoSelf& ns, Stack& st,
+                                              Counters& cnt, HitState h, bool overflow) {
+    uint4 out = make_uint4(WR_NONE, __float_as_uint(-1.f), 0u, 0u);
+    bool failed;
+    // the winner's record is fetched alongside the verification's first fetch
+    const uint32_t rec0 = h.rec;
+    wr_tri T{};
+    if (rec0 != WR_NONE) T = tr.tris[rec0];
+    finish_hit<NOSELF, COUNT>(tr, r, ns, st, cnt, h, overflow, failed);
+    if (h.rec != WR_NONE) {
+        if (h.rec != rec0) T = tr.tris[h.rec];
+        float u1, u2;
+        bary(T, r.o, r.d, h.t, u1, u2);
+        out = make_uint4(T.prim, __float_as_uint(h.t), __float_as_uint(u1), __float_as_uint(u2));
+    }
+    if (failed) out.x = 0xFFFFFFFEu;  // stack overflow: reported, never silently wrong
+    return out;
+}
+
+// Completion of k_closest_hit's records, one lane per ray, so the verification
+// walks of a wave run together.
+template <bool NOSELF, bool COUNT, int D>
 __global__ __launch_bounds__(256) void k_closest_hit_finish(SceneDev S, wr_tree_hdr H,
-                                                            const float* __restrict__ rays, uint64_t n,
-                                                            uint4* __restrict__ hits, unsigned long long* counters) {
+                                                            const uint32_t* __restrict__ rays, uint64_t n,
+                                                            uint4* __restrict__ hits, unsigned long long* counters,
+                                                            unsigned long long* work) {
+    if (blockIdx.x == 0 && threadIdx.x < kXcds) work[kWorkStride * threadIdx.x] = 0ull;  // for the next launch
     const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
     const uint64_t i = (uint64_t)b * 256 + threadIdx.x;
     Counters cnt{0, 0, 0};
@@ -178,62 +257,49 @@ __global__ __launch_bounds__(256) void k_closest_hit_finish(SceneDev S, wr_tree_
     LaneStackT<D> st(&spill);
     if (i < n) {
         const uint4 f = hits[i];
-        HitState h{__uint_as_float(f.y), f.x, f.z};
+        const HitState h{__uint_as_float(f.y), f.x, f.z};
         const bool overflow = f.w != 0;
         uint4 out = make_uint4(WR_NONE, __float_as_uint(-1.f), 0u, 0u);
         if (h.rec != WR_NONE || overflow) {
-            const float* rp = rays + 6 * i;
-            const f3 o = mk(rp[0], rp[1], rp[2]);
-            const f3 d = mk(rp[3], rp[4], rp[5]);
+            f3 o, d;
+            uint32_t inside, contact;
+            load_ray<NOSELF>(rays, i, o, d, inside, contact);
             const Tree tr = make_tree(H, S);
             const RayPre r = make_ray(o, d, tr.scale);
-            const NoSelf ns{};
-            bool failed;
-            // the winner's record is fetched alongside the verification's first fetch
-            const uint32_t rec0 = h.rec;
-            wr_tri T{};
-            if (rec0 != WR_NONE) T = tr.tris[rec0];
-            finish_hit<false, COUNT>(tr, r, ns, st, cnt, h, overflow, failed);
-            if (h.rec != WR_NONE) {
-                if (h.rec != rec0) T = tr.tris[h.rec];
-                float u1, u2;
-                bary(T, o, d, h.t, u1, u2);
-                out = make_uint4(T.prim, __float_as_uint(h.t), __float_as_uint(u1), __float_as_uint(u2));
-            }
-            if (failed) out.x = 0xFFFFFFFEu;  // stack overflow: reported, never silently wrong
+            out = complete_hit<NOSELF, COUNT>(tr, r, make_noself<NOSELF>(S, H, inside, contact), st, cnt, h, overflow);
         }
         hits[i] = out;
     }
     if (COUNT) add_counters(counters, cnt);
 }
 
-__global__ __launch_bounds__(256) void k_closest_hit_path(SceneDev S, wr_tree_hdr H, const uint32_t* __restrict__ rays,
-                                                          uint64_t n, uint4* __restrict__ hits) {
-    const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
-    const uint64_t i = (uint64_t)b * 256 + threadIdx.x;
-    if (i >= n) return;
+// The whole query in one launch, one lane per ray: the first `width` lanes of
+// every wave take a ray each.  A small batch is bound by the latency of its
+// longest traversal (about 40 us), and lanes that share a wave lengthen it:
+// they wait for each other's triangle and node steps, and their 64 B fetches
+// go through one CU's cache one line at a time.  So few rays are spread over
+// many waves.  1,000 / 16,000 / 65,537 rays on the 512-object field: 60 / 77 /
+// 80 us with 16 lanes, 46 / 106 / 207 us with one, 67 / 95 / 91 us with 64.
+template <bool NOSELF>
+__global__ __launch_bounds__(256) void k_closest_hit_small(SceneDev S, wr_tree_hdr H,
+                                                           const uint32_t* __restrict__ rays, uint64_t n,
+                                                           uint32_t width, uint4* __restrict__ hits) {
+    const uint32_t lane = threadIdx.x & 63u, wave = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const uint64_t i = (uint64_t)wave * width + lane;
+    if (lane >= width || i >= n) return;
     StackSpill spill;
     LaneStack st(&spill);
-    const uint32_t* rp = rays + 8 * i;
-    const f3 o = mk(__uint_as_float(rp[0]), __uint_as_float(rp[1]), __uint_as_float(rp[2]));
-    const f3 d = mk(__uint_as_float(rp[3]), __uint_as_float(rp[4]), __uint_as_float(rp[5]));
+    f3 o, d;
+    uint32_t inside, contact;
+    load_ray<NOSELF>(rays, i, o, d, inside, contact);
     const Tree tr = make_tree(H, S);
     const RayPre r = make_ray(o, d, tr.scale);
-    NoSelf ns{rp[6], rp[7], S.rec_nrm + 9 * (size_t)H.rec_base, S.obj_has_normals};
+    const NoSelf ns = make_noself<NOSELF>(S, H, inside, contact);
     Counters cnt{0, 0, 0};
-    bool failed;
-    const HitState h = closest_hit<true, false>(tr, r, ns, st, cnt, failed);
-    uint4 out;
-    if (h.rec != WR_NONE) {
-        float u1, u2;
-        bary(tr.tris[h.rec], o, d, h.t, u1, u2);
-        out = make_uint4(tr.tris[h.rec].prim, __float_as_uint(h.t), __float_as_uint(u1),
-                         __float_as_uint(u2));
-    } else {
-        out = make_uint4(WR_NONE, __float_as_uint(-1.f), 0u, 0u);
-    }
-    if (failed) out.x = 0xFFFFFFFEu;
-    hits[i] = out;
+    HitState h;
+    bool overflow;
+    traverse_wide<NOSELF, false>(tr, r, ns, st, h, overflow, cnt);
+    hits[i] = complete_hit<NOSELF, false>(tr, r, ns, st, cnt, h, overflow);
 }
 
 __global__ __launch_bounds__(256) void k_inside_object(SceneDev S, const uint32_t* __restrict__ rays, uint64_t n,
@@ -286,14 +352,14 @@ hipError_t launch_hit_sources(const SceneDev& S, uint32_t n_tris, const void* hi
 
 // Workgroups of the persistent kernel with D LDS stack levels: per_cu per CU
 // (0: as many as fit).
-template <int D>
+template <bool NOSELF, int D>
 static uint32_t persistent_blocks(uint64_t n, uint32_t per_cu_want) {
     static int cus = 0, per_cu_max = 0;
     if (!cus) {
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_max, wrd::k_closest_hit<false, D>, 256,
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_max, wrd::k_closest_hit<NOSELF, false, D>, 256,
                                                          wrd::stack_lds_bytes<D>()) != hipSuccess ||
             cus <= 0 || per_cu_max <= 0) {
             cus = 256;
@@ -306,30 +372,60 @@ static uint32_t persistent_blocks(uint64_t n, uint32_t per_cu_want) {
     return (uint32_t)(need < resident ? need : resident);
 }
 
-template <int D>
-static hipError_t launch_closest_hit_d(const SceneDev& S, const wr_tree_hdr& H, const float* rays, uint64_t n,
+// Waves that k_closest_hit_small spreads a small batch over: four per SIMD.
+constexpr uint64_t kSmallWaves = 4096;
+// Largest batch for k_closest_hit_small; a larger one has more rays than the
+// persistent kernel's resident lanes (8 waves on each of 1,024 SIMDs), so that
+// refilling lanes pays.  Incoherent rays on the field, in us, small against
+// persistent: 400,009 rays 132 / 142, 700,001 rays 178 / 181, 1,000,003 rays
+// 229 / 207, 4M 762 / 459.  With the NoSelf test, whose normals leave both
+// kernels 5 waves per SIMD, rays from camera hits cross over later: 1M
+// 181 / 255, 2M 306 / 367, 4M 564 / 555.
+template <bool NOSELF>
+constexpr uint64_t kSmallMax = NOSELF ? 1ull << 21 : 1ull << 19;
+
+template <bool NOSELF, int D>
+static hipError_t launch_closest_hit_d(const SceneDev& S, const wr_tree_hdr& H, const uint32_t* rays, uint64_t n,
                                        void* hits, unsigned long long* counters, unsigned long long* work,
                                        uint32_t per_cu, uint32_t rmin, uint32_t nmin, uint32_t batch,
                                        hipStream_t st) {
-    const uint32_t pgrid = persistent_blocks<D>(n, per_cu);
+    uint4* out = (uint4*)hits;
+    if (n <= kSmallMax<NOSELF> && !counters) {
+        // the power of two nearest to the rays per wave
+        uint32_t width = 1;
+        while (width < 64 && 2 * n > 3ull * width * kSmallWaves) width *= 2;
+        const uint64_t waves = (n + width - 1) / width;
+        wrd::k_closest_hit_small<NOSELF>
+            <<<(uint32_t)((waves + 3) / 4), 256, wrd::kStackLdsBytes, st>>>(S, H, rays, n, width, out);
+        return hipGetLastError();
+    }
+    const uint32_t pgrid = persistent_blocks<NOSELF, D>(n, per_cu);
     const uint32_t grid = (uint32_t)((n + 255) / 256);
     const size_t lds = wrd::stack_lds_bytes<D>();
+    // units of 64 rays: a workgroup's first ones, one for each of its waves; then at most `batch` rays
+    // at a time, fewer where it would come back less than eight times; stripes of at most 64
+    const uint64_t units = (n + 63) / 64;
+    const uint32_t first = (uint32_t)std::min<uint64_t>((units + pgrid - 1) / pgrid, 4);
+    const uint64_t left = units > (uint64_t)first * pgrid ? units - (uint64_t)first * pgrid : 0;
+    const uint32_t take = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(batch / 64, left / (8ull * pgrid)));
+    const uint32_t stripe = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(64, units / (16 * kXcds)));
     if (counters) {
-        wrd::k_closest_hit<true, D><<<pgrid, 256, lds, st>>>(S, H, rays, n, (uint4*)hits, counters, work, rmin, nmin,
-                                                                 batch);
-        wrd::k_closest_hit_finish<true, D><<<grid, 256, lds, st>>>(S, H, rays, n, (uint4*)hits, counters);
+        wrd::k_closest_hit<NOSELF, true, D>
+            <<<pgrid, 256, lds, st>>>(S, H, rays, n, out, counters, work, rmin, nmin, take, first, stripe);
+        wrd::k_closest_hit_finish<NOSELF, true, D><<<grid, 256, lds, st>>>(S, H, rays, n, out, counters, work);
     } else {
-        wrd::k_closest_hit<false, D><<<pgrid, 256, lds, st>>>(S, H, rays, n, (uint4*)hits, nullptr, work, rmin, nmin,
-                                                                  batch);
-        wrd::k_closest_hit_finish<false, D><<<grid, 256, lds, st>>>(S, H, rays, n, (uint4*)hits, nullptr);
+        wrd::k_closest_hit<NOSELF, false, D>
+            <<<pgrid, 256, lds, st>>>(S, H, rays, n, out, nullptr, work, rmin, nmin, take, first, stripe);
+        wrd::k_closest_hit_finish<NOSELF, false, D><<<grid, 256, lds, st>>>(S, H, rays, n, out, nullptr, work);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_closest_hit(const SceneDev& S, const wr_tree_hdr& H, const float* rays, uint64_t n, void* hits,
+hipError_t launch_closest_hit(const SceneDev& S, const wr_tree_hdr& H, const float* rays_f, uint64_t n, void* hits,
                               unsigned long long* counters, unsigned long long* work, const ChTune& tune,
                               hipStream_t st) {
     if (n == 0) return hipSuccess;
+    const uint32_t* rays = (const uint32_t*)rays_f;
     // refill_min in [1, 64]; node_phase_min in [1, 65] (0 would never leave the node phase; 65 disables it)
     const uint32_t rmin = tune.refill_min < 1 ? 1 : (tune.refill_min > 64 ? 64 : tune.refill_min);
     const uint32_t nmin = tune.node_phase_min < 1 ? 1 : (tune.node_phase_min > 65 ? 65 : tune.node_phase_min);
@@ -338,20 +434,20 @@ hipError_t launch_closest_hit(const SceneDev& S, const wr_tree_hdr& H, const flo
     const uint32_t pc = tune.blocks_per_cu;
     switch (tune.lds_levels) {
         case 4:
-            return launch_closest_hit_d<4>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
+            return launch_closest_hit_d<false, 4>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
         case 16:
-            return launch_closest_hit_d<16>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
+            return launch_closest_hit_d<false, 16>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
         default:
-            return launch_closest_hit_d<8>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
+            return launch_closest_hit_d<false, 8>(S, H, rays, n, hits, counters, work, pc, rmin, nmin, batch, st);
     }
 }
 
 hipError_t launch_closest_hit_path(const SceneDev& S, const wr_tree_hdr& H, const uint32_t* rays, uint64_t n,
-                                   void* hits, hipStream_t st) {
+                                   void* hits, unsigned long long* work, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const uint32_t grid = (uint32_t)((n + 255) / 256);
-    wrd::k_closest_hit_path<<<grid, 256, wrd::kStackLdsBytes, st>>>(S, H, rays, n, (uint4*)hits);
-    return hipGetLastError();
+    const ChTune t;
+    return launch_closest_hit_d<true, 8>(S, H, rays, n, hits, nullptr, work, t.blocks_per_cu, t.refill_min,
+                                         t.node_phase_min, t.batch, st);
 }
 
 hipError_t launch_inside_object(const SceneDev& S, uint32_t max_obj_depth, const uint32_t* rays, uint64_t n,

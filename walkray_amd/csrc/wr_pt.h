@@ -165,6 +165,7 @@ struct BdptQueue {
     uint32_t* count;
     uint32_t cap;
     uint32_t* counts;  // 2 per pixel and pass: the eye and light sub-path record counts
+    unsigned long long* work;  // work counters of the batch queries on this stream (wr_ctx::d_work)
 };
 constexpr size_t kBdptQueueEntryBytes = 32 + 16 + 4 + 16;
 size_t bdpt_vertex_bytes();
