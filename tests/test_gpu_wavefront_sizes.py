@@ -1,0 +1,30 @@
+"""Wavefront films at the numbers of live paths where its trace stage changes the paths per wave
+(a unit of 1, 2, 4, ... 64 paths) and starts to draw units from its counters: bit-identical to the
+megakernel's films."""
+import numpy as np
+import pytest
+
+from walkray_amd import _lib as W
+from walkray_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width,height,spp,slots", [
+    (1, 1, 1, 0), (96, 64, 1, 0), (5, 1229, 1, 0), (193, 97, 1, 0), (384, 256, 1, 0), (391, 503, 1, 0),
+    (391, 503, 2, 0),        # 393,346 paths: more full units than the resident waves
+    (701, 467, 4, 0),        # 1.3M paths: units from the counters, two at a time
+    (200, 150, 3, 20000),    # a pool smaller than a pass
+])
+@pytest.mark.parametrize("nee", [False, True])
+def test_paths_per_wave(ctx, width, height, spp, slots, nee):
+    objs, cam = S.random_field(n_objects=40, seed=5, width=width, height=height)
+    sc = W.Scene(ctx, objs)
+    films = []
+    for mode in (W.WR_MEGAKERNEL, W.WR_WAVEFRONT):
+        film = W.Film(ctx, width, height)
+        for k in range(2):  # two calls: the counters are left ready for the next
+            W.render(sc, cam, film, spp, 6, 99, mode, wave_slots=slots if mode == W.WR_WAVEFRONT else 0, nee=nee)
+        films.append(film.read())
+    for k in ("sum", "comp", "sumsq"):
+        assert np.array_equal(films[0][k].view(np.uint32), films[1][k].view(np.uint32)), k

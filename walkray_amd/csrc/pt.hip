@@ -24,10 +24,6 @@
 
 namespace wrd {
 
-using wr::kWorkDone;
-using wr::kWorkStride;
-using wr::kXcds;
-
 template <bool NEE>
 __global__ __launch_bounds__(256) void k_pt_mega(SceneDev S, CamDev cam, uint32_t max_depth, uint64_t seed,
                                                  uint32_t pass, FilmDev film, uint32_t npix) {
@@ -195,24 +191,17 @@ __device__ __forceinline__ void block_count_done(uint32_t* addr, bool want) {
 // k_closest_hit).  The fast-pass result goes to ht / hrec / hobj (first record
 // of the leaf) and the overflow flag; k_wf_finish completes it.
 constexpr uint32_t kOverflow = 4u;
-constexpr uint32_t kTraceRefillMin = 16;
-// Work ranges and batches: the live paths are cut into kXcds contiguous
-// ranges, range q handed out by its own counter to the workgroups of XCD q
-// (workgroups are dispatched to the XCDs round-robin), so neighbouring paths
-// share one XCD's L2 and each counter takes an eighth of the atomics; a wave
-// whose range is used up moves on round the others.  Paths a wave takes at a
-// time: guided self-scheduling (Polychronopoulos and Kuck, 1987), the paths
-// left in the range over sixteen times the XCD's waves, clamped to
-// [kTraceBatchMin, kTraceBatchMax] and rounded up to whole waves.  Large
-// batches early keep the waves off the counters while most paths remain;
-// small ones at the end keep the tail short.  A fixed 64 left a single
-// counter contended on large iterations, a fixed 256 stretched the tail of
-// small ones; with a counter per XCD a share of 16 beat 8, 4 and 2 (on the
-// 512-object field's iterations of about 8M paths it takes 64-128 paths).
-constexpr uint32_t kTraceBatchMin = 64;
-constexpr uint32_t kTraceBatchMax = 1024;
-constexpr uint32_t kTraceBatchShare = 16;
-constexpr uint32_t kTraceNodePhaseMin = 32;
+constexpr uint32_t kTraceRefillMin = 16;     // idle lanes before a full wave takes new paths
+constexpr uint32_t kTraceNodePhaseMin = 32;  // lanes of a full wave at wide nodes for a node-only step
+// Units of a UnitQueue, their size by the live paths.  An iteration with few
+// paths is bound by the latency of its longest traversal, and lanes that share
+// a wave lengthen it, so its paths are spread over kTraceSpread waves, a unit
+// of up to 64 paths for each and no more lanes of it at work than that (as in
+// k_closest_hit_small); with full units a workgroup comes back for one at a
+// time, or for two when it would come back for eight or more.  4,096 paths in the
+// Cornell box ran on 64 waves of 16 CUs, 92 us an iteration; now 43 us (with
+// 8,192 waves, more than fit, 1 to 6% slower; with 2,048 the same).
+constexpr uint32_t kTraceSpread = 4096;
 
 // D: traversal stack levels in LDS (4, 8 or 16; the wavefront autotuner's stack-depth knob).
 // COUNT: add the fast pass's node and triangle records fetched to the engine's
@@ -221,68 +210,62 @@ template <int D, bool COUNT = false>
 __global__ __launch_bounds__(256) void k_wf_trace(EngineDev E, uint32_t par) {
     const PathBuf& A = E.buf[par];
     const uint32_t n = E.cnt->n[par];
-    unsigned long long* work = E.cnt->trace_work;
-    // workgroups beyond what n paths need leave at once (and are not counted below)
-    const uint32_t used = (uint32_t)(((uint64_t)n + 255) / 256 < gridDim.x ? ((uint64_t)n + 255) / 256 : gridDim.x);
-    if (blockIdx.x >= used) return;
+    // paths of a unit: the power of two nearest to the paths per spread wave
+    uint32_t width = 1;
+    while (width < 64 && 2ull * n > 3ull * width * kTraceSpread) width *= 2;
+    const uint32_t units = (uint32_t)(((uint64_t)n + width - 1) / width);
+    // workgroups beyond what the units need (a unit per wave, every XCD alike) leave at once
+    const uint32_t used = min((units + 31) / 32 * 8, gridDim.x);
+    if (blockIdx.x >= used || n == 0) return;
     StackSpillT<D> spill;
     LaneStackT<D> st(&spill);
     Counters cnt{0, 0, 0};
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t bnext = 0, bend = 0;  // the wave's current batch of paths [bnext, bend)
-    uint32_t q = blockIdx.x % kXcds;  // the work range of this workgroup's XCD
-    uint32_t used_up = 0;             // ranges this wave has found used up (each once: they stay so)
-    const uint32_t xcd_waves = used * 4u / kXcds > 0u ? used * 4u / kXcds : 1u;
+    const uint64_t lanes = width < 64 ? (1ull << width) - 1ull : ~0ull;  // the lanes that take paths
+    const uint32_t refill_min = width < 64 ? 1u : kTraceRefillMin;
+    const uint32_t node_phase_min = (width * kTraceNodePhaseMin + 63) / 64;
+    __shared__ unsigned long long pool;
+    UnitQueue queue;
+    queue.init(&pool, E.cnt->trace_work, units, used, 4, units / used > 12 ? 2 : 1,
+               units > 4 * used ? min(max(units / (16 * wr::kXcds), 1u), 64u) : 1u);
+    uint32_t bnext = 0, bend = 0;  // the paths of the wave's current unit [bnext, bend)
     bool exhausted = false;
     bool active = false, overflow = false;
-    uint32_t pid = 0, ref = 0;
+    uint32_t pid = 0, ref = 0, job = WR_NONE;
     RayPre r{};
     HitState h{};
     Tree tr{};
     NoSelf ns{};
     for (;;) {
-        uint64_t idle = __ballot(!active);
-        if (!exhausted && (uint32_t)__popcll(idle) >= kTraceRefillMin) {
+        uint64_t idle = __ballot(!active) & lanes;
+        if (!exhausted && (uint32_t)__popcll(idle) >= refill_min) {
             while (idle != 0) {
                 if (bnext == bend) {
-                    // next batch: from range q, or the next range once q is used up
-                    bool got = false;
-                    while (used_up < kXcds) {
-                        const uint32_t lo = (uint32_t)((uint64_t)n * q / kXcds);
-                        const uint32_t hi = (uint32_t)((uint64_t)n * (q + 1) / kXcds);
-                        const uint32_t from = bend >= lo && bend < hi ? bend : lo;  // progress estimate
-                        uint32_t take = (hi - from) / (xcd_waves * kTraceBatchShare);
-                        take = take < kTraceBatchMin ? kTraceBatchMin : (take > kTraceBatchMax ? kTraceBatchMax : take);
-                        take = (take + 63u) & ~63u;
-                        unsigned long long base = 0;
-                        if (lane == 0) base = atomicAdd(work + kWorkStride * q, (unsigned long long)take);
-                        base = __shfl(base, 0);
-                        if (lo + base < hi) {
-                            bnext = lo + (uint32_t)base;
-                            bend = lo + base + take < hi ? lo + (uint32_t)base + take : hi;
-                            got = true;
-                            break;
-                        }
-                        q = q + 1 < kXcds ? q + 1 : 0;
-                        used_up++;
-                    }
-                    if (!got) {
+                    const uint32_t u = queue.next();
+                    if (u == WR_NONE) {
                         exhausted = true;
                         break;
                     }
+                    bnext = u * width;
+                    bend = n - bnext > width ? bnext + width : n;
                 }
                 const uint32_t avail = bend - bnext;
                 const uint32_t rank = (uint32_t)__popcll(idle & below);
-                if (!active && rank < avail) {
+                if (!active && lane < width && rank < avail) {
                     pid = bnext + rank;
-                    const SceneDev& S = E.scenes[E.jobs[A.job[pid]].scene];
-                    const wr_tree_hdr H = S.hdrs[0];
-                    tr = make_tree(H, S);
+                    if (A.job[pid] != job) {  // another job than the lane's last path: its scene
+                        job = A.job[pid];
+                        const SceneDev& S = E.scenes[E.jobs[job].scene];
+                        const wr_tree_hdr H = S.hdrs[0];
+                        tr = make_tree(H, S);
+                        ns.rec_nrm = S.rec_nrm + 9 * (size_t)H.rec_base;
+                        ns.obj_flags = S.obj_has_normals;
+                    }
                     r = make_ray(mk(A.ox[pid], A.oy[pid], A.oz[pid]), mk(A.dx[pid], A.dy[pid], A.dz[pid]), tr.scale);
                     const bool primary = A.flags[pid] & kPrimary;
-                    ns = NoSelf{primary ? WR_NONE : A.inside[pid], primary ? WR_NONE : A.contact[pid],
-                                S.rec_nrm + 9 * (size_t)H.rec_base, S.obj_has_normals};
+                    ns.inside = primary ? WR_NONE : A.inside[pid];
+                    ns.contact = primary ? WR_NONE : A.contact[pid];
                     overflow = false;
                     if (wide_begin(tr, r, st, h, ref)) {
                         active = true;
@@ -292,13 +275,13 @@ __global__ __launch_bounds__(256) void k_wf_trace(EngineDev E, uint32_t par) {
                 }
                 const uint32_t took = (uint32_t)__popcll(idle);
                 bnext += took < avail ? took : avail;
-                idle = __ballot(!active);
+                idle = __ballot(!active) & lanes;
             }
         }
-        if (__ballot(active) == 0) break;  // only once the counter is exhausted
+        if (__ballot(active) == 0) break;  // only once the queue is empty
         for (;;) {
             const bool at_node = active && !(ref & WR_LEAF_BIT);
-            if ((uint32_t)__popcll(__ballot(at_node)) < kTraceNodePhaseMin) break;
+            if ((uint32_t)__popcll(__ballot(at_node)) < node_phase_min) break;
             if (at_node && !wide_step<true, COUNT>(tr, r, ns, st, h, ref, overflow, cnt)) {
                 active = false;
                 A.ht[pid] = h.t;
@@ -327,13 +310,6 @@ __global__ __launch_bounds__(256) void k_wf_trace(EngineDev E, uint32_t par) {
             atomicAdd(&E.cnt->trace_tris, b);
         }
     }
-    if (lane == 0) {
-        const unsigned long long waves = (unsigned long long)used * (blockDim.x / 64);
-        if (atomicAdd(work + kWorkDone, 1ull) == waves - 1) {
-            for (uint32_t k = 0; k < kXcds; k++) atomicExch(work + kWorkStride * k, 0ull);
-            atomicExch(work + kWorkDone, 0ull);
-        }
-    }
 }
 
 // extend, part 2 (one lane per path): binary fast pass after an overflow,
@@ -346,6 +322,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const PathBuf& A = E.buf[par];
     const PathBuf& B = E.buf[par ^ 1];
     const uint32_t n = E.cnt->n[par];
+    if (blockIdx.x == 0) UnitQueue::clear(E.cnt->trace_work);  // for the next iteration's trace
     StackSpill spill;
     LaneStack st(&spill);
     // the workgroup steps through the slots together: the paths that end here

@@ -21,9 +21,6 @@
 
 namespace wrd {
 
-using wr::kWorkStride;
-using wr::kXcds;
-
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t G) {
     const uint32_t xcd = b & 7u, local = b >> 3;
     const uint32_t per = G >> 3, rem = G & 7u;
@@ -84,23 +81,15 @@ __device__ __forceinline__ NoSelf make_noself(const SceneDev& S, const wr_tree_h
 // ends, so a wave never waits for its slowest ray.  The result of the fast
 // pass (record, t, first record of the leaf, overflow flag) goes to hits[ray];
 // k_closest_hit_finish completes it.
-// Work distribution: every XCD has a range of the units (workgroups are
-// dispatched to the XCDs round-robin), made of stripes of `stripe` units that
-// the XCDs take in turn: neighbouring rays share one XCD's L2, and every range
-// sees the whole ray array, so the ranges end together and none needs another
-// XCD's help.  What bounds the distribution is the shared counters: an atomic
-// on one address takes about 65 ns here whatever the number of waves, and so
-// does a load that other XCDs' atomics keep out of L2.  So a workgroup's first
-// `first` units need no counter, later ones come `batch` at a time from the
-// range's counter into a pool in LDS that its four waves share, and a wave
-// that finds the range used up is done: no probing of other ranges, no count
-// of finished waves (k_closest_hit_finish zeroes the counters).  With one
-// counter atomic per wave and 256 rays, probing of the other seven ranges and
-// the count, 400,009 incoherent rays on the 512-object field took 242 us and
-// 8M camera rays 0.93 ms; now 142 us and 0.80 ms (with the finishing kernel; 16.8M rays on the 2.1M-triangle heightfield, where
-// the traversal itself is all, stay at 2.6 ms coherent, 3.2 ms incoherent).  Compiled for 8 waves per SIMD (64
-// VGPRs): more waves in flight hide more of the node-fetch latency; with the
-// NoSelf test for the 5 that its registers allow.
+// The units come from a UnitQueue.  With one counter atomic per wave and 256
+// rays, probing of the other seven ranges at the end and a count of finished
+// waves, 400,009 incoherent rays on the 512-object field took 242 us and 8M
+// camera rays 0.93 ms; now 142 us and 0.80 ms (with the finishing kernel;
+// 16.8M rays on the 2.1M-triangle heightfield, where the traversal itself is
+// all, stay at 2.6 ms coherent, 3.2 ms incoherent).
+// Compiled for 8 waves per SIMD (64 VGPRs): more waves in flight hide more of
+// the node-fetch latency; with the NoSelf test for the 5 that its registers
+// allow.
 // Scheduling knobs (ChTune, chosen by the autotuner): idle lanes are refilled
 // once at least refill_min are idle; a wave runs node-only steps while at
 // least node_phase_min lanes sit at wide nodes (a mixed step pays for both the
@@ -118,22 +107,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NOSELF ? 5 
     NoSelf ns{};
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = (1ull << lane) - 1ull;
-    // the workgroup's units of its range: next | end << 32
     __shared__ unsigned long long pool;
-    const uint32_t ranges = gridDim.x < kXcds ? gridDim.x : kXcds;
-    const uint32_t q = blockIdx.x % ranges;
-    const uint32_t units = (uint32_t)((n + 63) / 64), row = stripe * ranges;
-    // units of range q: whole rows of stripes, and its part of the last one
-    const uint32_t rest = units % row;
-    const uint32_t len = units / row * stripe + (rest > q * stripe ? min(rest - q * stripe, stripe) : 0u);
-    const uint32_t firsts = (gridDim.x - q + ranges - 1) / ranges * first;  // taken without the counter
-    if (threadIdx.x == 0) {
-        const uint32_t a = blockIdx.x / ranges * first;
-        pool = a < len ? (a | (unsigned long long)min(a + first, len) << 32) : 0ull;
-    }
-    __syncthreads();
-    uint32_t kept = 0, kept_end = 0;  // units of the range that this wave keeps to itself
-    uint64_t bnext = 0, bend = 0;     // the rays of its current unit [bnext, bend)
+    UnitQueue queue;
+    queue.init(&pool, work, (uint32_t)((n + 63) / 64), gridDim.x, first, batch, stripe);
+    uint64_t bnext = 0, bend = 0;  // the rays of the wave's current unit [bnext, bend)
     bool exhausted = false;
     bool active = false, overflow = false;
     uint64_t rid = 0;
@@ -145,41 +122,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NOSELF ? 5 
         if (!exhausted && (uint32_t)__popcll(idle) >= refill_min) {
             while (idle != 0) {
                 if (bnext == bend) {
-                    uint32_t a = kept < kept_end ? kept++ : len;
-                    if (a == len) {
-                        unsigned long long p = 0;
-                        if (lane == 0) p = atomicAdd(&pool, 1ull);
-                        p = __shfl(p, 0);
-                        if ((uint32_t)p < (uint32_t)(p >> 32)) a = (uint32_t)p;
-                    }
-                    if (a == len && firsts < len) {  // the pool is empty: the next units of the range
-                        unsigned long long c = 0, pub = 0;
-                        if (lane == 0) {
-                            c = firsts + atomicAdd(work + kWorkStride * q, (unsigned long long)batch);
-                            if (c + 1 < len) {  // all but the first go to the pool, if no other wave has filled it
-                                const unsigned long long next = (c + 1) | min(c + batch, (unsigned long long)len) << 32;
-                                unsigned long long cur = atomicAdd(&pool, 0ull);
-                                while (!pub && (uint32_t)cur >= (uint32_t)(cur >> 32)) {
-                                    const unsigned long long old = atomicCAS(&pool, cur, next);
-                                    pub = old == cur;
-                                    cur = old;
-                                }
-                            }
-                        }
-                        c = __shfl(c, 0);
-                        if (c < len) {
-                            a = (uint32_t)c;
-                            if (!__shfl(pub, 0)) {  // another wave filled it: this one keeps its units
-                                kept = a + 1;
-                                kept_end = (uint32_t)min(c + batch, (unsigned long long)len);
-                            }
-                        }
-                    }
-                    if (a == len) {
+                    const uint32_t u = queue.next();
+                    if (u == WR_NONE) {
                         exhausted = true;
                         break;
                     }
-                    const uint32_t u = a / stripe * row + q * stripe + a % stripe;
                     bnext = 64ull * u;
                     bend = bnext + 64 < n ? bnext + 64 : n;
                 }
@@ -249,7 +196,7 @@ __global__ __launch_bounds__(256) void k_closest_hit_finish(SceneDev S, wr_tree_
                                                             const uint32_t* __restrict__ rays, uint64_t n,
                                                             uint4* __restrict__ hits, unsigned long long* counters,
                                                             unsigned long long* work) {
-    if (blockIdx.x == 0 && threadIdx.x < kXcds) work[kWorkStride * threadIdx.x] = 0ull;  // for the next launch
+    if (blockIdx.x == 0) UnitQueue::clear(work);  // for the next launch
     const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
     const uint64_t i = (uint64_t)b * 256 + threadIdx.x;
     Counters cnt{0, 0, 0};

@@ -610,6 +610,95 @@ __device__ __forceinline__ void traverse_wide(const Tree& tr, const RayPre& r, c
     }
 }
 
+// Work distribution of a persistent traversal kernel of 256-lane workgroups:
+// units of consecutive rays, one at a time to a wave.  Every XCD has a range
+// of the units (workgroups are dispatched to the XCDs round-robin), made of
+// stripes of `stripe` units that the XCDs take in turn: neighbouring rays share
+// one XCD's L2, and every range sees the whole ray array, so the ranges end
+// together and none needs another XCD's help.  What bounds the distribution is
+// the shared counters: an atomic on one address takes about 65 ns here however
+// many waves there are, and so does a load of a line that other XCDs' atomics
+// keep changing.  So a workgroup's first `first` units need no counter, later
+// ones come `batch` at a time from the range's counter into a pool in LDS that
+// its four waves share, and a wave that finds the range used up is done: no
+// probing of other ranges (seven probes per wave cost up to 25%, one or two
+// gain nothing) and no count of finished waves: a later kernel of the same
+// stream clears the counters.
+struct UnitQueue {
+    unsigned long long* pool;     // LDS: the workgroup's units of its range, next | end << 32
+    unsigned long long* counter;  // the range's units handed out after the first ones
+    uint32_t q, stripe, row;
+    uint32_t len;                 // units of the range
+    uint32_t firsts;              // of those, the first ones of its workgroups
+    uint32_t batch;
+    uint32_t kept, kept_end;      // units that this wave keeps to itself
+
+    // work: one counter per XCD, zero at the start of the kernel.  blocks: the
+    // workgroups that take part, the first ones of the grid.  Every thread of
+    // a workgroup makes the call.
+    __device__ __forceinline__ void init(unsigned long long* lds_pool, unsigned long long* work, uint32_t units,
+                                         uint32_t blocks, uint32_t first, uint32_t take, uint32_t stripe_units) {
+        const uint32_t ranges = blocks < wr::kXcds ? blocks : wr::kXcds;
+        pool = lds_pool;
+        q = blockIdx.x % ranges;
+        counter = work + wr::kWorkStride * q;
+        stripe = stripe_units;
+        row = stripe * ranges;
+        // whole rows of stripes, and the range's part of the last one
+        const uint32_t rest = units % row;
+        len = units / row * stripe + (rest > q * stripe ? min(rest - q * stripe, stripe) : 0u);
+        firsts = (blocks - q + ranges - 1) / ranges * first;
+        batch = take;
+        kept = kept_end = 0;
+        if (threadIdx.x == 0) {
+            const uint32_t a = blockIdx.x / ranges * first;
+            *pool = a < len ? (a | (unsigned long long)min(a + first, len) << 32) : 0ull;
+        }
+        __syncthreads();
+    }
+
+    // The wave's next unit, WR_NONE when there is none; the whole wave makes the call.
+    __device__ __forceinline__ uint32_t next() {
+        const uint32_t lane = threadIdx.x & 63u;
+        uint32_t a = kept < kept_end ? kept++ : len;
+        if (a == len) {
+            unsigned long long p = 0;
+            if (lane == 0) p = atomicAdd(pool, 1ull);
+            p = __shfl(p, 0);
+            if ((uint32_t)p < (uint32_t)(p >> 32)) a = (uint32_t)p;
+        }
+        if (a == len && firsts < len) {  // the pool is empty: the next units of the range
+            unsigned long long c = 0, pub = 0;
+            if (lane == 0) {
+                c = firsts + atomicAdd(counter, (unsigned long long)batch);
+                if (c + 1 < len) {  // all but the first go to the pool, if no other wave has filled it
+                    const unsigned long long fill = (c + 1) | min(c + batch, (unsigned long long)len) << 32;
+                    unsigned long long cur = atomicAdd(pool, 0ull);
+                    while (!pub && (uint32_t)cur >= (uint32_t)(cur >> 32)) {
+                        const unsigned long long old = atomicCAS(pool, cur, fill);
+                        pub = old == cur;
+                        cur = old;
+                    }
+                }
+            }
+            c = __shfl(c, 0);
+            if (c < len) {
+                a = (uint32_t)c;
+                if (!__shfl(pub, 0)) {  // another wave filled it: this one keeps its units
+                    kept = a + 1;
+                    kept_end = (uint32_t)min(c + batch, (unsigned long long)len);
+                }
+            }
+        }
+        return a == len ? WR_NONE : a / stripe * row + q * stripe + a % stripe;
+    }
+
+    // Clears the counters for the next launch: by one workgroup of a later kernel.
+    static __device__ __forceinline__ void clear(unsigned long long* work) {
+        if (threadIdx.x < wr::kXcds) work[wr::kWorkStride * threadIdx.x] = 0ull;
+    }
+};
+
 // Re-check the winner's root-to-leaf chain with the reference box test.  The
 // ten levels nearest the leaf come from the leaf's chain record (two lines,
 // five levels each; the leaf key is its index, so its fetch does not wait for

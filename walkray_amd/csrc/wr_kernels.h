@@ -60,12 +60,11 @@ struct ChTune {
     uint32_t lds_levels = 8;       // traversal stack levels kept in LDS: 4, 8 or 16 (deeper ones spill)
     uint32_t batch = 128;          // most rays a workgroup takes from its XCD's work counter at a time (64..4096)
 };
-// The persistent closest-hit kernel's work counters: one per XCD, each on its
-// own 128 B line, and the count of finished waves after them.
+// The persistent traversal kernels' work counters: one per XCD, each on its
+// own 128 B line.
 constexpr uint32_t kXcds = 8;
-constexpr uint32_t kWorkStride = 16;                    // 64-bit words between counters
-constexpr uint32_t kWorkDone = kXcds * kWorkStride;     // the finished-wave count
-constexpr uint32_t kWorkWords = kWorkDone + kWorkStride;
+constexpr uint32_t kWorkStride = 16;  // 64-bit words between counters
+constexpr uint32_t kWorkWords = kXcds * kWorkStride;
 // work: kWorkWords zeroed 64-bit words owned by the caller's stream; the call
 // leaves them zeroed again when it ends.
 hipError_t launch_closest_hit(const SceneDev& S, const wr_tree_hdr& H, const float* rays, uint64_t n, void* hits,
