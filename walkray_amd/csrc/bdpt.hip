@@ -10,7 +10,8 @@
 //   3. every (light length, eye length) split of every joined length
 //      (bidirPathTracer.cpp:53-140): connectEdge (294-324), the visibility
 //      test (mcRenderer.cpp:59-65), connectingColorProb (266-291) and
-//      connectingMisWeight (142-221) with linkVertex (228-243), in one sweep;
+//      connectingMisWeight (142-221) with linkVertex (228-243), from the
+//      connection's two records and their sub-paths' prefixes (BPrefix);
 //   4. contributions with an eye side of two or more vertices go to the
 //      lane's pixel, light-tracing ones (the camera vertex alone on the eye
 //      side) are splatted to the pixel Camera::convToRaster names
@@ -44,7 +45,6 @@ namespace wrd {
 constexpr uint32_t kBdptLightVertex = 0x80000000u;  // as the light sub-paths of photon.hip
 constexpr uint32_t kCameraObj = 0xFFFFFFFEu;        // the camera as a NoSelf contact: not an object, not NULL
 constexpr uint32_t kVDelta = 1u, kVCamera = 2u;
-constexpr int kBdptMaxJoined = 2 * (wr::kBdptMaxDepth + 3);
 
 // One Ray of a Path as the estimator reads it (ray.h:8-37).
 struct BVert {
@@ -174,213 +174,183 @@ __device__ float eval_dir_prob(const SceneDev& S, const CamDev& cam, uint32_t pi
     return p * (float)(((double)ob.power + 1.0) * (double)powf(cos_theta, ob.power) * (kInvPi * 0.5));
 }
 
-// The joined path light[0..nl) + reversed eye[0..ne), with the two connection
-// records (indices cl, cl + 1) replaced by their edited copies once connected.
-struct Joined {
-    const BVert* L;
-    const BVert* E;
-    int nl, ne, n, cl;
-    bool edited;
-    BVert lc, ec;
-    __device__ __forceinline__ BVert at(int i) const {
-        if (edited && i == cl) return lc;
-        if (edited && i == cl + 1) return ec;
-        return i < nl ? L[i] : E[ne - 1 - (i - nl)];
-    }
-    __device__ __forceinline__ bool delta(int i) const { return (at(i).flags & kVDelta) != 0; }
+__device__ __forceinline__ bool is_delta(const BVert& v) { return (v.flags & kVDelta) != 0; }
+
+// max(|a - b|, EPSILON)
+__device__ __forceinline__ float vert_dist(const BVert& a, const BVert& b) {
+    const float l = len(sub(a.o, b.o));
+    return (double)l > kEps ? l : (float)kEps;
+}
+
+// PdfWtoA's factor cosine / distance^2.
+__device__ __forceinline__ double area_factor(float cosine, float dist) {
+    return (double)(1.0f * fabsf(cosine) / (dist * dist));
+}
+
+// linkVertex (bidirPathTracer.cpp:228-243): record v re-aimed at its neighbour.
+__device__ __forceinline__ BVert link_to(const BVert& v, const BVert& to) {
+    BVert l = v;
+    l.d = normalize(sub(to.o, v.o));
+    l.inside = to.inside;
+    return l;
+}
+
+// What a connection or merge needs of all the records before one of its two
+// records, i.e. the part of connectingColorProb (bidirPathTracer.cpp:266-291)
+// and of the weight (142-221; vcmTracer.cpp:221-320) that does not depend on
+// the other sub-path.
+//
+// Write the joined path light[0..c], eye[e..0]; direct[i] and reverse[i] are
+// the weight's two recurrences, and the weight's sum is
+//   sum over i of direct[i] * reverse[i + 1] * (vc_i + K * vm_i),
+// vc_i = 1 for two non-delta neighbours, vm_i the merging strategy's factor at
+// vertex i + 1 and K = pi r^2 * merging light paths.  On the light side,
+// direct[i] does not depend on the connection up to i = c, and reverse[i] =
+// reverse[c] * (factors f[i] .. f[c - 1] of single edges); on the eye side the
+// same holds with the roles exchanged.  So
+//   sum over i < c = reverse[c] * sum(direct[i] * (..) * f[i + 1] .. f[c - 1]),
+// whose second factor obeys S[c + 1] = f[c] * S[c] + direct[c] * (..): one
+// multiply-add per record.  The same holds for the products of the colour and
+// of the probability.  These prefixes, kept per record by k_bdpt_prefix, leave
+// each connection and each merge the two records and the edge between them,
+// instead of a sweep over the joined path with its dozen arrays in scratch
+// (3.5 KB a lane): Cornell 256^2 x 8 passes, maxPathLen 8, 14.7 ms in k_bdpt
+// before, 7.5 and 0.36 in k_bdpt_prefix now; the merges of a 201 x 151 VCM
+// render 0.83 and 0.29 ms.
+struct BPrefix {
+    double run;     // direct[i] of a light record, reverse of an eye record
+    double vc, vm;  // S of the connections and of the merging factors (without K)
+    double all;     // product of the edge factors: reverse[0] = reverse[c] * all
+    f3 color;       // product over the records before this one (radiance * cosine)
+    float prob;     // product of their probabilities
+    uint32_t flags; // kPAny, kPEmissive
+    uint32_t pad;
 };
+constexpr uint32_t kPAny = 1u;       // some neighbours among the records up to this one are both non-delta
+constexpr uint32_t kPEmissive = 2u;  // the record's contact is an emitter
 
-// pathCanNotConnect (bidirPathTracer.cpp:251-257)
-__device__ __forceinline__ bool cannot_connect(const Joined& P) {
-    for (int i = 0; i + 1 < P.n; i++)
-        if (!P.delta(i) && !P.delta(i + 1)) return false;
-    return true;
-}
-
-// connectEdge (bidirPathTracer.cpp:294-324): edits the copies lc / ec; the
-// previous records are read after the edits (for cl = 0, and for an eye side
-// of one record, the previous record is the connection record itself).
-__device__ bool connect_edge(const SceneDev& S, Joined& P) {
-    P.lc = P.at(P.cl);
-    P.ec = P.at(P.cl + 1);
-    if ((P.lc.flags & kVDelta) || (P.ec.flags & kVDelta)) return false;
-    P.edited = true;
-    const int last = P.n - 1;
-    const int il = P.cl - 1 > 0 ? P.cl - 1 : 0;
-    const int ie = P.cl + 2 < last ? P.cl + 2 : last;
-    P.lc.d = normalize(sub(P.ec.o, P.lc.o));
-    P.ec.d = mk(-P.lc.d.x, -P.lc.d.y, -P.lc.d.z);
-    P.lc.dp = 1.f;
-    P.lc.flags &= ~kVDelta;
-    {
-        const BVert pre = P.at(il);  // lc itself when il == cl
-        P.lc.rad = eval_bsdf(S, pre, P.lc);
-        if (P.lc.contact != WR_NONE && P.cl > 0)
-            P.lc.inside = dot(P.lc.n, P.lc.d) > 0.f ? pre.inside : P.lc.contact;
-    }
-    P.ec.dp = 1.f;
-    P.ec.flags &= ~kVDelta;
-    {
-        const BVert pre = P.at(ie);  // ec itself when ie == cl + 1
-        P.ec.rad = eval_bsdf(S, pre, P.ec);
-        if (P.ec.contact != WR_NONE && P.cl < last - 1)
-            P.ec.inside = dot(P.ec.n, P.ec.d) > 0.f ? pre.inside : P.ec.contact;
-    }
-    return true;
-}
-
-// connectingColorProb (bidirPathTracer.cpp:266-291; no participating media)
-// and connectingMisWeight (142-221, expTerm 1; every evalOriginProbability
-// there compares two temporaries, so it is 1) in one sweep over the joined
-// path, each record read once.  linkVertex(j, reverse = false) is record j
-// re-aimed at j + 1 when j > cl, linkVertex(j, true) record j re-aimed at
-// j - 1 when j <= cl; the weight reads only the cosine term and the
-// direction probability of those links (evalDirectionProbability ignores its
-// incoming ray), so the sweep keeps those per record and the two recurrences
-// run over them afterwards, in the reference's order.
-// With vt (VCMTracer) the colour and probability are connectingColorProb of
-// vcmTracer.cpp:329-362 (a merge also takes the merging disc, the area
-// density of the merged vertex and, inside a medium, the sphere's extra length)
-// and the weight is vcmMisWeight (vcmTracer.cpp:221-320, expTerm 1, nVC = 1):
-// the same two recurrences, with every merging strategy beside every
-// connection in the sum.
 struct VcmTerms {
     float r;     // the pass's merging radius
     double nvm;  // light sub-paths of the pass (one per pixel)
     bool vm;     // a merge (VM), else a connection (VC)
 };
 
-// insideObj && !contactObj: a point inside a medium (the camera is a contact)
-__device__ __forceinline__ bool in_volume(const BVert& v) {
-    return v.inside != WR_NONE && v.contact == WR_NONE && !(v.flags & kVCamera);
-}
-
-__device__ float color_prob_weight(const SceneDev& S, const CamDev& cam, uint32_t pixel, const Joined& P, f3& color,
-                                   float& prob, const VcmTerms* vt = nullptr) {
-    float cos_f[kBdptMaxJoined], cos_b[kBdptMaxJoined], dp_f[kBdptMaxJoined], dp_b[kBdptMaxJoined];
-    float dist[kBdptMaxJoined], op[kBdptMaxJoined];
-    uint8_t delta[kBdptMaxJoined], vol[kBdptMaxJoined];
-    const int n = P.n, cl = P.cl;
-    color = mk(1.f, 1.f, 1.f);
-    prob = 1.f;
-    BVert prev = P.at(0), cur = prev, next = prev;
-    for (int j = 0; j < n; j++) {
-        if (j + 1 < n) next = P.at(j + 1);
-        BVert f = cur, b = cur;
-        if (j > cl) {  // linkVertex(j, false)
-            const BVert& e = j + 1 < n ? next : cur;
-            f.d = normalize(sub(e.o, cur.o));
-            f.inside = e.inside;
-        }
-        if (j <= cl) {  // linkVertex(j, true)
-            const BVert& e = j > 0 ? prev : cur;
-            b.d = normalize(sub(e.o, cur.o));
-            b.inside = e.inside;
-        }
-        cos_f[j] = cos_term_v(f);
-        cos_b[j] = cos_term_v(b);
-        dp_f[j] = eval_dir_prob(S, cam, pixel, f, f, j == 0);
-        dp_b[j] = eval_dir_prob(S, cam, pixel, b, b, j == n - 1);
-        delta[j] = (cur.flags & kVDelta) ? 1 : 0;
-        vol[j] = in_volume(cur) ? 1 : 0;
-        op[j] = cur.op;
-        if (j > 0) {
-            const float l = len(sub(cur.o, prev.o));
-            dist[j] = (double)l > kEps ? l : (float)kEps;
-        }
-        // connectingColorProb
-        color = mulv(color, cur.rad);
-        if (j == cl && j < n - 1) {
-            const float l = len(sub(cur.o, next.o));
-            const float d = (double)l > kEps ? l : (float)kEps;
-            color = muls(color, cos_term_v(cur) * cos_term_v(next) / (d * d));
-        }
-        if (j != cl && j != cl + 1) color = muls(color, cos_term_v(cur));
-        prob *= cur.dp * cur.op;
-        if (vt && vt->vm && j == cl) {  // a merge: cl + 1 (the eye-side vertex) always exists
-            const float l = len(sub(cur.o, next.o));
-            const float d = (double)l > kEps ? l : (float)kEps;
-            prob = (float)((double)prob * (kPi * (double)vt->r * (double)vt->r));
-            prob *= 1.0f * fabsf(cos_term_v(next)) / (d * d);  // PdfWtoA at the eye-side vertex
-            if (in_volume(next)) prob = (float)((double)prob * (4.0 / 3 * (double)vt->r));
-        }
-        prev = cur;
-        cur = next;
+// The weight, colour and probability of the path light[0..c], eye[e..0] joined
+// by its two records as connectEdge left them (evalOriginProbability compares
+// two temporaries there, so it is 1; no participating media, so expTerm is 1
+// and no record lies inside a medium).  The doubles are the reference's.
+__device__ __forceinline__ float color_prob_weight(const SceneDev& S, const CamDev& cam, uint32_t pixel,
+                                                   const BVert& lc, const BPrefix& pl, int c, const BVert& ec,
+                                                   const BPrefix& pe, int e, f3& color, float& prob,
+                                                   const VcmTerms* vt = nullptr) {
+    const float d = vert_dist(ec, lc);
+    const float cos_l = cos_term_v(lc), cos_e = cos_term_v(ec);
+    color = mulv(pl.color, lc.rad);
+    color = muls(color, cos_l * cos_e / (d * d));
+    color = mulv(color, ec.rad);
+    color = mulv(color, pe.color);
+    prob = pl.prob * (lc.dp * lc.op);
+    if (vt && vt->vm) {  // a merge: the merging disc and the area density at the eye-side vertex
+        prob = (float)((double)prob * (kPi * (double)vt->r * (double)vt->r));
+        prob *= 1.0f * fabsf(cos_e) / (d * d);
     }
+    prob *= ec.dp * ec.op;
+    prob *= pe.prob;
     if (prob == 0.f || len(color) == 0.f) return 0.f;  // the caller skips these
-    double direct[kBdptMaxJoined], reverse[kBdptMaxJoined];
-    direct[0] = op[0];
-    for (int i = 1; i < n; i++) {
-        const float d = dist[i];
-        direct[i] = direct[i - 1] * (double)(1.0f * fabsf(cos_b[i]) / (d * d));  // PdfWtoA
-        if (delta[i - 1]) continue;
-        direct[i] *= dp_f[i - 1] * 1.f;
-    }
-    reverse[n - 1] = op[n - 1];
-    for (int i = n - 2; i >= 0; i--) {
-        const float d = dist[i + 1];
-        reverse[i] = reverse[i + 1] * (double)(1.0f * fabsf(cos_f[i]) / (d * d));
-        if (delta[i + 1]) continue;
-        reverse[i] *= dp_b[i + 1] * 1.f;
-    }
-    double all = 0.0;
-    bool cannot = true;  // pathCanNotConnect (bidirPathTracer.cpp:251-257)
+    const bool dl = is_delta(lc), de = is_delta(ec);
+    const double pf = dl ? 1.0 : (double)eval_dir_prob(S, cam, pixel, lc, lc, c == 0);
+    const double pb = de ? 1.0 : (double)eval_dir_prob(S, cam, pixel, ec, ec, e == 0);
+    const double next = pl.run * area_factor(cos_e, d) * pf;  // direct[c + 1]
+    const double back = pe.run * area_factor(cos_l, d) * pb;  // reverse[c]
+    const double join = pl.run * pe.run;
+    double all = back * pl.vc + next * pe.vc;
+    const bool connects = !dl && !de;
+    if (connects) all += join;
     if (!vt) {
-        for (int i = 0; i < n - 1; i++) {
-            if (!delta[i] && !delta[i + 1]) {
-                all += direct[i] * reverse[i + 1];
-                cannot = false;
-            }
-        }
-        if (cannot) all += reverse[0];
-        const double self = cl == -1 ? reverse[0] : direct[cl] * reverse[cl + 1];
-        const double w = self / all;
+        const double w = join / all;
         return (float)(w > 0.0 ? w : 0.0);
     }
-    double self = cl == -1 ? reverse[0] : direct[cl] * reverse[cl + 1];
-    for (int i = 0; i < n - 1; i++) {
-        if (!delta[i] && !delta[i + 1]) {  // VC
-            all += direct[i] * reverse[i + 1] * 1.0;
-            cannot = false;
-        }
-        if (i < n - 2 && !delta[i + 1]) {  // VM at vertex i + 1
-            double p = direct[i] * reverse[i + 1];
-            if (!delta[i]) p *= dp_f[i];
-            p *= 1.f;  // evalOriginProbability of two temporaries
-            p *= (double)(1.0f * fabsf(cos_b[i + 1]) / (dist[i + 1] * dist[i + 1]));
-            p *= kPi * (double)vt->r * (double)vt->r;
-            if (vol[i + 1]) p *= 4.0 / 3 * (double)vt->r;
-            if (vt->vm && i == cl) self = p;
-            all += p * vt->nvm;
-        }
-    }
-    if (cannot) all += reverse[0];
-    self *= vt->vm ? vt->nvm : 1.0;
-    const double w = self / all;
+    const double disc = kPi * (double)vt->r * (double)vt->r;
+    // merging at the eye-side vertex, unless it is the camera
+    const double merge = e > 0 && !de ? pe.run * next * disc : 0.0;
+    all += (back * pl.vm + next * pe.vm) * disc * vt->nvm + merge * vt->nvm;
+    if (!connects && !((pl.flags | pe.flags) & kPAny)) all += back * pl.all;  // pathCanNotConnect
+    const double w = (vt->vm ? merge * vt->nvm : join) / all;
     if (!(w >= 0.0)) return 0.f;
     return (float)w;
+}
+
+// connectEdge (bidirPathTracer.cpp:294-324) on copies lc / ec of light[c] and
+// eye[e]; the previous records are read after the edits (for c = 0, and for an
+// eye side of one record, the previous record is the connection record itself).
+__device__ __forceinline__ bool connect_edge(const SceneDev& S, const BVert* L, int c, const BVert* E, int e, BVert& lc,
+                                             BVert& ec) {
+    if (is_delta(lc) || is_delta(ec)) return false;
+    lc.d = normalize(sub(ec.o, lc.o));
+    ec.d = mk(-lc.d.x, -lc.d.y, -lc.d.z);
+    lc.dp = 1.f;
+    {
+        BVert pre = lc;
+        if (c > 0) {
+            pre.d = L[c - 1].d;
+            pre.inside = L[c - 1].inside;
+        }
+        lc.rad = eval_bsdf(S, pre, lc);
+        if (lc.contact != WR_NONE && c > 0) lc.inside = dot(lc.n, lc.d) > 0.f ? pre.inside : lc.contact;
+    }
+    ec.dp = 1.f;
+    {
+        BVert pre = ec;
+        if (e > 0) {
+            pre.d = E[e - 1].d;
+            pre.inside = E[e - 1].inside;
+        }
+        ec.rad = eval_bsdf(S, pre, ec);
+        if (ec.contact != WR_NONE && e > 0) ec.inside = dot(ec.n, ec.d) > 0.f ? pre.inside : ec.contact;
+    }
+    return true;
 }
 
 // connectEdge for a merge (vcmTracer.cpp:366-398 with VM): both directions are
 // re-aimed, only the eye-side record is edited (radiance, probability, delta,
 // inside); its previous record is an eye record (the merged eye vertex is at
 // least the second of its path).
-__device__ bool connect_edge_vm(const SceneDev& S, Joined& P) {
-    P.lc = P.at(P.cl);
-    P.ec = P.at(P.cl + 1);
-    if (P.ec.flags & kVDelta) return false;
-    P.edited = true;
-    const int last = P.n - 1;
-    const int ie = P.cl + 2 < last ? P.cl + 2 : last;
-    P.lc.d = normalize(sub(P.ec.o, P.lc.o));
-    P.ec.d = mk(-P.lc.d.x, -P.lc.d.y, -P.lc.d.z);
-    P.ec.dp = 1.f;
-    P.ec.flags &= ~kVDelta;
-    const BVert pre = P.at(ie);
-    P.ec.rad = eval_bsdf(S, pre, P.ec);
-    if (P.ec.contact != WR_NONE && P.cl < last - 1)
-        P.ec.inside = dot(P.ec.n, P.ec.d) > 0.f ? pre.inside : P.ec.contact;
+__device__ __forceinline__ bool connect_edge_vm(const SceneDev& S, const BVert* E, int e, BVert& lc, BVert& ec) {
+    if (is_delta(ec)) return false;
+    lc.d = normalize(sub(ec.o, lc.o));
+    ec.d = mk(-lc.d.x, -lc.d.y, -lc.d.z);
+    ec.dp = 1.f;
+    BVert pre = ec;
+    pre.d = E[e - 1].d;
+    pre.inside = E[e - 1].inside;
+    ec.rad = eval_bsdf(S, pre, ec);
+    if (ec.contact != WR_NONE) ec.inside = dot(ec.n, ec.d) > 0.f ? pre.inside : ec.contact;
     return true;
+}
+
+// A path that the eye side found alone: eye[e..0], eye[e] on an emitter (e >= 1).
+// Only paths that pathCanNotConnect rejects for every connection are taken.
+// Its sum has no connection terms; with vt, the merging ones.
+__device__ __forceinline__ float eye_path_weight(const BVert* E, const BPrefix* PE, int e, const BVert& last, f3& color,
+                                                 float& prob, const VcmTerms* vt = nullptr) {
+    const BPrefix pe = PE[e];
+    color = mulv(last.rad, pe.color);
+    prob = last.dp * last.op * pe.prob;
+    if (prob == 0.f || len(color) == 0.f) return 0.f;
+    double all = 0.0;
+    if (vt) {
+        // the emitter's record starts the path: its direction probability is that of an emission
+        const double pf = is_delta(last) ? 1.0 : (double)((float)(kInvPi * 0.25f) * 2.f);
+        const BVert prev = E[e - 1];
+        const BPrefix pp = PE[e - 1];
+        const double next = last.op * area_factor(cos_term_v(prev), vert_dist(last, prev)) * pf;
+        const double disc = kPi * (double)vt->r * (double)vt->r * vt->nvm;
+        if (e > 1 && !is_delta(prev)) all += pp.run * next * disc;
+        all += next * pp.vm * disc;
+    }
+    all += pe.run;
+    const double w = pe.run / all;
+    return (float)(w > 0.0 ? w : 0.0);
 }
 
 __device__ __forceinline__ bool emissive(const SceneDev& S, uint32_t obj) {
@@ -495,53 +465,95 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     counts[2 * lane + 1] = nl;
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt(SceneDev S, CamDev cam, uint32_t max_depth, uint64_t seed,
-                                              uint32_t pass0, uint32_t npass, uint32_t npix, uint32_t maxv,
-                                              BVert* verts, const uint32_t* counts, float* pix_all, VisQueue Q) {
-    (void)max_depth;
-    (void)seed;
-    (void)pass0;
-    const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (lane >= (uint64_t)npass * npix) return;
-    const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
-    float* pix = pix_all + 3 * (size_t)k * npix;
-    StackSpill spill;
-    LaneStack st(&spill);
-    const SceneCtx sc = make_scene_ctx(S);
-    BVert* E = verts + lane * 2 * maxv;
-    BVert* L = E + maxv;
-    const uint32_t ne = counts[2 * lane], nl = counts[2 * lane + 1];
-    const int max_eye = (int)(ne < maxv ? ne : maxv), max_light = (int)(nl < maxv ? nl : maxv);
+// The prefixes of every sub-path (BPrefix), one lane per sub-path: side 0 the
+// light sub-path, side 1 the eye sub-path of each lane of k_bdpt_subpaths.
+__global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uint32_t npix, uint32_t lanes,
+                                                     uint32_t maxv, const BVert* verts, const uint32_t* counts,
+                                                     BPrefix* prefix) {
+    const uint32_t id = blockIdx.x * 256 + threadIdx.x;
+    if (id >= 2 * lanes) return;
+    const bool eye = id >= lanes;
+    const uint32_t lane = eye ? id - lanes : id;
+    const size_t first = (size_t)lane * 2 * maxv + (eye ? 0 : maxv);
+    const BVert* V = verts + first;
+    BPrefix* P = prefix + first;
+    const uint32_t n = min(counts[2 * lane + (eye ? 0 : 1)], maxv), pixel = lane % npix;
+    if (n == 0) return;
+    BVert prev = V[0];
+    BPrefix p;
+    p.run = prev.op;
+    p.vc = p.vm = 0.0;
+    p.all = 1.0;
+    p.color = mk(1.f, 1.f, 1.f);
+    p.prob = 1.f;
+    p.flags = emissive(S, prev.contact) ? kPEmissive : 0u;
+    p.pad = 0;
+    P[0] = p;
+    for (uint32_t i = 1; i < n; i++) {
+        const BVert cur = V[i];
+        const BVert link = link_to(cur, prev);
+        const float d = vert_dist(cur, prev);
+        const bool dp = is_delta(prev), dc = is_delta(cur);
+        const float cos_prev = cos_term_v(prev);
+        const double own = area_factor(cos_prev, d);             // of the edge, at prev
+        const double at = area_factor(cos_term_v(link), d);      // of the edge, at cur
+        const double own_p = dp ? 1.0 : (double)eval_dir_prob(S, cam, pixel, prev, prev, !eye && i == 1);
+        const double link_p = dc ? 1.0 : (double)eval_dir_prob(S, cam, pixel, link, link, false);
+        const double edge = own * link_p;  // the other recurrence's factor from cur to prev
+        // merging at the far vertex of the pair: at cur on the light side, at prev on the eye side
+        // (the camera merges with nothing)
+        double merge = 0.0;
+        if (!eye && !dc) merge = own_p * at;
+        if (eye && i > 1 && !dp) merge = edge;
+        const bool connects = !dp && !dc;
+        p.vc = edge * p.vc + (connects ? p.run : 0.0);
+        p.vm = edge * p.vm + merge * p.run;
+        p.all *= edge;
+        p.run = p.run * at * own_p;
+        p.color = muls(mulv(p.color, prev.rad), cos_prev);
+        p.prob *= prev.dp * prev.op;
+        p.flags = (p.flags & kPAny) | (connects ? kPAny : 0u) | (emissive(S, cur.contact) ? kPEmissive : 0u);
+        P[i] = p;
+        prev = cur;
+    }
+}
+
+// The connections of one lane (throughput of bidirPathTracer.cpp:53-140, and of
+// vcmTracer.cpp:88-173 with vt): every eye record with no light record, and with
+// every light record.  Returns what goes to the lane's own pixel at once.
+__device__ __forceinline__ f3 connect_all(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
+                                          uint32_t k, uint32_t p, const BVert* E, const BPrefix* PE, int max_eye,
+                                          const BVert* L, const BPrefix* PL, int max_light, float* pix,
+                                          const VisQueue& Q, LaneStack& st, const VcmTerms* vt) {
     f3 own = mk(0.f, 0.f, 0.f);
-    for (int whole = 2; whole <= max_eye + max_light; whole++) {
-        const int min_l = whole - max_eye > 0 ? whole - max_eye : 0;
-        const int max_l = whole - 1 >= max_light ? max_light : whole - 1;
-        for (int light_len = min_l; light_len <= max_l; light_len++) {
-            Joined P;
-            P.L = L;
-            P.E = E;
-            P.nl = light_len;
-            P.ne = whole - light_len;
-            P.n = whole;
-            P.cl = light_len - 1;
-            P.edited = false;
-            if (!emissive(S, P.at(0).contact)) continue;
-            if (light_len == 0 && !cannot_connect(P)) continue;
-            const bool connected = P.ne > 0 && light_len > 0;
-            if (connected) {
-                if (light_len > 1 && emissive(S, P.at(P.cl).contact)) continue;
-                if (emissive(S, P.at(P.cl + 1).contact)) continue;
-                if (!connect_edge(S, P)) continue;
+    // light paths that start on no emitter (an empty light sample) connect to nothing
+    if (max_light > 0 && !(PL[0].flags & kPEmissive)) max_light = 0;
+    for (int e = 0; e < max_eye; e++) {
+        const BPrefix pe = PE[e];
+        const BVert ev = E[e];
+        f3 color;
+        float prob;
+        if (pe.flags & kPEmissive) {
+            // an emitter: the eye path alone, if no connection could have made it; no connections
+            if (e > 0 && !(pe.flags & kPAny)) {
+                const float w = eye_path_weight(E, PE, e, ev, color, prob, vt);
+                if (prob != 0.f && len(color) != 0.f) own = add(own, muls(divs(color, prob), w));
             }
-            f3 color;
-            float prob;
-            const float w = color_prob_weight(S, cam, p, P, color, prob);
+            continue;
+        }
+        if (is_delta(ev)) continue;
+        for (int c = 0; c < max_light; c++) {
+            const BPrefix pl = PL[c];
+            if (c > 0 && (pl.flags & kPEmissive)) continue;
+            BVert lc = L[c], ec = ev;
+            if (!connect_edge(S, L, c, E, e, lc, ec)) continue;
+            const float w = color_prob_weight(S, cam, p, lc, pl, c, ec, pe, e, color, prob, vt);
             if (prob == 0.f) continue;
             if (len(color) == 0.f) continue;
             f3 contrib = muls(divs(color, prob), w);
             uint32_t target = p;
-            if (P.ne <= 1) {  // light tracing: splat to the pixel the camera sees the point in
-                const f3 v = sub(P.at(whole - 2).o, cam.pos);
+            if (e == 0) {  // light tracing: splat to the pixel the camera sees the point in
+                const f3 v = sub(lc.o, cam.pos);
                 const float vfd = dot(v, cam.front);
                 const float scale = cam.dist / vfd;
                 const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
@@ -552,33 +564,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
                 contrib = muls(contrib, factor / (float)npix);
             }
-            if (!connected) {  // no visibility test (a path found by the eye side alone)
-                if (target == p) own = add(own, contrib);
-                else atomic_add3(pix, target, contrib);
-                continue;
-            }
             // MCRenderer::visibilityTest from the eye-side connection record
-            const uint32_t contact = (P.ec.flags & kVCamera) ? kCameraObj : P.ec.contact;
-            const float dist = len(sub(P.ec.o, P.lc.o));
+            const uint32_t contact = (ec.flags & kVCamera) ? kCameraObj : ec.contact;
+            const float dist = len(sub(ec.o, lc.o));
             const uint32_t slot = wave_slot(Q.count);
             if (slot < Q.cap) {
                 uint32_t* r = Q.rays + 8 * (size_t)slot;
-                r[0] = __float_as_uint(P.ec.o.x); r[1] = __float_as_uint(P.ec.o.y); r[2] = __float_as_uint(P.ec.o.z);
-                r[3] = __float_as_uint(P.ec.d.x); r[4] = __float_as_uint(P.ec.d.y); r[5] = __float_as_uint(P.ec.d.z);
-                r[6] = P.ec.inside;
+                r[0] = __float_as_uint(ec.o.x); r[1] = __float_as_uint(ec.o.y); r[2] = __float_as_uint(ec.o.z);
+                r[3] = __float_as_uint(ec.d.x); r[4] = __float_as_uint(ec.d.y); r[5] = __float_as_uint(ec.d.z);
+                r[6] = ec.inside;
                 r[7] = contact;
                 float* y = Q.pay + 4 * (size_t)slot;
                 y[0] = contrib.x; y[1] = contrib.y; y[2] = contrib.z; y[3] = dist;
                 Q.dst[slot] = k * npix + target;
             } else {  // queue full: trace here
-                const PHit h = trace_scene<true>(sc, P.ec.o, P.ec.d, P.ec.inside, contact, st);
+                const PHit h = trace_scene<true>(sc, ec.o, ec.d, ec.inside, contact, st);
                 if (!nee_visible(h.rec, h.t, dist)) continue;
                 if (target == p) own = add(own, contrib);
                 else atomic_add3(pix, target, contrib);
             }
         }
     }
-    atomic_add3(pix, p, own);
+    return own;
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt(
+    SceneDev S, CamDev cam, uint32_t npass, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* prefix,
+    const uint32_t* counts, float* pix_all, VisQueue Q) {
+    const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (lane >= (uint64_t)npass * npix) return;
+    const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
+    float* pix = pix_all + 3 * (size_t)k * npix;
+    StackSpill spill;
+    LaneStack st(&spill);
+    const SceneCtx sc = make_scene_ctx(S);
+    const size_t ei = lane * 2 * maxv, li = ei + maxv;
+    const uint32_t ne = counts[2 * lane], nl = counts[2 * lane + 1];
+    atomic_add3(pix, p, connect_all(S, sc, cam, npix, k, p, verts + ei, prefix + ei, (int)min(ne, maxv), verts + li,
+                                    prefix + li, (int)min(nl, maxv), pix, Q, st, nullptr));
 }
 
 // The queued visibility tests, answered by the batch NoSelf query (hits:
@@ -699,29 +722,24 @@ struct MergeQueue {
 // lane `lane` with light point pi of the lane's pass.  Returns the contribution
 // (before the division by the pixel count); zero when the merge gives nothing.
 __device__ __forceinline__ f3 vcm_merge(const SceneDev& S, const CamDev& cam, uint32_t npix, uint32_t maxv,
-                                        const BVert* verts, const VcmGrid& G, uint64_t lane, int i, uint32_t pi) {
+                                        const BVert* verts, const BPrefix* prefix, const VcmGrid& G, uint64_t lane,
+                                        int i, uint32_t pi) {
     const uint32_t p = (uint32_t)(lane % npix);
     const uint32_t k = G.src[2 * (size_t)pi], j = G.src[2 * (size_t)pi + 1];
-    Joined P;
-    P.L = verts + (size_t)k * 2 * maxv + maxv;
-    P.E = verts + lane * 2 * maxv;
-    P.nl = (int)j;
-    P.ne = i + 1;
-    P.n = (int)j + i + 1;
-    P.cl = (int)j - 1;
-    P.edited = false;
-    if (!connect_edge_vm(S, P)) return mk(0.f, 0.f, 0.f);
+    const size_t li = (size_t)k * 2 * maxv + maxv + (j - 1), ei = lane * 2 * maxv;
+    BVert lc = verts[li], ec = verts[ei + i];
+    if (!connect_edge_vm(S, verts + ei, i, lc, ec)) return mk(0.f, 0.f, 0.f);
     const VcmTerms vm{G.r, (double)npix, true};
     f3 color;
     float prob;
-    const float w = color_prob_weight(S, cam, p, P, color, prob, &vm);
+    const float w = color_prob_weight(S, cam, p, lc, prefix[li], (int)j - 1, ec, prefix[ei + i], i, color, prob, &vm);
     if (len(color) == 0.f || prob == 0.f) return mk(0.f, 0.f, 0.f);
     return divs(muls(color, w), prob);
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm(SceneDev S, CamDev cam, uint32_t npix, uint32_t npass, uint32_t maxv,
-                                             const BVert* verts, const uint32_t* counts, float* pix_all, VisQueue Q,
-                                             const VcmGrid* grids, MergeQueue M) {
+                                             const BVert* verts, const BPrefix* prefix, const uint32_t* counts,
+                                             float* pix_all, VisQueue Q, const VcmGrid* grids, MergeQueue M) {
     // every lane of a wave stays to the end (the merge reservations below are
     // wave-wide scans); a lane past the last one stands in for lane 0 and does
     // nothing
@@ -734,77 +752,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
-    const BVert* E = verts + lane * 2 * maxv;
-    const BVert* L = E + maxv;
+    const size_t ei = lane * 2 * maxv, li = ei + maxv;
+    const BVert* E = verts + ei;
     const uint32_t ne = counts[2 * lane], nl = counts[2 * lane + 1];
     const int max_eye = (int)(ne < maxv ? ne : maxv), max_light = (int)(nl < maxv ? nl : maxv);
     const VcmTerms vc{G.r, (double)npix, false};
-    f3 own = mk(0.f, 0.f, 0.f);
-    // throughputByConnecting (vcmTracer.cpp:88-173): k_bdpt's loop with vcmMisWeight
-    for (int whole = 2; valid && whole <= max_eye + max_light; whole++) {
-        const int min_l = whole - max_eye > 0 ? whole - max_eye : 0;
-        const int max_l = whole - 1 >= max_light ? max_light : whole - 1;
-        for (int light_len = min_l; light_len <= max_l; light_len++) {
-            Joined P;
-            P.L = L;
-            P.E = E;
-            P.nl = light_len;
-            P.ne = whole - light_len;
-            P.n = whole;
-            P.cl = light_len - 1;
-            P.edited = false;
-            if (!emissive(S, P.at(0).contact)) continue;
-            if (light_len == 0 && !cannot_connect(P)) continue;
-            const bool connected = P.ne > 0 && light_len > 0;
-            if (connected) {
-                if (light_len > 1 && emissive(S, P.at(P.cl).contact)) continue;
-                if (emissive(S, P.at(P.cl + 1).contact)) continue;
-                if (!connect_edge(S, P)) continue;
-            }
-            f3 color;
-            float prob;
-            const float w = color_prob_weight(S, cam, p, P, color, prob, &vc);
-            if (prob == 0.f) continue;
-            if (len(color) == 0.f) continue;
-            f3 contrib = muls(divs(color, prob), w);
-            uint32_t target = p;
-            if (P.ne <= 1) {  // light tracing: splat to the pixel the camera sees the point in
-                const f3 v = sub(P.at(whole - 2).o, cam.pos);
-                const float vfd = dot(v, cam.front);
-                const float scale = cam.dist / vfd;
-                const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
-                const float ry = (float)(cam.H / 2.0 - (double)(dot(v, cam.top) * scale));
-                const int x = (int)rx, y = (int)ry;  // checkPixelBound truncates (camera.cpp:164-170)
-                if (!(x >= 0 && y >= 0 && x < (int)cam.W && y < (int)cam.H)) continue;
-                target = (uint32_t)(y * (int)cam.W + x);
-                const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
-                contrib = muls(contrib, factor / (float)npix);
-            }
-            if (!connected) {
-                if (target == p) own = add(own, contrib);
-                else atomic_add3(pix, target, contrib);
-                continue;
-            }
-            const uint32_t contact = (P.ec.flags & kVCamera) ? kCameraObj : P.ec.contact;
-            const float dist = len(sub(P.ec.o, P.lc.o));
-            const uint32_t slot = wave_slot(Q.count);
-            if (slot < Q.cap) {
-                uint32_t* r = Q.rays + 8 * (size_t)slot;
-                r[0] = __float_as_uint(P.ec.o.x); r[1] = __float_as_uint(P.ec.o.y); r[2] = __float_as_uint(P.ec.o.z);
-                r[3] = __float_as_uint(P.ec.d.x); r[4] = __float_as_uint(P.ec.d.y); r[5] = __float_as_uint(P.ec.d.z);
-                r[6] = P.ec.inside;
-                r[7] = contact;
-                float* y = Q.pay + 4 * (size_t)slot;
-                y[0] = contrib.x; y[1] = contrib.y; y[2] = contrib.z; y[3] = dist;
-                Q.dst[slot] = kb * npix + target;
-            } else {  // queue full: trace here
-                const PHit h = trace_scene<true>(sc, P.ec.o, P.ec.d, P.ec.inside, contact, st);
-                if (!nee_visible(h.rec, h.t, dist)) continue;
-                if (target == p) own = add(own, contrib);
-                else atomic_add3(pix, target, contrib);
-            }
-        }
-    }
+    // throughputByConnecting (vcmTracer.cpp:88-173): k_bdpt's connections with vcmMisWeight
+    f3 own = connect_all(S, sc, cam, npix, kb, p, E, prefix + ei, valid ? max_eye : 0, verts + li, prefix + li,
+                         max_light, pix, Q, st, &vc);
     // throughputByMerging (vcmTracer.cpp:175-217): the light points within the
     // radius of every non-delta eye vertex before an emitter, in the grid's
     // order (HashGrid::Process); the default points have no path and give
@@ -866,7 +821,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         M.ent[2 * (size_t)k + 1] = pi;
                         k++;
                     } else {  // queue full: merge here
-                        contrib = add(contrib, vcm_merge(S, cam, npix, maxv, verts, G, lane, i, pi));
+                        contrib = add(contrib, vcm_merge(S, cam, npix, maxv, verts, prefix, G, lane, i, pi));
                         k++;
                     }
                 }
@@ -880,7 +835,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
 // The queued merges of k_vcm, one per lane, each added to its pixel of its pass.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm_merge(SceneDev S, CamDev cam, uint32_t npix, uint32_t maxv,
-                                                   const BVert* verts, float* pix_all, MergeQueue M,
+                                                   const BVert* verts, const BPrefix* prefix, float* pix_all, MergeQueue M,
                                                    const VcmGrid* grids) {
     const uint32_t n = min(M.ent[2 * (size_t)M.cap], M.cap);
     for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
@@ -888,7 +843,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const uint32_t lane = w0 & 0xFFFFFFu;
         const int i = (int)(w0 >> 24);
         const uint32_t kb = lane / npix, p = lane % npix;
-        const f3 c = vcm_merge(S, cam, npix, maxv, verts, grids[kb], lane, i, pi);
+        const f3 c = vcm_merge(S, cam, npix, maxv, verts, prefix, grids[kb], lane, i, pi);
         if (c.x != 0.f || c.y != 0.f || c.z != 0.f) atomic_add3(pix_all + 3 * (size_t)kb * npix, p, divs(c, (float)npix));
     }
 }
@@ -903,6 +858,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // 670-674).  No object here is a volume or an anisotropic glossy object, so
 // every photon is a surface photon and every estimate the plain range query.
 constexpr uint32_t kMergeLen = 10;
+
+// The throughput of every light path before each of its records (radiance /
+// directionProb / originProb * cosine of the records before it), kept in the
+// radiance of the eye-side record of the same index, which PhotonMap has no
+// other use for: a photon in reach costs one record instead of its whole path
+// (k_ppm 2.99 -> 2.35 ms for Cornell 256^2 x 8 passes, and 0.11 here).
+__global__ __launch_bounds__(256) void k_ppm_throughput(uint32_t lanes, uint32_t maxv, BVert* verts,
+                                                        const uint32_t* counts) {
+    const uint32_t lane = blockIdx.x * 256 + threadIdx.x;
+    if (lane >= lanes) return;
+    BVert* out = verts + (size_t)lane * 2 * maxv;
+    const BVert* L = out + maxv;
+    const uint32_t n = min(counts[2 * lane + 1], maxv);
+    f3 thr = mk(1.f, 1.f, 1.f);
+    for (uint32_t m = 0; m < n; m++) {
+        out[m].rad = thr;
+        const BVert lm = L[m];
+        thr = mulv(thr, divs(divs(lm.rad, lm.dp), lm.op));
+        thr = muls(thr, cos_term_v(lm));
+    }
+}
 
 // Query::Process for the photons around outRay (the eye vertex, its direction
 // towards the previous eye vertex).
@@ -927,12 +903,7 @@ __device__ f3 ppm_density(const SceneDev& S, const VcmGrid& G, const BVert* vert
             if (!grid_near(G.g, G.pos, outRay.o, pi)) continue;
             const uint32_t k = G.src[2 * (size_t)pi], j = G.src[2 * (size_t)pi + 1];
             const BVert* L = verts + (size_t)k * 2 * maxv + maxv;
-            f3 thr = mk(1.f, 1.f, 1.f);
-            for (uint32_t m = 0; m < j; m++) {
-                const BVert lm = L[m];
-                thr = mulv(thr, divs(divs(lm.rad, lm.dp), lm.op));
-                thr = muls(thr, cos_term_v(lm));
-            }
+            f3 thr = (L - maxv)[j].rad;  // k_ppm_throughput
             BVert ph = L[j];
             thr = divs(thr, ph.op);
             ph.d = L[j - 1].d;
@@ -1024,6 +995,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 namespace wr {
 
 size_t bdpt_vertex_bytes() { return sizeof(wrd::BVert); }
+size_t bdpt_prefix_bytes() { return sizeof(wrd::BPrefix); }
 
 float vcm_radius(float base, uint32_t pass) {
     const float alpha = (float)(2.0 / 3);  // vcmTracer.h:39
@@ -1112,6 +1084,8 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
         destroy();
         return rc;
     }
+    wrd::BPrefix* prefix = (wrd::BPrefix*)q.prefix;
+    wrd::k_bdpt_prefix<<<(2 * lanes + 255) / 256, 256, 0, st>>>(S, cam, npix, lanes, maxv, V, q.counts, prefix);
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
     const wrd::MergeQueue M{vb.mq, vb.mq_cap};
     e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint32_t), st);
@@ -1119,12 +1093,11 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
         destroy();
         return hip_fail(ctx, e, "wr_render_vcm");
     }
-    wrd::k_vcm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, q.counts, pix, Q,
+    wrd::k_vcm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q,
                                                         (const wrd::VcmGrid*)vb.grids, M);
     e = hipGetLastError();
     if (e == hipSuccess) {
-        wrd::k_vcm_merge<<<4096, 256, 0, st>>>(S, cam, npix, maxv, V, pix, M,
-                                                                (const wrd::VcmGrid*)vb.grids);
+        wrd::k_vcm_merge<<<4096, 256, 0, st>>>(S, cam, npix, maxv, V, prefix, pix, M, (const wrd::VcmGrid*)vb.grids);
         e = hipGetLastError();
     }
     uint32_t nq = 0;
@@ -1163,6 +1136,7 @@ int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const CamHost& ch, uint32_
         destroy();
         return rc;
     }
+    wrd::k_ppm_throughput<<<blocks, 256, 0, st>>>(lanes, maxv, V, counts);
     wrd::k_ppm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, seed, pass0, pix,
                                                         (const wrd::VcmGrid*)vb.grids);
     wrd::k_bdpt_fold<<<(npix + 255) / 256, 256, 0, st>>>(cam, npass, npix, pix,
@@ -1195,8 +1169,10 @@ hipError_t launch_bdpt_passes(const SceneDev& S, const wr_tree_hdr& H, const Cam
     const uint32_t blocks = (uint32_t)((lanes + 255) / 256);
     wrd::k_bdpt_subpaths<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, max_depth, seed, pass0, npass, npix, maxv,
                                                                   (wrd::BVert*)verts, q.counts);
-    wrd::k_bdpt<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, max_depth, seed, pass0, npass, npix, maxv,
-                                                         (wrd::BVert*)verts, q.counts, pix, Q);
+    wrd::k_bdpt_prefix<<<(uint32_t)((2 * lanes + 255) / 256), 256, 0, st>>>(
+        S, cam, npix, (uint32_t)lanes, maxv, (const wrd::BVert*)verts, q.counts, (wrd::BPrefix*)q.prefix);
+    wrd::k_bdpt<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npass, npix, maxv, (const wrd::BVert*)verts,
+                                                         (const wrd::BPrefix*)q.prefix, q.counts, pix, Q);
     uint32_t nq = 0;
     e = hipMemcpyAsync(&nq, q.count, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -280,6 +280,7 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     hipError_t e = hipMalloc(&verts, per_pass * batch);
     if (e == hipSuccess) e = hipMalloc((void**)&pix, sizeof(float) * 3 * npix * batch);
     if (e == hipSuccess) e = hipMalloc(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
+    if (e == hipSuccess) e = hipMalloc(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * npix * batch);
     if (e == hipSuccess) e = hipMalloc((void**)&q.counts, sizeof(uint32_t) * 2 * npix * batch);
     if (e == hipSuccess) {
         char* b = (char*)qbuf;
@@ -304,6 +305,7 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     (void)hipFree(verts);
     (void)hipFree(pix);
     (void)hipFree(qbuf);
+    (void)hipFree(q.prefix);
     (void)hipFree(q.counts);
     if (e != hipSuccess) {
         film->broken = film->broken || launched;
@@ -360,6 +362,7 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = hipMalloc((void**)&pix, sizeof(float) * 3 * lanes);
     if (e == hipSuccess) e = hipMalloc((void**)&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 1));
     if (e == hipSuccess) e = hipMalloc(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
+    if (e == hipSuccess) e = hipMalloc(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * lanes);
     if (e == hipSuccess) e = hipMalloc((void**)&q.counts, sizeof(uint32_t) * 2 * lanes);
     if (e == hipSuccess) e = hipMalloc((void**)&vb.pc, sizeof(uint32_t) * (lanes + 1));
     if (e == hipSuccess) e = hipMalloc((void**)&vb.offs, sizeof(uint32_t) * (lanes + 1));
@@ -377,7 +380,7 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
         q.count = (uint32_t*)(b + 68 * (size_t)q.cap + 128);
     }
     auto release = [&]() {
-        for (void* ptr : {verts, (void*)pix, qbuf, (void*)q.counts, (void*)vb.pc, (void*)vb.offs, (void*)vb.starts,
+        for (void* ptr : {verts, (void*)pix, qbuf, q.prefix, (void*)q.counts, (void*)vb.pc, (void*)vb.offs, (void*)vb.starts,
                           vb.scan, (void*)vb.pos, (void*)vb.src, vb.grids, (void*)vb.mq})
             (void)hipFree(ptr);
     };
