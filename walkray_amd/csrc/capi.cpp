@@ -34,11 +34,88 @@ int hip_fail(wr_ctx* ctx, hipError_t e, const char* what) {
     return fail(ctx, WR_EHIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+hipError_t WorkPool::get(void** out, size_t bytes) {
+    *out = nullptr;
+    // whole MiB above one, so that calls of similar sizes share buffers
+    bytes = bytes > (1u << 20) ? (bytes + (1u << 20) - 1) >> 20 << 20 : std::max<size_t>((bytes + 255) / 256 * 256, 256);
+    std::lock_guard<std::mutex> lk(mu);
+    Buf* best = nullptr;
+    for (Buf& b : bufs)  // the smallest that fits, unless it is several times too large
+        if (!b.out && b.bytes >= bytes && b.bytes / 4 <= bytes && (!best || b.bytes < best->bytes)) best = &b;
+    if (best) {
+        best->out = true;
+        *out = best->p;
+        return hipSuccess;
+    }
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // must not surface at a later launch check
+        free_idle(0);
+        e = hipMalloc(&p, bytes);
+    }
+    if (e != hipSuccess) return e;
+    bufs.push_back(Buf{p, bytes, true});
+    *out = p;
+    return hipSuccess;
+}
+
+void WorkPool::put(void* p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t k = 0; k < bufs.size(); k++)
+        if (bufs[k].p == p) {
+            Buf b = bufs[k];
+            b.out = false;
+            bufs.erase(bufs.begin() + (long)k);
+            bufs.push_back(b);  // the newest of the unused ones
+            break;
+        }
+    free_idle(closed ? 0 : kIdleMax);
+}
+
+void WorkPool::free_idle(size_t keep) {
+    size_t idle = 0;
+    for (const Buf& b : bufs) idle += b.out ? 0 : b.bytes;
+    for (size_t k = 0; k < bufs.size() && idle > keep;) {
+        if (bufs[k].out) {
+            k++;
+            continue;
+        }
+        idle -= bufs[k].bytes;
+        (void)hipFree(bufs[k].p);
+        bufs.erase(bufs.begin() + (long)k);
+    }
+}
+
+void WorkPool::trim() {
+    std::lock_guard<std::mutex> lk(mu);
+    free_idle(0);
+}
+
+void WorkPool::close() {
+    std::lock_guard<std::mutex> lk(mu);
+    closed = true;
+    free_idle(0);
+}
+
+// hipMalloc; when the device is out of memory, once more without the
+// context's unused buffers.
+static hipError_t alloc_trimmed(wr_ctx* ctx, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        ctx->pool->trim();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 template <class T>
 static int upload(wr_ctx* ctx, const T* v, size_t n, T** d, uint64_t& bytes) {
     *d = nullptr;
     const size_t b = std::max<size_t>(n, 1) * sizeof(T);
-    hipError_t e = hipMalloc((void**)d, b);
+    hipError_t e = alloc_trimmed(ctx, (void**)d, b);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(scene)");
     bytes += b;
     if (n) {
@@ -108,6 +185,7 @@ int wr_ctx_create(int device, wr_ctx** out) {
     if (e != hipSuccess) return hip_fail(nullptr, e, "hipSetDevice");
     std::unique_ptr<wr_ctx> c(new wr_ctx);
     c->device = device;
+    c->pool = std::make_shared<wr::WorkPool>(device);
     if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess)
         return hip_fail(nullptr, e, "hipStreamCreate");
     if ((e = hipEventCreate(&c->ev0)) != hipSuccess) return hip_fail(nullptr, e, "hipEventCreate");
@@ -126,6 +204,8 @@ void wr_ctx_destroy(wr_ctx* ctx) {
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
     (void)hipFree(ctx->d_work);
+    ctx->pool->close();
+    if (ctx->film_back) (void)hipHostFree(ctx->film_back);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -140,7 +220,7 @@ int wr_synchronize(wr_ctx* ctx) {
 int wr_device_alloc(wr_ctx* ctx, size_t bytes, void** d_out) {
     if (!ctx || !d_out) return fail(ctx, WR_EINVAL, "wr_device_alloc: bad argument");
     (void)hipSetDevice(ctx->device);
-    hipError_t e = hipMalloc(d_out, std::max<size_t>(bytes, 1));
+    hipError_t e = alloc_trimmed(ctx, d_out, std::max<size_t>(bytes, 1));
     if (e != hipSuccess) return fail(ctx, WR_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return WR_OK;
 }

@@ -469,24 +469,6 @@ using wr::hip_fail;
         if (e_ != hipSuccess) return hip_fail(ctx, e_, what); \
     } while (0)
 
-namespace {
-// Device scratch owned by one call, freed on every exit.
-struct Scratch {
-    std::vector<void*> p;
-    ~Scratch() {
-        for (void* q : p) (void)hipFree(q);
-    }
-    template <class T>
-    hipError_t get(T** out, size_t bytes) {
-        void* q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(bytes, 4));
-        if (e == hipSuccess) p.push_back(q);
-        *out = (T*)q;
-        return e;
-    }
-};
-}  // namespace
-
 extern "C" {
 
 int wr_light_paths(wr_ctx* ctx, const wr_scene* s, uint32_t max_depth, uint64_t seed, uint32_t pass, uint32_t path0,
@@ -515,7 +497,7 @@ int wr_photons_collect(wr_ctx* ctx, const wr_scene* s, const wr_path_vertex* d_v
     if (n_paths >= (1u << 31)) return fail(ctx, WR_EINVAL, "wr_photons_collect: too many paths");
     (void)hipSetDevice(ctx->device);
     hipStream_t st = ctx->stream;
-    Scratch sc;
+    wr::Scratch sc(*ctx->pool);
     uint32_t* pc = nullptr;
     uint64_t* offs = nullptr;
     PH_CHECK(sc.get(&pc, sizeof(uint32_t) * (n_paths + 1)), "hipMalloc(photons)");
@@ -575,7 +557,7 @@ int wr_hashgrid_build(wr_ctx* ctx, const float* d_pos, uint64_t n, float radius,
     hipError_t e = hipMalloc((void**)&g->ends, sizeof(int) * n_cells);
     if (e == hipSuccess) e = hipMalloc((void**)&g->idx, sizeof(uint32_t) * std::max<uint64_t>(n, 1));
     if (e != hipSuccess) return bail(e, "hipMalloc(hashgrid)");
-    Scratch sc;
+    wr::Scratch sc(*ctx->pool);
     int* keys6 = nullptr;
     uint32_t *ckeys = nullptr, *ckeys2 = nullptr, *vals = nullptr, *cnt = nullptr;
     if ((e = sc.get(&keys6, 6 * sizeof(int))) != hipSuccess) return bail(e, "hipMalloc(hashgrid)");

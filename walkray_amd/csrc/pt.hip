@@ -688,22 +688,26 @@ __global__ __launch_bounds__(64) void k_wf_advance(EngineDev E, uint32_t par) {
     }
 }
 
-// run_wavefront's admission in one launch: scene slot 0, job slot 0 (running,
-// with the engine iteration it starts at) and the job's pass counters zeroed.
-// Nothing else runs on the engine meanwhile (the previous call ended with a
-// synchronisation).
+// A job's admission in one launch, without a copy or a synchronisation: its
+// record in its slot (running, with the engine iteration it starts at), its
+// pass counters zeroed and, for run_wavefront's one job, its scene in scene
+// slot 0.  Nothing else runs on the engine meanwhile.
 __global__ __launch_bounds__(256) void k_wf_admit(SceneDev* scenes, wr::JobDesc* jobs, wr::JobCtl* ctl,
-                                                  const wr::EngineCounters* cnt, SceneDev S, wr::JobDesc J) {
+                                                  const wr::EngineCounters* cnt, uint32_t slot, wr::JobDesc J,
+                                                  bool set_scene, SceneDev S) {
     for (uint32_t k = threadIdx.x; k < J.R; k += 256) J.pass_done[k] = 0;
     if (threadIdx.x == 0) {
-        scenes[0] = S;
-        jobs[0] = J;
+        if (set_scene) scenes[0] = S;
+        jobs[slot] = J;
         wr::JobCtl c{};
         c.state = wr::kJobRunning;
         c.start_iter = cnt->iteration;
-        ctl[0] = c;
+        ctl[slot] = c;
     }
 }
+
+// Frees a job slot.
+__global__ void k_wf_free_slot(wr::JobCtl* ctl, uint32_t slot) { ctl[slot] = wr::JobCtl{}; }
 
 }  // namespace wrd
 
@@ -907,12 +911,9 @@ hipError_t Engine::set_scene(uint32_t slot, const SceneDev& S, hipStream_t st) {
 }
 
 // Admits a job into a free slot (between replays, on the engine's stream).
-hipError_t Engine::admit(uint32_t slot, const JobDesc& J, hipStream_t st) {
-    WR_CHECK(hipMemcpyAsync(jobs + slot, &J, sizeof(JobDesc), hipMemcpyHostToDevice, st));
-    JobCtl c{};
-    c.state = kJobRunning;
-    WR_CHECK(hipMemcpyAsync(ctl + slot, &c, sizeof(JobCtl), hipMemcpyHostToDevice, st));
-    return hipStreamSynchronize(st);  // the sources are host stack copies
+hipError_t Engine::admit(uint32_t slot, const JobDesc& J, hipStream_t st, const SceneDev* scene) {
+    k_wf_admit<<<1, 256, 0, st>>>(scenes, jobs, ctl, cnt, slot, J, scene != nullptr, scene ? *scene : SceneDev{});
+    return hipGetLastError();
 }
 
 hipError_t Engine::cancel_slot(uint32_t slot, hipStream_t st) {
@@ -922,9 +923,8 @@ hipError_t Engine::cancel_slot(uint32_t slot, hipStream_t st) {
 }
 
 hipError_t Engine::release_slot(uint32_t slot, hipStream_t st) {
-    JobCtl c{};
-    WR_CHECK(hipMemcpyAsync(ctl + slot, &c, sizeof(JobCtl), hipMemcpyHostToDevice, st));
-    return hipStreamSynchronize(st);
+    k_wf_free_slot<<<1, 1, 0, st>>>(ctl, slot);
+    return hipGetLastError();
 }
 
 // One replay of the iteration graph, then a read-back of the job states.
@@ -1030,8 +1030,7 @@ static hipError_t run_wavefront_once(const SceneDev& S, const CamHost& cam, uint
     J.fsumsq = film.sumsq;
     EngineCounters c0{};
     if (ev) WR_CHECK(hipMemcpy(&c0, E.cnt, sizeof(EngineCounters), hipMemcpyDeviceToHost));
-    k_wf_admit<<<1, 256, 0, st>>>(E.scenes, E.jobs, E.ctl, E.cnt, S, J);
-    WR_CHECK(hipGetLastError());
+    WR_CHECK(E.admit(0, J, st, &S));
     // every pass is generated within npass window turns and drains in at most
     // max_depth + 2 iterations after its last path is issued
     const uint64_t it_bound = 4 * (uint64_t)(max_depth + 4) * (total / E.cap + npass + 2) + 64;

@@ -5,6 +5,8 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -14,8 +16,9 @@
 
 struct wr_film {
     wr_ctx* ctx = nullptr;
+    std::shared_ptr<wr::WorkPool> pool;
     uint32_t W = 0, H = 0;
-    float* sum = nullptr;
+    float* sum = nullptr;  // one allocation: the sums, then comp, then sumsq
     float* comp = nullptr;
     float* sumsq = nullptr;
     uint32_t passes = 0;
@@ -62,6 +65,56 @@ wr::CamHost make_cam(const wr_camera& c) {
 
 }  // namespace
 
+namespace wr {
+
+// The film of 3 n floats (sums, compensation, square sums) at `film` to host
+// arrays, each nullable, and the mean over `passes`.  A small film comes in one
+// copy through pinned memory of the context: three copies to pageable memory
+// take about 20 us each however small they are.
+hipError_t read_film(wr_ctx* ctx, const float* film, size_t n, uint32_t passes, float* mean, float* sum, float* comp,
+                     float* sumsq) {
+    constexpr size_t kPinnedMax = 1u << 20;
+    const size_t b = n * sizeof(float);
+    const float* host = nullptr;  // the film's three arrays in pinned memory
+    std::unique_lock<std::mutex> lk(ctx->film_mu, std::defer_lock);
+    if (3 * b <= kPinnedMax) {
+        lk.lock();
+        if (!ctx->film_back && hipHostMalloc((void**)&ctx->film_back, kPinnedMax, hipHostMallocDefault) != hipSuccess)
+            (void)hipGetLastError();  // must not surface at a later launch check
+        host = ctx->film_back;
+    }
+    hipError_t e = hipSuccess;
+    std::vector<float> tmp;
+    const float* s = host;
+    if (host) {
+        e = hipMemcpyAsync((void*)host, film, 3 * b, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return e;
+        if (sum) std::memcpy(sum, host, b);
+        if (comp) std::memcpy(comp, host + n, b);
+        if (sumsq) std::memcpy(sumsq, host + 2 * n, b);
+    } else {
+        float* to = sum;
+        if (!to && mean) {
+            tmp.resize(n);
+            to = tmp.data();
+        }
+        if (to) e = hipMemcpyAsync(to, film, b, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess && comp) e = hipMemcpyAsync(comp, film + n, b, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess && sumsq) e = hipMemcpyAsync(sumsq, film + 2 * n, b, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return e;
+        s = to;
+    }
+    if (mean) {
+        const float inv = passes ? 1.f / (float)passes : 0.f;
+        for (size_t i = 0; i < n; i++) mean[i] = passes ? s[i] * inv : 0.f;
+    }
+    return hipSuccess;
+}
+
+}  // namespace wr
+
 using namespace wr;
 
 extern "C" {
@@ -74,12 +127,14 @@ int wr_film_create(wr_ctx* ctx, uint32_t width, uint32_t height, wr_film** out) 
     f->ctx = ctx;
     f->W = width;
     f->H = height;
-    const size_t b = sizeof(float) * 3 * (size_t)width * height;
-    if (hipMalloc((void**)&f->sum, b) != hipSuccess || hipMalloc((void**)&f->comp, b) != hipSuccess ||
-        hipMalloc((void**)&f->sumsq, b) != hipSuccess) {
-        wr_film_destroy(f);
+    const size_t n = 3 * (size_t)width * height;
+    if (ctx->pool->get(&f->sum, sizeof(float) * 3 * n) != hipSuccess) {
+        delete f;
         return fail(ctx, WR_ENOMEM, "wr_film_create: out of device memory");
     }
+    f->pool = ctx->pool;
+    f->comp = f->sum + n;
+    f->sumsq = f->comp + n;
     int rc = wr_film_clear(f);
     if (rc) {
         wr_film_destroy(f);
@@ -91,19 +146,14 @@ int wr_film_create(wr_ctx* ctx, uint32_t width, uint32_t height, wr_film** out) 
 
 void wr_film_destroy(wr_film* f) {
     if (!f) return;
-    (void)hipStreamSynchronize(f->ctx->stream);
-    if (f->sum) (void)hipFree(f->sum);
-    if (f->comp) (void)hipFree(f->comp);
-    if (f->sumsq) (void)hipFree(f->sumsq);
+    f->pool->put(f->sum);
     delete f;
 }
 
 int wr_film_clear(wr_film* f) {
     if (!f) return fail(nullptr, WR_EINVAL, "wr_film_clear: film is NULL");
     const size_t b = sizeof(float) * 3 * (size_t)f->W * f->H;
-    hipError_t e = hipMemsetAsync(f->sum, 0, b, f->ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(f->comp, 0, b, f->ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(f->sumsq, 0, b, f->ctx->stream);
+    hipError_t e = hipMemsetAsync(f->sum, 0, 3 * b, f->ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(f->ctx->stream);
     if (e != hipSuccess) return hip_fail(f->ctx, e, "wr_film_clear");
     f->passes = 0;
@@ -119,23 +169,8 @@ static int film_broken(wr_film* f, const char* who) {
 int wr_film_read(wr_film* f, float* mean_rgb, float* sum, float* comp, float* sumsq, uint32_t* passes) {
     if (!f) return fail(nullptr, WR_EINVAL, "wr_film_read: film is NULL");
     if (f->broken) return film_broken(f, "wr_film_read");
-    const size_t n = 3 * (size_t)f->W * f->H;
-    std::vector<float> tmp;
-    float* s = sum;
-    if (!s && mean_rgb) {
-        tmp.resize(n);
-        s = tmp.data();
-    }
-    hipError_t e = hipSuccess;
-    if (s) e = hipMemcpyAsync(s, f->sum, n * sizeof(float), hipMemcpyDeviceToHost, f->ctx->stream);
-    if (e == hipSuccess && comp) e = hipMemcpyAsync(comp, f->comp, n * sizeof(float), hipMemcpyDeviceToHost, f->ctx->stream);
-    if (e == hipSuccess && sumsq) e = hipMemcpyAsync(sumsq, f->sumsq, n * sizeof(float), hipMemcpyDeviceToHost, f->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(f->ctx->stream);
+    const hipError_t e = read_film(f->ctx, f->sum, 3 * (size_t)f->W * f->H, f->passes, mean_rgb, sum, comp, sumsq);
     if (e != hipSuccess) return hip_fail(f->ctx, e, "wr_film_read");
-    if (mean_rgb) {
-        const float inv = f->passes ? 1.f / (float)f->passes : 0.f;
-        for (size_t i = 0; i < n; i++) mean_rgb[i] = f->passes ? s[i] * inv : 0.f;
-    }
     if (passes) *passes = f->passes;
     return WR_OK;
 }
@@ -277,11 +312,12 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     q.work = ctx->d_work;
     q.cap = prm->wave_slots ? prm->wave_slots : (uint32_t)std::min<uint64_t>(32ull * npix * batch, 24ull << 20);
     void* qbuf = nullptr;
-    hipError_t e = hipMalloc(&verts, per_pass * batch);
-    if (e == hipSuccess) e = hipMalloc((void**)&pix, sizeof(float) * 3 * npix * batch);
-    if (e == hipSuccess) e = hipMalloc(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
-    if (e == hipSuccess) e = hipMalloc(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * npix * batch);
-    if (e == hipSuccess) e = hipMalloc((void**)&q.counts, sizeof(uint32_t) * 2 * npix * batch);
+    Scratch mem(*ctx->pool);
+    hipError_t e = mem.get(&verts, per_pass * batch);
+    if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * npix * batch);
+    if (e == hipSuccess) e = mem.get(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
+    if (e == hipSuccess) e = mem.get(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * npix * batch);
+    if (e == hipSuccess) e = mem.get(&q.counts, sizeof(uint32_t) * 2 * npix * batch);
     if (e == hipSuccess) {
         char* b = (char*)qbuf;
         q.rays = (uint32_t*)b;
@@ -302,11 +338,7 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     if (e == hipSuccess) e = hipEventSynchronize(ctx->ev1);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
-    (void)hipFree(verts);
-    (void)hipFree(pix);
-    (void)hipFree(qbuf);
-    (void)hipFree(q.prefix);
-    (void)hipFree(q.counts);
+    if (e != hipSuccess) (void)hipStreamSynchronize(ctx->stream);  // before the buffers go back
     if (e != hipSuccess) {
         film->broken = film->broken || launched;
         return hip_fail(ctx, e, "wr_render_bdpt");
@@ -358,19 +390,20 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     vb.mq_cap = (uint32_t)std::min<uint64_t>(64ull * lanes, 48ull << 20);  // beyond it a lane merges in place
     void *verts = nullptr, *qbuf = nullptr;
     float* pix = nullptr;
-    hipError_t e = hipMalloc(&verts, per_pass * batch);
-    if (e == hipSuccess) e = hipMalloc((void**)&pix, sizeof(float) * 3 * lanes);
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 1));
-    if (e == hipSuccess) e = hipMalloc(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
-    if (e == hipSuccess) e = hipMalloc(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * lanes);
-    if (e == hipSuccess) e = hipMalloc((void**)&q.counts, sizeof(uint32_t) * 2 * lanes);
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.pc, sizeof(uint32_t) * (lanes + 1));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.offs, sizeof(uint32_t) * (lanes + 1));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.starts, sizeof(uint32_t) * (batch + 1));
-    if (e == hipSuccess) e = hipMalloc(&vb.scan, std::max<size_t>(vb.scan_bytes, 4));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.pos, sizeof(float) * 3 * vb.cap);
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.src, sizeof(uint32_t) * 2 * vb.cap);
-    if (e == hipSuccess) e = hipMalloc(&vb.grids, vcm_grid_bytes() * batch);
+    Scratch mem(*ctx->pool);
+    hipError_t e = mem.get(&verts, per_pass * batch);
+    if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * lanes);
+    if (e == hipSuccess) e = mem.get(&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 1));
+    if (e == hipSuccess) e = mem.get(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
+    if (e == hipSuccess) e = mem.get(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * lanes);
+    if (e == hipSuccess) e = mem.get(&q.counts, sizeof(uint32_t) * 2 * lanes);
+    if (e == hipSuccess) e = mem.get(&vb.pc, sizeof(uint32_t) * (lanes + 1));
+    if (e == hipSuccess) e = mem.get(&vb.offs, sizeof(uint32_t) * (lanes + 1));
+    if (e == hipSuccess) e = mem.get(&vb.starts, sizeof(uint32_t) * (batch + 1));
+    if (e == hipSuccess) e = mem.get(&vb.scan, std::max<size_t>(vb.scan_bytes, 4));
+    if (e == hipSuccess) e = mem.get(&vb.pos, sizeof(float) * 3 * vb.cap);
+    if (e == hipSuccess) e = mem.get(&vb.src, sizeof(uint32_t) * 2 * vb.cap);
+    if (e == hipSuccess) e = mem.get(&vb.grids, vcm_grid_bytes() * batch);
     if (e == hipSuccess) {
         char* b = (char*)qbuf;
         q.rays = (uint32_t*)b;
@@ -379,16 +412,8 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
         q.dst = (uint32_t*)(b + 64 * (size_t)q.cap);
         q.count = (uint32_t*)(b + 68 * (size_t)q.cap + 128);
     }
-    auto release = [&]() {
-        for (void* ptr : {verts, (void*)pix, qbuf, q.prefix, (void*)q.counts, (void*)vb.pc, (void*)vb.offs, (void*)vb.starts,
-                          vb.scan, (void*)vb.pos, (void*)vb.src, vb.grids, (void*)vb.mq})
-            (void)hipFree(ptr);
-    };
     if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
-    if (e != hipSuccess) {
-        release();
-        return hip_fail(ctx, e, "wr_render_vcm");
-    }
+    if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     const FilmBufs fb{film->sum, film->comp, film->sumsq};
     for (uint32_t k = 0; k < prm->spp; k += (uint32_t)batch) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, prm->spp - k);
@@ -396,7 +421,6 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
                                          base_radius, maxv, verts, pix, q, vb, fb);
         if (rc != WR_OK) {  // the film may hold part of this call's passes
             (void)hipStreamSynchronize(ctx->stream);
-            release();
             film->broken = true;
             return rc;
         }
@@ -405,8 +429,8 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = hipEventSynchronize(ctx->ev1);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
-    release();
     if (e != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);  // before the buffers go back
         film->broken = film->broken || prm->spp > 0;
         return hip_fail(ctx, e, "wr_render_vcm");
     }
@@ -450,26 +474,19 @@ extern "C" int wr_render_ppm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     void* verts = nullptr;
     float* pix = nullptr;
     uint32_t* counts = nullptr;
-    hipError_t e = hipMalloc(&verts, per_pass * batch);
-    if (e == hipSuccess) e = hipMalloc((void**)&pix, sizeof(float) * 3 * lanes);
-    if (e == hipSuccess) e = hipMalloc((void**)&counts, sizeof(uint32_t) * 2 * lanes);
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.pc, sizeof(uint32_t) * (lanes + 1));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.offs, sizeof(uint32_t) * (lanes + 1));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.starts, sizeof(uint32_t) * (batch + 1));
-    if (e == hipSuccess) e = hipMalloc(&vb.scan, std::max<size_t>(vb.scan_bytes, 4));
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.pos, sizeof(float) * 3 * vb.cap);
-    if (e == hipSuccess) e = hipMalloc((void**)&vb.src, sizeof(uint32_t) * 2 * vb.cap);
-    if (e == hipSuccess) e = hipMalloc(&vb.grids, vcm_grid_bytes() * batch);
-    auto release = [&]() {
-        for (void* ptr : {verts, (void*)pix, (void*)counts, (void*)vb.pc, (void*)vb.offs, (void*)vb.starts, vb.scan,
-                          (void*)vb.pos, (void*)vb.src, vb.grids})
-            (void)hipFree(ptr);
-    };
+    Scratch mem(*ctx->pool);
+    hipError_t e = mem.get(&verts, per_pass * batch);
+    if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * lanes);
+    if (e == hipSuccess) e = mem.get(&counts, sizeof(uint32_t) * 2 * lanes);
+    if (e == hipSuccess) e = mem.get(&vb.pc, sizeof(uint32_t) * (lanes + 1));
+    if (e == hipSuccess) e = mem.get(&vb.offs, sizeof(uint32_t) * (lanes + 1));
+    if (e == hipSuccess) e = mem.get(&vb.starts, sizeof(uint32_t) * (batch + 1));
+    if (e == hipSuccess) e = mem.get(&vb.scan, std::max<size_t>(vb.scan_bytes, 4));
+    if (e == hipSuccess) e = mem.get(&vb.pos, sizeof(float) * 3 * vb.cap);
+    if (e == hipSuccess) e = mem.get(&vb.src, sizeof(uint32_t) * 2 * vb.cap);
+    if (e == hipSuccess) e = mem.get(&vb.grids, vcm_grid_bytes() * batch);
     if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
-    if (e != hipSuccess) {
-        release();
-        return hip_fail(ctx, e, "wr_render_ppm");
-    }
+    if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_ppm");
     const FilmBufs fb{film->sum, film->comp, film->sumsq};
     for (uint32_t k = 0; k < prm->spp; k += (uint32_t)batch) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, prm->spp - k);
@@ -477,7 +494,6 @@ extern "C" int wr_render_ppm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
                                          maxv, verts, counts, pix, vb, fb);
         if (rc != WR_OK) {  // the film may hold part of this call's passes
             (void)hipStreamSynchronize(ctx->stream);
-            release();
             film->broken = true;
             return rc;
         }
@@ -486,8 +502,8 @@ extern "C" int wr_render_ppm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = hipEventSynchronize(ctx->ev1);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
-    release();
     if (e != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);  // before the buffers go back
         film->broken = film->broken || prm->spp > 0;
         return hip_fail(ctx, e, "wr_render_ppm");
     }

@@ -39,8 +39,8 @@ struct Job {
     wr_job_status st{};
     int slot = -1;
     uint32_t R = 0;
-    float *sum = nullptr, *comp = nullptr, *sumsq = nullptr, *contrib = nullptr;
-    uint32_t* pass_done = nullptr;
+    float* film = nullptr;    // the sums, then comp, then sumsq
+    float* contrib = nullptr; // the sample window, then its pass counters
     uint64_t film_bytes = 0, window_bytes = 0;
     uint64_t total = 0;  // camera paths of the job (spp x pixels)
 };
@@ -70,18 +70,14 @@ using namespace wr;
 // reused once the next replay has dropped the job's paths from the pool.
 static constexpr int64_t kDraining = -2;
 
-static void free_job_window(Job& j) {
-    if (j.contrib) (void)hipFree(j.contrib);
-    if (j.pass_done) (void)hipFree(j.pass_done);
+static void free_job_window(wr_server* s, Job& j) {
+    s->ctx->pool->put(j.contrib);
     j.contrib = nullptr;
-    j.pass_done = nullptr;
 }
 
-static void free_job_film(Job& j) {
-    if (j.sum) (void)hipFree(j.sum);
-    if (j.comp) (void)hipFree(j.comp);
-    if (j.sumsq) (void)hipFree(j.sumsq);
-    j.sum = j.comp = j.sumsq = nullptr;
+static void free_job_film(wr_server* s, Job& j) {
+    s->ctx->pool->put(j.film);
+    j.film = nullptr;
 }
 
 extern "C" {
@@ -111,8 +107,8 @@ void wr_server_destroy(wr_server* s) {
     if (!s) return;
     (void)hipStreamSynchronize(s->ctx->stream);
     for (auto& kv : s->jobs) {
-        free_job_window(kv.second);
-        free_job_film(kv.second);
+        free_job_window(s, kv.second);
+        free_job_film(s, kv.second);
     }
     delete s;
 }
@@ -172,18 +168,13 @@ static hipError_t admit_one(wr_server* s, Job& j, int slot) {
         s->inject_admit_failures--;
         return hipErrorOutOfMemory;
     }
-    hipError_t e = hipMalloc((void**)&j.sum, fb);
-    if (e == hipSuccess) e = hipMalloc((void**)&j.comp, fb);
-    if (e == hipSuccess) e = hipMalloc((void**)&j.sumsq, fb);
-    if (e == hipSuccess) e = hipMalloc((void**)&j.contrib, sizeof(float) * 3 * (size_t)j.R * npix);
-    if (e == hipSuccess) e = hipMalloc((void**)&j.pass_done, sizeof(uint32_t) * j.R);
-    if (e == hipSuccess) e = hipMemsetAsync(j.sum, 0, fb, st);
-    if (e == hipSuccess) e = hipMemsetAsync(j.comp, 0, fb, st);
-    if (e == hipSuccess) e = hipMemsetAsync(j.sumsq, 0, fb, st);
-    if (e == hipSuccess) e = hipMemsetAsync(j.pass_done, 0, sizeof(uint32_t) * j.R, st);
+    const size_t window = 3 * (size_t)j.R * npix;
+    hipError_t e = s->ctx->pool->get(&j.film, 3 * fb);
+    if (e == hipSuccess) e = s->ctx->pool->get(&j.contrib, sizeof(float) * window + sizeof(uint32_t) * j.R);
+    if (e == hipSuccess) e = hipMemsetAsync(j.film, 0, 3 * fb, st);
     if (e != hipSuccess) {
-        free_job_window(j);
-        free_job_film(j);
+        free_job_window(s, j);
+        free_job_film(s, j);
         return e;
     }
     wr_camera c = j.desc.cam;
@@ -211,15 +202,15 @@ static hipError_t admit_one(wr_server* s, Job& j, int slot) {
     j.total = (uint64_t)j.desc.spp * npix;
     J.R = j.R;
     J.contrib = j.contrib;
-    J.pass_done = j.pass_done;
-    J.fsum = j.sum;
-    J.fcomp = j.comp;
-    J.fsumsq = j.sumsq;
+    J.pass_done = (uint32_t*)(j.contrib + window);
+    J.fsum = j.film;
+    J.fcomp = j.film + 3 * (size_t)npix;
+    J.fsumsq = j.film + 6 * (size_t)npix;
     e = s->engine.admit((uint32_t)slot, J, st);
     if (e != hipSuccess) {
         (void)hipStreamSynchronize(st);
-        free_job_window(j);
-        free_job_film(j);
+        free_job_window(s, j);
+        free_job_film(s, j);
         return e;
     }
     j.slot = slot;
@@ -286,7 +277,7 @@ int wr_server_step(wr_server* s, uint32_t* n_active) {
             Job& j = s->jobs[(uint64_t)s->slot_job[k]];
             j.st.state = WR_JOB_DONE;
             j.st.done_s = t;
-            free_job_window(j);
+            free_job_window(s, j);
             s->used -= j.window_bytes;
             e = s->engine.release_slot(k, st);
             if (e != hipSuccess) return hip_fail(s->ctx, e, "wr_server_step: release");
@@ -317,8 +308,8 @@ int wr_job_cancel(wr_server* s, uint64_t id) {
         // the slot waits for the next replay
         hipError_t e = s->engine.cancel_slot((uint32_t)j.slot, s->ctx->stream);
         if (e != hipSuccess) return hip_fail(s->ctx, e, "wr_job_cancel");
-        free_job_window(j);
-        free_job_film(j);
+        free_job_window(s, j);
+        free_job_film(s, j);
         s->used -= j.film_bytes + j.window_bytes;
         s->slot_job[j.slot] = kDraining;
         j.slot = -1;
@@ -347,25 +338,10 @@ int wr_job_read(wr_server* s, uint64_t id, float* mean_rgb, float* sum, float* c
     auto it = s->jobs.find(id);
     if (it == s->jobs.end()) return fail(s->ctx, WR_EINVAL, "wr_job_read: unknown job");
     Job& j = it->second;
-    if (j.st.state != WR_JOB_DONE || !j.sum) return fail(s->ctx, WR_ESTATE, "wr_job_read: job not finished");
+    if (j.st.state != WR_JOB_DONE || !j.film) return fail(s->ctx, WR_ESTATE, "wr_job_read: job not finished");
     const size_t n = 3 * (size_t)j.desc.cam.width * j.desc.cam.height;
-    hipStream_t st = s->ctx->stream;
-    std::vector<float> tmp;
-    float* sp = sum;
-    if (!sp && mean_rgb) {
-        tmp.resize(n);
-        sp = tmp.data();
-    }
-    hipError_t e = hipSuccess;
-    if (sp) e = hipMemcpyAsync(sp, j.sum, n * sizeof(float), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && comp) e = hipMemcpyAsync(comp, j.comp, n * sizeof(float), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && sumsq) e = hipMemcpyAsync(sumsq, j.sumsq, n * sizeof(float), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    const hipError_t e = read_film(s->ctx, j.film, n, j.desc.spp, mean_rgb, sum, comp, sumsq);
     if (e != hipSuccess) return hip_fail(s->ctx, e, "wr_job_read");
-    if (mean_rgb) {
-        const float inv = 1.f / (float)j.desc.spp;
-        for (size_t i = 0; i < n; i++) mean_rgb[i] = sp[i] * inv;
-    }
     if (passes) *passes = j.desc.spp;
     return WR_OK;
 }
@@ -378,8 +354,8 @@ int wr_job_release(wr_server* s, uint64_t id) {
     if (j.st.state == WR_JOB_RUNNING || j.st.state == WR_JOB_QUEUED)
         return fail(s->ctx, WR_EBUSY, "wr_job_release: job still queued or running");
     (void)hipStreamSynchronize(s->ctx->stream);
-    if (j.sum) s->used -= j.film_bytes;
-    free_job_film(j);
+    if (j.film) s->used -= j.film_bytes;
+    free_job_film(s, j);
     s->jobs.erase(it);
     return WR_OK;
 }

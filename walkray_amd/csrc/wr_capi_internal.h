@@ -13,11 +13,71 @@
 #include "wr_pt.h"
 #include "wr_sceneio.h"
 
+namespace wr {
+// Device memory that a context's calls use again: scratch and result buffers
+// of calls that used to allocate and free them each time (a 256^2
+// BidirectionalPathTracer call's 4 GB took 1 to 20 ms of hipMalloc and
+// hipFree).  A buffer is handed out to one call (or one grid or served job)
+// at a time, whichever thread makes it, and comes back when that ends; all
+// work on a context runs on its stream, so a buffer's next user is ordered
+// behind its last one.  At most kIdleMax bytes stay with the pool unused; they
+// go back to the device when an allocation fails for want of memory, and with
+// the context.  Buffers still out then (a grid that outlives its context) are
+// freed when they come back.
+class WorkPool {
+public:
+    explicit WorkPool(int dev) : device(dev) {}
+    ~WorkPool() { close(); }
+    hipError_t get(void** out, size_t bytes);
+    template <class T>
+    hipError_t get(T** out, size_t bytes) {
+        return get((void**)out, bytes);
+    }
+    void put(void* p);  // nullptr: nothing
+    void trim();        // gives the unused buffers back
+    void close();
+    const int device;
+
+private:
+    static constexpr size_t kIdleMax = 6ull << 30;  // 2% of the device's memory
+    struct Buf {
+        void* p;
+        size_t bytes;
+        bool out;
+    };
+    void free_idle(size_t keep);  // frees unused buffers, the oldest first, until at most `keep` bytes of them are left
+    std::mutex mu;
+    std::vector<Buf> bufs;
+    bool closed = false;
+};
+// Buffers of one call, given back on every exit.
+struct Scratch {
+    WorkPool& pool;
+    std::vector<void*> p;
+    explicit Scratch(WorkPool& w) : pool(w) {}
+    Scratch(const Scratch&) = delete;
+    ~Scratch() {
+        for (void* q : p) pool.put(q);
+    }
+    template <class T>
+    hipError_t get(T** out, size_t bytes) {
+        void* q = nullptr;
+        const hipError_t e = pool.get(&q, bytes);
+        if (e == hipSuccess) p.push_back(q);
+        *out = (T*)q;
+        return e;
+    }
+};
+}  // namespace wr
+
 struct wr_ctx {
     int device = 0;
+    std::shared_ptr<wr::WorkPool> pool;  // shared with the grids built in it
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     std::string err;
+    float* film_back = nullptr;  // pinned, for small films on their way to the host (read_film)
+    std::mutex film_mu;          // held by the read that uses it
     unsigned long long* d_work = nullptr;  // work counters of the persistent closest-hit kernel (each call leaves them zero)
     wr::Engine engine;  // wavefront engine of wr_render, reused across calls
     uint32_t tuned_slots = 0, tuned_grid = 0;  // wr_autotune_render's choice (0 = defaults)
@@ -39,6 +99,8 @@ struct HostObject {
 int fail(wr_ctx* ctx, int code, const std::string& msg);
 int hip_fail(wr_ctx* ctx, hipError_t e, const char* what);
 void scene_free_device(wr_scene* s);
+hipError_t read_film(wr_ctx* ctx, const float* film, size_t n, uint32_t passes, float* mean, float* sum, float* comp,
+                     float* sumsq);
 // Places a moving object with transform M: vertices M (v, 1), corner normals
 // transpose(inverse(M)) (n, 0) (mesh.h:47-77,106).
 void place_object(HostObject& o, const io::Mat4& M);
