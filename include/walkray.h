@@ -400,7 +400,7 @@ int wr_photons_collect(wr_ctx* ctx, const wr_scene* scene, const wr_path_vertex*
                        uint32_t n_paths, uint32_t max_vertices, uint64_t n_leading, float* d_pos, uint32_t* d_src,
                        uint64_t cap, uint64_t* n_out);
 /* HashGrid (hashgrid.hxx:15-203): Reserve(n_cells) + Build(points, radius)
- * over n points (d_pos, device, read again by queries: keep it alive), and
+ * over n points (d_pos, device; the grid keeps a copy in its own order), and
  * Process as a range query: for each query point (device, 3 floats), the
  * points handed to the query in the reference's order (8 cells, a cell
  * reached twice through a hash collision visited twice), the first cap of

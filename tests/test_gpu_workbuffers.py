@@ -72,3 +72,10 @@ def test_film_read(ctx, width, height):
     assert np.array_equal(mean, got["mean"])
     film.clear()
     assert film.read()["passes"] == 0 and not film.read()["sumsq"].any()
+
+
+def test_grid_outlives_context():
+    c = W.Context(0)
+    g = W.HashGrid.from_points(c, np.random.default_rng(1).random((500, 3)), 0.1, 64)
+    c.close()
+    g.close()

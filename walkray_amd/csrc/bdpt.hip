@@ -699,15 +699,8 @@ __global__ void k_vcm_pass_starts(const uint32_t* offs, uint32_t npix, uint32_t 
     if (b <= npass) starts[b] = offs[(size_t)b * npix];
 }
 
-// One pass's grid: pos / src point at the pass's block, idx indexes it.
-struct VcmGrid {
-    GridDev g;
-    const int* ends;
-    const uint32_t* idx;
-    const float* pos;
-    const uint32_t* src;
-    float r;
-};
+// One pass's grid: src and idx are of the pass's block of points.
+using VcmGrid = GridView;
 
 // The merges of the VCM lanes, one entry per light point in reach of an eye
 // vertex: word 0 = lane | eye vertex << 24 (lanes < 2^22), word 1 = the light
@@ -812,8 +805,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     else hi = mid;
                 }
                 for (; a < b; a++) {
+                    if (!grid_near(G.g, G.pos, ev.o, a)) continue;
                     const uint32_t pi = G.idx[a];
-                    if (!grid_near(G.g, G.pos, ev.o, pi)) continue;
                     if (!pass2) {
                         cnt++;
                     } else if (k < M.cap) {
@@ -899,8 +892,8 @@ __device__ f3 ppm_density(const SceneDev& S, const VcmGrid& G, const BVert* vert
             else hi = mid;
         }
         for (; a < b; a++) {
+            if (!grid_near(G.g, G.pos, outRay.o, a)) continue;
             const uint32_t pi = G.idx[a];
-            if (!grid_near(G.g, G.pos, outRay.o, pi)) continue;
             const uint32_t k = G.src[2 * (size_t)pi], j = G.src[2 * (size_t)pi + 1];
             const BVert* L = verts + (size_t)k * 2 * maxv + maxv;
             f3 thr = (L - maxv)[j].rad;  // k_ppm_throughput
@@ -1016,16 +1009,18 @@ static wrd::CamDev make_cam_dev(const CamHost& ch) {
 }
 
 // The light sub-paths of passes [pass0, pass0 + npass) (and their eye sub-paths
-// when eye), their light points and one grid per pass, uploaded to vb.grids;
-// the grids go to `grids` (the caller destroys them).
-static int light_point_grids(wr_ctx* ctx, const SceneDev& S, const wrd::CamDev& cam, uint32_t npix, uint32_t max_depth,
-                             uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv,
-                             wrd::BVert* V, uint32_t* counts, const VcmBufs& vb, bool eye,
-                             std::vector<wr_hashgrid*>& grids, const char* who) {
+// when eye), their light points and one grid per pass, described in vb.grids;
+// the grids' buffers come from mem.  vb.err is set on the device if a pass's
+// points spread over too many cells.
+static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const wrd::CamDev& cam, uint32_t npix,
+                             uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius,
+                             uint32_t maxv, wrd::BVert* V, uint32_t* counts, const VcmBufs& vb, bool eye,
+                             const char* who) {
     hipStream_t st = ctx->stream;
     const uint32_t lanes = npass * npix;  // the caller keeps npass * npix below 2^31
     const uint32_t blocks = (lanes + 255) / 256;
     hipError_t e = hipMemsetAsync(vb.pc + lanes, 0, sizeof(uint32_t), st);
+    if (e == hipSuccess) e = hipMemsetAsync(vb.err, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, who);
     wrd::k_bdpt_subpaths<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, max_depth, seed, pass0, npass, npix, maxv, V,
                                                                   counts, eye);
@@ -1046,20 +1041,22 @@ static int light_point_grids(wr_ctx* ctx, const SceneDev& S, const wrd::CamDev& 
     wrd::k_vcm_point_write<<<blocks, 256, 0, st>>>(S, V, counts, npix, lanes, maxv, vb.offs, vb.pos, vb.src);
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, who);
     // per pass: HashGrid::Reserve(pixels) + Build(its light points, its radius)
-    // (vcmTracer.cpp:30,33,57; photonMap.cpp:48,56,93)
-    grids.assign(npass, nullptr);
-    std::vector<wrd::VcmGrid> G(npass);
+    // (vcmTracer.cpp:30,33,57; photonMap.cpp:48,56,93), all passes together
+    std::vector<wrd::GridParams> params(npass);
     for (uint32_t b = 0; b < npass; b++) {
-        const uint64_t block = (uint64_t)b * npix + starts[b];
-        const uint64_t n = (uint64_t)npix + (starts[b + 1] - starts[b]);
         const float r = vcm_radius(base_radius, pass0 + b);
-        const int rc = wr_hashgrid_build(ctx, vb.pos + 3 * block, n, r, npix, &grids[b]);
-        if (rc != WR_OK) return rc;
-        G[b] = wrd::VcmGrid{grids[b]->g, grids[b]->ends, grids[b]->idx, vb.pos + 3 * block, vb.src + 2 * block, r};
+        params[b] = wrd::GridParams{1.f / (r * 2.f), r * r, r};
     }
-    if ((e = hipMemcpyAsync(vb.grids, G.data(), sizeof(wrd::VcmGrid) * npass, hipMemcpyHostToDevice, st)) != hipSuccess)
-        return hip_fail(ctx, e, who);
+    e = build_grids(ctx, mem, vb.pos, vb.src, (uint64_t)lanes + starts[npass], vb.starts, npix, npass, npix,
+                    params.data(), (wrd::GridView*)vb.grids, vb.err, nullptr);
+    if (e != hipSuccess) return hip_fail(ctx, e, who);
     return WR_OK;
+}
+
+// Once the stream has been synchronised: the error of a pass's grid.
+static int check_grids(wr_ctx* ctx, uint32_t err, const char* who) {
+    if (!err) return WR_OK;
+    return fail(ctx, WR_EINVAL, std::string(who) + ": too many cells across the light points' box for this radius");
 }
 
 int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
@@ -1074,25 +1071,16 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     hipError_t e = hipMemsetAsync(pix, 0, sizeof(float) * 3 * (size_t)lanes, st);
     if (e == hipSuccess) e = hipMemsetAsync(q.count, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
-    std::vector<wr_hashgrid*> grids;
-    auto destroy = [&]() {
-        for (wr_hashgrid* g : grids) wr_hashgrid_destroy(g);
-    };
-    int rc = light_point_grids(ctx, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, q.counts, vb,
-                               true, grids, "wr_render_vcm");
-    if (rc != WR_OK) {
-        destroy();
-        return rc;
-    }
+    Scratch mem(*ctx->pool);  // the grids'
+    int rc = light_point_grids(ctx, mem, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, q.counts,
+                               vb, true, "wr_render_vcm");
+    if (rc != WR_OK) return rc;
     wrd::BPrefix* prefix = (wrd::BPrefix*)q.prefix;
     wrd::k_bdpt_prefix<<<(2 * lanes + 255) / 256, 256, 0, st>>>(S, cam, npix, lanes, maxv, V, q.counts, prefix);
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
     const wrd::MergeQueue M{vb.mq, vb.mq_cap};
     e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint32_t), st);
-    if (e != hipSuccess) {
-        destroy();
-        return hip_fail(ctx, e, "wr_render_vcm");
-    }
+    if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     wrd::k_vcm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q,
                                                         (const wrd::VcmGrid*)vb.grids, M);
     e = hipGetLastError();
@@ -1100,11 +1088,12 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
         wrd::k_vcm_merge<<<4096, 256, 0, st>>>(S, cam, npix, maxv, V, prefix, pix, M, (const wrd::VcmGrid*)vb.grids);
         e = hipGetLastError();
     }
-    uint32_t nq = 0;
+    uint32_t nq = 0, grid_err = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&nq, q.count, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(&grid_err, vb.err, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    destroy();
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
+    if ((rc = check_grids(ctx, grid_err, "wr_render_vcm")) != WR_OK) return rc;
     if (nq > q.cap) nq = q.cap;
     if (nq) {
         if ((e = launch_closest_hit_path(S, H, q.rays, nq, q.hits, q.work, st)) != hipSuccess)
@@ -1126,26 +1115,21 @@ int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const CamHost& ch, uint32_
     const uint32_t lanes = npass * npix;
     const uint32_t blocks = (lanes + 255) / 256;
     wrd::BVert* V = (wrd::BVert*)verts;
-    std::vector<wr_hashgrid*> grids;
-    auto destroy = [&]() {
-        for (wr_hashgrid* g : grids) wr_hashgrid_destroy(g);
-    };
-    int rc = light_point_grids(ctx, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts, vb,
-                               false, grids, "wr_render_ppm");
-    if (rc != WR_OK) {
-        destroy();
-        return rc;
-    }
+    Scratch mem(*ctx->pool);  // the grids'
+    int rc = light_point_grids(ctx, mem, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts, vb,
+                               false, "wr_render_ppm");
+    if (rc != WR_OK) return rc;
     wrd::k_ppm_throughput<<<blocks, 256, 0, st>>>(lanes, maxv, V, counts);
     wrd::k_ppm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, seed, pass0, pix,
                                                         (const wrd::VcmGrid*)vb.grids);
     wrd::k_bdpt_fold<<<(npix + 255) / 256, 256, 0, st>>>(cam, npass, npix, pix,
                                                          wrd::FilmDev{film.sum, film.comp, film.sumsq});
+    uint32_t grid_err = 0;
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);  // the grids are read until k_ppm ends
-    destroy();
+    if (e == hipSuccess) e = hipMemcpyAsync(&grid_err, vb.err, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_ppm");
-    return WR_OK;
+    return check_grids(ctx, grid_err, "wr_render_ppm");  // an error marks the film as part-written
 }
 
 size_t vcm_grid_bytes() { return sizeof(wrd::VcmGrid); }

@@ -25,9 +25,11 @@ __device__ __forceinline__ uint32_t grid_hash(const GridDev& g, int cx, int cy, 
     return ((x * 73856093u) ^ (y * 19349663u) ^ (z * 83492791u)) % g.n_cells;
 }
 
-// The distance test of HashGrid::Process (hashgrid.hxx:142-147): |q - p|^2 <= r^2.
-__device__ __forceinline__ bool grid_near(const GridDev& g, const float* pos, f3 qp, uint32_t pi) {
-    const f3 dv = mk(qp.x - pos[3 * pi], qp.y - pos[3 * pi + 1], qp.z - pos[3 * pi + 2]);
+// The distance test of HashGrid::Process (hashgrid.hxx:142-147): |q - p|^2 <= r^2,
+// p the a-th point in the grid's order.
+__device__ __forceinline__ bool grid_near(const GridDev& g, const float* sorted_pos, f3 qp, int a) {
+    const float* p = sorted_pos + 3 * (size_t)a;
+    const f3 dv = mk(qp.x - p[0], qp.y - p[1], qp.z - p[2]);
     const float dist = len(dv);
     return dist * dist <= g.r2;
 }
@@ -54,17 +56,49 @@ __device__ __forceinline__ uint32_t query_cell(const GridDev& g, const int p[6],
     return grid_hash(g, (j & 4) ? p[3] : p[0], (j & 2) ? p[4] : p[1], (j & 1) ? p[5] : p[2]);
 }
 
+// One grid as its users see it.  pos holds the positions in the grid's order
+// (mIndices), so that a cell's points are read next to each other and their
+// indices only where a point is in reach.
+struct GridView {
+    GridDev g;
+    const int* ends;      // mCellEnds (n_cells)
+    const uint32_t* idx;  // mIndices
+    const float* pos;     // 3 floats per entry of idx
+    const uint32_t* src;  // the caller's: 2 words per point (nullptr: none)
+    float r;
+};
+
+// What the host knows of a grid before its points.
+struct GridParams {
+    float inv, r2, r;
+};
+
 }  // namespace wrd
 
-// A built grid: mCellEnds (inclusive ends per cell) and mIndices over the
-// caller's points.
+namespace wr {
+// Builds `nseg` grids of n_cells cells each over consecutive blocks of points
+// in one go (photon.hip).  Block b starts at point b * lead + starts[b]
+// (starts: nseg + 1 device words; nullptr with one block of all the points) and
+// its grid has the parameters params[b] (host).  `total` points in all (below
+// 2^31), nseg * n_cells below 2^31.  Enqueued on the context's stream: views
+// (nseg device records) describe the grids in buffers taken from mem; *err (a
+// zeroed device word) is set if a grid has too many cells across.  boxes
+// (nullable): the bounding box of every kGridChunk entries of the order.
+constexpr uint32_t kGridChunk = 256;
+hipError_t build_grids(wr_ctx* ctx, Scratch& mem, const float* d_pos, const uint32_t* d_src, uint64_t total,
+                       const uint32_t* starts, uint32_t lead, uint32_t nseg, uint32_t n_cells,
+                       const wrd::GridParams* params, wrd::GridView* views, uint32_t* err, float** boxes);
+}  // namespace wr
+
+// A built grid: mCellEnds (inclusive ends per cell), mIndices and the positions
+// in its order, in buffers of the context's pool.
 struct wr_hashgrid {
     wr_ctx* ctx = nullptr;
-    wrd::GridDev g{};
-    const float* pos = nullptr;  // the caller's points
+    std::shared_ptr<wr::WorkPool> pool;
+    std::unique_ptr<wr::Scratch> mem;
+    wrd::GridView v{};
+    const float* boxes = nullptr;  // per kGridChunk entries of the order: min xyz, max xyz
     uint64_t n = 0;
-    int* ends = nullptr;         // n_cells
-    uint32_t* idx = nullptr;     // n
-    uint32_t* defer = nullptr;   // query calls: deferred-query counter and list (grown on demand)
-    uint64_t defer_cap = 0;      // entries of defer
+    uint32_t* defer = nullptr;     // query calls: deferred-query counter and list (grown on demand)
+    uint64_t defer_cap = 0;        // entries of defer
 };

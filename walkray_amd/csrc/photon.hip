@@ -7,11 +7,11 @@
 //                   every Ray of the Path written as a 64 B record.
 //  photon collect   count, scan and write the light points VCM / PPM keep
 //                   (vcmTracer.cpp:42-55): deterministic, path-major order.
-//  hash grid        HashGrid::Build (hashgrid.hxx:24-75) as bbox reduction,
-//                   per-cell counts, an inclusive scan (mCellEnds) and a stable
-//                   radix sort of (cell, point) pairs (mIndices: the serial
-//                   scatter keeps input order inside a cell, so does a stable
-//                   sort); HashGrid::Process (hashgrid.hxx:77-158) as a range
+//  hash grid        HashGrid::Build (hashgrid.hxx:24-75) as bbox reduction and
+//                   a stable radix sort of (cell, point) pairs (mIndices: the
+//                   serial scatter keeps input order inside a cell, so does a
+//                   stable sort; mCellEnds: the cells' ends in the sorted
+//                   pairs); HashGrid::Process (hashgrid.hxx:77-158) as a range
 //                   query, one lane per query point.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -184,26 +184,36 @@ __global__ __launch_bounds__(256) void k_fill_leading(uint64_t n, uint64_t cap, 
 }
 
 // ---- hash grid ------------------------------------------------------------
-// Order-preserving map of floats onto signed ints, for atomic min / max.
-__device__ __forceinline__ int fkey(float f) {
-    const int i = __float_as_int(f);
-    return i >= 0 ? i : i ^ 0x7FFFFFFF;
-}
-static inline int fkey_host(float f) {
-    int i;
-    std::memcpy(&i, &f, 4);
-    return i >= 0 ? i : i ^ 0x7FFFFFFF;
-}
-static inline float fkey_inv(int k) {
-    const int i = k >= 0 ? k : k ^ 0x7FFFFFFF;
-    float f;
-    std::memcpy(&f, &i, 4);
-    return f;
-}
+// The grids of several passes are built together: every kernel below covers all
+// blocks of points (segments), and one sort orders them by (segment, cell).
+// Built one by one, the eight grids of a 256^2 PhotonMap call (1M points) took
+// 1.6 ms in 190 launches, with two synchronisations each; now 0.18 ms in 12.
+struct GridSegs {
+    const uint32_t* starts;  // nullptr: one segment
+    uint32_t lead, nseg, total;
+    __device__ __forceinline__ uint32_t first(uint32_t b) const {
+        return starts ? b * lead + starts[b] : (b ? total : 0u);
+    }
+    // the segment of point i
+    __device__ __forceinline__ uint32_t of(uint32_t i) const {
+        uint32_t lo = 0, hi = nseg;  // first(lo) <= i < first(hi)
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (first(mid) <= i) lo = mid;
+            else hi = mid;
+        }
+        return lo;
+    }
+};
 
-__global__ __launch_bounds__(256) void k_grid_bbox(const float* pos, uint64_t n, int* keys) {
+// Partial bounding boxes: `parts` workgroups per segment, their boxes in part
+// (6 floats each).  No atomics: 13,000 of them on six words took most of the
+// 155 us that 568,000 points' box took.
+__global__ __launch_bounds__(256) void k_grid_bbox(GridSegs G, const float* pos, uint32_t parts, float* part) {
+    const uint32_t b = blockIdx.x / parts, k = blockIdx.x % parts;
+    const uint32_t end = G.first(b + 1);
     float mn[3] = {1e36f, 1e36f, 1e36f}, mx[3] = {-1e36f, -1e36f, -1e36f};
-    for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
+    for (uint64_t i = (uint64_t)G.first(b) + k * 256 + threadIdx.x; i < end; i += (uint64_t)parts * 256) {
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             const float v = pos[3 * i + a];
@@ -218,47 +228,129 @@ __global__ __launch_bounds__(256) void k_grid_bbox(const float* pos, uint64_t n,
             mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off));
         }
     }
-    // the block's four waves meet in LDS: one set of atomics per block
-    __shared__ float part[4][6];
+    __shared__ float wave[4][6];
     const uint32_t w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
         for (int a = 0; a < 3; a++) {
-            part[w][a] = mn[a];
-            part[w][3 + a] = mx[a];
+            wave[w][a] = mn[a];
+            wave[w][3 + a] = mx[a];
         }
     __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            float lo = part[0][a], hi = part[0][3 + a];
-            for (int k = 1; k < 4; k++) {
-                lo = fminf(lo, part[k][a]);
-                hi = fmaxf(hi, part[k][3 + a]);
-            }
-            atomicMin(keys + a, fkey(lo));
-            atomicMax(keys + 3 + a, fkey(hi));
-        }
+    if (threadIdx.x < 6) {
+        float v = wave[0][threadIdx.x];
+        for (int k2 = 1; k2 < 4; k2++)
+            v = threadIdx.x < 3 ? fminf(v, wave[k2][threadIdx.x]) : fmaxf(v, wave[k2][threadIdx.x]);
+        part[6 * (size_t)blockIdx.x + threadIdx.x] = v;
     }
 }
 
-__global__ __launch_bounds__(256) void k_grid_keys(GridDev g, const float* pos, uint32_t n, uint32_t* keys,
-                                                   uint32_t* vals, uint32_t* cell_count) {
+// The view of every segment's grid, one wave per segment: its box from the
+// partial ones, and the check that the integer cell coordinates stay
+// representable.
+__global__ __launch_bounds__(64) void k_grid_views(GridSegs G, const float* part, uint32_t parts,
+                                                   const GridParams* params, uint32_t n_cells, const int* ends,
+                                                   const uint32_t* idx, const float* sorted_pos, const uint32_t* src,
+                                                   GridView* views, uint32_t* err) {
+    const uint32_t b = blockIdx.x;
+    float mn[3] = {1e36f, 1e36f, 1e36f}, mx[3] = {-1e36f, -1e36f, -1e36f};
+    for (uint32_t k = threadIdx.x; k < parts; k += 64)
+        for (int a = 0; a < 3; a++) {
+            mn[a] = fminf(mn[a], part[6 * (size_t)(b * parts + k) + a]);
+            mx[a] = fmaxf(mx[a], part[6 * (size_t)(b * parts + k) + 3 + a]);
+        }
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        for (int off = 32; off > 0; off >>= 1) {
+            mn[a] = fminf(mn[a], __shfl_xor(mn[a], off));
+            mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off));
+        }
+    }
+    if (threadIdx.x != 0) return;
+    const GridParams P = params[b];
+    const size_t first = G.first(b);
+    GridView v;
+    bool fits = true;
+    for (int a = 0; a < 3; a++) {
+        v.g.bmin[a] = mn[a];
+        v.g.bmax[a] = mx[a];
+        fits = fits && (mx[a] - mn[a]) * P.inv < 2147483520.f;
+    }
+    v.g.inv = P.inv;
+    v.g.r2 = P.r2;
+    v.g.n_cells = n_cells;
+    v.ends = ends + (size_t)b * n_cells;
+    v.idx = idx + first;
+    v.pos = sorted_pos + 3 * first;
+    v.src = src ? src + 2 * first : nullptr;
+    v.r = P.r;
+    views[b] = v;
+    if (!fits && G.first(b + 1) > first) *err = 1u;
+}
+
+// Each point's sort key (its segment, then its cell: GetCellIndex(Vec3f),
+// hashgrid.hxx:180-190) and its index within the segment.
+__global__ __launch_bounds__(256) void k_grid_keys(GridSegs G, const GridView* views, const float* pos, uint32_t* keys,
+                                                   uint32_t* vals) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    // GetCellIndex(Vec3f) (hashgrid.hxx:180-190)
-    const float dx = pos[3 * i] - g.bmin[0], dy = pos[3 * i + 1] - g.bmin[1], dz = pos[3 * i + 2] - g.bmin[2];
-    const uint32_t c = grid_hash(g, (int)floorf(g.inv * dx), (int)floorf(g.inv * dy), (int)floorf(g.inv * dz));
-    keys[i] = c;
-    vals[i] = i;
-    // one atomic for a wave whose points share a cell (many coincident points,
-    // such as VCM's leading ones), else one per point
-    const uint64_t act = __ballot(1);
-    const uint32_t leader = __ffsll((unsigned long long)act) - 1;
-    const uint64_t same = __ballot(c == __shfl(c, leader));
-    if (same == act) {
-        if ((threadIdx.x & 63) == leader) atomicAdd(cell_count + c, (uint32_t)__popcll(act));
-    } else {
-        atomicAdd(cell_count + c, 1u);
+    if (i >= G.total) return;
+    const uint32_t b = G.of(i);
+    const GridDev g = views[b].g;
+    const float* p = pos + 3 * (size_t)i;
+    const float dx = p[0] - g.bmin[0], dy = p[1] - g.bmin[1], dz = p[2] - g.bmin[2];
+    keys[i] = b * g.n_cells + grid_hash(g, (int)floorf(g.inv * dx), (int)floorf(g.inv * dy), (int)floorf(g.inv * dz));
+    vals[i] = i - G.first(b);
+}
+
+// From the sorted keys: the end of every cell (the entries of its segment with
+// a key up to its own, by binary search: no counts, so no atomics and no scan
+// of the cells) and the positions in the grid's order.
+__global__ __launch_bounds__(256) void k_grid_finish(GridSegs G, const float* pos, const uint32_t* keys,
+                                                     const uint32_t* idx, uint32_t n_cells, int* ends,
+                                                     float* sorted_pos) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < G.nseg * n_cells) {
+        uint32_t lo = 0, n = G.total;  // the first entry with a larger key
+        while (n > 0) {
+            const uint32_t half = n >> 1;
+            if (keys[lo + half] <= i) {
+                lo += half + 1;
+                n -= half + 1;
+            } else {
+                n = half;
+            }
+        }
+        ends[i] = (int)(lo - G.first(i / n_cells));
+    }
+    if (i < G.total) {
+        const size_t from = (size_t)G.first(keys[i] / n_cells) + idx[i];
+        for (int a = 0; a < 3; a++) sorted_pos[3 * (size_t)i + a] = pos[3 * from + a];
+    }
+}
+
+// The bounding box of every kGridChunk entries, one workgroup each.
+__global__ __launch_bounds__(256) void k_grid_boxes(uint32_t total, const float* sorted_pos, float* boxes) {
+    static_assert(wr::kGridChunk == 256, "one lane per entry");
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    float v[6];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const bool in = i < total;
+        const float x = in ? sorted_pos[3 * (size_t)i + a] : 0.f;
+        v[a] = in ? x : 1e38f;
+        v[3 + a] = in ? x : -1e38f;
+        for (int off = 32; off > 0; off >>= 1) {
+            v[a] = fminf(v[a], __shfl_xor(v[a], off));
+            v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], off));
+        }
+    }
+    __shared__ float wave[4][6];
+    if ((threadIdx.x & 63) == 0)
+        for (int a = 0; a < 6; a++) wave[threadIdx.x >> 6][a] = v[a];
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        float r = wave[0][threadIdx.x];
+        for (int k = 1; k < 4; k++) r = threadIdx.x < 3 ? fminf(r, wave[k][threadIdx.x]) : fmaxf(r, wave[k][threadIdx.x]);
+        boxes[6 * (size_t)blockIdx.x + threadIdx.x] = r;
     }
 }
 
@@ -271,12 +363,15 @@ constexpr int kLongRange = 64;
 constexpr int kHugeRange = 2048;
 
 // defer: [0] the number of deferred queries, then their indices.
-__global__ __launch_bounds__(256) void k_grid_query(GridDev g, const float* pos, const int* ends, const uint32_t* idx,
-                                                    const float* q, uint32_t nq, uint32_t cap, uint32_t* counts,
+__global__ __launch_bounds__(256) void k_grid_query(GridView G, const float* q, uint32_t nq, uint32_t cap, uint32_t* counts,
                                                     uint32_t* out, uint32_t* defer) {
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = (1ull << lane) - 1ull;
+    const GridDev& g = G.g;
+    const int* ends = G.ends;
+    const uint32_t* idx = G.idx;
+    const float* pos = G.pos;
     // every lane stays to the end: the long ranges are scanned by the whole wave
     bool valid = k < nq;
     f3 qp = mk(0.f, 0.f, 0.f);
@@ -309,9 +404,8 @@ __global__ __launch_bounds__(256) void k_grid_query(GridDev g, const float* pos,
         const bool long_range = b - a > kLongRange;
         if (!long_range) {
             for (; a < b; a++) {
-                const uint32_t pi = idx[a];
-                if (grid_near(g, pos, qp, pi)) {
-                    if (m < cap) out[(size_t)k * cap + m] = pi;
+                if (grid_near(g, pos, qp, a)) {
+                    if (m < cap) out[(size_t)k * cap + m] = idx[a];
                     m++;
                 }
             }
@@ -327,22 +421,18 @@ __global__ __launch_bounds__(256) void k_grid_query(GridDev g, const float* pos,
             // sixteen 64-point steps per iteration: their loads are in flight together
             // (a single wave walks the whole range, so its loads in flight set the pace)
             for (int base = la; base < lb; base += 16 * 64) {
-                uint32_t pi[16];
                 bool hit[16];
 #pragma unroll
                 for (int u = 0; u < 16; u++) {
                     const int ai = base + 64 * u + (int)lane;
-                    pi[u] = ai < lb ? idx[ai] : 0u;
+                    hit[u] = ai < lb && grid_near(g, pos, lq, ai);
                 }
-#pragma unroll
-                for (int u = 0; u < 16; u++)
-                    hit[u] = base + 64 * u + (int)lane < lb && grid_near(g, pos, lq, pi[u]);
 #pragma unroll
                 for (int u = 0; u < 16; u++) {
                     const uint64_t hm = __ballot(hit[u]);
                     if (hit[u]) {
                         const uint32_t slot = lm + (uint32_t)__popcll(hm & below);
-                        if (slot < cap) out[(size_t)lk * cap + slot] = pi[u];
+                        if (slot < cap) out[(size_t)lk * cap + slot] = idx[base + 64 * u + (int)lane];
                     }
                     lm += (uint32_t)__popcll(hm);
                 }
@@ -354,17 +444,24 @@ __global__ __launch_bounds__(256) void k_grid_query(GridDev g, const float* pos,
 }
 
 // The deferred queries, one workgroup per query: the workgroup walks the
-// query's 8 cells in the reference's order, 256 points a step and kWideSteps
-// steps per iteration.  Step u, wave w, lane l holds point base + 256u + 64w + l,
-// so a hit's slot is the hits before it in that order: the query's count so
-// far, the wave counts of the earlier steps and waves (LDS), and its rank in
-// its wave's ballot.  Every loop bound is the same for the whole workgroup.
-constexpr int kWideSteps = 16;
-
-__global__ __launch_bounds__(256) void k_grid_query_wide(GridDev g, const float* pos, const int* ends,
-                                                         const uint32_t* idx, const float* q, uint32_t cap,
+// query's 8 cells in the reference's order, in chunks of kGridChunk entries of
+// the grid's order, and skips every chunk whose bounding box is out of reach (a
+// long range is mostly points that have nothing in common but their bucket, or
+// one coincident heap such as VCM's leading points).  The test is exact: the
+// distance to the box is formed by the operations of the distance to a point,
+// each of them monotone under rounding, from per-axis distances no larger than
+// any of its points', so a chunk is skipped only if every point of it would
+// fail.  256 chunks are tested at a time; the points of the ones left are
+// tested one per lane, and a hit's slot is the query's count so far, the hits
+// of the earlier waves (LDS) and its rank in its wave's ballot, which keeps the
+// serial order.  Every loop bound is the same for the whole workgroup.  Point
+// by point, 260,000 queries over 568,000 points of which 307,200 share a
+// bucket took 566 us; now 15 us.
+__global__ __launch_bounds__(256) void k_grid_query_wide(GridView G, const float* boxes, const float* q, uint32_t cap,
                                                          uint32_t* counts, uint32_t* out, const uint32_t* defer) {
-    __shared__ uint32_t wcnt[kWideSteps][4];
+    __shared__ uint64_t near[4];   // the chunks in reach, a bit each
+    __shared__ uint32_t wcnt[4];
+    const GridDev& g = G.g;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
     const uint32_t nd = defer[0];
@@ -376,42 +473,46 @@ __global__ __launch_bounds__(256) void k_grid_query_wide(GridDev g, const float*
         uint32_t m = 0;
         for (int j = 0; j < 8; j++) {
             const uint32_t c = query_cell(g, p, j);
-            const int a = c == 0 ? 0 : ends[c - 1];
-            const int b = ends[c];
-            for (int base = a; base < b; base += kWideSteps * 256) {
-                uint32_t pi[kWideSteps];
-                bool hit[kWideSteps];
-#pragma unroll
-                for (int u = 0; u < kWideSteps; u++) {
-                    const int ai = base + 256 * u + (int)threadIdx.x;
-                    pi[u] = ai < b ? idx[ai] : 0u;
+            const int a = c == 0 ? 0 : G.ends[c - 1];
+            const int b = G.ends[c];
+            if (a >= b) continue;
+            const uint32_t last = (uint32_t)(b - 1) / wr::kGridChunk;
+            for (uint32_t c0 = (uint32_t)a / wr::kGridChunk; c0 <= last; c0 += 256) {
+                const uint32_t ch = c0 + threadIdx.x;
+                bool reach = false;
+                if (ch <= last) {
+                    const float* B = boxes + 6 * (size_t)ch;
+                    const f3 dv = mk(fmaxf(fmaxf(B[0] - qp.x, qp.x - B[3]), 0.f),
+                                     fmaxf(fmaxf(B[1] - qp.y, qp.y - B[4]), 0.f),
+                                     fmaxf(fmaxf(B[2] - qp.z, qp.z - B[5]), 0.f));
+                    const float dist = len(dv);
+                    reach = dist * dist <= g.r2;
                 }
-#pragma unroll
-                for (int u = 0; u < kWideSteps; u++)
-                    hit[u] = base + 256 * u + (int)threadIdx.x < b && grid_near(g, pos, qp, pi[u]);
-                uint64_t hm[kWideSteps];
-#pragma unroll
-                for (int u = 0; u < kWideSteps; u++) {
-                    hm[u] = __ballot(hit[u]);
-                    if (lane == 0) wcnt[u][wave] = (uint32_t)__popcll(hm[u]);
-                }
+                const uint64_t rm = __ballot(reach);
+                if (lane == 0) near[wave] = rm;
                 __syncthreads();
-                uint32_t off = m;
-#pragma unroll
-                for (int u = 0; u < kWideSteps; u++) {
-                    uint32_t before = 0, all = 0;
-                    for (uint32_t w = 0; w < 4; w++) {
-                        before += w < wave ? wcnt[u][w] : 0u;
-                        all += wcnt[u][w];
+                for (uint32_t w = 0; w < 4; w++) {
+                    for (uint64_t left = near[w]; left != 0; left &= left - 1) {
+                        const uint32_t chunk = c0 + 64 * w + (uint32_t)__ffsll((unsigned long long)left) - 1;
+                        const int ai = (int)(chunk * wr::kGridChunk + threadIdx.x);
+                        const bool hit = ai >= a && ai < b && grid_near(g, G.pos, qp, ai);
+                        const uint64_t hm = __ballot(hit);
+                        if (lane == 0) wcnt[wave] = (uint32_t)__popcll(hm);
+                        __syncthreads();
+                        uint32_t before = 0, all = 0;
+                        for (uint32_t v = 0; v < 4; v++) {
+                            before += v < wave ? wcnt[v] : 0u;
+                            all += wcnt[v];
+                        }
+                        if (hit) {
+                            const uint32_t slot = m + before + (uint32_t)__popcll(hm & below);
+                            if (slot < cap) out[(size_t)k * cap + slot] = G.idx[ai];
+                        }
+                        m += all;
+                        __syncthreads();  // wcnt serves the next chunk
                     }
-                    if (hit[u]) {
-                        const uint32_t slot = off + before + (uint32_t)__popcll(hm[u] & below);
-                        if (slot < cap) out[(size_t)k * cap + slot] = pi[u];
-                    }
-                    off += all;
                 }
-                m = off;
-                __syncthreads();  // wcnt is rewritten by the next iteration
+                __syncthreads();  // near serves the next 256 chunks
             }
         }
         if (threadIdx.x == 0) counts[k] = m;
@@ -468,6 +569,63 @@ using wr::hip_fail;
         hipError_t e_ = (call);                      \
         if (e_ != hipSuccess) return hip_fail(ctx, e_, what); \
     } while (0)
+
+namespace wr {
+
+hipError_t build_grids(wr_ctx* ctx, Scratch& mem, const float* d_pos, const uint32_t* d_src, uint64_t total,
+                       const uint32_t* starts, uint32_t lead, uint32_t nseg, uint32_t n_cells,
+                       const GridParams* params, GridView* views, uint32_t* err, float** boxes) {
+    hipStream_t st = ctx->stream;
+    const uint32_t cells = nseg * n_cells;
+    // workgroups of 256 per segment's box: one per 1,024 points, at most 128
+    const uint32_t parts = (uint32_t)std::min<uint64_t>(128, std::max<uint64_t>(1, total / nseg / 1024));
+    int end_bit = 1;
+    while (end_bit < 32 && (cells - 1) >> end_bit) end_bit++;
+    size_t tb = 0;
+    hipError_t e = hipSuccess;
+    if (total)
+        e = hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (uint32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
+                                               (uint32_t*)nullptr, (int)total, 0, end_bit, st);
+    if (e != hipSuccess) return e;
+    // what the grids keep, and what the build alone needs
+    int* ends;
+    uint32_t* idx;
+    float* pos;
+    if ((e = mem.get(&ends, sizeof(int) * (size_t)cells)) != hipSuccess) return e;
+    if ((e = mem.get(&idx, sizeof(uint32_t) * total)) != hipSuccess) return e;
+    if ((e = mem.get(&pos, sizeof(float) * 3 * total)) != hipSuccess) return e;
+    if (boxes && (e = mem.get(boxes, sizeof(float) * 6 * ((total + kGridChunk - 1) / kGridChunk))) != hipSuccess)
+        return e;
+    Scratch sc(*ctx->pool);
+    float* part;
+    GridParams* d_params;
+    uint32_t* keys;
+    void* tmp;
+    const size_t n4 = sizeof(uint32_t) * total;
+    if ((e = sc.get(&part, sizeof(float) * 6 * (size_t)nseg * parts)) != hipSuccess) return e;
+    if ((e = sc.get(&d_params, sizeof(GridParams) * nseg)) != hipSuccess) return e;
+    if ((e = sc.get(&keys, 3 * n4)) != hipSuccess) return e;
+    if ((e = sc.get(&tmp, tb)) != hipSuccess) return e;
+    uint32_t *sorted_keys = keys + total, *vals = sorted_keys + total;
+    if ((e = hipMemcpyAsync(d_params, params, sizeof(GridParams) * nseg, hipMemcpyHostToDevice, st)) != hipSuccess)
+        return e;
+    const GridSegs G{starts, lead, nseg, (uint32_t)total};
+    k_grid_bbox<<<nseg * parts, 256, 0, st>>>(G, d_pos, parts, part);
+    k_grid_views<<<nseg, 64, 0, st>>>(G, part, parts, d_params, n_cells, ends, idx, pos, d_src, views, err);
+    const uint32_t blocks = (uint32_t)((total + 255) / 256);
+    if (total) {
+        k_grid_keys<<<blocks, 256, 0, st>>>(G, views, d_pos, keys, vals);
+        // stable: points of one cell keep their input order, as the serial scatter does
+        e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, sorted_keys, vals, idx, (int)total, 0, end_bit, st);
+        if (e != hipSuccess) return e;
+    }
+    const uint32_t most = (uint32_t)std::max<uint64_t>(total, cells);
+    k_grid_finish<<<(most + 255) / 256, 256, 0, st>>>(G, d_pos, sorted_keys, idx, n_cells, ends, pos);
+    if (boxes && total) k_grid_boxes<<<blocks, 256, 0, st>>>((uint32_t)total, pos, *boxes);
+    return hipGetLastError();
+}
+
+}  // namespace wr
 
 extern "C" {
 
@@ -539,77 +697,35 @@ int wr_hashgrid_build(wr_ctx* ctx, const float* d_pos, uint64_t n, float radius,
     if (!(radius > 0.f) || !std::isfinite(radius)) return fail(ctx, WR_EINVAL, "wr_hashgrid_build: radius must be > 0");
     (void)hipSetDevice(ctx->device);
     hipStream_t st = ctx->stream;
-    wr_hashgrid* g = new wr_hashgrid;
+    std::unique_ptr<wr_hashgrid> g(new wr_hashgrid);
     g->ctx = ctx;
-    g->pos = d_pos;
+    g->pool = ctx->pool;
+    g->mem.reset(new wr::Scratch(*g->pool));
     g->n = n;
     // Build with aMaxDist = 0: mCellSize = 2 * radius (hashgrid.hxx:28-35)
     float max_dist = 0.f;
     if (std::fabs(max_dist) < 1e-5) max_dist = radius;
     const float cell = max_dist * 2.f;
-    g->g.inv = 1.f / cell;
-    g->g.r2 = radius * radius;
-    g->g.n_cells = n_cells;
-    auto bail = [&](hipError_t e, const char* what) {
-        wr_hashgrid_destroy(g);
-        return hip_fail(ctx, e, what);
-    };
-    hipError_t e = hipMalloc((void**)&g->ends, sizeof(int) * n_cells);
-    if (e == hipSuccess) e = hipMalloc((void**)&g->idx, sizeof(uint32_t) * std::max<uint64_t>(n, 1));
-    if (e != hipSuccess) return bail(e, "hipMalloc(hashgrid)");
+    const GridParams P{1.f / cell, radius * radius, radius};
     wr::Scratch sc(*ctx->pool);
-    int* keys6 = nullptr;
-    uint32_t *ckeys = nullptr, *ckeys2 = nullptr, *vals = nullptr, *cnt = nullptr;
-    if ((e = sc.get(&keys6, 6 * sizeof(int))) != hipSuccess) return bail(e, "hipMalloc(hashgrid)");
-    const int init[6] = {fkey_host(1e36f), fkey_host(1e36f), fkey_host(1e36f),
-                         fkey_host(-1e36f), fkey_host(-1e36f), fkey_host(-1e36f)};
-    if ((e = hipMemcpyAsync(keys6, init, sizeof(init), hipMemcpyHostToDevice, st)) != hipSuccess)
-        return bail(e, "wr_hashgrid_build");
-    if (n) {
-        k_grid_bbox<<<(unsigned)std::min<uint64_t>((n + 255) / 256, 4096), 256, 0, st>>>(d_pos, n, keys6);
-        if ((e = hipGetLastError()) != hipSuccess) return bail(e, "wr_hashgrid_build");
-    }
-    int hk[6];
-    if ((e = hipMemcpyAsync(hk, keys6, sizeof(hk), hipMemcpyDeviceToHost, st)) != hipSuccess ||
-        (e = hipStreamSynchronize(st)) != hipSuccess)
-        return bail(e, "wr_hashgrid_build");
-    for (int a = 0; a < 3; a++) {
-        g->g.bmin[a] = fkey_inv(hk[a]);
-        g->g.bmax[a] = fkey_inv(hk[3 + a]);
-        // the integer cell coordinates must stay representable
-        if (n && !((g->g.bmax[a] - g->g.bmin[a]) * g->g.inv < 2147483520.f)) {
-            wr_hashgrid_destroy(g);
-            return fail(ctx, WR_EINVAL, "wr_hashgrid_build: too many cells across the points' box for this radius");
-        }
-    }
-    if ((e = hipMemsetAsync(g->ends, 0, sizeof(int) * n_cells, st)) != hipSuccess) return bail(e, "wr_hashgrid_build");
-    if (n) {
-        if ((e = sc.get(&ckeys, 4 * n)) != hipSuccess || (e = sc.get(&ckeys2, 4 * n)) != hipSuccess ||
-            (e = sc.get(&vals, 4 * n)) != hipSuccess || (e = sc.get(&cnt, 4ull * n_cells)) != hipSuccess)
-            return bail(e, "hipMalloc(hashgrid)");
-        if ((e = hipMemsetAsync(cnt, 0, 4ull * n_cells, st)) != hipSuccess) return bail(e, "wr_hashgrid_build");
-        k_grid_keys<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(g->g, d_pos, (uint32_t)n, ckeys, vals, cnt);
-        if ((e = hipGetLastError()) != hipSuccess) return bail(e, "wr_hashgrid_build");
-        // mCellEnds = inclusive prefix sum of the counts
-        size_t tb = 0, tb2 = 0;
-        if ((e = hipcub::DeviceScan::InclusiveSum(nullptr, tb, cnt, g->ends, (int)n_cells, st)) != hipSuccess)
-            return bail(e, "hipcub scan");
-        int end_bit = 1;
-        while (end_bit < 32 && (n_cells - 1) >> end_bit) end_bit++;
-        if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, tb2, ckeys, ckeys2, vals, g->idx, (int)n, 0, end_bit,
-                                                    st)) != hipSuccess)
-            return bail(e, "hipcub sort");
-        void* tmp = nullptr;
-        if ((e = sc.get(&tmp, std::max(tb, tb2))) != hipSuccess) return bail(e, "hipMalloc(hashgrid)");
-        if ((e = hipcub::DeviceScan::InclusiveSum(tmp, tb, cnt, g->ends, (int)n_cells, st)) != hipSuccess)
-            return bail(e, "hipcub scan");
-        // stable: points of one cell keep their input order, as the serial scatter does
-        if ((e = hipcub::DeviceRadixSort::SortPairs(tmp, tb2, ckeys, ckeys2, vals, g->idx, (int)n, 0, end_bit,
-                                                    st)) != hipSuccess)
-            return bail(e, "hipcub sort");
-    }
-    if ((e = hipStreamSynchronize(st)) != hipSuccess) return bail(e, "wr_hashgrid_build");
-    *out = g;
+    GridView* view = nullptr;
+    float* boxes = nullptr;
+    struct {
+        GridView v;
+        uint32_t err;
+    } back;
+    PH_CHECK(sc.get(&view, sizeof(back)), "hipMalloc(hashgrid)");
+    uint32_t* err = (uint32_t*)((char*)view + ((char*)&back.err - (char*)&back));
+    k_clear_word<<<1, 1, 0, st>>>(err);
+    PH_CHECK(wr::build_grids(ctx, *g->mem, d_pos, nullptr, n, nullptr, 0, 1, n_cells, &P, view, err, &boxes),
+             "wr_hashgrid_build");
+    PH_CHECK(hipMemcpyAsync(&back, view, sizeof(back), hipMemcpyDeviceToHost, st), "wr_hashgrid_build");
+    PH_CHECK(hipStreamSynchronize(st), "wr_hashgrid_build");
+    if (back.err)
+        return fail(ctx, WR_EINVAL, "wr_hashgrid_build: too many cells across the points' box for this radius");
+    g->v = back.v;
+    g->boxes = boxes;
+    *out = g.release();
     return WR_OK;
 }
 
@@ -619,13 +735,13 @@ int wr_hashgrid_export(const wr_hashgrid* g, float* bbox, int32_t* cell_ends, in
     (void)hipSetDevice(ctx->device);
     if (bbox)
         for (int a = 0; a < 3; a++) {
-            bbox[a] = g->g.bmin[a];
-            bbox[3 + a] = g->g.bmax[a];
+            bbox[a] = g->v.g.bmin[a];
+            bbox[3 + a] = g->v.g.bmax[a];
         }
     if (cell_ends)
-        PH_CHECK(hipMemcpy(cell_ends, g->ends, sizeof(int) * g->g.n_cells, hipMemcpyDeviceToHost), "wr_hashgrid_export");
+        PH_CHECK(hipMemcpy(cell_ends, g->v.ends, sizeof(int) * g->v.g.n_cells, hipMemcpyDeviceToHost), "wr_hashgrid_export");
     if (indices && g->n)
-        PH_CHECK(hipMemcpy(indices, g->idx, sizeof(uint32_t) * g->n, hipMemcpyDeviceToHost), "wr_hashgrid_export");
+        PH_CHECK(hipMemcpy(indices, g->v.idx, sizeof(uint32_t) * g->n, hipMemcpyDeviceToHost), "wr_hashgrid_export");
     return WR_OK;
 }
 
@@ -638,20 +754,18 @@ int wr_hashgrid_query(wr_hashgrid* g, const float* d_queries, uint64_t nq, uint3
     if (nq == 0) return WR_OK;
     (void)hipSetDevice(ctx->device);
     if (g->defer_cap < nq + 1) {
-        if (g->defer) PH_CHECK(hipFree(g->defer), "wr_hashgrid_query");
+        g->pool->put(g->defer);
         g->defer = nullptr;
         g->defer_cap = 0;
-        PH_CHECK(hipMalloc((void**)&g->defer, sizeof(uint32_t) * (nq + 1)), "hipMalloc(hashgrid query)");
+        PH_CHECK(g->pool->get(&g->defer, sizeof(uint32_t) * (nq + 1)), "hipMalloc(hashgrid query)");
         g->defer_cap = nq + 1;
     }
     PH_CHECK(hipMemsetAsync(g->defer, 0, sizeof(uint32_t), ctx->stream), "wr_hashgrid_query");
-    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->g, g->pos, g->ends, g->idx, d_queries,
-                                                                         (uint32_t)nq, cap, d_counts, d_idx, g->defer);
+    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts, d_idx, g->defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query");
     // the deferred queries: a workgroup each, as many workgroups as fill the device twice
     const unsigned wide_grid = (unsigned)std::min<uint64_t>(nq, 2048);
-    k_grid_query_wide<<<wide_grid, 256, 0, ctx->stream>>>(g->g, g->pos, g->ends, g->idx, d_queries, cap, d_counts,
-                                                          d_idx, g->defer);
+    k_grid_query_wide<<<wide_grid, 256, 0, ctx->stream>>>(g->v, g->boxes, d_queries, cap, d_counts, d_idx, g->defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query");
     PH_CHECK(hipStreamSynchronize(ctx->stream), "wr_hashgrid_query");
     return WR_OK;
@@ -672,22 +786,19 @@ int wr_hashgrid_query_noalloc(wr_hashgrid* g, const float* d_queries, uint64_t n
     // the list keeps the previous call's contents: only its counter must start at zero
     k_clear_word<<<1, 1, 0, ctx->stream>>>(defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query_noalloc");
-    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->g, g->pos, g->ends, g->idx, d_queries,
-                                                                         (uint32_t)nq, cap, d_counts, d_idx, defer);
+    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts, d_idx, defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query_noalloc");
     const unsigned wide_grid = (unsigned)std::min<uint64_t>(nq, 2048);
-    k_grid_query_wide<<<wide_grid, 256, 0, ctx->stream>>>(g->g, g->pos, g->ends, g->idx, d_queries, cap, d_counts,
-                                                          d_idx, defer);
+    k_grid_query_wide<<<wide_grid, 256, 0, ctx->stream>>>(g->v, g->boxes, d_queries, cap, d_counts, d_idx, defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query_noalloc");
     return WR_OK;
 }
 
 void wr_hashgrid_destroy(wr_hashgrid* g) {
     if (!g) return;
-    (void)hipSetDevice(g->ctx->device);
-    if (g->ends) (void)hipFree(g->ends);
-    if (g->idx) (void)hipFree(g->idx);
-    if (g->defer) (void)hipFree(g->defer);
+    (void)hipSetDevice(g->pool->device);
+    g->pool->put(g->defer);
+    g->mem.reset();
     delete g;
 }
 

@@ -404,6 +404,7 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = mem.get(&vb.pos, sizeof(float) * 3 * vb.cap);
     if (e == hipSuccess) e = mem.get(&vb.src, sizeof(uint32_t) * 2 * vb.cap);
     if (e == hipSuccess) e = mem.get(&vb.grids, vcm_grid_bytes() * batch);
+    if (e == hipSuccess) e = mem.get(&vb.err, sizeof(uint32_t));
     if (e == hipSuccess) {
         char* b = (char*)qbuf;
         q.rays = (uint32_t*)b;
@@ -485,6 +486,7 @@ extern "C" int wr_render_ppm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = mem.get(&vb.pos, sizeof(float) * 3 * vb.cap);
     if (e == hipSuccess) e = mem.get(&vb.src, sizeof(uint32_t) * 2 * vb.cap);
     if (e == hipSuccess) e = mem.get(&vb.grids, vcm_grid_bytes() * batch);
+    if (e == hipSuccess) e = mem.get(&vb.err, sizeof(uint32_t));
     if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_ppm");
     const FilmBufs fb{film->sum, film->comp, film->sumsq};
