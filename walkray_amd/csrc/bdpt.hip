@@ -223,11 +223,16 @@ struct BPrefix {
     double all;     // product of the edge factors: reverse[0] = reverse[c] * all
     f3 color;       // product over the records before this one (radiance * cosine)
     float prob;     // product of their probabilities
-    uint32_t flags; // kPAny, kPEmissive
+    uint32_t flags; // kPAny, kPEmissive, kPDelta
     uint32_t pad;
 };
 constexpr uint32_t kPAny = 1u;       // some neighbours among the records up to this one are both non-delta
 constexpr uint32_t kPEmissive = 2u;  // the record's contact is an emitter
+constexpr uint32_t kPDelta = 4u;     // the record is a delta scatter (or an end)
+
+// One pass's grid (VCMTracer, PhotonMap): src and idx are of the pass's block of
+// light points.
+using VcmGrid = GridView;
 
 struct VcmTerms {
     float r;     // the pass's merging radius
@@ -486,7 +491,7 @@ __global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uin
     p.all = 1.0;
     p.color = mk(1.f, 1.f, 1.f);
     p.prob = 1.f;
-    p.flags = emissive(S, prev.contact) ? kPEmissive : 0u;
+    p.flags = (emissive(S, prev.contact) ? kPEmissive : 0u) | (is_delta(prev) ? kPDelta : 0u);
     p.pad = 0;
     P[0] = p;
     for (uint32_t i = 1; i < n; i++) {
@@ -512,77 +517,127 @@ __global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uin
         p.run = p.run * at * own_p;
         p.color = muls(mulv(p.color, prev.rad), cos_prev);
         p.prob *= prev.dp * prev.op;
-        p.flags = (p.flags & kPAny) | (connects ? kPAny : 0u) | (emissive(S, cur.contact) ? kPEmissive : 0u);
+        p.flags = (p.flags & kPAny) | (connects ? kPAny : 0u) | (emissive(S, cur.contact) ? kPEmissive : 0u) |
+                  (dc ? kPDelta : 0u);
         P[i] = p;
         prev = cur;
     }
 }
 
-// The connections of one lane (throughput of bidirPathTracer.cpp:53-140, and of
-// vcmTracer.cpp:88-173 with vt): every eye record with no light record, and with
-// every light record.  Returns what goes to the lane's own pixel at once.
-__device__ __forceinline__ f3 connect_all(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
-                                          uint32_t k, uint32_t p, const BVert* E, const BPrefix* PE, int max_eye,
-                                          const BVert* L, const BPrefix* PL, int max_light, float* pix,
-                                          const VisQueue& Q, LaneStack& st, const VcmTerms* vt) {
+// Index of the n-th set bit.
+__device__ __forceinline__ int nth_bit(uint64_t mask, uint32_t n) {
+    for (; n > 0; n--) mask &= mask - 1;
+    return __ffsll((unsigned long long)mask) - 1;
+}
+
+// The pairs of records that a wave's lanes connect, for connect_wave.
+struct PairTable {
+    uint64_t eye[64], light[64];  // per lane: the records that connect to something, a bit each
+    uint32_t upto[64];            // pairs of the lanes up to this one
+};
+
+// The connections of a wave's lanes (bidirPathTracer.cpp:53-140, and with grids
+// vcmTracer.cpp:88-173): every eye record with no light record, and with every
+// light record.  Sub-paths differ in length, and a lane that walked its own
+// pairs would keep its wave for the longest of 64 products (k_bdpt: 7.5 ms for
+// Cornell 256^2 x 8 passes); so each lane notes which of its records connect
+// at all (neither delta nor an emitter), and the wave deals its lanes' pairs
+// out one to each lane at a time (1.6 ms).  Every lane of the wave makes the
+// call; lane0: the wave's first lane; max_eye, max_light: 0 where there is
+// none.  Adds what needs no visibility test to the lane's own pixel.
+__device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
+                                           uint32_t maxv, uint64_t lane0, const BVert* verts, const BPrefix* prefix,
+                                           int max_eye, int max_light, float* pix_all, const VisQueue& Q,
+                                           LaneStack& st, const VcmGrid* grids, PairTable& T) {
+    static_assert(wr::kBdptMaxDepth + 3 <= 64, "a record per bit");
+    const uint32_t wl = threadIdx.x & 63u;
     f3 own = mk(0.f, 0.f, 0.f);
-    // light paths that start on no emitter (an empty light sample) connect to nothing
-    if (max_light > 0 && !(PL[0].flags & kPEmissive)) max_light = 0;
-    for (int e = 0; e < max_eye; e++) {
-        const BPrefix pe = PE[e];
-        const BVert ev = E[e];
-        f3 color;
-        float prob;
-        if (pe.flags & kPEmissive) {
-            // an emitter: the eye path alone, if no connection could have made it; no connections
-            if (e > 0 && !(pe.flags & kPAny)) {
-                const float w = eye_path_weight(E, PE, e, ev, color, prob, vt);
+    uint64_t eye = 0, light = 0;
+    {
+        const size_t ei = (lane0 + wl) * 2 * maxv, li = ei + maxv;
+        for (int e = 0; e < max_eye; e++) {
+            const uint32_t fl = prefix[ei + e].flags;
+            if (!(fl & kPEmissive)) {
+                if (!(fl & kPDelta)) eye |= 1ull << e;
+            } else if (e > 0 && !(fl & kPAny)) {
+                // an emitter: the eye path alone, if no connection could have made it
+                const VcmTerms vt{grids ? grids[(lane0 + wl) / npix].r : 0.f, (double)npix, false};
+                f3 color;
+                float prob;
+                const float w = eye_path_weight(verts + ei, prefix + ei, e, verts[ei + e], color, prob,
+                                                grids ? &vt : nullptr);
                 if (prob != 0.f && len(color) != 0.f) own = add(own, muls(divs(color, prob), w));
             }
-            continue;
         }
-        if (is_delta(ev)) continue;
-        for (int c = 0; c < max_light; c++) {
-            const BPrefix pl = PL[c];
-            if (c > 0 && (pl.flags & kPEmissive)) continue;
-            BVert lc = L[c], ec = ev;
-            if (!connect_edge(S, L, c, E, e, lc, ec)) continue;
-            const float w = color_prob_weight(S, cam, p, lc, pl, c, ec, pe, e, color, prob, vt);
-            if (prob == 0.f) continue;
-            if (len(color) == 0.f) continue;
-            f3 contrib = muls(divs(color, prob), w);
-            uint32_t target = p;
-            if (e == 0) {  // light tracing: splat to the pixel the camera sees the point in
-                const f3 v = sub(lc.o, cam.pos);
-                const float vfd = dot(v, cam.front);
-                const float scale = cam.dist / vfd;
-                const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
-                const float ry = (float)(cam.H / 2.0 - (double)(dot(v, cam.top) * scale));
-                const int x = (int)rx, y = (int)ry;  // checkPixelBound truncates (camera.cpp:164-170)
-                if (!(x >= 0 && y >= 0 && x < (int)cam.W && y < (int)cam.H)) continue;
-                target = (uint32_t)(y * (int)cam.W + x);
-                const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
-                contrib = muls(contrib, factor / (float)npix);
+        // light paths that start on no emitter (an empty light sample) connect to nothing
+        if (max_light > 0 && eye != 0 && (prefix[li].flags & kPEmissive)) {
+            for (int c = 0; c < max_light; c++) {
+                const uint32_t fl = prefix[li + c].flags;
+                if (!(fl & kPDelta) && (c == 0 || !(fl & kPEmissive))) light |= 1ull << c;
             }
-            // MCRenderer::visibilityTest from the eye-side connection record
-            const uint32_t contact = (ec.flags & kVCamera) ? kCameraObj : ec.contact;
-            const float dist = len(sub(ec.o, lc.o));
-            const uint32_t slot = wave_slot(Q.count);
-            if (slot < Q.cap) {
-                uint32_t* r = Q.rays + 8 * (size_t)slot;
-                r[0] = __float_as_uint(ec.o.x); r[1] = __float_as_uint(ec.o.y); r[2] = __float_as_uint(ec.o.z);
-                r[3] = __float_as_uint(ec.d.x); r[4] = __float_as_uint(ec.d.y); r[5] = __float_as_uint(ec.d.z);
-                r[6] = ec.inside;
-                r[7] = contact;
-                float* y = Q.pay + 4 * (size_t)slot;
-                y[0] = contrib.x; y[1] = contrib.y; y[2] = contrib.z; y[3] = dist;
-                Q.dst[slot] = k * npix + target;
-            } else {  // queue full: trace here
-                const PHit h = trace_scene<true>(sc, ec.o, ec.d, ec.inside, contact, st);
-                if (!nee_visible(h.rec, h.t, dist)) continue;
-                if (target == p) own = add(own, contrib);
-                else atomic_add3(pix, target, contrib);
-            }
+        }
+    }
+    uint32_t upto = (uint32_t)(__popcll(eye) * __popcll(light));
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t t = __shfl_up(upto, off, 64);
+        if (wl >= (uint32_t)off) upto += t;
+    }
+    T.eye[wl] = eye;
+    T.light[wl] = light;
+    T.upto[wl] = upto;
+    __builtin_amdgcn_wave_barrier();  // the table is this wave's own: LDS operations of a wave stay in order
+    const uint32_t total = __shfl(upto, 63, 64);
+    for (uint32_t t = wl; t < total; t += 64) {
+        uint32_t o = 0;  // the first lane with upto > t
+#pragma unroll
+        for (uint32_t step = 32; step > 0; step >>= 1)
+            if (T.upto[o + step - 1] <= t) o += step;
+        const uint32_t r = o ? t - T.upto[o - 1] : t;
+        const uint64_t lights = T.light[o];
+        const uint32_t nl = (uint32_t)__popcll(lights);
+        const int e = nth_bit(T.eye[o], r / nl), c = nth_bit(lights, r % nl);
+        const uint64_t lane = lane0 + o;
+        const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
+        const size_t ei = lane * 2 * maxv, li = ei + maxv;
+        BVert lc = verts[li + c], ec = verts[ei + e];
+        if (!connect_edge(S, verts + li, c, verts + ei, e, lc, ec)) continue;
+        const VcmTerms vt{grids ? grids[k].r : 0.f, (double)npix, false};
+        f3 color;
+        float prob;
+        const float w = color_prob_weight(S, cam, p, lc, prefix[li + c], c, ec, prefix[ei + e], e, color, prob,
+                                          grids ? &vt : nullptr);
+        if (prob == 0.f) continue;
+        if (len(color) == 0.f) continue;
+        f3 contrib = muls(divs(color, prob), w);
+        uint32_t target = p;
+        if (e == 0) {  // light tracing: splat to the pixel the camera sees the point in
+            const f3 v = sub(lc.o, cam.pos);
+            const float vfd = dot(v, cam.front);
+            const float scale = cam.dist / vfd;
+            const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
+            const float ry = (float)(cam.H / 2.0 - (double)(dot(v, cam.top) * scale));
+            const int x = (int)rx, y = (int)ry;  // checkPixelBound truncates (camera.cpp:164-170)
+            if (!(x >= 0 && y >= 0 && x < (int)cam.W && y < (int)cam.H)) continue;
+            target = (uint32_t)(y * (int)cam.W + x);
+            const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
+            contrib = muls(contrib, factor / (float)npix);
+        }
+        // MCRenderer::visibilityTest from the eye-side connection record
+        const uint32_t contact = (ec.flags & kVCamera) ? kCameraObj : ec.contact;
+        const float dist = len(sub(ec.o, lc.o));
+        const uint32_t slot = wave_slot(Q.count);
+        if (slot < Q.cap) {
+            uint32_t* ray = Q.rays + 8 * (size_t)slot;
+            ray[0] = __float_as_uint(ec.o.x); ray[1] = __float_as_uint(ec.o.y); ray[2] = __float_as_uint(ec.o.z);
+            ray[3] = __float_as_uint(ec.d.x); ray[4] = __float_as_uint(ec.d.y); ray[5] = __float_as_uint(ec.d.z);
+            ray[6] = ec.inside;
+            ray[7] = contact;
+            float* y = Q.pay + 4 * (size_t)slot;
+            y[0] = contrib.x; y[1] = contrib.y; y[2] = contrib.z; y[3] = dist;
+            Q.dst[slot] = k * npix + target;
+        } else {  // queue full: trace here
+            const PHit h = trace_scene<true>(sc, ec.o, ec.d, ec.inside, contact, st);
+            if (nee_visible(h.rec, h.t, dist)) atomic_add3(pix_all + 3 * (size_t)k * npix, target, contrib);
         }
     }
     return own;
@@ -591,29 +646,47 @@ __device__ __forceinline__ f3 connect_all(const SceneDev& S, const SceneCtx& sc,
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt(
     SceneDev S, CamDev cam, uint32_t npass, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* prefix,
     const uint32_t* counts, float* pix_all, VisQueue Q) {
+    __shared__ PairTable tables[4];
     const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (lane >= (uint64_t)npass * npix) return;
-    const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
-    float* pix = pix_all + 3 * (size_t)k * npix;
+    const bool valid = lane < (uint64_t)npass * npix;
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
-    const size_t ei = lane * 2 * maxv, li = ei + maxv;
-    const uint32_t ne = counts[2 * lane], nl = counts[2 * lane + 1];
-    atomic_add3(pix, p, connect_all(S, sc, cam, npix, k, p, verts + ei, prefix + ei, (int)min(ne, maxv), verts + li,
-                                    prefix + li, (int)min(nl, maxv), pix, Q, st, nullptr));
+    const uint32_t ne = valid ? counts[2 * lane] : 0u, nl = valid ? counts[2 * lane + 1] : 0u;
+    const f3 own = connect_wave(S, sc, cam, npix, maxv, lane & ~63ull, verts, prefix, (int)min(ne, maxv),
+                                (int)min(nl, maxv), pix_all, Q, st, nullptr, tables[threadIdx.x >> 6]);
+    if (valid) atomic_add3(pix_all + 3 * (size_t)(lane / npix) * npix, (uint32_t)(lane % npix), own);
 }
 
 // The queued visibility tests, answered by the batch NoSelf query (hits:
 // prim WR_NONE on a miss, t): visible connections add their contribution.
+// Connections of one pixel follow each other in the queue (connect_wave deals
+// them out in that order), so a wave first sums every run of entries with one
+// target and adds a run with one set of atomics (5.9M entries: 936 us with one
+// set per entry, 96 us).
 __global__ __launch_bounds__(256) void k_bdpt_accum(uint32_t n, const float* pay, const uint32_t* dst,
                                                     const uint4* hits, float* pix_all) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const uint4 h = hits[i];
-    const float* y = pay + 4 * (size_t)i;
-    if (!nee_visible(h.x == WR_NONE ? WR_NONE : 0u, __uint_as_float(h.y), y[3])) return;
-    atomic_add3(pix_all, dst[i], mk(y[0], y[1], y[2]));
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t to = WR_NONE;
+    f3 v = mk(0.f, 0.f, 0.f);
+    if (i < n) {
+        const uint4 h = hits[i];
+        const float* y = pay + 4 * (size_t)i;
+        if (nee_visible(h.x == WR_NONE ? WR_NONE : 0u, __uint_as_float(h.y), y[3])) v = mk(y[0], y[1], y[2]);
+        to = dst[i];
+    }
+    const uint32_t prev = __shfl_up(to, 1);
+    const uint64_t heads = __ballot(lane == 0 || to != prev);
+    // the lanes of this run that follow: up to the next head
+    const uint64_t later = heads & ~((2ull << lane) - 1ull);
+    const uint32_t end = later ? (uint32_t)__ffsll((unsigned long long)later) - 1 : 64u;
+#pragma unroll
+    for (uint32_t off = 1; off < 64; off <<= 1) {
+        const f3 o = mk(__shfl_down(v.x, off), __shfl_down(v.y, off), __shfl_down(v.z, off));
+        if (lane + off < end) v = add(v, o);
+    }
+    if (i < n && ((heads >> lane) & 1) && (v.x != 0.f || v.y != 0.f || v.z != 0.f)) atomic_add3(pix_all, to, v);
 }
 
 // Each pass's pixel values, in pass order: isLegalColor, fixVignetting, the Kahan film.
@@ -699,9 +772,6 @@ __global__ void k_vcm_pass_starts(const uint32_t* offs, uint32_t npix, uint32_t 
     if (b <= npass) starts[b] = offs[(size_t)b * npix];
 }
 
-// One pass's grid: src and idx are of the pass's block of points.
-using VcmGrid = GridView;
-
 // The merges of the VCM lanes, one entry per light point in reach of an eye
 // vertex: word 0 = lane | eye vertex << 24 (lanes < 2^22), word 1 = the light
 // point; count at ent[2 * cap].  A separate kernel takes one merge per lane, so
@@ -745,14 +815,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
-    const size_t ei = lane * 2 * maxv, li = ei + maxv;
-    const BVert* E = verts + ei;
+    const BVert* E = verts + lane * 2 * maxv;
     const uint32_t ne = counts[2 * lane], nl = counts[2 * lane + 1];
     const int max_eye = (int)(ne < maxv ? ne : maxv), max_light = (int)(nl < maxv ? nl : maxv);
-    const VcmTerms vc{G.r, (double)npix, false};
     // throughputByConnecting (vcmTracer.cpp:88-173): k_bdpt's connections with vcmMisWeight
-    f3 own = connect_all(S, sc, cam, npix, kb, p, E, prefix + ei, valid ? max_eye : 0, verts + li, prefix + li,
-                         max_light, pix, Q, st, &vc);
+    __shared__ PairTable tables[4];
+    f3 own = connect_wave(S, sc, cam, npix, maxv, lane_id & ~63ull, verts, prefix, valid ? max_eye : 0,
+                          valid ? max_light : 0, pix_all, Q, st, grids, tables[threadIdx.x >> 6]);
     // throughputByMerging (vcmTracer.cpp:175-217): the light points within the
     // radius of every non-delta eye vertex before an emitter, in the grid's
     // order (HashGrid::Process); the default points have no path and give
