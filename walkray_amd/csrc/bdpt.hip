@@ -36,6 +36,7 @@
 
 #include "grid_dev.h"
 #include "pt_dev.h"
+#include "walk_dev.h"
 #include "wr_pt.h"
 
 #pragma clang fp contract(off)
@@ -53,11 +54,6 @@ struct BVert {
     uint32_t inside, contact, flags, pad;
 };
 
-__device__ __forceinline__ void put(BVert* V, uint32_t& nv, uint32_t maxv, const BVert& v) {
-    if (nv < maxv) V[nv] = v;
-    nv++;
-}
-
 // terminateRay (mcRenderer.cpp:20-27) after a ray from o.
 __device__ __forceinline__ BVert terminate_at(f3 o) {
     BVert t;
@@ -72,53 +68,6 @@ __device__ __forceinline__ BVert terminate_at(f3 o) {
     t.flags = kVDelta;
     t.pad = 0;
     return t;
-}
-
-// samplePath from v0 (already traced: hit) with vertex counters vbase + depth + 1.
-__device__ void walk(const SceneCtx& sc, const BVert& v0, PHit hit, uint32_t max_depth, uint64_t seed, uint32_t p,
-                     uint32_t pass, uint32_t vbase, BVert* V, uint32_t& nv, uint32_t maxv, LaneStack& st) {
-    put(V, nv, maxv, v0);
-    f3 o = v0.o, d = v0.d;
-    uint32_t inside = v0.inside;
-    for (uint32_t depth = 0;; depth++) {
-        const uint32_t self = inside != WR_NONE ? inside : hit.obj;
-        if (self == WR_NONE || hit.rec == WR_NONE) {
-            put(V, nv, maxv, terminate_at(o));
-            return;
-        }
-        float rn[4];
-        rng4(seed, p, pass, vbase + depth + 1, rn);
-        const Out r = scatter(sc, self, o, d, hit, inside, rn, st);
-        BVert nx;
-        nx.o = r.o;
-        nx.d = r.d;
-        nx.rad = r.rad;
-        nx.n = r.n;
-        nx.op = r.op;
-        nx.dp = r.dp;
-        nx.inside = r.inside;
-        nx.contact = r.contact;
-        nx.flags = r.delta ? kVDelta : 0u;
-        nx.pad = 0;
-        if ((double)len(r.d) < 0.5) {
-            put(V, nv, maxv, nx);
-            return;
-        }
-        if (depth + 1 > max_depth) {
-            put(V, nv, maxv, terminate_at(o));
-            return;
-        }
-        const PHit nh = trace_scene<true>(sc, r.o, r.d, r.inside, r.contact, st);
-        put(V, nv, maxv, nx);
-        if (nh.rec == WR_NONE) {
-            put(V, nv, maxv, terminate_at(o));
-            return;
-        }
-        o = r.o;
-        d = r.d;
-        inside = r.inside;
-        hit = nh;
-    }
 }
 
 // Camera::getPixelSolidAngle (camera.cpp:124-131).
@@ -391,84 +340,127 @@ __device__ __forceinline__ void atomic_add3(float* buf, uint32_t p, f3 v) {
     atomicAdd(buf + 3 * p + 2, v.z);
 }
 
-// The two sub-paths of one pixel and pass (kept apart from the connections:
-// this half traverses at a register count that lets several waves share a
-// SIMD); counts[2 * lane] = eye records, counts[2 * lane + 1] = light records.
-// 4 waves per SIMD (128 VGPRs, the rest spilled) for both kernels: 80 -> 43 ms on the
-// Cornell box against the unconstrained 264 / 190 registers.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt_subpaths(SceneDev S, CamDev cam, uint32_t max_depth, uint64_t seed,
-                                                       uint32_t pass0, uint32_t npass, uint32_t npix, uint32_t maxv,
-                                                       BVert* verts, uint32_t* counts, bool eye = true) {
-    const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (lane >= (uint64_t)npass * npix) return;
-    const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
-    const uint32_t pass = pass0 + k;
-    StackSpill spill;
-    LaneStack st(&spill);
-    const SceneCtx sc = make_scene_ctx(S);
-    BVert* E = verts + lane * 2 * maxv;
-    BVert* L = E + maxv;
-    uint32_t ne = 0, nl = 0;
-    float rn[4];
-    // eye sub-path: the camera ray (camera.cpp:6-60) then samplePath (PhotonMap forms its own)
-    if (eye) {
-        rng4(seed, p, pass, 0, rn);
-        BVert c;
-        c.o = cam.pos;
-        c.d = cam_dir(cam, p, rn[0], rn[1]);
-        c.rad = mk(1.f, 1.f, 1.f);
-        c.n = cam.front;
-        c.op = 1.f;
-        c.dp = 1.f;
-        c.contact = WR_NONE;
-        c.flags = kVCamera;
-        c.pad = 0;
-        const PHit h = trace_scene<false>(sc, c.o, c.d, WR_NONE, WR_NONE, st);
-        c.inside = find_inside(S, c.o, c.d, WR_NONE, st);
-        walk(sc, c, h, max_depth, seed, p, pass, 0u, E, ne, maxv, st);
+// The sub-paths of every lane (pixel and pass) as a path walk: paths [0, eyes)
+// are the eye sub-paths of the lanes in order, the others their light
+// sub-paths (eyes = 0: PhotonMap forms its own).  counts[2 * lane] = eye
+// records, counts[2 * lane + 1] = light records.  Record k + 1 is written by
+// step k; max_depth + 3 records hold the longest sub-path: its first ray,
+// max_depth scatters, the end.
+struct SubpathWalk {
+    CamDev cam;
+    uint32_t max_depth, pass0, npix, maxv, eyes;
+    uint64_t seed;
+    BVert* verts;
+    uint32_t* counts;
+
+    __device__ __forceinline__ void split(uint32_t path, bool& eye, uint32_t& lane, uint32_t& p, uint32_t& pass,
+                                          BVert*& V) const {
+        eye = path < eyes;
+        lane = eye ? path : path - eyes;
+        p = lane % npix;
+        pass = pass0 + lane / npix;
+        V = verts + ((size_t)lane * 2 + (eye ? 0 : 1)) * maxv;
     }
-    // light sub-path (as k_light_paths)
-    {
-        rng4(seed, p, pass, kBdptLightVertex, rn);
-        const LightSample ls = sample_light(sc, rn);
+
+    __device__ __forceinline__ bool begin(const SceneCtx& sc, uint32_t path, LaneStack& st, f3& o, f3& d,
+                                          uint32_t& inside, uint32_t& contact) const {
+        bool eye;
+        uint32_t lane, p, pass;
+        BVert* V;
+        split(path, eye, lane, p, pass, V);
+        float rn[4];
         BVert r;
-        r.o = mk(0.f, 0.f, 0.f);
-        r.d = r.o;
-        r.rad = r.o;
-        r.n = r.o;
         r.op = 1.f;
         r.dp = 1.f;
         r.inside = WR_NONE;
         r.contact = WR_NONE;
-        r.flags = 0;
         r.pad = 0;
-        PHit hit;
-        hit.t = -1.f;
-        hit.rec = WR_NONE;
-        hit.obj = WR_NONE;
-        if (ls.ok) {
-            rng4(seed, p, pass, kBdptLightVertex + 1, rn);
-            const float term1 = (float)(2.0 * kPi * (double)rn[0]);  // uniformSphereSampler.h:6-20
-            const float term2 = 2.f * sqrtf(rn[1] - rn[1] * rn[1]);
-            f3 d = mk(cosf(term1) * term2, 1.f - 2.f * rn[1], sinf(term1) * term2);
-            r.dp = (float)(kInvPi * 0.25f);
-            if (dot(d, ls.n) < 0.f) d = mk(-d.x, -d.y, -d.z);
-            r.o = ls.o;
-            r.n = ls.n;
-            r.d = d;
-            r.rad = ls.rad;
-            r.contact = ls.obj;
-            r.inside = find_inside(S, r.o, r.d, ls.obj, st);
-            r.dp *= 2.f;
-            r.op = ls.op;
-            const PHit h = trace_scene<true>(sc, r.o, r.d, r.inside, r.contact, st);
-            if (h.rec != WR_NONE && h.t > 0.f) hit = h;
+        bool go = true;
+        inside = contact = WR_NONE;
+        if (eye) {  // the camera ray (camera.cpp:6-60), traced without a condition
+            rng4(seed, p, pass, 0, rn);
+            r.o = cam.pos;
+            r.d = cam_dir(cam, p, rn[0], rn[1]);
+            r.rad = mk(1.f, 1.f, 1.f);
+            r.n = cam.front;
+            r.flags = kVCamera;
+            r.inside = find_inside(sc.S, r.o, r.d, WR_NONE, st);
+        } else {  // the light ray (as k_light_paths' first)
+            rng4(seed, p, pass, kBdptLightVertex, rn);
+            const LightSample ls = sample_light(sc, rn);
+            r.o = mk(0.f, 0.f, 0.f);
+            r.d = r.o;
+            r.rad = r.o;
+            r.n = r.o;
+            r.flags = 0;
+            go = ls.ok;
+            if (ls.ok) {
+                rng4(seed, p, pass, kBdptLightVertex + 1, rn);
+                const float term1 = (float)(2.0 * kPi * (double)rn[0]);  // uniformSphereSampler.h:6-20
+                const float term2 = 2.f * sqrtf(rn[1] - rn[1] * rn[1]);
+                f3 dir = mk(cosf(term1) * term2, 1.f - 2.f * rn[1], sinf(term1) * term2);
+                r.dp = (float)(kInvPi * 0.25f);
+                if (dot(dir, ls.n) < 0.f) dir = mk(-dir.x, -dir.y, -dir.z);
+                r.o = ls.o;
+                r.n = ls.n;
+                r.d = dir;
+                r.rad = ls.rad;
+                r.contact = ls.obj;
+                r.inside = find_inside(sc.S, r.o, r.d, ls.obj, st);
+                r.dp *= 2.f;
+                r.op = ls.op;
+                inside = r.inside;
+                contact = r.contact;
+            }
         }
-        walk(sc, r, hit, max_depth, seed, p, pass, kBdptLightVertex + 1, L, nl, maxv, st);
+        V[0] = r;
+        if (!go) {  // an empty light sample: its ray hits nothing
+            V[1] = terminate_at(r.o);
+            counts[2 * lane + 1] = 2;
+        }
+        o = r.o;
+        d = r.d;
+        return go;
     }
-    counts[2 * lane] = ne;
-    counts[2 * lane + 1] = nl;
-}
+
+    __device__ __forceinline__ bool step(const SceneCtx& sc, uint32_t path, uint32_t s, f3 o, f3 d, const PHit& hit,
+                                         LaneStack& st, Out& out) const {
+        bool eye;
+        uint32_t lane, p, pass;
+        BVert* V;
+        split(path, eye, lane, p, pass, V);
+        uint32_t* count = counts + 2 * lane + (eye ? 0 : 1);
+        *count = s + 2;  // of a path that ends here; a later step overwrites it
+        // an escaped ray ends the path at the origin before its own; a light
+        // ray's hit counts only at dist > 0 (abstractObj.cpp:46)
+        if (hit.rec == WR_NONE || (!eye && s == 0 && !(hit.t > 0.f))) {
+            V[s + 1] = terminate_at(s == 0 ? o : V[s - 1].o);
+            return false;
+        }
+        const uint32_t inside = V[s].inside;
+        float rn[4];
+        rng4(seed, p, pass, (eye ? 0u : kBdptLightVertex + 1) + s + 1, rn);
+        out = scatter(sc, inside != WR_NONE ? inside : hit.obj, o, d, hit, inside, rn, st);
+        const bool absorbed = (double)len(out.d) < 0.5;
+        if (!absorbed && s + 1 > max_depth) {
+            V[s + 1] = terminate_at(o);
+            return false;
+        }
+        BVert nx;
+        nx.o = out.o;
+        nx.d = out.d;
+        nx.rad = out.rad;
+        nx.n = out.n;
+        nx.op = out.op;
+        nx.dp = out.dp;
+        nx.inside = out.inside;
+        nx.contact = out.contact;
+        nx.flags = out.delta ? kVDelta : 0u;
+        nx.pad = 0;
+        V[s + 1] = nx;
+        return !absorbed;
+    }
+};
 
 // The prefixes of every sub-path (BPrefix), one lane per sub-path: side 0 the
 // light sub-path, side 1 the eye sub-path of each lane of k_bdpt_subpaths.
@@ -912,7 +904,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
 // ---- PhotonMap (photonMap.cpp:21-680), progressive photon mapping ----------
 // The light points and per-pass grids of VCMTracer (the same light paths);
-// k_ppm, one lane per pixel and pass: the eye "merge path" (samplePath with
+// the eye "merge path" of every pixel and pass (PpmWalk: samplePath with
 // maxPathLen MERGE_LEN = 10, photonMap.cpp:10,150-190) up to its first
 // emitter (its emitted radiance) or first non-specular, i.e. diffuse, vertex
 // (the kernel density estimate of the photons around it, photonMap.cpp:
@@ -925,7 +917,7 @@ constexpr uint32_t kMergeLen = 10;
 // directionProb / originProb * cosine of the records before it), kept in the
 // radiance of the eye-side record of the same index, which PhotonMap has no
 // other use for: a photon in reach costs one record instead of its whole path
-// (k_ppm 2.99 -> 2.35 ms for Cornell 256^2 x 8 passes, and 0.11 here).
+// (Cornell 256^2 x 8 passes: 0.6 ms less in the estimates, 0.11 here).
 __global__ __launch_bounds__(256) void k_ppm_throughput(uint32_t lanes, uint32_t maxv, BVert* verts,
                                                         const uint32_t* counts) {
     const uint32_t lane = blockIdx.x * 256 + threadIdx.x;
@@ -983,70 +975,88 @@ __device__ f3 ppm_density(const SceneDev& S, const VcmGrid& G, const BVert* vert
     return contrib;
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_ppm(SceneDev S, CamDev cam, uint32_t npix, uint32_t npass, uint32_t maxv,
-                                             const BVert* verts, uint64_t seed, uint32_t pass0, float* pix_all,
-                                             const VcmGrid* grids) {
-    const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (lane >= (uint64_t)npass * npix) return;
-    const uint32_t kb = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
-    const uint32_t pass = pass0 + kb;
-    const VcmGrid G = grids[kb];
-    StackSpill spill;
-    LaneStack st(&spill);
-    const SceneCtx sc = make_scene_ctx(S);
-    float rn[4];
-    rng4(seed, p, pass, 0, rn);
-    BVert c;
-    c.o = cam.pos;
-    c.d = cam_dir(cam, p, rn[0], rn[1]);
-    c.rad = mk(1.f, 1.f, 1.f);
-    c.n = cam.front;
-    c.op = 1.f;
-    c.dp = 1.f;
-    c.contact = WR_NONE;
-    c.flags = kVCamera;
-    c.pad = 0;
-    PHit hit = trace_scene<false>(sc, c.o, c.d, WR_NONE, WR_NONE, st);
-    c.inside = find_inside(S, c.o, c.d, WR_NONE, st);
-    f3 surface = mk(0.f, 0.f, 0.f);
-    f3 o = c.o, d = c.d;
-    uint32_t inside = c.inside;
-    for (uint32_t depth = 0;; depth++) {
-        const uint32_t self = inside != WR_NONE ? inside : hit.obj;
-        if (self == WR_NONE || hit.rec == WR_NONE) break;  // the terminating record: no contact
-        rng4(seed, p, pass, depth + 1, rn);
-        const Out r = scatter(sc, self, o, d, hit, inside, rn, st);
-        const bool absorbed = (double)len(r.d) < 0.5;
-        if (!absorbed && depth + 1 > kMergeLen) break;  // the terminating record
-        if (emissive(S, r.contact)) {  // the eye path hit a light
-            surface = r.rad;
-            break;
-        }
-        if (r.contact != WR_NONE && S.objs[r.contact].mat == WR_MAT_DIFFUSE) {  // nonSpecular()
-            BVert out;
-            out.o = r.o;
-            out.d = mk(-d.x, -d.y, -d.z);
-            out.rad = r.rad;
-            out.n = r.n;
-            out.op = r.op;
-            out.dp = r.dp;
-            out.inside = r.inside;
-            out.contact = r.contact;
-            out.flags = 0;
-            out.pad = 0;
-            surface = ppm_density(S, G, verts, maxv, npix, out);
-            break;
-        }
-        if (absorbed) break;
-        const PHit nh = trace_scene<true>(sc, r.o, r.d, r.inside, r.contact, st);
-        if (nh.rec == WR_NONE) break;
-        o = r.o;
-        d = r.d;
-        inside = r.inside;
-        hit = nh;
+// The eye merge paths as a path walk, one per pixel and pass.  What the walk
+// keeps of a path lies in its first two eye-side records, of which PhotonMap
+// otherwise uses the radiance only (k_ppm_throughput): record 0 the path's
+// inside object, then kPpmDensity or 0 in flags and the light it found in n;
+// record 1 the vertex whose density k_ppm_density estimates.  (With the
+// estimate inside the walk's steps, the lanes of a step waited for the
+// longest list of photons in a kernel of 128 registers: 2.3 ms for 256^2 x 8
+// passes; 0.36 and 0.47 ms apart.)
+constexpr uint32_t kPpmDensity = 1u;
+struct PpmWalk {
+    CamDev cam;
+    uint32_t pass0, npix, maxv;
+    uint64_t seed;
+    BVert* verts;
+
+    __device__ __forceinline__ bool begin(const SceneCtx& sc, uint32_t lane, LaneStack& st, f3& o, f3& d,
+                                          uint32_t& inside, uint32_t& contact) const {
+        float rn[4];
+        rng4(seed, lane % npix, pass0 + lane / npix, 0, rn);
+        o = cam.pos;
+        d = cam_dir(cam, lane % npix, rn[0], rn[1]);
+        BVert* first = verts + (size_t)lane * 2 * maxv;
+        first->inside = find_inside(sc.S, o, d, WR_NONE, st);
+        first->n = mk(0.f, 0.f, 0.f);
+        first->flags = 0;
+        inside = contact = WR_NONE;  // traced without a condition
+        return true;
     }
-    const f3 color = mulv(mulv(mk(1.f, 1.f, 1.f), surface), divs(divs(muls(c.rad, cos_term_v(c)), c.dp), c.op));
-    float* px = pix_all + 3 * lane;
+
+    __device__ __forceinline__ bool step(const SceneCtx& sc, uint32_t lane, uint32_t s, f3 o, f3 d, const PHit& hit,
+                                         LaneStack& st, Out& out) const {
+        if (hit.rec == WR_NONE) return false;
+        BVert* first = verts + (size_t)lane * 2 * maxv;
+        const uint32_t inside = first->inside;
+        float rn[4];
+        rng4(seed, lane % npix, pass0 + lane / npix, s + 1, rn);
+        out = scatter(sc, inside != WR_NONE ? inside : hit.obj, o, d, hit, inside, rn, st);
+        first->inside = out.inside;
+        const bool absorbed = (double)len(out.d) < 0.5;
+        if (!absorbed && s + 1 > kMergeLen) return false;  // the terminating record
+        if (emissive(sc.S, out.contact)) {                 // the eye path hit a light
+            first->n = out.rad;
+            return false;
+        }
+        if (out.contact != WR_NONE && sc.S.objs[out.contact].mat == WR_MAT_DIFFUSE) {  // nonSpecular()
+            first->flags = kPpmDensity;
+            BVert* v = first + 1;
+            v->o = out.o;
+            v->d = mk(-d.x, -d.y, -d.z);
+            v->n = out.n;
+            v->inside = out.inside;
+            v->contact = out.contact;
+            return false;
+        }
+        return !absorbed;
+    }
+};
+
+// Each pixel's value: the camera vertex's factor times what its path found.
+__global__ __launch_bounds__(256) void k_ppm_density(SceneDev S, CamDev cam, uint32_t npix, uint32_t lanes,
+                                                     uint32_t maxv, const BVert* verts, uint64_t seed, uint32_t pass0,
+                                                     float* pix_all, const VcmGrid* grids) {
+    const uint32_t lane = blockIdx.x * 256 + threadIdx.x;
+    if (lane >= lanes) return;
+    const uint32_t kb = lane / npix, p = lane % npix;
+    const BVert* first = verts + (size_t)lane * 2 * maxv;
+    f3 surface = first->n;
+    if (first->flags & kPpmDensity) {
+        BVert v = first[1];
+        v.flags = 0;
+        surface = ppm_density(S, grids[kb], verts, maxv, npix, v);
+    }
+    float rn[4];
+    rng4(seed, p, pass0 + kb, 0, rn);
+    BVert c;
+    c.d = cam_dir(cam, p, rn[0], rn[1]);
+    c.n = cam.front;
+    c.flags = kVCamera;
+    c.contact = WR_NONE;
+    const f3 color = mulv(mulv(mk(1.f, 1.f, 1.f), surface),
+                          divs(divs(muls(mk(1.f, 1.f, 1.f), cos_term_v(c)), 1.f), 1.f));
+    float* px = pix_all + 3 * (size_t)lane;
     px[0] = color.x;
     px[1] = color.y;
     px[2] = color.z;
@@ -1077,12 +1087,20 @@ static wrd::CamDev make_cam_dev(const CamHost& ch) {
     return cam;
 }
 
+// The light sub-paths of `lanes` lanes, and their eye sub-paths when eye.
+static hipError_t run_subpaths(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const wrd::CamDev& cam,
+                               uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t lanes, uint32_t npix,
+                               uint32_t maxv, wrd::BVert* V, uint32_t* counts, bool eye) {
+    const wrd::SubpathWalk P{cam, max_depth, pass0, npix, maxv, eye ? lanes : 0u, seed, V, counts};
+    return run_walk(ctx, S, H, P, eye ? 2 * lanes : lanes, max_depth + 1);
+}
+
 // The light sub-paths of passes [pass0, pass0 + npass) (and their eye sub-paths
 // when eye), their light points and one grid per pass, described in vb.grids;
 // the grids' buffers come from mem.  vb.err is set on the device if a pass's
 // points spread over too many cells.
-static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const wrd::CamDev& cam, uint32_t npix,
-                             uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius,
+static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const wr_tree_hdr& H,
+                             const wrd::CamDev& cam, uint32_t npix, uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius,
                              uint32_t maxv, wrd::BVert* V, uint32_t* counts, const VcmBufs& vb, bool eye,
                              const char* who) {
     hipStream_t st = ctx->stream;
@@ -1091,8 +1109,8 @@ static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const
     hipError_t e = hipMemsetAsync(vb.pc + lanes, 0, sizeof(uint32_t), st);
     if (e == hipSuccess) e = hipMemsetAsync(vb.err, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, who);
-    wrd::k_bdpt_subpaths<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, max_depth, seed, pass0, npass, npix, maxv, V,
-                                                                  counts, eye);
+    if ((e = run_subpaths(ctx, S, H, cam, max_depth, seed, pass0, lanes, npix, maxv, V, counts, eye)) != hipSuccess)
+        return hip_fail(ctx, e, who);
     wrd::k_vcm_point_count<<<blocks, 256, 0, st>>>(S, V, counts, lanes, maxv, vb.pc);
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail(ctx, e, who);
     size_t tb = vb.scan_bytes;
@@ -1141,7 +1159,7 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     if (e == hipSuccess) e = hipMemsetAsync(q.count, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     Scratch mem(*ctx->pool);  // the grids'
-    int rc = light_point_grids(ctx, mem, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, q.counts,
+    int rc = light_point_grids(ctx, mem, S, H, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, q.counts,
                                vb, true, "wr_render_vcm");
     if (rc != WR_OK) return rc;
     wrd::BPrefix* prefix = (wrd::BPrefix*)q.prefix;
@@ -1175,7 +1193,7 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     return WR_OK;
 }
 
-int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const CamHost& ch, uint32_t max_depth, uint64_t seed,
+int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth, uint64_t seed,
                       uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts, uint32_t* counts,
                       float* pix, const VcmBufs& vb, const FilmBufs& film) {
     hipStream_t st = ctx->stream;
@@ -1185,16 +1203,19 @@ int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const CamHost& ch, uint32_
     const uint32_t blocks = (lanes + 255) / 256;
     wrd::BVert* V = (wrd::BVert*)verts;
     Scratch mem(*ctx->pool);  // the grids'
-    int rc = light_point_grids(ctx, mem, S, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts, vb,
+    int rc = light_point_grids(ctx, mem, S, H, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts, vb,
                                false, "wr_render_ppm");
     if (rc != WR_OK) return rc;
     wrd::k_ppm_throughput<<<blocks, 256, 0, st>>>(lanes, maxv, V, counts);
-    wrd::k_ppm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, seed, pass0, pix,
-                                                        (const wrd::VcmGrid*)vb.grids);
+    const wrd::PpmWalk P{cam, pass0, npix, maxv, seed, V};
+    hipError_t e = run_walk(ctx, S, H, P, lanes, wrd::kMergeLen + 1);
+    if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_ppm");
+    wrd::k_ppm_density<<<blocks, 256, 0, st>>>(S, cam, npix, lanes, maxv, V, seed, pass0, pix,
+                                               (const wrd::VcmGrid*)vb.grids);
     wrd::k_bdpt_fold<<<(npix + 255) / 256, 256, 0, st>>>(cam, npass, npix, pix,
                                                          wrd::FilmDev{film.sum, film.comp, film.sumsq});
     uint32_t grid_err = 0;
-    hipError_t e = hipGetLastError();
+    e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&grid_err, vb.err, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_ppm");
@@ -1209,9 +1230,10 @@ size_t vcm_scan_bytes(uint32_t lanes) {
     return tb;
 }
 
-hipError_t launch_bdpt_passes(const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
+hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
                               uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
-                              const BdptQueue& q, const FilmBufs& film, hipStream_t st) {
+                              const BdptQueue& q, const FilmBufs& film) {
+    hipStream_t st = ctx->stream;
     const wrd::CamDev cam = make_cam_dev(ch);
     const uint32_t npix = ch.W * ch.H;
     const uint64_t lanes = (uint64_t)npass * npix;
@@ -1220,8 +1242,9 @@ hipError_t launch_bdpt_passes(const SceneDev& S, const wr_tree_hdr& H, const Cam
     if (e != hipSuccess) return e;
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
     const uint32_t blocks = (uint32_t)((lanes + 255) / 256);
-    wrd::k_bdpt_subpaths<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, max_depth, seed, pass0, npass, npix, maxv,
-                                                                  (wrd::BVert*)verts, q.counts);
+    e = run_subpaths(ctx, S, H, cam, max_depth, seed, pass0, (uint32_t)lanes, npix, maxv, (wrd::BVert*)verts, q.counts,
+                     true);
+    if (e != hipSuccess) return e;
     wrd::k_bdpt_prefix<<<(uint32_t)((2 * lanes + 255) / 256), 256, 0, st>>>(
         S, cam, npix, (uint32_t)lanes, maxv, (const wrd::BVert*)verts, q.counts, (wrd::BPrefix*)q.prefix);
     wrd::k_bdpt<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npass, npix, maxv, (const wrd::BVert*)verts,

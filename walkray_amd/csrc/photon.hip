@@ -1,9 +1,9 @@
 // photon.hip -- light sub-paths and the photon hash grid (gfx950), with their
 // C ABI entry points.
 //
-//  k_light_paths    one lane per light path: Scene::genLightSample as
-//                   AbstractObject::genSurfaceSample (abstractObj.cpp:18-52)
-//                   and MCRenderer::samplePath (mcRenderer.cpp:16-57) from it,
+//  light paths      Scene::genLightSample as AbstractObject::genSurfaceSample
+//                   (abstractObj.cpp:18-52) and MCRenderer::samplePath
+//                   (mcRenderer.cpp:16-57) from it as a path walk (LightWalk),
 //                   every Ray of the Path written as a 64 B record.
 //  photon collect   count, scan and write the light points VCM / PPM keep
 //                   (vcmTracer.cpp:42-55): deterministic, path-major order.
@@ -23,6 +23,7 @@
 
 #include "grid_dev.h"
 #include "pt_dev.h"
+#include "walk_dev.h"
 #include "wr_capi_internal.h"
 
 #pragma clang fp contract(off)
@@ -33,55 +34,49 @@ namespace wrd {
 // point), kLightVertex + 1 (direction), kLightVertex + 2 + d (scatter at depth d).
 constexpr uint32_t kLightVertex = 0x80000000u;
 
-__device__ __forceinline__ void put_vertex(wr_path_vertex* V, uint32_t& nv, uint32_t maxv, f3 o, f3 d, f3 rad,
-                                           float op, float dp, uint32_t contact, uint32_t ctri, uint32_t inside,
-                                           bool delta) {
-    if (nv < maxv) {
-        wr_path_vertex& v = V[nv];
-        v.origin[0] = o.x; v.origin[1] = o.y; v.origin[2] = o.z;
-        v.direction[0] = d.x; v.direction[1] = d.y; v.direction[2] = d.z;
-        v.radiance[0] = rad.x; v.radiance[1] = rad.y; v.radiance[2] = rad.z;
-        v.origin_prob = op;
-        v.direction_prob = dp;
-        v.contact_obj = contact;
-        v.contact_tri = contact == WR_NONE ? 0u : ctri;
-        v.inside_obj = inside;
-        v.flags = delta ? (uint32_t)WR_VERTEX_DELTA : 0u;
-        v.pad = 0u;
-    }
-    nv++;
+__device__ __forceinline__ void put_vertex(wr_path_vertex& v, f3 o, f3 d, f3 rad, float op, float dp, uint32_t contact,
+                                           uint32_t ctri, uint32_t inside, bool delta) {
+    v.origin[0] = o.x; v.origin[1] = o.y; v.origin[2] = o.z;
+    v.direction[0] = d.x; v.direction[1] = d.y; v.direction[2] = d.z;
+    v.radiance[0] = rad.x; v.radiance[1] = rad.y; v.radiance[2] = rad.z;
+    v.origin_prob = op;
+    v.direction_prob = dp;
+    v.contact_obj = contact;
+    v.contact_tri = contact == WR_NONE ? 0u : ctri;
+    v.inside_obj = inside;
+    v.flags = delta ? (uint32_t)WR_VERTEX_DELTA : 0u;
+    v.pad = 0u;
 }
 
 // terminateRay (mcRenderer.cpp:20-27): the origin of the ray passed in.
-__device__ __forceinline__ void put_terminate(wr_path_vertex* V, uint32_t& nv, uint32_t maxv, f3 o) {
+__device__ __forceinline__ void put_terminate(wr_path_vertex& v, f3 o) {
     const f3 z = mk(0.f, 0.f, 0.f);
-    put_vertex(V, nv, maxv, o, z, z, 1.f, 1.f, WR_NONE, 0u, WR_NONE, true);
+    put_vertex(v, o, z, z, 1.f, 1.f, WR_NONE, 0u, WR_NONE, true);
 }
 
-// 4 waves per SIMD (128 VGPRs, the rest spilled): 12.8 -> 9.3 ms for 2M light paths on the field.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_light_paths(SceneDev S, uint32_t max_depth, uint64_t seed, uint32_t pass,
-                                                     uint32_t path0, uint32_t n, uint32_t maxv, wr_path_vertex* out,
-                                                     uint32_t* counts) {
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    StackSpill spill;
-    LaneStack st(&spill);
-    const SceneCtx sc = make_scene_ctx(S);
-    const uint32_t path = path0 + k;
-    wr_path_vertex* V = out + (size_t)k * maxv;
-    uint32_t nv = 0;
-    float rn[4];
-    rng4(seed, path, pass, kLightVertex, rn);
-    const LightSample L = sample_light(sc, rn);
-    f3 o = mk(0.f, 0.f, 0.f), d = o;
-    uint32_t inside = WR_NONE;
-    PHit hit;
-    hit.rec = WR_NONE;
-    hit.obj = WR_NONE;
-    hit.t = -1.f;
-    if (!L.ok) {  // the reference's empty-mesh light ray: no direction, radiance or contact
-        put_vertex(V, nv, maxv, o, d, o, 1.f, 1.f, WR_NONE, 0u, WR_NONE, false);
-    } else {
+// The light paths path0 + k, k < n, as a path walk (walk_dev.h): record s + 1 of
+// path k is written by step s.  As one kernel, a lane per path, 307,200 paths
+// of the object field (maxPathLen 16) took 2.0 ms; in steps XXX ms.
+struct LightWalk {
+    uint32_t max_depth, pass, path0, maxv;
+    uint64_t seed;
+    wr_path_vertex* out;
+    uint32_t* counts;
+
+    __device__ __forceinline__ bool begin(const SceneCtx& sc, uint32_t k, LaneStack& st, f3& o, f3& d,
+                                          uint32_t& inside, uint32_t& contact) const {
+        const uint32_t path = path0 + k;
+        wr_path_vertex* V = out + (size_t)k * maxv;
+        float rn[4];
+        rng4(seed, path, pass, kLightVertex, rn);
+        const LightSample L = sample_light(sc, rn);
+        if (!L.ok) {  // the reference's empty-mesh light ray: no direction, radiance or contact, and it hits nothing
+            const f3 z = mk(0.f, 0.f, 0.f);
+            put_vertex(V[0], z, z, z, 1.f, 1.f, WR_NONE, 0u, WR_NONE, false);
+            put_terminate(V[1], z);
+            counts[k] = 2;
+            return false;
+        }
         rng4(seed, path, pass, kLightVertex + 1, rn);
         // UniformSphereSampler::sample (uniformSphereSampler.h:6-20)
         const float term1 = (float)(2.0 * kPi * (double)rn[0]);
@@ -90,42 +85,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         float dp = (float)(kInvPi * 0.25f);
         if (dot(d, L.n) < 0.f) d = mk(-d.x, -d.y, -d.z);
         o = L.o;
-        inside = find_inside(S, o, d, L.obj, st);
+        inside = find_inside(sc.S, o, d, L.obj, st);
+        contact = L.obj;
         dp *= 2.f;
-        const PHit h = trace_scene<true>(sc, o, d, inside, L.obj, st);
-        if (h.rec != WR_NONE && h.t > 0.f) hit = h;  // intersectObj is set only for dist > 0
-        put_vertex(V, nv, maxv, o, d, L.rad, L.op, dp, L.obj, L.tri, inside, false);
+        put_vertex(V[0], o, d, L.rad, L.op, dp, L.obj, L.tri, inside, false);
+        return true;
     }
-    for (uint32_t depth = 0;; depth++) {
-        const uint32_t self = inside != WR_NONE ? inside : hit.obj;
-        if (self == WR_NONE || hit.rec == WR_NONE) {  // nothing to scatter (an open inside object as well)
-            put_terminate(V, nv, maxv, o);
-            break;
+
+    __device__ __forceinline__ bool step(const SceneCtx& sc, uint32_t k, uint32_t s, f3 o, f3 d, const PHit& hit,
+                                         LaneStack& st, Out& r) const {
+        wr_path_vertex* V = out + (size_t)k * maxv;
+        counts[k] = s + 2;  // of a path that ends here; a later step overwrites it
+        // an escaped ray ends the path at the origin before its own; the light
+        // ray's hit counts only at dist > 0 (abstractObj.cpp:46)
+        if (hit.rec == WR_NONE || (s == 0 && !(hit.t > 0.f))) {
+            const float* e = V[s == 0 ? 0 : s - 1].origin;
+            put_terminate(V[s + 1], mk(e[0], e[1], e[2]));
+            return false;
         }
-        rng4(seed, path, pass, kLightVertex + 2 + depth, rn);
-        const Out r = scatter(sc, self, o, d, hit, inside, rn, st);
-        const uint32_t ctri = S.tris[hit.rec].prim - S.objs[hit.obj].prim_base;  // intersectTriangleID
-        if ((double)len(r.d) < 0.5) {
-            put_vertex(V, nv, maxv, r.o, r.d, r.rad, r.op, r.dp, r.contact, ctri, r.inside, r.delta);
-            break;
+        const uint32_t inside = V[s].inside_obj;
+        float rn[4];
+        rng4(seed, path0 + k, pass, kLightVertex + 2 + s, rn);
+        r = scatter(sc, inside != WR_NONE ? inside : hit.obj, o, d, hit, inside, rn, st);
+        const bool absorbed = (double)len(r.d) < 0.5;
+        if (!absorbed && s + 1 > max_depth) {
+            put_terminate(V[s + 1], o);
+            return false;
         }
-        if (depth + 1 > max_depth) {
-            put_terminate(V, nv, maxv, o);
-            break;
-        }
-        const PHit nh = trace_scene<true>(sc, r.o, r.d, r.inside, r.contact, st);
-        put_vertex(V, nv, maxv, r.o, r.d, r.rad, r.op, r.dp, r.contact, ctri, r.inside, r.delta);
-        if (nh.rec == WR_NONE) {
-            put_terminate(V, nv, maxv, o);
-            break;
-        }
-        o = r.o;
-        d = r.d;
-        inside = r.inside;
-        hit = nh;
+        const uint32_t ctri = sc.S.tris[hit.rec].prim - sc.S.objs[hit.obj].prim_base;  // intersectTriangleID
+        put_vertex(V[s + 1], r.o, r.d, r.rad, r.op, r.dp, r.contact, ctri, r.inside, r.delta);
+        return !absorbed;
     }
-    counts[k] = nv;
-}
+};
 
 // Light points of one path: vertices 1.. before the first emissive contact,
 // without the delta ones.
@@ -638,10 +629,8 @@ int wr_light_paths(wr_ctx* ctx, const wr_scene* s, uint32_t max_depth, uint64_t 
     if ((uint64_t)path0 + n_paths > 0x100000000ull) return fail(ctx, WR_EINVAL, "wr_light_paths: path ids overflow");
     if (n_paths == 0) return WR_OK;
     (void)hipSetDevice(ctx->device);
-    k_light_paths<<<(n_paths + 255) / 256, 256, kStackLdsBytes, ctx->stream>>>(s->dev, max_depth, seed, pass, path0,
-                                                                               n_paths, max_vertices, d_vertices,
-                                                                               d_counts);
-    PH_CHECK(hipGetLastError(), "wr_light_paths");
+    const LightWalk P{max_depth, pass, path0, max_vertices, seed, d_vertices, d_counts};
+    PH_CHECK(wr::run_walk(ctx, s->dev, s->hdrs[0], P, n_paths, max_depth + 1), "wr_light_paths");
     PH_CHECK(hipStreamSynchronize(ctx->stream), "wr_light_paths");
     return WR_OK;
 }

@@ -289,6 +289,29 @@ __device__ Out scatter(const SceneCtx& sc, uint32_t self, f3 in_o, f3 in_d, cons
     return out;
 }
 
+// ---- workgroup helpers ----------------------------------------------------------
+// One slot per lane that wants one, for the whole 256-lane workgroup with a
+// single atomic; every thread of the workgroup must make the call.  Slots go
+// out in thread order.
+__device__ __forceinline__ uint32_t block_append(uint32_t* counter, bool want) {
+    __shared__ uint32_t s_cnt[4];
+    __shared__ uint32_t s_base;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint64_t mask = __ballot(want);
+    if (lane == 0) s_cnt[w] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t t = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+        s_base = t ? atomicAdd(counter, t) : 0u;
+    }
+    __syncthreads();
+    uint32_t off = s_base;
+    for (uint32_t v = 0; v < w; v++) off += s_cnt[v];
+    off += (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+    __syncthreads();  // s_cnt and s_base serve the next call
+    return off;
+}
+
 // ---- next-event estimation (PathTracer's useNextEventEstimation branch) -------
 // Vertex counter of the light sample's uniforms; path vertices use 0 .. max_depth + 1.
 constexpr uint32_t kNeeVertex = 0xFFFFFFFFu;

@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "trace_dev.h"
+#include "walk_dev.h"
 #include "wr_kernels.h"
 
 #pragma clang fp contract(off)
@@ -249,6 +250,86 @@ __global__ __launch_bounds__(256) void k_closest_hit_small(SceneDev S, wr_tree_h
     hits[i] = complete_hit<NOSELF, false>(tr, r, ns, st, cnt, h, overflow);
 }
 
+// The fast pass of a path walk's step (walk_dev.h): the *n_dev rays, NoSelf,
+// spread over the chip as k_wf_trace spreads its paths: a unit of up to 64 rays
+// for each of kSpread waves, and no more lanes of a wave at work than that.
+__global__ __launch_bounds__(256) void k_walk_trace(SceneDev S, wr_tree_hdr H, const uint32_t* __restrict__ rays,
+                                                    const uint32_t* n_dev, uint4* __restrict__ hits,
+                                                    unsigned long long* work) {
+    constexpr uint32_t kSpread = 4096, kRefillMin = 16, kNodePhaseMin = 32;
+    const uint32_t n = *n_dev;
+    uint32_t width = 1;
+    while (width < 64 && 2ull * n > 3ull * width * kSpread) width *= 2;
+    const uint32_t units = (uint32_t)(((uint64_t)n + width - 1) / width);
+    const uint32_t used = min((units + 31) / 32 * 8, gridDim.x);
+    if (blockIdx.x >= used || n == 0) return;
+    const Tree tr = make_tree(H, S);
+    StackSpill spill;
+    LaneStack st(&spill);
+    Counters cnt{0, 0, 0};
+    NoSelf ns{};
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint64_t lanes = width < 64 ? (1ull << width) - 1ull : ~0ull;  // the lanes that take rays
+    const uint32_t refill_min = width < 64 ? 1u : kRefillMin;
+    const uint32_t node_phase_min = (width * kNodePhaseMin + 63) / 64;
+    __shared__ unsigned long long pool;
+    UnitQueue queue;
+    queue.init(&pool, work, units, used, 4, units / used > 12 ? 2 : 1,
+               units > 4 * used ? min(max(units / (16 * wr::kXcds), 1u), 64u) : 1u);
+    uint32_t bnext = 0, bend = 0;  // the rays of the wave's current unit [bnext, bend)
+    bool exhausted = false;
+    bool active = false, overflow = false;
+    uint32_t rid = 0, ref = 0;
+    RayPre r{};
+    HitState h{};
+    for (;;) {
+        uint64_t idle = __ballot(!active) & lanes;
+        if (!exhausted && (uint32_t)__popcll(idle) >= refill_min) {
+            while (idle != 0) {
+                if (bnext == bend) {
+                    const uint32_t u = queue.next();
+                    if (u == WR_NONE) {
+                        exhausted = true;
+                        break;
+                    }
+                    bnext = u * width;
+                    bend = n - bnext > width ? bnext + width : n;
+                }
+                const uint32_t avail = bend - bnext;
+                const uint32_t rank = (uint32_t)__popcll(idle & below);
+                if (!active && lane < width && rank < avail) {
+                    rid = bnext + rank;
+                    f3 o, d;
+                    uint32_t inside, contact;
+                    load_ray<true>(rays, rid, o, d, inside, contact);
+                    r = make_ray(o, d, tr.scale);
+                    ns = make_noself<true>(S, H, inside, contact);
+                    overflow = false;
+                    if (wide_begin(tr, r, st, h, ref)) active = true;
+                    else hits[rid] = make_uint4(WR_NONE, 0u, 0u, 0u);  // misses the root box
+                }
+                const uint32_t took = (uint32_t)__popcll(idle);
+                bnext += took < avail ? took : avail;
+                idle = __ballot(!active) & lanes;
+            }
+        }
+        if (__ballot(active) == 0) break;  // only once the queue is empty
+        for (;;) {
+            const bool at_node = active && !(ref & WR_LEAF_BIT);
+            if ((uint32_t)__popcll(__ballot(at_node)) < node_phase_min) break;
+            if (at_node && !wide_step<true, false>(tr, r, ns, st, h, ref, overflow, cnt)) {
+                hits[rid] = make_uint4(h.rec, __float_as_uint(h.t), h.leaf, overflow ? 1u : 0u);
+                active = false;
+            }
+        }
+        if (active && !wide_step<true, false>(tr, r, ns, st, h, ref, overflow, cnt)) {
+            hits[rid] = make_uint4(h.rec, __float_as_uint(h.t), h.leaf, overflow ? 1u : 0u);
+            active = false;
+        }
+    }
+}
+
 __global__ __launch_bounds__(256) void k_inside_object(SceneDev S, const uint32_t* __restrict__ rays, uint64_t n,
                                                        uint32_t* __restrict__ out) {
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
@@ -395,6 +476,23 @@ hipError_t launch_closest_hit_path(const SceneDev& S, const wr_tree_hdr& H, cons
     const ChTune t;
     return launch_closest_hit_d<true, 8>(S, H, rays, n, hits, nullptr, work, t.blocks_per_cu, t.refill_min,
                                          t.node_phase_min, t.batch, st);
+}
+
+hipError_t launch_walk_trace(const SceneDev& S, const wr_tree_hdr& H, const uint32_t* rays, const uint32_t* n,
+                             uint32_t max_n, uint4* hits, unsigned long long* work, hipStream_t st) {
+    // as many workgroups as fit (5 waves per SIMD), or as the rays can use
+    static const uint32_t resident = [] {
+        int dev = 0, cus = 0, per_cu = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wrd::k_walk_trace, 256, wrd::kStackLdsBytes) !=
+                hipSuccess || cus <= 0 || per_cu <= 0)
+            return 256u;
+        return (uint32_t)(cus * per_cu);
+    }();
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)max_n + 31) / 32 * 8, resident);
+    wrd::k_walk_trace<<<grid, 256, wrd::kStackLdsBytes, st>>>(S, H, rays, n, hits, work);
+    return hipGetLastError();
 }
 
 hipError_t launch_inside_object(const SceneDev& S, uint32_t max_obj_depth, const uint32_t* rays, uint64_t n,

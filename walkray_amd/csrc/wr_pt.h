@@ -7,6 +7,8 @@
 
 #include "wr_kernels.h"
 
+struct wr_ctx;
+
 namespace wr {
 
 // Camera basis computed on the host with the reference's float semantics
@@ -171,9 +173,9 @@ struct BdptQueue {
 constexpr size_t kBdptQueueEntryBytes = 32 + 16 + 4 + 16;
 size_t bdpt_vertex_bytes();
 size_t bdpt_prefix_bytes();
-hipError_t launch_bdpt_passes(const SceneDev& S, const wr_tree_hdr& H, const CamHost& cam, uint32_t max_depth,
+hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& cam, uint32_t max_depth,
                               uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
-                              const BdptQueue& q, const FilmBufs& film, hipStream_t st);
+                              const BdptQueue& q, const FilmBufs& film);
 
 hipError_t run_wavefront(const SceneDev& S, const CamHost& cam, uint32_t max_depth, uint64_t seed, uint32_t pass0,
                          uint32_t npass, bool nee, const FilmBufs& film, Engine& engine, uint32_t cap, uint32_t grid,
