@@ -385,7 +385,7 @@ struct SubpathWalk {
             r.n = cam.front;
             r.flags = kVCamera;
             r.inside = find_inside(sc.S, r.o, r.d, WR_NONE, st);
-        } else {  // the light ray (as k_light_paths' first)
+        } else {  // the light ray (as LightWalk's first)
             rng4(seed, p, pass, kBdptLightVertex, rn);
             const LightSample ls = sample_light(sc, rn);
             r.o = mk(0.f, 0.f, 0.f);
@@ -463,7 +463,7 @@ struct SubpathWalk {
 };
 
 // The prefixes of every sub-path (BPrefix), one lane per sub-path: side 0 the
-// light sub-path, side 1 the eye sub-path of each lane of k_bdpt_subpaths.
+// light sub-path, side 1 the eye sub-path of each lane's SubpathWalk.
 __global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uint32_t npix, uint32_t lanes,
                                                      uint32_t maxv, const BVert* verts, const uint32_t* counts,
                                                      BPrefix* prefix) {
@@ -696,7 +696,7 @@ __global__ __launch_bounds__(256) void k_bdpt_fold(CamDev cam, uint32_t npass, u
 
 // ---- VCMTracer (vcmTracer.cpp:6-446) ---------------------------------------
 // Several passes side by side (lane = pass x pixel, as k_bdpt), each with its
-// own light points, radius and grid: the sub-paths of k_bdpt_subpaths (one
+// own light points, radius and grid: the sub-paths of SubpathWalk (one
 // light path per pixel); per pass the light points (vcmTracer.cpp:42-55: the
 // pixel count of default-constructed ones, then every non-delta vertex past
 // the first of each light path, up to an emitter, path-major) in a block of

@@ -258,11 +258,12 @@ __global__ __launch_bounds__(256) void k_walk_trace(SceneDev S, wr_tree_hdr H, c
                                                     unsigned long long* work) {
     constexpr uint32_t kSpread = 4096, kRefillMin = 16, kNodePhaseMin = 32;
     const uint32_t n = *n_dev;
+    if (n <= wr::kWalkFew) return;  // k_walk_shade traces the last paths itself
     uint32_t width = 1;
     while (width < 64 && 2ull * n > 3ull * width * kSpread) width *= 2;
     const uint32_t units = (uint32_t)(((uint64_t)n + width - 1) / width);
     const uint32_t used = min((units + 31) / 32 * 8, gridDim.x);
-    if (blockIdx.x >= used || n == 0) return;
+    if (blockIdx.x >= used) return;
     const Tree tr = make_tree(H, S);
     StackSpill spill;
     LaneStack st(&spill);

@@ -21,6 +21,17 @@
 
 #pragma clang fp contract(off)
 
+namespace wr {
+// A step with at most this many live paths ends the walk: what bounds it is the
+// latency of one traversal and one vertex, about 45 us, to which two kernels'
+// launches and the lists add 25 us, so k_walk_shade takes the paths to their
+// ends, spread over the chip.  307,200 light paths of the object field
+// (maxPathLen 16) with their photons and grid 2.30 ms without, 2.0 ms up to
+// 16,384 paths, 1.91 up to 32,768, 1.79 up to 65,536 and 131,072, where
+// PhotonMap loses 1.5%.
+constexpr uint32_t kWalkFew = 65536;
+}  // namespace wr
+
 namespace wrd {
 
 // The live paths of two consecutive steps: rays in the batch NoSelf layout (8
@@ -72,6 +83,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
+    if (n <= wr::kWalkFew) {  // the rest of every path, the trace included
+        uint32_t width = 1;   // lanes of a wave that take a path
+        while (width < 64 && (uint64_t)width * gridDim.x * 4 < n) width *= 2;
+        const uint32_t lane = threadIdx.x & 63u;
+        const uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane;
+        if (lane >= width || i >= n) return;
+        const uint32_t path = W.path[s & 1][i];
+        const uint32_t* rp = W.rays[s & 1] + 8 * (size_t)i;
+        Out out;
+        out.o = mk(__uint_as_float(rp[0]), __uint_as_float(rp[1]), __uint_as_float(rp[2]));
+        out.d = mk(__uint_as_float(rp[3]), __uint_as_float(rp[4]), __uint_as_float(rp[5]));
+        out.inside = rp[6];
+        out.contact = rp[7];
+        for (uint32_t k = s;; k++) {
+            const f3 o = out.o, d = out.d;
+            const PHit hit = trace_scene<true>(sc, o, d, out.inside, out.contact, st);
+            if (!policy.step(sc, path, k, o, d, hit, st, out)) return;
+        }
+    }
     for (uint32_t i0 = blockIdx.x * 256; i0 < n; i0 += gridDim.x * 256) {
         const uint32_t i = i0 + threadIdx.x;
         bool go = false;
@@ -138,11 +168,13 @@ hipError_t run_walk(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const 
         const uint32_t n = n_paths - p < chunk ? n_paths - p : chunk;
         const uint32_t blocks = (n + 255) / 256;
         if ((e = hipMemsetAsync(W.n, 0, sizeof(uint32_t) * (steps + 1), st)) != hipSuccess) return e;
+        // at least one wave per SIMD for a few paths' ends
+        const uint32_t shade = blocks < 256 ? 256 : (blocks < 2048 ? blocks : 2048);
         wrd::k_walk_begin<P><<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, p, n);
         for (uint32_t s = 0; s < steps; s++) {
             e = launch_walk_trace(S, H, W.rays[s & 1], W.n + s, n, W.hits, W.work, st);
             if (e != hipSuccess) return e;
-            wrd::k_walk_shade<P><<<blocks < 2048 ? blocks : 2048, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s);
+            wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s);
         }
         p += n;
     }
