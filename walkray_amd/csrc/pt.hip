@@ -76,6 +76,7 @@ struct EngineDev {
     const SceneDev* scenes;
     uint32_t* exit_list;
     uint32_t cap;
+    uint32_t few;  // an iteration with at most this many live paths takes them to their ends (wf_rest)
 };
 
 __device__ __forceinline__ CamDev job_cam(const wr::JobDesc& J) {
@@ -188,13 +189,14 @@ template <int D, bool COUNT = false>
 __global__ __launch_bounds__(256) void k_wf_trace(EngineDev E, uint32_t par) {
     const PathBuf& A = E.buf[par];
     const uint32_t n = E.cnt->n[par];
+    if (n <= E.few) return;  // wf_rest traces them
     // paths of a unit: the power of two nearest to the paths per spread wave
     uint32_t width = 1;
     while (width < 64 && 2ull * n > 3ull * width * kTraceSpread) width *= 2;
     const uint32_t units = (uint32_t)(((uint64_t)n + width - 1) / width);
     // workgroups beyond what the units need (a unit per wave, every XCD alike) leave at once
     const uint32_t used = min((units + 31) / 32 * 8, gridDim.x);
-    if (blockIdx.x >= used || n == 0) return;
+    if (blockIdx.x >= used || n == 0) return;  // n: with few = 0
     StackSpillT<D> spill;
     LaneStackT<D> st(&spill);
     Counters cnt{0, 0, 0};
@@ -300,6 +302,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const PathBuf& A = E.buf[par];
     const PathBuf& B = E.buf[par ^ 1];
     const uint32_t n = E.cnt->n[par];
+    if (n <= E.few) return;  // wf_rest completes them
     if (blockIdx.x == 0) UnitQueue::clear(E.cnt->trace_work);  // for the next iteration's trace
     StackSpill spill;
     LaneStack st(&spill);
@@ -365,6 +368,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
 }
 
+// The rest of one live path or connection entry, in one lane: extend and shade
+// until it ends, the connection of the next-event branch included.  Returns
+// the completion counter of its pass (nullptr for a cancelled job's path).
+template <bool NEE>
+__device__ __forceinline__ uint32_t* wf_rest(const EngineDev& E, const PathBuf& A, uint32_t i, LaneStack& st) {
+    const uint32_t jb = A.job[i];
+    if (E.ctl[jb].state != wr::kJobRunning) return nullptr;
+    const wr::JobDesc& J = E.jobs[jb];
+    const SceneCtx sc = make_scene_ctx(E.scenes[J.scene]);
+    const uint32_t p = A.pixel[i], ps = A.pass[i], fl = A.flags[i];
+    f3 o = mk(A.ox[i], A.oy[i], A.oz[i]), d = mk(A.dx[i], A.dy[i], A.dz[i]);
+    f3 T = mk(A.tx[i], A.ty[i], A.tz[i]);
+    uint32_t inside = A.inside[i], contact = A.contact[i], depth = A.depth[i];
+    if (NEE && (fl & kShadow)) {  // MCRenderer::visibilityTest (mcRenderer.cpp:59-65)
+        const PHit h = trace_scene<true>(sc, o, d, inside, contact, st);
+        return finish_value(J, job_cam(J), p, ps, nee_visible(h.rec, h.t, A.ux[i]) ? T : mk(0.f, 0.f, 0.f));
+    }
+    const bool nee = NEE && (J.flags & wr::kJobNee) != 0;
+    f3 U = T, P = T;  // the branch-order products with and without the current ray
+    uint32_t crec = WR_NONE;
+    bool front = false, primary = (fl & kPrimary) != 0;
+    if (nee) {
+        U = mk(A.ux[i], A.uy[i], A.uz[i]);
+        if (!primary) {
+            P = mk(A.px[i], A.py[i], A.pz[i]);
+            crec = A.crec[i];
+            front = (fl & kFront) != 0;
+        }
+    }
+    f3 color = mk(0.f, 0.f, 0.f);
+    float rn[4];
+    for (;;) {
+        // a camera ray's inside and contact are WR_NONE: no condition
+        const PHit h = trace_scene<true>(sc, o, d, inside, contact, st);
+        if (primary) inside = find_inside(sc.S, o, d, WR_NONE, st);
+        bool connect = h.rec == WR_NONE && !primary;  // escaped: from the ray's origin
+        if (h.rec != WR_NONE) {
+            rng4(J.seed, p, J.pass0 + ps, depth + 1, rn);
+            const Out out = scatter(sc, inside != WR_NONE ? inside : h.obj, o, d, h, inside, rn, st);
+            if ((double)len(out.d) < 0.5) {  // emission / absorption ends the path
+                color = mulv(T, divs(divs(out.rad, out.op), out.dp));
+                break;
+            }
+            connect = depth + 1 > J.max_depth && depth >= 1;  // at the limit: from this ray's origin
+            if (depth + 1 <= J.max_depth) {
+                T = muls(T, cosine_term(out));
+                T = mulv(T, divs(divs(out.rad, out.op), out.dp));
+                if (nee) {
+                    P = U;
+                    U = mulv(U, divs(divs(out.rad, out.op), out.dp));
+                    U = muls(U, cosine_term(out));
+                    crec = h.rec;
+                    front = dot(d, out.n) <= 0.f;
+                }
+                o = out.o;
+                d = out.d;
+                inside = out.inside;
+                contact = out.contact;
+                primary = false;
+                depth++;
+                continue;
+            }
+        }
+        if (nee && connect)
+            color = nee_sample(sc, o, contact, crec, front, P, inside, J.seed, p, J.pass0 + ps, st);
+        break;
+    }
+    return finish_value(J, job_cam(J), p, ps, color);
+}
+
 // shade: scatter + Russian roulette of every path whose ray hit (MCRenderer::
 // samplePath, mcRenderer.cpp:30-41), survivors appended to the next buffer.
 // EXITS = false shades every live path except refraction exits, whose scatter
@@ -383,6 +456,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXITS ? 1 :
     const uint32_t n = EXITS ? E.cnt->n_exit : E.cnt->n[par];
     StackSpill spill;
     LaneStack st(&spill);
+    if (E.cnt->n[par] <= E.few) return;  // k_wf_rest takes them to their ends
     // the workgroup steps through the slots together: each step's survivors,
     // connection entries and refraction exits take their slots with one
     // atomic per workgroup (block_append) instead of one per wave
@@ -485,6 +559,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXITS ? 1 :
             B.job[j] = jb;
         }
     }
+}
+
+// Few live paths: their rest in this one launch.  What bounds such an iteration
+// is the latency of one ray and one vertex, about 45 us, to which its other
+// kernels add as much again, every iteration anew.  The lanes of a wave that
+// take a path: as few as give each of the waves that fit (two on each of 1,024
+// SIMDs) one at least.  Renders without and with it: 64x64, 1 spp 965 and
+// 535 us; 256x256, 16 spp 3.14 and 3.09 ms; field 1280x720, 16 spp, next-event
+// 25.1 and 23.4 ms; ten small jobs of a server 4.47 and 3.93 ms.  A kernel of
+// its own: inside the refraction exits' shade it cost that kernel registers,
+// 0.1 ms of the 256x256 render.
+template <bool NEE>
+__global__ __launch_bounds__(256) void k_wf_rest(EngineDev E, uint32_t par) {
+    const PathBuf& A = E.buf[par];
+    const uint32_t n = E.cnt->n[par];
+    if (n > E.few) return;
+    const uint32_t waves = min(gridDim.x * 4, 2048u);
+    uint32_t width = 1;
+    while (width < 64 && width * waves < n) width *= 2;
+    if (blockIdx.x * 4 * width >= n) return;
+    StackSpill spill;
+    LaneStack st(&spill);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane;
+    uint32_t* done = nullptr;
+    if (lane < width && i < n) done = wf_rest<NEE>(E, A, i, st);
+    block_count_done(done, done != nullptr);
 }
 
 // Number of consecutive complete passes of a job starting at its fold cursor.
@@ -836,6 +937,8 @@ static EngineDev engine_dev(const Engine& En) {
     E.scenes = En.scenes;
     E.exit_list = En.exit_list;
     E.cap = En.cap;
+    // the last workgroups of the grid must reach the last of the few paths
+    E.few = std::min<uint32_t>(kWaveFew, En.grid * 256);
     return E;
 }
 
@@ -850,7 +953,8 @@ static void launch_trace(const EngineDev& E, uint32_t lds_levels, uint32_t trace
 }
 
 hipError_t Engine::enqueue(int iters, hipStream_t st, hipEvent_t* ev, bool nee) {
-    const EngineDev E = engine_dev(*this);
+    EngineDev E = engine_dev(*this);
+    if (ev) E.few = 0;  // the statistics count every segment
     int k = 0;
     auto mark = [&]() -> hipError_t { return ev ? hipEventRecord(ev[k++], st) : hipSuccess; };
     WR_CHECK(mark());
@@ -871,6 +975,10 @@ hipError_t Engine::enqueue(int iters, hipStream_t st, hipEvent_t* ev, bool nee) 
             k_wf_shade<true, false><<<grid, 256, kStackLdsBytes, st>>>(E, par);
         }
         WR_CHECK(mark());
+        if (E.few) {
+            if (nee) k_wf_rest<true><<<grid, 256, kStackLdsBytes, st>>>(E, par);
+            else k_wf_rest<false><<<grid, 256, kStackLdsBytes, st>>>(E, par);
+        }
         k_wf_plan<<<1, 64, 0, st>>>(E, par);
         WR_CHECK(mark());
         k_wf_generate<<<grid, 256, 0, st>>>(E, par);
@@ -1014,10 +1122,12 @@ static hipError_t run_wavefront_once(const SceneDev& S, const CamHost& cam, uint
     const uint64_t it_bound = 4 * (uint64_t)(max_depth + 4) * (total / E.cap + npass + 2) + 64;
     // every camera path fits the pool and the window: all are issued in the
     // first iteration, so the first replay is followed by a tail replay at once
-    // (with per-stage events every replay is read back on its own)
-    bool chain_tail = total <= E.cap && npass <= J.R && !ev;
+    // (with per-stage events every replay is read back on its own); few enough
+    // to be taken to their ends by the second iteration, a tail replay is all
+    const bool at_once = total <= E.cap && npass <= J.R && !ev;
+    bool tail = at_once && total <= std::min<uint32_t>(kWaveFew, E.grid * 256);
+    bool chain_tail = at_once && !tail;
     uint64_t iters = 0;
-    bool tail = false;
     JobCtl& back = *E.ctl_back;
     hipError_t e = hipSuccess;
     auto replay = [&](bool short_one) -> hipError_t {

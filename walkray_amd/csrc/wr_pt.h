@@ -32,6 +32,11 @@ constexpr uint32_t kMaxJobs = 64;        // concurrently admitted jobs
 constexpr uint32_t kMaxScenes = 64;      // resident scenes of one engine
 constexpr int kGraphIters = 8;           // wavefront iterations per graph replay (even)
 constexpr int kTailIters = 2;            // iterations per replay once every job has issued all its paths (even)
+// Live paths up to which an iteration takes them to their ends (k_wf_rest): 64
+// per wave that fits.  Renders of cornell 256x256, 4 spp and field 640x360, 8 spp:
+// 2,128 and 4,244 us at 32,768; 1,940 and 4,196 at 65,536; 1,833 and 4,029 at
+// 131,072; 2,362 and 4,698 at 262,144, where the lists are the faster.
+constexpr uint32_t kWaveFew = 131072;
 constexpr uint32_t kDefaultPathSlots = 1u << 22;  // 4M paths in flight: 2 x 416 MB of path state
 constexpr uint32_t kBdptMaxDepth = 32;           // BidirectionalPathTracer: maxPathLen limit of wr_render_bdpt
 
