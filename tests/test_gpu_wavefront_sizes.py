@@ -1,6 +1,6 @@
 """Wavefront films at the numbers of live paths where its trace stage changes the paths per wave
-(a unit of 1, 2, 4, ... 64 paths) and starts to draw units from its counters: bit-identical to the
-megakernel's films."""
+(a unit of 1, 2, 4, ... 64 paths), starts to draw units from its counters, and where an iteration
+takes its paths to their ends: bit-identical to the megakernel's films."""
 import numpy as np
 import pytest
 
@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("width,height,spp,slots", [
     (1, 1, 1, 0), (96, 64, 1, 0), (5, 1229, 1, 0), (193, 97, 1, 0), (384, 256, 1, 0), (391, 503, 1, 0),
+    (512, 256, 1, 0), (43691, 3, 1, 0),  # the most paths taken to their ends at once, and one more
     (391, 503, 2, 0),        # 393,346 paths: more full units than the resident waves
     (701, 467, 4, 0),        # 1.3M paths: units from the counters, two at a time
     (200, 150, 3, 20000),    # a pool smaller than a pass

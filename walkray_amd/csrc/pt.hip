@@ -571,7 +571,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXITS ? 1 :
 // its own: inside the refraction exits' shade it cost that kernel registers,
 // 0.1 ms of the 256x256 render.
 template <bool NEE>
-__global__ __launch_bounds__(256) void k_wf_rest(EngineDev E, uint32_t par) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_wf_rest(EngineDev E, uint32_t par) {
     const PathBuf& A = E.buf[par];
     const uint32_t n = E.cnt->n[par];
     if (n > E.few) return;
