@@ -311,18 +311,6 @@ __device__ __forceinline__ bool emissive(const SceneDev& S, uint32_t obj) {
     return obj != WR_NONE && S.objs[obj].mat == WR_MAT_EMISSIVE;
 }
 
-// One slot of a queue per active lane, one atomic per wave.
-__device__ __forceinline__ uint32_t wave_slot(uint32_t* counter) {
-    const uint64_t mask = __ballot(1);
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t leader = __ffsll((unsigned long long)mask) - 1;
-    const uint32_t rank = __popcll(mask & ((1ull << lane) - 1));
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    return base + rank;
-}
-
 // The visibility queue: rays in the batch NoSelf layout (o, d, inside,
 // contact), per entry the contribution and the distance to the light-side
 // record, and the target (pass buffer offset + pixel).
@@ -522,6 +510,13 @@ __device__ __forceinline__ int nth_bit(uint64_t mask, uint32_t n) {
     return __ffsll((unsigned long long)mask) - 1;
 }
 
+// Queue slots that a wave of connect_wave reserves ahead at most.  The one
+// counter bounds the connections: with an atomic of each wave for every 64
+// pairs k_bdpt took 1.6 ms for Cornell 256^2 x 8 passes (5.9M entries), of which
+// its arithmetic is 0.6 ms.  With the expected number of entries reserved at
+// once (slots that stay empty hold rays that leave the scene) the render takes 4.97 ms instead of 6.04; 192 ahead instead of 448: 5.00 ms.
+constexpr uint32_t kReserve = 448;
+
 // The pairs of records that a wave's lanes connect, for connect_wave.
 struct PairTable {
     uint64_t eye[64], light[64];  // per lane: the records that connect to something, a bit each
@@ -534,9 +529,9 @@ struct PairTable {
 // pairs would keep its wave for the longest of 64 products (k_bdpt: 7.5 ms for
 // Cornell 256^2 x 8 passes); so each lane notes which of its records connect
 // at all (neither delta nor an emitter), and the wave deals its lanes' pairs
-// out one to each lane at a time (1.6 ms).  Every lane of the wave makes the
-// call; lane0: the wave's first lane; max_eye, max_light: 0 where there is
-// none.  Adds what needs no visibility test to the lane's own pixel.
+// out one to each lane at a time.  Every lane of the wave makes the
+// call; lane0: the lane (pixel and pass) of the wave's first; max_eye,
+// max_light: 0 where a lane of the wave has none.  Adds what needs no visibility test to the lane's own pixel.
 __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
                                            uint32_t maxv, uint64_t lane0, const BVert* verts, const BPrefix* prefix,
                                            int max_eye, int max_light, float* pix_all, const VisQueue& Q,
@@ -579,45 +574,75 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
     T.upto[wl] = upto;
     __builtin_amdgcn_wave_barrier();  // the table is this wave's own: LDS operations of a wave stay in order
     const uint32_t total = __shfl(upto, 63, 64);
-    for (uint32_t t = wl; t < total; t += 64) {
-        uint32_t o = 0;  // the first lane with upto > t
+    uint32_t kept = 0, kept_end = 0, used = 0;  // the wave's reserved queue slots, and its entries so far
+    for (uint32_t t0 = 0; t0 < total; t0 += 64) {
+        BVert ec{};
+        f3 contrib{};
+        uint32_t target = 0, k = 0;
+        float dist = 0.f;
+        auto connect = [&](uint32_t t) {
+            uint32_t o = 0;  // the first lane with upto > t
 #pragma unroll
-        for (uint32_t step = 32; step > 0; step >>= 1)
-            if (T.upto[o + step - 1] <= t) o += step;
-        const uint32_t r = o ? t - T.upto[o - 1] : t;
-        const uint64_t lights = T.light[o];
-        const uint32_t nl = (uint32_t)__popcll(lights);
-        const int e = nth_bit(T.eye[o], r / nl), c = nth_bit(lights, r % nl);
-        const uint64_t lane = lane0 + o;
-        const uint32_t k = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
-        const size_t ei = lane * 2 * maxv, li = ei + maxv;
-        BVert lc = verts[li + c], ec = verts[ei + e];
-        if (!connect_edge(S, verts + li, c, verts + ei, e, lc, ec)) continue;
-        const VcmTerms vt{grids ? grids[k].r : 0.f, (double)npix, false};
-        f3 color;
-        float prob;
-        const float w = color_prob_weight(S, cam, p, lc, prefix[li + c], c, ec, prefix[ei + e], e, color, prob,
-                                          grids ? &vt : nullptr);
-        if (prob == 0.f) continue;
-        if (len(color) == 0.f) continue;
-        f3 contrib = muls(divs(color, prob), w);
-        uint32_t target = p;
-        if (e == 0) {  // light tracing: splat to the pixel the camera sees the point in
-            const f3 v = sub(lc.o, cam.pos);
-            const float vfd = dot(v, cam.front);
-            const float scale = cam.dist / vfd;
-            const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
-            const float ry = (float)(cam.H / 2.0 - (double)(dot(v, cam.top) * scale));
-            const int x = (int)rx, y = (int)ry;  // checkPixelBound truncates (camera.cpp:164-170)
-            if (!(x >= 0 && y >= 0 && x < (int)cam.W && y < (int)cam.H)) continue;
-            target = (uint32_t)(y * (int)cam.W + x);
-            const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
-            contrib = muls(contrib, factor / (float)npix);
+            for (uint32_t step = 32; step > 0; step >>= 1)
+                if (T.upto[o + step - 1] <= t) o += step;
+            const uint32_t r = o ? t - T.upto[o - 1] : t;
+            const uint64_t lights = T.light[o];
+            const uint32_t nl = (uint32_t)__popcll(lights);
+            const int e = nth_bit(T.eye[o], r / nl), c = nth_bit(lights, r % nl);
+            const uint64_t lane = lane0 + o;
+            const uint32_t p = (uint32_t)(lane % npix);
+            k = (uint32_t)(lane / npix);
+            const size_t ei = lane * 2 * maxv, li = ei + maxv;
+            BVert lc = verts[li + c];
+            ec = verts[ei + e];
+            if (!connect_edge(S, verts + li, c, verts + ei, e, lc, ec)) return false;
+            const VcmTerms vt{grids ? grids[k].r : 0.f, (double)npix, false};
+            f3 color;
+            float prob;
+            const float w = color_prob_weight(S, cam, p, lc, prefix[li + c], c, ec, prefix[ei + e], e, color, prob,
+                                              grids ? &vt : nullptr);
+            if (prob == 0.f) return false;
+            if (len(color) == 0.f) return false;
+            contrib = muls(divs(color, prob), w);
+            target = p;
+            if (e == 0) {  // light tracing: splat to the pixel the camera sees the point in
+                const f3 v = sub(lc.o, cam.pos);
+                const float vfd = dot(v, cam.front);
+                const float scale = cam.dist / vfd;
+                const float rx = (float)(cam.W / 2.0 + (double)(dot(v, cam.right) * scale));
+                const float ry = (float)(cam.H / 2.0 - (double)(dot(v, cam.top) * scale));
+                const int x = (int)rx, y = (int)ry;  // checkPixelBound truncates (camera.cpp:164-170)
+                if (!(x >= 0 && y >= 0 && x < (int)cam.W && y < (int)cam.H)) return false;
+                target = (uint32_t)(y * (int)cam.W + x);
+                const float factor = (float)(1.0 / (double)pixel_solid_angle(cam, target));
+                contrib = muls(contrib, factor / (float)npix);
+            }
+            dist = len(sub(ec.o, lc.o));
+            return true;
+        };
+        const bool want = t0 + wl < total && connect(t0 + wl);
+        const uint64_t m = __ballot(want);
+        if (m == 0) continue;
+        // the slots: what is left of the wave's reservation, then of a new one
+        // for as many more entries as its pairs so far let expect
+        const uint32_t n = (uint32_t)__popcll(m), avail = kept_end - kept;
+        used += n;
+        uint32_t first = kept, fresh = 0;
+        if (n > avail) {
+            const uint32_t seen = min(t0 + 64, total);
+            const uint32_t take = n - avail + min((uint32_t)((uint64_t)(total - seen) * used / seen), kReserve);
+            if (wl == 0) fresh = atomicAdd(Q.count, take);
+            fresh = __shfl(fresh, 0, 64);
+            kept = fresh + (n - avail);
+            kept_end = fresh + take;
+        } else {
+            kept += n;
         }
+        if (!want) continue;
+        const uint32_t rank = (uint32_t)__popcll(m & ((1ull << wl) - 1ull));
+        const uint32_t slot = rank < avail ? first + rank : fresh + (rank - avail);
         // MCRenderer::visibilityTest from the eye-side connection record
         const uint32_t contact = (ec.flags & kVCamera) ? kCameraObj : ec.contact;
-        const float dist = len(sub(ec.o, lc.o));
-        const uint32_t slot = wave_slot(Q.count);
         if (slot < Q.cap) {
             uint32_t* ray = Q.rays + 8 * (size_t)slot;
             ray[0] = __float_as_uint(ec.o.x); ray[1] = __float_as_uint(ec.o.y); ray[2] = __float_as_uint(ec.o.z);
@@ -632,20 +657,30 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
             if (nee_visible(h.rec, h.t, dist)) atomic_add3(pix_all + 3 * (size_t)k * npix, target, contrib);
         }
     }
+    // slots reserved for more entries than came: rays that leave the scene, contributing nothing
+    for (uint32_t slot = kept + wl; slot < min(kept_end, Q.cap); slot += 64) {
+        uint32_t* ray = Q.rays + 8 * (size_t)slot;
+        for (int a = 0; a < 6; a++) ray[a] = __float_as_uint(a < 3 ? 1e18f : 1.f);
+        ray[6] = ray[7] = WR_NONE;
+        float* y = Q.pay + 4 * (size_t)slot;
+        y[0] = y[1] = y[2] = y[3] = 0.f;
+        Q.dst[slot] = WR_NONE;
+    }
     return own;
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt(
     SceneDev S, CamDev cam, uint32_t npass, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* prefix,
-    const uint32_t* counts, float* pix_all, VisQueue Q) {
+    const uint32_t* counts, float* pix_all, VisQueue Q, uint32_t width) {
     __shared__ PairTable tables[4];
-    const uint64_t lane = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool valid = lane < (uint64_t)npass * npix;
+    const uint32_t wl = threadIdx.x & 63u;
+    const uint64_t lane0 = (uint64_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * width, lane = lane0 + wl;
+    const bool valid = wl < width && lane < (uint64_t)npass * npix;
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
     const uint32_t ne = valid ? counts[2 * lane] : 0u, nl = valid ? counts[2 * lane + 1] : 0u;
-    const f3 own = connect_wave(S, sc, cam, npix, maxv, lane & ~63ull, verts, prefix, (int)min(ne, maxv),
+    const f3 own = connect_wave(S, sc, cam, npix, maxv, lane0, verts, prefix, (int)min(ne, maxv),
                                 (int)min(nl, maxv), pix_all, Q, st, nullptr, tables[threadIdx.x >> 6]);
     if (valid) atomic_add3(pix_all + 3 * (size_t)(lane / npix) * npix, (uint32_t)(lane % npix), own);
 }
@@ -794,13 +829,14 @@ __device__ __forceinline__ f3 vcm_merge(const SceneDev& S, const CamDev& cam, ui
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm(SceneDev S, CamDev cam, uint32_t npix, uint32_t npass, uint32_t maxv,
                                              const BVert* verts, const BPrefix* prefix, const uint32_t* counts,
-                                             float* pix_all, VisQueue Q, const VcmGrid* grids, MergeQueue M) {
+                                             float* pix_all, VisQueue Q, const VcmGrid* grids, MergeQueue M, uint32_t width) {
     // every lane of a wave stays to the end (the merge reservations below are
     // wave-wide scans); a lane past the last one stands in for lane 0 and does
     // nothing
-    const uint64_t lane_id = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool valid = lane_id < (uint64_t)npass * npix;
-    const uint64_t lane = valid ? lane_id : 0;
+    const uint32_t wl = threadIdx.x & 63u;
+    const uint64_t lane0 = (uint64_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * width;
+    const bool valid = wl < width && lane0 + wl < (uint64_t)npass * npix;
+    const uint64_t lane = valid ? lane0 + wl : 0;
     const uint32_t kb = (uint32_t)(lane / npix), p = (uint32_t)(lane % npix);
     const VcmGrid G = grids[kb];
     float* pix = pix_all + 3 * (size_t)kb * npix;
@@ -812,7 +848,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int max_eye = (int)(ne < maxv ? ne : maxv), max_light = (int)(nl < maxv ? nl : maxv);
     // throughputByConnecting (vcmTracer.cpp:88-173): k_bdpt's connections with vcmMisWeight
     __shared__ PairTable tables[4];
-    f3 own = connect_wave(S, sc, cam, npix, maxv, lane_id & ~63ull, verts, prefix, valid ? max_eye : 0,
+    f3 own = connect_wave(S, sc, cam, npix, maxv, lane0, verts, prefix, valid ? max_eye : 0,
                           valid ? max_light : 0, pix_all, Q, st, grids, tables[threadIdx.x >> 6]);
     // throughputByMerging (vcmTracer.cpp:175-217): the light points within the
     // radius of every non-delta eye vertex before an emitter, in the grid's
@@ -820,7 +856,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // nothing.  Each merge is queued for k_vcm_merge: per eye vertex the lane
     // counts its points in reach, the wave reserves their slots with one
     // atomic (an exclusive scan of the counts), and the lane writes them.
-    const uint32_t wl = threadIdx.x & 63u;
     uint32_t* mcount = M.ent + 2 * (size_t)M.cap;
     bool alive = valid;
     for (int i = 1; i < (int)maxv; i++) {
@@ -1146,6 +1181,20 @@ static int check_grids(wr_ctx* ctx, uint32_t err, const char* who) {
     return fail(ctx, WR_EINVAL, std::string(who) + ": too many cells across the light points' box for this radius");
 }
 
+// Lanes (pixel and pass) of each wave of the connection kernels: fewer than 64
+// while that leaves fewer than `waves` waves, so that a small image fills the
+// chip (the lanes without a pixel still take their share of the pairs).  Cornell
+// 64x64, 1 pass: BidirectionalPathTracer 1,018 -> 916 us, VCMTracer 1,615 ->
+// 1,278 us; 100x100, 2 passes, VCMTracer 2.01 -> 1.81 ms.  k_vcm's merges are a
+// lane's own: with its line at 4,096 waves 256x256, 4 passes took 7.5 ms, 7.1 at 1,024.
+constexpr uint64_t kBdptWaves = 2048, kVcmWaves = 1024;
+
+static uint32_t connect_width(uint64_t lanes, uint64_t waves) {
+    uint32_t width = 64;
+    while (width > 4 && lanes < waves * width) width /= 2;
+    return width;
+}
+
 int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
                       uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts,
                       float* pix, const BdptQueue& q, const VcmBufs& vb, const FilmBufs& film) {
@@ -1153,7 +1202,6 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     const wrd::CamDev cam = make_cam_dev(ch);
     const uint32_t npix = ch.W * ch.H;
     const uint32_t lanes = npass * npix;
-    const uint32_t blocks = (lanes + 255) / 256;
     wrd::BVert* V = (wrd::BVert*)verts;
     hipError_t e = hipMemsetAsync(pix, 0, sizeof(float) * 3 * (size_t)lanes, st);
     if (e == hipSuccess) e = hipMemsetAsync(q.count, 0, sizeof(uint32_t), st);
@@ -1168,8 +1216,9 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     const wrd::MergeQueue M{vb.mq, vb.mq_cap};
     e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
-    wrd::k_vcm<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q,
-                                                        (const wrd::VcmGrid*)vb.grids, M);
+    const uint32_t width = connect_width(lanes, kVcmWaves);
+    wrd::k_vcm<<<(lanes + 4 * width - 1) / (4 * width), 256, wrd::kStackLdsBytes, st>>>(
+        S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q, (const wrd::VcmGrid*)vb.grids, M, width);
     e = hipGetLastError();
     if (e == hipSuccess) {
         wrd::k_vcm_merge<<<4096, 256, 0, st>>>(S, cam, npix, maxv, V, prefix, pix, M, (const wrd::VcmGrid*)vb.grids);
@@ -1241,14 +1290,14 @@ hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr&
     if (e == hipSuccess) e = hipMemsetAsync(q.count, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return e;
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
-    const uint32_t blocks = (uint32_t)((lanes + 255) / 256);
     e = run_subpaths(ctx, S, H, cam, max_depth, seed, pass0, (uint32_t)lanes, npix, maxv, (wrd::BVert*)verts, q.counts,
                      true);
     if (e != hipSuccess) return e;
     wrd::k_bdpt_prefix<<<(uint32_t)((2 * lanes + 255) / 256), 256, 0, st>>>(
         S, cam, npix, (uint32_t)lanes, maxv, (const wrd::BVert*)verts, q.counts, (wrd::BPrefix*)q.prefix);
-    wrd::k_bdpt<<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, cam, npass, npix, maxv, (const wrd::BVert*)verts,
-                                                         (const wrd::BPrefix*)q.prefix, q.counts, pix, Q);
+    const uint32_t width = connect_width(lanes, kBdptWaves);
+    wrd::k_bdpt<<<(uint32_t)((lanes + 4 * width - 1) / (4 * width)), 256, wrd::kStackLdsBytes, st>>>(
+        S, cam, npass, npix, maxv, (const wrd::BVert*)verts, (const wrd::BPrefix*)q.prefix, q.counts, pix, Q, width);
     uint32_t nq = 0;
     e = hipMemcpyAsync(&nq, q.count, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
