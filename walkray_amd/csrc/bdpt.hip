@@ -514,7 +514,8 @@ __device__ __forceinline__ int nth_bit(uint64_t mask, uint32_t n) {
 // counter bounds the connections: with an atomic of each wave for every 64
 // pairs k_bdpt took 1.6 ms for Cornell 256^2 x 8 passes (5.9M entries), of which
 // its arithmetic is 0.6 ms.  With the expected number of entries reserved at
-// once (slots that stay empty hold rays that leave the scene) the render takes 4.97 ms instead of 6.04; 192 ahead instead of 448: 5.00 ms.
+// once (slots that stay empty hold rays that leave the scene) the render takes
+// 4.97 ms instead of 6.04; 192 ahead instead of 448: 5.00 ms.
 constexpr uint32_t kReserve = 448;
 
 // The pairs of records that a wave's lanes connect, for connect_wave.
