@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "grid_dev.h"
+#include "merge_entry.h"
 #include "pt_dev.h"
 #include "walk_dev.h"
 #include "wr_pt.h"
@@ -801,9 +802,9 @@ __global__ void k_vcm_pass_starts(const uint32_t* offs, uint32_t npix, uint32_t 
 }
 
 // The merges of the VCM lanes, one entry per light point in reach of an eye
-// vertex: word 0 = lane | eye vertex << 24 (lanes < 2^22), word 1 = the light
-// point; count at ent[2 * cap].  A separate kernel takes one merge per lane, so
-// the uneven number of merges per pixel does not leave most lanes of a wave idle.
+// vertex: word 0 the eye vertex (merge_entry.h), word 1 the light point; count
+// at ent[2 * cap].  A separate kernel takes one merge per lane, so the uneven
+// number of merges per pixel does not leave most lanes of a wave idle.
 struct MergeQueue {
     uint32_t* ent;
     uint32_t cap;
@@ -907,7 +908,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     if (!pass2) {
                         cnt++;
                     } else if (k < M.cap) {
-                        M.ent[2 * (size_t)k] = (uint32_t)lane | ((uint32_t)i << 24);
+                        M.ent[2 * (size_t)k] = wr::merge_entry((uint32_t)lane, (uint32_t)i, maxv);
                         M.ent[2 * (size_t)k + 1] = pi;
                         k++;
                     } else {  // queue full: merge here
@@ -930,8 +931,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const uint32_t n = min(M.ent[2 * (size_t)M.cap], M.cap);
     for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
         const uint32_t w0 = M.ent[2 * (size_t)e], pi = M.ent[2 * (size_t)e + 1];
-        const uint32_t lane = w0 & 0xFFFFFFu;
-        const int i = (int)(w0 >> 24);
+        const uint32_t lane = wr::merge_lane(w0, maxv);
+        const int i = (int)wr::merge_vertex(w0, maxv);
         const uint32_t kb = lane / npix, p = lane % npix;
         const f3 c = vcm_merge(S, cam, npix, maxv, verts, prefix, grids[kb], lane, i, pi);
         if (c.x != 0.f || c.y != 0.f || c.z != 0.f) atomic_add3(pix_all + 3 * (size_t)kb * npix, p, divs(c, (float)npix));
