@@ -66,3 +66,20 @@ def test_persistent_launch_choices(field, tuning):
         _check(sc.closest_hit(rays[:333], counters=True)[0], ref, idx[:333], f"{tuning} counted")
     finally:
         sc.set_closest_hit_tuning(16, 32)
+
+
+@pytest.mark.parametrize("n_objects", [24, 100])  # on both sides of the tree size where NoSelf batches change their order
+@pytest.mark.parametrize("n", [49152, 49153, 65537, 98305, 196608, 196609])
+def test_noself_orders(ctx, field, n_objects, n):
+    """The one-launch NoSelf batch at the sizes where its lanes per wave and the order of its rays change.
+    The larger scene's rays are compared with the same rays in small batches."""
+    idx = np.arange(n) % BASE
+    if n_objects == 24:
+        sc, path, inside, contact, ref = (field[k] for k in (0, 3, 4, 5, 6))
+        _check(sc.closest_hit_noself(path[idx], inside[idx], contact[idx]), ref, idx, f"{n} NoSelf rays")
+        return
+    objs, _ = S.random_field(n_objects=n_objects, seed=8)
+    assert sum(len(o["tris"]) for o in objs) > 81920
+    sc, path, contact = W.Scene(ctx, objs), field[3], np.full(BASE, O.NONE, np.uint32)
+    base = sc.closest_hit_noself(path, contact, contact)
+    _check(sc.closest_hit_noself(path[idx], contact[idx], contact[idx]), base, idx, f"{n} NoSelf rays")

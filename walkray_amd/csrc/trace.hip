@@ -231,8 +231,9 @@ __global__ __launch_bounds__(256) void k_closest_hit_finish(SceneDev S, wr_tree_
 template <bool NOSELF>
 __global__ __launch_bounds__(256) void k_closest_hit_small(SceneDev S, wr_tree_hdr H,
                                                            const uint32_t* __restrict__ rays, uint64_t n,
-                                                           uint32_t width, uint4* __restrict__ hits) {
-    const uint32_t lane = threadIdx.x & 63u, wave = blockIdx.x * 4 + (threadIdx.x >> 6);
+                                                           uint32_t width, bool by_xcd, uint4* __restrict__ hits) {
+    const uint32_t block = by_xcd ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, wave = block * 4 + (threadIdx.x >> 6);
     const uint64_t i = (uint64_t)wave * width + lane;
     if (lane >= width || i >= n) return;
     StackSpill spill;
@@ -413,6 +414,19 @@ constexpr uint64_t kSmallWaves = 4096;
 template <bool NOSELF>
 constexpr uint64_t kSmallMax = NOSELF ? 1ull << 21 : 1ull << 19;
 
+// NoSelf batches continue paths: neighbouring rays start near each other, their
+// normals leave the kernel 5 waves per SIMD, and in a small tree they mostly
+// read what the XCD's L2 already holds.  There, between these numbers of rays,
+// full waves in the order in which each XCD walks its own range are the faster:
+// 100,000 rays on 16 / 40 / 64 objects 50 / 61 / 68 us so, 58 / 67 / 73 us spread
+// (150,000: 55 / 65 / 74 and 65 / 74 / 83); from 200,000 rays on, or from 100
+// objects (96,000 triangles) on, spreading is.
+constexpr uint64_t kLocalMin = 49152, kLocalMax = 196608;
+constexpr uint32_t kLocalTris = 81920;
+// In a larger tree eight lanes a wave up to this number of rays (two rounds of
+// the waves that fit): 50,000 rays on 512 objects 86 us, 104 with sixteen.
+constexpr uint64_t kNarrowMax = 65536;
+
 template <bool NOSELF, int D>
 static hipError_t launch_closest_hit_d(const SceneDev& S, const wr_tree_hdr& H, const uint32_t* rays, uint64_t n,
                                        void* hits, unsigned long long* counters, unsigned long long* work,
@@ -423,9 +437,12 @@ static hipError_t launch_closest_hit_d(const SceneDev& S, const wr_tree_hdr& H, 
         // the power of two nearest to the rays per wave
         uint32_t width = 1;
         while (width < 64 && 2 * n > 3ull * width * kSmallWaves) width *= 2;
+        const bool by_xcd = NOSELF && H.n_recs <= kLocalTris && n > kLocalMin && n <= kLocalMax;
+        if (by_xcd) width = 64;
+        else if (NOSELF && n <= kNarrowMax) width = std::min(width, 8u);
         const uint64_t waves = (n + width - 1) / width;
         wrd::k_closest_hit_small<NOSELF>
-            <<<(uint32_t)((waves + 3) / 4), 256, wrd::kStackLdsBytes, st>>>(S, H, rays, n, width, out);
+            <<<(uint32_t)((waves + 3) / 4), 256, wrd::kStackLdsBytes, st>>>(S, H, rays, n, width, by_xcd, out);
         return hipGetLastError();
     }
     const uint32_t pgrid = persistent_blocks<NOSELF, D>(n, per_cu);
