@@ -29,3 +29,15 @@ def test_paths_per_wave(ctx, width, height, spp, slots, nee):
         films.append(film.read())
     for k in ("sum", "comp", "sumsq"):
         assert np.array_equal(films[0][k].view(np.uint32), films[1][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("nee", [False, True])
+def test_small_pool_is_refilled(ctx, nee):
+    """A pool much smaller than a pass takes new paths as others end; only the last are taken to their ends
+    in one iteration.  (An iteration that ended every path of a full pool would make one turn per pool of
+    paths and wait for the longest path each time; a path of the Cornell box has three segments or more.)"""
+    objs, cam = S.cornell(k=2, width=400, height=300)
+    slots = 16384
+    st = W.render(W.Scene(ctx, objs), cam, W.Film(ctx, 400, 300), 2, 8, 5, W.WR_WAVEFRONT, wave_slots=slots, nee=nee)
+    turns = -(-st["paths"] // slots)
+    assert st["iterations"] > 1.5 * turns, (st["iterations"], turns)

@@ -898,7 +898,8 @@ hipError_t Engine::init(uint32_t want_cap, uint32_t want_grid, hipStream_t st, u
     const size_t trace_lds = lds_levels == 4 ? stack_lds_bytes<4>() : lds_levels == 16 ? stack_lds_bytes<16>()
                                                                                        : stack_lds_bytes<8>();
     WR_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trace_fn, 256, trace_lds));
-    trace_grid = (uint32_t)std::max(1, std::min<int>(cus * std::max(per_cu, 1), (int)(cap / 256)));
+    // (at most what cap paths of one unit each can use, as k_wf_trace counts them)
+    trace_grid = (uint32_t)std::min<uint64_t>((uint64_t)cus * std::max(per_cu, 1), ((uint64_t)cap + 31) / 32 * 8);
     ready = true;
     return hipSuccess;
 }
@@ -927,6 +928,14 @@ hipError_t Engine::ensure_graphs(hipStream_t st, bool nee) {
     return hipSuccess;
 }
 
+// Live paths up to which an iteration takes them to their ends: at most
+// kWaveFew; no more than the last workgroups of the grid reach; and never a full
+// pool, which has others waiting for its slots (a pool of kWaveFew slots or
+// fewer would do nothing else, each round waiting for its longest path: field
+// 640x360, 8 spp, next-event, with pools of 16,384 / 65,536 / 131,072 slots 68 /
+// 31 / 22.6 ms so, 39 / 15.4 / 11.4 ms refilled).
+uint32_t Engine::few() const { return std::min<uint32_t>({kWaveFew, grid * 256, cap - 1}); }
+
 static EngineDev engine_dev(const Engine& En) {
     EngineDev E;
     E.buf[0] = to_pathbuf(En.words[0]);
@@ -937,8 +946,7 @@ static EngineDev engine_dev(const Engine& En) {
     E.scenes = En.scenes;
     E.exit_list = En.exit_list;
     E.cap = En.cap;
-    // the last workgroups of the grid must reach the last of the few paths
-    E.few = std::min<uint32_t>(kWaveFew, En.grid * 256);
+    E.few = En.few();
     return E;
 }
 
@@ -1125,7 +1133,7 @@ static hipError_t run_wavefront_once(const SceneDev& S, const CamHost& cam, uint
     // (with per-stage events every replay is read back on its own); few enough
     // to be taken to their ends by the second iteration, a tail replay is all
     const bool at_once = total <= E.cap && npass <= J.R && !ev;
-    bool tail = at_once && total <= std::min<uint32_t>(kWaveFew, E.grid * 256);
+    bool tail = at_once && total <= E.few();
     bool chain_tail = at_once && !tail;
     uint64_t iters = 0;
     JobCtl& back = *E.ctl_back;

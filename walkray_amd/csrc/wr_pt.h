@@ -143,6 +143,7 @@ struct Engine {
     bool ready = false;  // buffers allocated and zeroed for (cap, grid, lds_levels)
     hipError_t init(uint32_t cap, uint32_t grid, hipStream_t st, uint32_t lds_levels = 8);
     hipError_t ensure_graphs(hipStream_t st, bool nee);
+    uint32_t few() const;  // live paths up to which an iteration takes them to their ends (k_wf_rest)
     hipError_t set_scene(uint32_t slot, const SceneDev& S, hipStream_t st);
     hipError_t admit(uint32_t slot, const JobDesc& J, hipStream_t st, const SceneDev* scene = nullptr);  // scene: into scene slot 0
     hipError_t release_slot(uint32_t slot, hipStream_t st);
