@@ -30,6 +30,12 @@ namespace wr {
 // 16,384 paths, 1.91 up to 32,768, 1.79 up to 65,536 and 131,072, where
 // PhotonMap loses 1.5%.
 constexpr uint32_t kWalkFew = 65536;
+// List steps of a walk: every step of the renderers (maxPathLen up to 32).  A
+// longer walk's paths that are still alive then are taken to their ends like
+// the last few, so that a call's launches do not grow with its path length:
+// 1,000 light paths of at most 1,000 scatters launched 2,000 kernels that found
+// nothing to do, 10 ms.
+constexpr uint32_t kWalkListSteps = 33;
 }  // namespace wr
 
 namespace wrd {
@@ -75,32 +81,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // Step s: completes every live path's hit and takes the path one vertex on.
 // P::step(sc, path, s, o, d, hit, st, out): the vertex at the hit (hit.rec
 // WR_NONE: the ray escaped); true if the path goes on with out.
+// last: the walk's last launch, which takes any number of paths to their ends.
 template <class P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_shade(SceneDev S, P policy,
-                                                                                           WalkLists W, uint32_t s) {
+                                                                                           WalkLists W, uint32_t s,
+                                                                                           bool last) {
     const uint32_t n = W.n[s];
     if (blockIdx.x == 0) UnitQueue::clear(W.work);  // for the next step's trace
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
-    if (n <= wr::kWalkFew) {  // the rest of every path, the trace included
-        uint32_t width = 1;   // lanes of a wave that take a path
+    if (n <= wr::kWalkFew || last) {  // the rest of every path, the trace included
+        uint32_t width = 1;           // lanes of a wave that take a path
         while (width < 64 && (uint64_t)width * gridDim.x * 4 < n) width *= 2;
         const uint32_t lane = threadIdx.x & 63u;
-        const uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane;
-        if (lane >= width || i >= n) return;
-        const uint32_t path = W.path[s & 1][i];
-        const uint32_t* rp = W.rays[s & 1] + 8 * (size_t)i;
-        Out out;
-        out.o = mk(__uint_as_float(rp[0]), __uint_as_float(rp[1]), __uint_as_float(rp[2]));
-        out.d = mk(__uint_as_float(rp[3]), __uint_as_float(rp[4]), __uint_as_float(rp[5]));
-        out.inside = rp[6];
-        out.contact = rp[7];
-        for (uint32_t k = s;; k++) {
-            const f3 o = out.o, d = out.d;
-            const PHit hit = trace_scene<true>(sc, o, d, out.inside, out.contact, st);
-            if (!policy.step(sc, path, k, o, d, hit, st, out)) return;
+        if (lane >= width) return;
+        for (uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane; i < n; i += gridDim.x * 4 * width) {
+            const uint32_t path = W.path[s & 1][i];
+            const uint32_t* rp = W.rays[s & 1] + 8 * (size_t)i;
+            Out out;
+            out.o = mk(__uint_as_float(rp[0]), __uint_as_float(rp[1]), __uint_as_float(rp[2]));
+            out.d = mk(__uint_as_float(rp[3]), __uint_as_float(rp[4]), __uint_as_float(rp[5]));
+            out.inside = rp[6];
+            out.contact = rp[7];
+            for (uint32_t k = s;; k++) {
+                const f3 o = out.o, d = out.d;
+                const PHit hit = trace_scene<true>(sc, o, d, out.inside, out.contact, st);
+                if (!policy.step(sc, path, k, o, d, hit, st, out)) break;
+            }
         }
+        return;
     }
     for (uint32_t i0 = blockIdx.x * 256; i0 < n; i0 += gridDim.x * 256) {
         const uint32_t i = i0 + threadIdx.x;
@@ -160,22 +170,25 @@ hipError_t run_walk(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const 
         chunk /= 4;
     }
     if (e != hipSuccess) return e;
-    if ((e = mem.get(&W.n, sizeof(uint32_t) * (steps + 1))) != hipSuccess) return e;
+    const uint32_t lists_max = steps < kWalkListSteps ? steps : kWalkListSteps;
+    if ((e = mem.get(&W.n, sizeof(uint32_t) * (lists_max + 1))) != hipSuccess) return e;
     for (int k = 0; k < 2; k++) W.rays[k] = (uint32_t*)(lists + 32ull * chunk * k);
     W.hits = (uint4*)(lists + 64ull * chunk);
     for (int k = 0; k < 2; k++) W.path[k] = (uint32_t*)(lists + (80ull + 4 * k) * chunk);
     for (uint32_t p = 0; p < n_paths;) {
         const uint32_t n = n_paths - p < chunk ? n_paths - p : chunk;
         const uint32_t blocks = (n + 255) / 256;
-        if ((e = hipMemsetAsync(W.n, 0, sizeof(uint32_t) * (steps + 1), st)) != hipSuccess) return e;
+        if ((e = hipMemsetAsync(W.n, 0, sizeof(uint32_t) * (lists_max + 1), st)) != hipSuccess) return e;
         // at least one wave per SIMD for a few paths' ends
         const uint32_t shade = blocks < 256 ? 256 : (blocks < 2048 ? blocks : 2048);
         wrd::k_walk_begin<P><<<blocks, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, p, n);
-        for (uint32_t s = 0; s < steps; s++) {
+        const uint32_t list_steps = n <= kWalkFew ? 0 : lists_max;  // a few paths end in the first shade
+        for (uint32_t s = 0; s < list_steps; s++) {
             e = launch_walk_trace(S, H, W.rays[s & 1], W.n + s, n, W.hits, W.work, st);
             if (e != hipSuccess) return e;
-            wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s);
+            wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s, false);
         }
+        if (list_steps < steps) wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, list_steps, true);
         p += n;
     }
     return hipGetLastError();
