@@ -730,7 +730,8 @@ class Scene:
         return {"refill_min": t.refill_min, "node_phase_min": t.node_phase_min, "blocks_per_cu": t.blocks_per_cu,
                 "lds_levels": t.lds_levels, "batch": t.batch, "ms": t.ms}
 
-    def set_closest_hit_tuning(self, refill_min, node_phase_min, blocks_per_cu=0, lds_levels=8, batch=256):
+    def set_closest_hit_tuning(self, refill_min, node_phase_min, blocks_per_cu=0, lds_levels=8, batch=0):
+        """wr_scene_set_closest_hit_tuning; batch 0 is the library's default."""
         t = ChTuning(refill_min, node_phase_min, blocks_per_cu, lds_levels, batch, 0.0)
         _check(lib().wr_scene_set_closest_hit_tuning(self.h, C.byref(t)), self.ctx.h,
                "wr_scene_set_closest_hit_tuning")
