@@ -190,7 +190,11 @@ int wr_closest_hit(wr_ctx* ctx, const wr_scene* scene, const wr_ray* d_rays, uin
  * per work-counter atomic), by coordinate descent from the
  * scene's current choice, and keeps the fastest for the scene; later
  * wr_closest_hit calls use it.  Results never depend on the configuration.
- * Synchronous; allocates 16 * n bytes of scratch while it runs. */
+ * Only batches of more than 2^19 rays run in the persistent kernel and use it
+ * (smaller ones are one launch without these choices, unless they count their
+ * traversal): with n up to 2^19 the scene's configuration is returned as it is,
+ * with the time of a call.
+ * Synchronous; takes 16 * n bytes of scratch while it runs. */
 typedef struct {
     uint32_t refill_min;     /* idle lanes of a wave before it takes new rays (1..64) */
     uint32_t node_phase_min; /* lanes at wide nodes for a node-only step (1..65; 65 = never) */

@@ -1053,16 +1053,19 @@ int wr_autotune_closest_hit(wr_ctx* ctx, wr_scene* s, const wr_ray* d_rays, uint
         return hipSuccess;
     };
     // coordinate descent over the knobs, starting from the current choice;
-    // a candidate must be 1% faster to replace it (timing noise stays put)
+    // a candidate must be 1% faster to replace it (timing noise stays put).
+    // A batch that runs as one launch reads none of them, so every difference
+    // would be noise, kept for the large batches: it leaves the choice alone.
     ChTune cur = s->ch_tune;
     float cur_ms = 0.f;
     e = time_of(cur, cur_ms);
+    const int passes = n > kClosestHitOneLaunch ? 2 : 0;
     const uint32_t nodes[] = {16, 24, 32, 40, 48, 65};
     const uint32_t refills[] = {4, 8, 16, 24, 32};
     const uint32_t blocks[] = {0, 7, 6, 5};
     const uint32_t levels[] = {4, 8, 16};
     const uint32_t batches[] = {64, 128, 256, 512};
-    for (int pass = 0; pass < 2 && e == hipSuccess; pass++) {
+    for (int pass = 0; pass < passes && e == hipSuccess; pass++) {
         for (uint32_t v : nodes) {
             ChTune t = cur;
             t.node_phase_min = v;

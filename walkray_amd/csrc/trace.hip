@@ -412,7 +412,7 @@ constexpr uint64_t kSmallWaves = 4096;
 // kernels 5 waves per SIMD, rays from camera hits cross over later: 1M
 // 181 / 255, 2M 306 / 367, 4M 564 / 555.
 template <bool NOSELF>
-constexpr uint64_t kSmallMax = NOSELF ? 1ull << 21 : 1ull << 19;
+constexpr uint64_t kSmallMax = NOSELF ? 1ull << 21 : kClosestHitOneLaunch;
 
 // NoSelf batches continue paths: neighbouring rays start near each other, their
 // normals leave the kernel 5 waves per SIMD, and in a small tree they mostly

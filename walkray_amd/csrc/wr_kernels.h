@@ -60,6 +60,9 @@ struct ChTune {
     uint32_t lds_levels = 8;       // traversal stack levels kept in LDS: 4, 8 or 16 (deeper ones spill)
     uint32_t batch = 128;          // most rays a workgroup takes from its XCD's work counter at a time (64..4096)
 };
+// Closest-hit batches of at most this many rays run as one launch, which has
+// none of ChTune's choices (trace.hip says why the line lies there).
+constexpr uint64_t kClosestHitOneLaunch = 1ull << 19;
 // The persistent traversal kernels' work counters: one per XCD, each on its
 // own 128 B line.
 constexpr uint32_t kXcds = 8;
