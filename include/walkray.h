@@ -89,6 +89,15 @@ int wr_ctx_create(int device, wr_ctx** out);
 void wr_ctx_destroy(wr_ctx* ctx);
 const char* wr_last_error(const wr_ctx* ctx);
 int wr_synchronize(wr_ctx* ctx);
+/* Work buffers that a context's calls share (scratch, films, served jobs' and
+ * grids' buffers): bytes in use, and bytes kept unused for later calls (at most
+ * 6 GiB; given back to the device when an allocation of the context fails for
+ * want of memory, and with the context). */
+int wr_ctx_work_memory(wr_ctx* ctx, uint64_t* in_use, uint64_t* unused);
+/* Test hook for calls at the end of memory: an allocation of the context that
+ * would take its work buffers past `bytes` fails as if the device had no more
+ * memory (0 = no limit). */
+int wr_ctx_limit_work_memory(wr_ctx* ctx, uint64_t bytes);
 int wr_device_alloc(wr_ctx* ctx, size_t bytes, void** d_out);
 int wr_device_free(wr_ctx* ctx, void* d_ptr);
 int wr_memcpy_htod(wr_ctx* ctx, void* d_dst, const void* src, size_t bytes);

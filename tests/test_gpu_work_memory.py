@@ -1,0 +1,70 @@
+"""The work buffers that a context keeps, at the end of device memory (wr_ctx_limit_work_memory): every
+allocation of the context gets the unused ones' memory before it fails."""
+import numpy as np
+import pytest
+
+from walkray_amd import _lib as W
+from walkray_amd import scenes as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _fill(ctx, sc, cam):
+    """Leaves the buffers of a BidirectionalPathTracer call unused."""
+    film = W.Film(ctx, cam["width"], cam["height"])
+    W.render_bdpt(sc, cam, film, 2, 4, 1)
+
+
+def _render(ctx, sc, cam, **kw):
+    W.render(sc, cam, W.Film(ctx, cam["width"], cam["height"]), 3, 4, 1, W.WR_WAVEFRONT, **kw)
+
+
+def _moving(ctx, sc, cam):
+    objs, _, motions = S.cornell_moving(k=2, width=cam["width"], height=cam["height"])
+    m = W.Scene(ctx, objs, build=False)
+    for obj, (t0, t1, a, b) in motions.items():
+        m.set_motion(obj, t0, t1, a, b)
+    m.build()
+    _render(ctx, m, cam)
+
+
+CALLS = {
+    "render": lambda ctx, sc, cam: _render(ctx, sc, cam, wave_slots=65536),
+    "moving": _moving,
+    "scene": lambda ctx, sc, cam: W.Scene(ctx, S.cornell(k=1)[0]),
+    "autotune": lambda ctx, sc, cam: sc.autotune_closest_hit(ctx.to_device(np.ones((999, 6), np.float32)), 999),
+    "server": lambda ctx, sc, cam: W.Server(ctx, path_slots=65536),
+    "alloc": lambda ctx, sc, cam: ctx.alloc(1 << 20),
+}
+
+
+@pytest.mark.parametrize("call", sorted(CALLS))
+def test_unused_buffers_are_given_back(call):
+    ctx = W.Context(0)
+    objs, cam = S.cornell(k=2, width=96, height=80)
+    sc = W.Scene(ctx, objs)
+    _fill(ctx, sc, cam)
+    used, unused = ctx.work_memory()
+    assert used == 0 and unused > 32 << 20
+    ctx.limit_work_memory(unused)  # the device has no more than the context holds
+    try:
+        CALLS[call](ctx, sc, cam)
+        assert ctx.work_memory()[1] < unused
+    finally:
+        ctx.limit_work_memory(0)
+
+
+def test_limit_is_reported():
+    """Past the limit a call fails with an error, and the next one within it succeeds."""
+    ctx = W.Context(0)
+    objs, cam = S.cornell(k=2, width=96, height=80)
+    sc = W.Scene(ctx, objs)
+    film = W.Film(ctx, 96, 80)
+    ctx.limit_work_memory(1 << 20)
+    with pytest.raises(Exception, match="memory"):
+        W.render_bdpt(sc, cam, film, 2, 4, 1)
+    with pytest.raises(Exception, match="memory"):
+        W.Film(ctx, 1000, 1000)
+    ctx.limit_work_memory(0)
+    W.render_bdpt(sc, cam, film, 2, 4, 1)
+    assert film.read()["sum"].any()

@@ -175,6 +175,8 @@ def lib():
         "wr_job_cancel": (i32, [vp, u64]),
         "wr_render_stage_stats": (i32, [vp, vp]),
         "wr_server_inject_admit_failures": (i32, [vp, u32]),
+        "wr_ctx_work_memory": (i32, [vp, vp, vp]),
+        "wr_ctx_limit_work_memory": (i32, [vp, u64]),
         "wr_hit_sources": (i32, [vp, vp, vp, u64, vp, vp]),
         "wr_server_clock": (C.c_double, [vp]),
         "wr_autotune_closest_hit": (i32, [vp, vp, vp, u64, P(ChTuning)]),
@@ -429,6 +431,16 @@ class Context:
 
     def synchronize(self):
         _check(lib().wr_synchronize(self.h), self.h, "wr_synchronize")
+
+    def work_memory(self):
+        """wr_ctx_work_memory: bytes of the shared work buffers in use, and kept unused."""
+        a, b = C.c_uint64(), C.c_uint64()
+        _check(lib().wr_ctx_work_memory(self.h, C.byref(a), C.byref(b)), self.h, "wr_ctx_work_memory")
+        return a.value, b.value
+
+    def limit_work_memory(self, nbytes):
+        """wr_ctx_limit_work_memory (test hook): allocations past nbytes of work buffers fail (0: no limit)."""
+        _check(lib().wr_ctx_limit_work_memory(self.h, nbytes), self.h, "wr_ctx_limit_work_memory")
 
     def copy(self, dst, src, nbytes):
         """Device-to-device copy (asynchronous on the context stream)."""

@@ -48,16 +48,45 @@ hipError_t WorkPool::get(void** out, size_t bytes) {
         return hipSuccess;
     }
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();  // must not surface at a later launch check
-        free_idle(0);
-        e = hipMalloc(&p, bytes);
-    }
+    const hipError_t e = malloc_trimmed(&p, bytes);
     if (e != hipSuccess) return e;
     bufs.push_back(Buf{p, bytes, true});
     *out = p;
     return hipSuccess;
+}
+
+hipError_t WorkPool::malloc_trimmed(void** out, size_t bytes) {
+    *out = nullptr;
+    hipError_t e = hipErrorOutOfMemory;
+    for (int attempt = 0; attempt < 2; attempt++) {
+        size_t total = bytes;
+        for (const Buf& b : bufs) total += b.bytes;
+        e = max_held && total > max_held ? hipErrorOutOfMemory : hipMalloc(out, bytes);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();  // must not surface at a later launch check
+        *out = nullptr;
+        if (e != hipErrorOutOfMemory) return e;
+        free_idle(0);
+    }
+    return e;
+}
+
+hipError_t WorkPool::lasting(void** out, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu);
+    return malloc_trimmed(out, std::max<size_t>(bytes, 4));
+}
+
+hipError_t device_alloc(WorkPool& pool, void** out, size_t bytes) { return pool.lasting(out, bytes); }
+
+void WorkPool::held(uint64_t* in_use, uint64_t* unused) {
+    std::lock_guard<std::mutex> lk(mu);
+    *in_use = *unused = 0;
+    for (const Buf& b : bufs) *(b.out ? in_use : unused) += b.bytes;
+}
+
+void WorkPool::limit(uint64_t bytes) {
+    std::lock_guard<std::mutex> lk(mu);
+    max_held = bytes;
 }
 
 void WorkPool::put(void* p) {
@@ -88,34 +117,17 @@ void WorkPool::free_idle(size_t keep) {
     }
 }
 
-void WorkPool::trim() {
-    std::lock_guard<std::mutex> lk(mu);
-    free_idle(0);
-}
-
 void WorkPool::close() {
     std::lock_guard<std::mutex> lk(mu);
     closed = true;
     free_idle(0);
 }
 
-// hipMalloc; when the device is out of memory, once more without the
-// context's unused buffers.
-static hipError_t alloc_trimmed(wr_ctx* ctx, void** p, size_t bytes) {
-    hipError_t e = hipMalloc(p, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        ctx->pool->trim();
-        e = hipMalloc(p, bytes);
-    }
-    return e;
-}
-
 template <class T>
 static int upload(wr_ctx* ctx, const T* v, size_t n, T** d, uint64_t& bytes) {
     *d = nullptr;
     const size_t b = std::max<size_t>(n, 1) * sizeof(T);
-    hipError_t e = alloc_trimmed(ctx, (void**)d, b);
+    hipError_t e = ctx->pool->lasting((void**)d, b);
     if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(scene)");
     bytes += b;
     if (n) {
@@ -190,7 +202,9 @@ int wr_ctx_create(int device, wr_ctx** out) {
         return hip_fail(nullptr, e, "hipStreamCreate");
     if ((e = hipEventCreate(&c->ev0)) != hipSuccess) return hip_fail(nullptr, e, "hipEventCreate");
     if ((e = hipEventCreate(&c->ev1)) != hipSuccess) return hip_fail(nullptr, e, "hipEventCreate");
-    if ((e = hipMalloc(&c->d_work, wr::kWorkWords * sizeof(unsigned long long))) != hipSuccess) return hip_fail(nullptr, e, "hipMalloc");
+    c->engine.pool = c->pool.get();
+    if ((e = c->pool->lasting((void**)&c->d_work, wr::kWorkWords * sizeof(unsigned long long))) != hipSuccess)
+        return hip_fail(nullptr, e, "hipMalloc");
     if ((e = hipMemset(c->d_work, 0, wr::kWorkWords * sizeof(unsigned long long))) != hipSuccess) return hip_fail(nullptr, e, "hipMemset");
     if ((e = wr::noalloc_scratch_init(device)) != hipSuccess) return hip_fail(nullptr, e, "hipGetSymbolAddress(scratch)");
     *out = c.release();
@@ -210,6 +224,18 @@ void wr_ctx_destroy(wr_ctx* ctx) {
     delete ctx;
 }
 
+int wr_ctx_work_memory(wr_ctx* ctx, uint64_t* in_use, uint64_t* unused) {
+    if (!ctx || !in_use || !unused) return fail(ctx, WR_EINVAL, "wr_ctx_work_memory: bad argument");
+    ctx->pool->held(in_use, unused);
+    return WR_OK;
+}
+
+int wr_ctx_limit_work_memory(wr_ctx* ctx, uint64_t bytes) {
+    if (!ctx) return fail(nullptr, WR_EINVAL, "wr_ctx_limit_work_memory: ctx is NULL");
+    ctx->pool->limit(bytes);
+    return WR_OK;
+}
+
 int wr_synchronize(wr_ctx* ctx) {
     if (!ctx) return fail(nullptr, WR_EINVAL, "wr_synchronize: ctx is NULL");
     hipError_t e = hipStreamSynchronize(ctx->stream);
@@ -220,7 +246,7 @@ int wr_synchronize(wr_ctx* ctx) {
 int wr_device_alloc(wr_ctx* ctx, size_t bytes, void** d_out) {
     if (!ctx || !d_out) return fail(ctx, WR_EINVAL, "wr_device_alloc: bad argument");
     (void)hipSetDevice(ctx->device);
-    hipError_t e = alloc_trimmed(ctx, d_out, std::max<size_t>(bytes, 1));
+    hipError_t e = ctx->pool->lasting(d_out, bytes);
     if (e != hipSuccess) return fail(ctx, WR_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return WR_OK;
 }
@@ -404,6 +430,7 @@ RebuildCache::~RebuildCache() {
 static hipError_t refit_on_device(RebuildCache& C, const wr_scene* built, size_t ti, wr_wnode* d_wnodes,
                                   const wr_tree_hdr& h, const wr_tri* d_tris, hipStream_t st) {
     const FlatTree& prev = built->trees[ti];
+    WorkPool& pool = *built->ctx->pool;
     if (C.d_order.size() < built->trees.size()) {
         C.d_order.resize(built->trees.size(), nullptr);
         C.level_start.resize(built->trees.size());
@@ -411,7 +438,7 @@ static hipError_t refit_on_device(RebuildCache& C, const wr_scene* built, size_t
     hipError_t e = hipSuccess;
     if (!C.d_order[ti]) {
         const std::vector<uint32_t> order = wide_levels(prev, C.level_start[ti]);
-        e = hipMalloc((void**)&C.d_order[ti], std::max<size_t>(order.size(), 1) * sizeof(uint32_t));
+        e = pool.lasting((void**)&C.d_order[ti], order.size() * sizeof(uint32_t));
         if (e != hipSuccess) return e;
         if (!order.empty())
             e = hipMemcpy(C.d_order[ti], order.data(), order.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -422,14 +449,14 @@ static hipError_t refit_on_device(RebuildCache& C, const wr_scene* built, size_t
         if (C.d_rec_of) (void)hipFree(C.d_rec_of);
         C.d_rec_of = nullptr;
         C.rec_cap = 0;
-        if ((e = hipMalloc((void**)&C.d_rec_of, nr * sizeof(uint32_t))) != hipSuccess) return e;
+        if ((e = pool.lasting((void**)&C.d_rec_of, nr * sizeof(uint32_t))) != hipSuccess) return e;
         C.rec_cap = nr;
     }
     if (C.box_cap < 6 * nw) {
         if (C.d_nbox) (void)hipFree(C.d_nbox);
         C.d_nbox = nullptr;
         C.box_cap = 0;
-        if ((e = hipMalloc((void**)&C.d_nbox, 6 * nw * sizeof(float))) != hipSuccess) return e;
+        if ((e = pool.lasting((void**)&C.d_nbox, 6 * nw * sizeof(float))) != hipSuccess) return e;
         C.box_cap = 6 * nw;
     }
     WideRefit R;
@@ -782,7 +809,7 @@ int scene_build(wr_scene* s, const wr_scene* reuse) {
             uint64_t built_wide = 0;
             for (const wr_tree_hdr& bh : reuse->hdrs) built_wide += bh.n_wide;
             if (built_wide != n_wide) return fail(ctx, WR_EINVAL, "wr_scene_build: fast-pass hierarchy size changed");
-            hipError_t e = hipMalloc((void**)&d_wnodes, std::max<uint64_t>(n_wide, 1) * sizeof(wr_wnode));
+            hipError_t e = ctx->pool->lasting((void**)&d_wnodes, std::max<uint64_t>(n_wide, 1) * sizeof(wr_wnode));
             if (e != hipSuccess) return hip_fail(ctx, e, "hipMalloc(scene)");
             s->dbufs.push_back(d_wnodes);
             bytes += std::max<uint64_t>(n_wide, 1) * sizeof(wr_wnode);
@@ -1033,7 +1060,8 @@ int wr_autotune_closest_hit(wr_ctx* ctx, wr_scene* s, const wr_ray* d_rays, uint
     if (!s->built) return fail(ctx, WR_ESTATE, "wr_autotune_closest_hit: scene not built");
     (void)hipSetDevice(ctx->device);
     void* d_hits = nullptr;
-    hipError_t e = hipMalloc(&d_hits, 16 * (size_t)n);
+    Scratch mem(*ctx->pool);
+    hipError_t e = mem.get(&d_hits, 16 * (size_t)n);
     if (e != hipSuccess) return fail(ctx, WR_ENOMEM, std::string("wr_autotune_closest_hit: ") + hipGetErrorString(e));
     // time of one call under t: best of three after one warm-up call
     auto time_of = [&](const ChTune& t, float& ms) -> hipError_t {
@@ -1106,7 +1134,6 @@ int wr_autotune_closest_hit(wr_ctx* ctx, wr_scene* s, const wr_ray* d_rays, uint
             if (m < 0.99f * cur_ms) cur = t, cur_ms = m;
         }
     }
-    (void)hipFree(d_hits);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_autotune_closest_hit");
     s->ch_tune = cur;
     if (best)

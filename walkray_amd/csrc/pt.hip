@@ -871,7 +871,7 @@ hipError_t Engine::init(uint32_t want_cap, uint32_t want_grid, hipStream_t st, u
     lds_levels = want_lds;
     auto alloc = [&](size_t bytes) -> void* {
         void* p = nullptr;
-        if (hipMalloc(&p, std::max<size_t>(bytes, 4)) != hipSuccess) return nullptr;
+        if (device_alloc(*pool, &p, bytes) != hipSuccess) return nullptr;
         bufs.push_back(p);
         return p;
     };
@@ -1106,14 +1106,14 @@ static hipError_t run_wavefront_once(const SceneDev& S, const CamHost& cam, uint
         if (E.contrib) WR_CHECK(hipFree(E.contrib));
         E.contrib = nullptr;
         E.contrib_floats = 0;
-        WR_CHECK(hipMalloc((void**)&E.contrib, sizeof(float) * want_floats));
+        WR_CHECK(device_alloc(*E.pool, (void**)&E.contrib, sizeof(float) * want_floats));
         E.contrib_floats = want_floats;
     }
     if (E.pass_slots < J.R) {
         if (E.pass_done) WR_CHECK(hipFree(E.pass_done));
         E.pass_done = nullptr;
         E.pass_slots = 0;
-        WR_CHECK(hipMalloc((void**)&E.pass_done, sizeof(uint32_t) * J.R));
+        WR_CHECK(device_alloc(*E.pool, (void**)&E.pass_done, sizeof(uint32_t) * J.R));
         E.pass_slots = J.R;
     }
     if (!E.ctl_back) WR_CHECK(hipHostMalloc((void**)&E.ctl_back, sizeof(JobCtl), hipHostMallocDefault));

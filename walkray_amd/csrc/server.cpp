@@ -94,6 +94,7 @@ int wr_server_create(wr_ctx* ctx, const wr_server_config* cfg, wr_server** out) 
     s->slot_job.assign(kMaxJobs, -1);
     s->slot_nee.assign(kMaxJobs, 0);
     (void)hipSetDevice(ctx->device);
+    s->engine.pool = ctx->pool.get();
     hipError_t e = s->engine.init(slots, 0, ctx->stream);
     if (e != hipSuccess) {
         delete s;

@@ -17,13 +17,13 @@ namespace wr {
 // Device memory that a context's calls use again: scratch and result buffers
 // of calls that used to allocate and free them each time (a 256^2
 // BidirectionalPathTracer call's 4 GB took 1 to 20 ms of hipMalloc and
-// hipFree).  A buffer is handed out to one call (or one grid or served job)
-// at a time, whichever thread makes it, and comes back when that ends; all
+// hipFree).  A buffer is handed out to one call (or one grid, film or served
+// job) at a time, whichever thread makes it, and comes back when that ends; all
 // work on a context runs on its stream, so a buffer's next user is ordered
 // behind its last one.  At most kIdleMax bytes stay with the pool unused; they
-// go back to the device when an allocation fails for want of memory, and with
-// the context.  Buffers still out then (a grid that outlives its context) are
-// freed when they come back.
+// go back to the device when any allocation of the context (device_alloc among
+// them) fails for want of memory, and with the context.  Buffers still out then
+// (a grid that outlives its context) are freed when they come back.
 class WorkPool {
 public:
     explicit WorkPool(int dev) : device(dev) {}
@@ -34,7 +34,14 @@ public:
         return get((void**)out, bytes);
     }
     void put(void* p);  // nullptr: nothing
-    void trim();        // gives the unused buffers back
+    // hipMalloc for a lasting buffer that its owner frees; when the device is out
+    // of memory, once more without the unused buffers.
+    hipError_t lasting(void** out, size_t bytes);
+    // Bytes of the buffers that are out, and of the unused ones.
+    void held(uint64_t* in_use, uint64_t* unused);
+    // An allocation that would take the buffers held past `bytes` fails as if the
+    // device had no more memory (0: no limit).
+    void limit(uint64_t bytes);
     void close();
     const int device;
 
@@ -45,9 +52,11 @@ private:
         size_t bytes;
         bool out;
     };
+    hipError_t malloc_trimmed(void** out, size_t bytes);
     void free_idle(size_t keep);  // frees unused buffers, the oldest first, until at most `keep` bytes of them are left
     std::mutex mu;
     std::vector<Buf> bufs;
+    size_t max_held = 0;  // 0: no limit
     bool closed = false;
 };
 // Buffers of one call, given back on every exit.

@@ -11,6 +11,10 @@ struct wr_ctx;
 
 namespace wr {
 
+class WorkPool;
+// hipMalloc for a context's lasting buffers (WorkPool::lasting).
+hipError_t device_alloc(WorkPool& pool, void** out, size_t bytes);
+
 // Camera basis computed on the host with the reference's float semantics
 // (camera.cpp:7-11): front = normalize(focus - pos), right =
 // normalize(front x up), top = right x front.
@@ -110,6 +114,7 @@ struct WaveStats {
 // The shared wavefront: path pool, job and scene tables, and the captured
 // iteration graph.  One per context (wr_render) or per server.
 struct Engine {
+    WorkPool* pool = nullptr;  // the context's, set by the owner before init
     uint32_t cap = 0, grid = 0, lds_levels = 0;  // lds_levels: k_wf_trace's traversal stack levels in LDS
     EngineCounters* cnt = nullptr;
     JobDesc* jobs = nullptr;
