@@ -68,3 +68,32 @@ def test_limit_is_reported():
     ctx.limit_work_memory(0)
     W.render_bdpt(sc, cam, film, 2, 4, 1)
     assert film.read()["sum"].any()
+
+
+def test_jobs_and_films_hold_their_size():
+    """A served job holds what its budget counts and a film its three arrays, also where larger unused
+    buffers would fit them."""
+    ctx = W.Context(0)
+    objs, cam = S.cornell(k=2, width=96, height=80)
+    sc = W.Scene(ctx, objs)
+    server = W.Server(ctx, path_slots=1 << 16)
+    sid = server.add_scene(sc)
+    cam2 = dict(cam, width=64, height=64)
+    sizes = []
+    for _ in range(2):  # the second job takes the first one's buffers
+        bufs = [W.Film(ctx, 80 + 10 * k, 80) for k in range(12)]  # a ladder of unused sizes
+        del bufs
+        _fill(ctx, sc, cam)
+        jid = server.submit(sid, cam2, 200, 4, 1)
+        server.step()
+        used = ctx.work_memory()[0]
+        while server.step():
+            pass
+        assert abs(used - server.status(jid)["device_bytes"]) <= 2 * 256
+        sizes.append(sum(ctx.work_memory()))
+        server.release(jid)
+    assert sizes[0] == sizes[1]
+    assert ctx.work_memory()[0] == 0
+    film = W.Film(ctx, 70, 64)
+    assert 0 <= ctx.work_memory()[0] - 3 * 12 * 70 * 64 <= 256
+    film.close()

@@ -34,14 +34,16 @@ int hip_fail(wr_ctx* ctx, hipError_t e, const char* what) {
     return fail(ctx, WR_EHIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-hipError_t WorkPool::get(void** out, size_t bytes) {
+hipError_t WorkPool::get(void** out, size_t bytes, bool exact) {
     *out = nullptr;
     // whole MiB above one, so that calls of similar sizes share buffers
-    bytes = bytes > (1u << 20) ? (bytes + (1u << 20) - 1) >> 20 << 20 : std::max<size_t>((bytes + 255) / 256 * 256, 256);
+    const size_t unit = bytes > (1u << 20) && !exact ? 1u << 20 : 256;
+    bytes = std::max<size_t>((bytes + unit - 1) / unit * unit, unit);
+    const size_t most = exact ? bytes : 4 * bytes;
     std::lock_guard<std::mutex> lk(mu);
     Buf* best = nullptr;
-    for (Buf& b : bufs)  // the smallest that fits, unless it is several times too large
-        if (!b.out && b.bytes >= bytes && b.bytes / 4 <= bytes && (!best || b.bytes < best->bytes)) best = &b;
+    for (Buf& b : bufs)  // the smallest that fits, unless it is too large
+        if (!b.out && b.bytes >= bytes && b.bytes <= most && (!best || b.bytes < best->bytes)) best = &b;
     if (best) {
         best->out = true;
         *out = best->p;

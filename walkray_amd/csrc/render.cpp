@@ -128,7 +128,7 @@ int wr_film_create(wr_ctx* ctx, uint32_t width, uint32_t height, wr_film** out) 
     f->W = width;
     f->H = height;
     const size_t n = 3 * (size_t)width * height;
-    if (ctx->pool->get(&f->sum, sizeof(float) * 3 * n) != hipSuccess) {
+    if (ctx->pool->get(&f->sum, sizeof(float) * 3 * n, true) != hipSuccess) {
         delete f;
         return fail(ctx, WR_ENOMEM, "wr_film_create: out of device memory");
     }

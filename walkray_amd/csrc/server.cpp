@@ -170,8 +170,9 @@ static hipError_t admit_one(wr_server* s, Job& j, int slot) {
         return hipErrorOutOfMemory;
     }
     const size_t window = 3 * (size_t)j.R * npix;
-    hipError_t e = s->ctx->pool->get(&j.film, 3 * fb);
-    if (e == hipSuccess) e = s->ctx->pool->get(&j.contrib, sizeof(float) * window + sizeof(uint32_t) * j.R);
+    // of the sizes that the budget counts
+    hipError_t e = s->ctx->pool->get(&j.film, 3 * fb, true);
+    if (e == hipSuccess) e = s->ctx->pool->get(&j.contrib, sizeof(float) * window + sizeof(uint32_t) * j.R, true);
     if (e == hipSuccess) e = hipMemsetAsync(j.film, 0, 3 * fb, st);
     if (e != hipSuccess) {
         free_job_window(s, j);

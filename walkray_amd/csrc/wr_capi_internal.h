@@ -28,10 +28,13 @@ class WorkPool {
 public:
     explicit WorkPool(int dev) : device(dev) {}
     ~WorkPool() { close(); }
-    hipError_t get(void** out, size_t bytes);
+    // A buffer of at least `bytes`, for a call's scratch: it may be several times
+    // as large.  exact: of `bytes` rounded up to 256, for what is held longer than
+    // a call (films and served jobs, whose sizes recur and are accounted for).
+    hipError_t get(void** out, size_t bytes, bool exact = false);
     template <class T>
-    hipError_t get(T** out, size_t bytes) {
-        return get((void**)out, bytes);
+    hipError_t get(T** out, size_t bytes, bool exact = false) {
+        return get((void**)out, bytes, exact);
     }
     void put(void* p);  // nullptr: nothing
     // hipMalloc for a lasting buffer that its owner frees; when the device is out
