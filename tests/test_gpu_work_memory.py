@@ -97,3 +97,27 @@ def test_jobs_and_films_hold_their_size():
     film = W.Film(ctx, 70, 64)
     assert 0 <= ctx.work_memory()[0] - 3 * 12 * 70 * 64 <= 256
     film.close()
+
+
+@pytest.mark.parametrize("kind", ["bdpt", "vcm"])
+@pytest.mark.parametrize("depth", [1, 5, 32])
+def test_prefixes_without_room(kind, depth):
+    """The prefixes of the sub-path records are 56 B beside a record's 72: an image whose records fit renders
+    without room for them all.  Sums of up to 4,096 nonnegative terms in any order agree to 4096 * 2^-24."""
+    objs, cam = S.cornell(k=2, width=96, height=80)
+    table = 56 * 2 * (depth + 3) * 96 * 80 * 2
+    args, films, held = () if kind == "bdpt" else (0.03,), [], 0
+    for room in (None, 0.6, 0.05):  # of the table
+        ctx = W.Context(0)
+        sc, film = W.Scene(ctx, objs), W.Film(ctx, 96, 80)
+        if room is not None:
+            ctx.limit_work_memory(int(held - (1 - room) * table))
+        getattr(W, f"render_{kind}")(sc, cam, film, 2, depth, 5, *args)
+        if room is None:
+            held = sum(ctx.work_memory())
+        else:
+            assert sum(ctx.work_memory()) <= held - (1 - room) * table
+        films.append(film.read()["sum"])
+    assert films[0].any()
+    for f in films[1:]:
+        assert np.allclose(f, films[0], rtol=2.5e-4, atol=1e-30)

@@ -283,12 +283,13 @@ __device__ __forceinline__ bool connect_edge_vm(const SceneDev& S, const BVert* 
     return true;
 }
 
-// A path that the eye side found alone: eye[e..0], eye[e] on an emitter (e >= 1).
+// A path that the eye side found alone: eye[e..0], eye[e] on an emitter (e >= 1);
+// pe, pp: the prefixes of eye[e] and eye[e - 1].
 // Only paths that pathCanNotConnect rejects for every connection are taken.
 // Its sum has no connection terms; with vt, the merging ones.
-__device__ __forceinline__ float eye_path_weight(const BVert* E, const BPrefix* PE, int e, const BVert& last, f3& color,
-                                                 float& prob, const VcmTerms* vt = nullptr) {
-    const BPrefix pe = PE[e];
+__device__ __forceinline__ float eye_path_weight(const BVert* E, const BPrefix& pe, const BPrefix& pp, int e,
+                                                 const BVert& last, f3& color, float& prob,
+                                                 const VcmTerms* vt = nullptr) {
     color = mulv(last.rad, pe.color);
     prob = last.dp * last.op * pe.prob;
     if (prob == 0.f || len(color) == 0.f) return 0.f;
@@ -297,7 +298,6 @@ __device__ __forceinline__ float eye_path_weight(const BVert* E, const BPrefix* 
         // the emitter's record starts the path: its direction probability is that of an emission
         const double pf = is_delta(last) ? 1.0 : (double)((float)(kInvPi * 0.25f) * 2.f);
         const BVert prev = E[e - 1];
-        const BPrefix pp = PE[e - 1];
         const double next = last.op * area_factor(cos_term_v(prev), vert_dist(last, prev)) * pf;
         const double disc = kPi * (double)vt->r * (double)vt->r * vt->nvm;
         if (e > 1 && !is_delta(prev)) all += pp.run * next * disc;
@@ -451,59 +451,104 @@ struct SubpathWalk {
     }
 };
 
-// The prefixes of every sub-path (BPrefix), one lane per sub-path: side 0 the
-// light sub-path, side 1 the eye sub-path of each lane's SubpathWalk.
-__global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uint32_t npix, uint32_t lanes,
-                                                     uint32_t maxv, const BVert* verts, const uint32_t* counts,
-                                                     BPrefix* prefix) {
-    const uint32_t id = blockIdx.x * 256 + threadIdx.x;
-    if (id >= 2 * lanes) return;
-    const bool eye = id >= lanes;
-    const uint32_t lane = eye ? id - lanes : id;
-    const size_t first = (size_t)lane * 2 * maxv + (eye ? 0 : maxv);
-    const BVert* V = verts + first;
-    BPrefix* P = prefix + first;
-    const uint32_t n = min(counts[2 * lane + (eye ? 0 : 1)], maxv), pixel = lane % npix;
-    if (n == 0) return;
-    BVert prev = V[0];
+// The prefix of a sub-path's first record.
+__device__ __forceinline__ BPrefix prefix_first(const SceneDev& S, const BVert& v) {
     BPrefix p;
-    p.run = prev.op;
+    p.run = v.op;
     p.vc = p.vm = 0.0;
     p.all = 1.0;
     p.color = mk(1.f, 1.f, 1.f);
     p.prob = 1.f;
-    p.flags = (emissive(S, prev.contact) ? kPEmissive : 0u) | (is_delta(prev) ? kPDelta : 0u);
+    p.flags = (emissive(S, v.contact) ? kPEmissive : 0u) | (is_delta(v) ? kPDelta : 0u);
     p.pad = 0;
+    return p;
+}
+
+// The prefix of record i > 0 (cur) from that of the record before it (prev).
+__device__ __forceinline__ void prefix_next(const SceneDev& S, const CamDev& cam, uint32_t pixel, bool eye, uint32_t i,
+                                            const BVert& prev, const BVert& cur, BPrefix& p) {
+    const BVert link = link_to(cur, prev);
+    const float d = vert_dist(cur, prev);
+    const bool dp = is_delta(prev), dc = is_delta(cur);
+    const float cos_prev = cos_term_v(prev);
+    const double own = area_factor(cos_prev, d);         // of the edge, at prev
+    const double at = area_factor(cos_term_v(link), d);  // of the edge, at cur
+    const double own_p = dp ? 1.0 : (double)eval_dir_prob(S, cam, pixel, prev, prev, !eye && i == 1);
+    const double link_p = dc ? 1.0 : (double)eval_dir_prob(S, cam, pixel, link, link, false);
+    const double edge = own * link_p;  // the other recurrence's factor from cur to prev
+    // merging at the far vertex of the pair: at cur on the light side, at prev on the eye side
+    // (the camera merges with nothing)
+    double merge = 0.0;
+    if (!eye && !dc) merge = own_p * at;
+    if (eye && i > 1 && !dp) merge = edge;
+    const bool connects = !dp && !dc;
+    p.vc = edge * p.vc + (connects ? p.run : 0.0);
+    p.vm = edge * p.vm + merge * p.run;
+    p.all *= edge;
+    p.run = p.run * at * own_p;
+    p.color = muls(mulv(p.color, prev.rad), cos_prev);
+    p.prob *= prev.dp * prev.op;
+    p.flags = (p.flags & kPAny) | (connects ? kPAny : 0u) | (emissive(S, cur.contact) ? kPEmissive : 0u) |
+              (dc ? kPDelta : 0u);
+}
+
+// The prefixes of every sub-path of the lanes [first, end), one lane per
+// sub-path: side 0 the light sub-path, side 1 the eye sub-path of each lane's
+// SubpathWalk.  table: of the records of lane `first` on.
+__global__ __launch_bounds__(256) void k_bdpt_prefix(SceneDev S, CamDev cam, uint32_t npix, uint32_t first,
+                                                     uint32_t end, uint32_t maxv, const BVert* verts,
+                                                     const uint32_t* counts, BPrefix* table) {
+    const uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t lanes = end - first;
+    if (id >= 2ull * lanes) return;
+    const bool eye = id >= lanes;
+    const uint32_t own = (uint32_t)(eye ? id - lanes : id), lane = first + own;
+    const BVert* V = verts + ((size_t)lane * 2 + (eye ? 0 : 1)) * maxv;
+    BPrefix* P = table + ((size_t)own * 2 + (eye ? 0 : 1)) * maxv;
+    const uint32_t n = min(counts[2 * (size_t)lane + (eye ? 0 : 1)], maxv), pixel = lane % npix;
+    if (n == 0) return;
+    BVert prev = V[0];
+    BPrefix p = prefix_first(S, prev);
     P[0] = p;
     for (uint32_t i = 1; i < n; i++) {
         const BVert cur = V[i];
-        const BVert link = link_to(cur, prev);
-        const float d = vert_dist(cur, prev);
-        const bool dp = is_delta(prev), dc = is_delta(cur);
-        const float cos_prev = cos_term_v(prev);
-        const double own = area_factor(cos_prev, d);             // of the edge, at prev
-        const double at = area_factor(cos_term_v(link), d);      // of the edge, at cur
-        const double own_p = dp ? 1.0 : (double)eval_dir_prob(S, cam, pixel, prev, prev, !eye && i == 1);
-        const double link_p = dc ? 1.0 : (double)eval_dir_prob(S, cam, pixel, link, link, false);
-        const double edge = own * link_p;  // the other recurrence's factor from cur to prev
-        // merging at the far vertex of the pair: at cur on the light side, at prev on the eye side
-        // (the camera merges with nothing)
-        double merge = 0.0;
-        if (!eye && !dc) merge = own_p * at;
-        if (eye && i > 1 && !dp) merge = edge;
-        const bool connects = !dp && !dc;
-        p.vc = edge * p.vc + (connects ? p.run : 0.0);
-        p.vm = edge * p.vm + merge * p.run;
-        p.all *= edge;
-        p.run = p.run * at * own_p;
-        p.color = muls(mulv(p.color, prev.rad), cos_prev);
-        p.prob *= prev.dp * prev.op;
-        p.flags = (p.flags & kPAny) | (connects ? kPAny : 0u) | (emissive(S, cur.contact) ? kPEmissive : 0u) |
-                  (dc ? kPDelta : 0u);
+        prefix_next(S, cam, pixel, eye, i, prev, cur, p);
         P[i] = p;
         prev = cur;
     }
 }
+
+// The prefixes as the connections and merges read them.  TABLE: from
+// k_bdpt_prefix's table; else, where the device has no room for the table (56 B
+// for each 72 B record), formed anew from the sub-path's records, which costs
+// about what a sweep over them costs.
+template <bool TABLE>
+struct Prefixes {
+    const BPrefix* table;  // indexed like verts
+    const BVert* verts;
+    uint32_t npix, maxv;
+    // of record i of a lane's eye or light sub-path
+    __device__ __forceinline__ BPrefix at(const SceneDev& S, const CamDev& cam, uint64_t lane, bool eye, int i) const {
+        const size_t first = (lane * 2 + (eye ? 0 : 1)) * maxv;
+        if (TABLE) return table[first + i];
+        BVert prev = verts[first];
+        BPrefix p = prefix_first(S, prev);
+        for (int k = 1; k <= i; k++) {
+            const BVert cur = verts[first + k];
+            prefix_next(S, cam, (uint32_t)(lane % npix), eye, (uint32_t)k, prev, cur, p);
+            prev = cur;
+        }
+        return p;
+    }
+    // the flags of record `rec`; before: those of the record before it, unless it is the first
+    __device__ __forceinline__ uint32_t flags(const SceneDev& S, size_t rec, bool first, uint32_t before) const {
+        if (TABLE) return table[rec].flags;
+        const BVert& v = verts[rec];
+        const bool d = is_delta(v);
+        const bool any = (before & kPAny) || (!first && !d && !(before & kPDelta));
+        return (any ? kPAny : 0u) | (emissive(S, v.contact) ? kPEmissive : 0u) | (d ? kPDelta : 0u);
+    }
+};
 
 // Index of the n-th set bit.
 __device__ __forceinline__ int nth_bit(uint64_t mask, uint32_t n) {
@@ -534,9 +579,10 @@ struct PairTable {
 // out one to each lane at a time.  Every lane of the wave makes the
 // call; lane0: the lane (pixel and pass) of the wave's first; max_eye,
 // max_light: 0 where a lane of the wave has none.  Adds what needs no visibility test to the lane's own pixel.
+template <bool TABLE>
 __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
-                                           uint32_t maxv, uint64_t lane0, const BVert* verts, const BPrefix* prefix,
-                                           int max_eye, int max_light, float* pix_all, const VisQueue& Q,
+                                           uint32_t maxv, uint64_t lane0, const BVert* verts,
+                                           const Prefixes<TABLE>& prefix, int max_eye, int max_light, float* pix_all, const VisQueue& Q,
                                            LaneStack& st, const VcmGrid* grids, PairTable& T) {
     static_assert(wr::kBdptMaxDepth + 3 <= 64, "a record per bit");
     const uint32_t wl = threadIdx.x & 63u;
@@ -544,8 +590,9 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
     uint64_t eye = 0, light = 0;
     {
         const size_t ei = (lane0 + wl) * 2 * maxv, li = ei + maxv;
+        uint32_t fl = 0;
         for (int e = 0; e < max_eye; e++) {
-            const uint32_t fl = prefix[ei + e].flags;
+            fl = prefix.flags(S, ei + e, e == 0, fl);
             if (!(fl & kPEmissive)) {
                 if (!(fl & kPDelta)) eye |= 1ull << e;
             } else if (e > 0 && !(fl & kPAny)) {
@@ -553,15 +600,17 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
                 const VcmTerms vt{grids ? grids[(lane0 + wl) / npix].r : 0.f, (double)npix, false};
                 f3 color;
                 float prob;
-                const float w = eye_path_weight(verts + ei, prefix + ei, e, verts[ei + e], color, prob,
-                                                grids ? &vt : nullptr);
+                const float w = eye_path_weight(verts + ei, prefix.at(S, cam, lane0 + wl, true, e),
+                                                prefix.at(S, cam, lane0 + wl, true, e - 1), e, verts[ei + e], color,
+                                                prob, grids ? &vt : nullptr);
                 if (prob != 0.f && len(color) != 0.f) own = add(own, muls(divs(color, prob), w));
             }
         }
         // light paths that start on no emitter (an empty light sample) connect to nothing
-        if (max_light > 0 && eye != 0 && (prefix[li].flags & kPEmissive)) {
+        if (max_light > 0 && eye != 0 && (prefix.flags(S, li, true, 0) & kPEmissive)) {
+            fl = 0;
             for (int c = 0; c < max_light; c++) {
-                const uint32_t fl = prefix[li + c].flags;
+                fl = prefix.flags(S, li + c, c == 0, fl);
                 if (!(fl & kPDelta) && (c == 0 || !(fl & kPEmissive))) light |= 1ull << c;
             }
         }
@@ -601,8 +650,8 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
             const VcmTerms vt{grids ? grids[k].r : 0.f, (double)npix, false};
             f3 color;
             float prob;
-            const float w = color_prob_weight(S, cam, p, lc, prefix[li + c], c, ec, prefix[ei + e], e, color, prob,
-                                              grids ? &vt : nullptr);
+            const float w = color_prob_weight(S, cam, p, lc, prefix.at(S, cam, lane, false, c), c, ec,
+                                              prefix.at(S, cam, lane, true, e), e, color, prob, grids ? &vt : nullptr);
             if (prob == 0.f) return false;
             if (len(color) == 0.f) return false;
             contrib = muls(divs(color, prob), w);
@@ -671,19 +720,21 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
     return own;
 }
 
+// The lanes [first, end); prefix: table indexed as if it held every lane's.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_bdpt(
-    SceneDev S, CamDev cam, uint32_t npass, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* prefix,
-    const uint32_t* counts, float* pix_all, VisQueue Q, uint32_t width) {
+    SceneDev S, CamDev cam, uint32_t first, uint32_t end, uint32_t npix, uint32_t maxv, const BVert* verts,
+    const BPrefix* prefix, const uint32_t* counts, float* pix_all, VisQueue Q, uint32_t width) {
     __shared__ PairTable tables[4];
     const uint32_t wl = threadIdx.x & 63u;
-    const uint64_t lane0 = (uint64_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * width, lane = lane0 + wl;
-    const bool valid = wl < width && lane < (uint64_t)npass * npix;
+    const uint64_t lane0 = first + (uint64_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * width, lane = lane0 + wl;
+    const bool valid = wl < width && lane < end;
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
     const uint32_t ne = valid ? counts[2 * lane] : 0u, nl = valid ? counts[2 * lane + 1] : 0u;
-    const f3 own = connect_wave(S, sc, cam, npix, maxv, lane0, verts, prefix, (int)min(ne, maxv),
-                                (int)min(nl, maxv), pix_all, Q, st, nullptr, tables[threadIdx.x >> 6]);
+    const f3 own = connect_wave(S, sc, cam, npix, maxv, lane0, verts, Prefixes<true>{prefix, verts, npix, maxv},
+                                (int)min(ne, maxv), (int)min(nl, maxv), pix_all, Q, st, nullptr,
+                                tables[threadIdx.x >> 6]);
     if (valid) atomic_add3(pix_all + 3 * (size_t)(lane / npix) * npix, (uint32_t)(lane % npix), own);
 }
 
@@ -813,9 +864,10 @@ struct MergeQueue {
 // One merge (throughputByMerging, vcmTracer.cpp:196-213): the eye vertex i of
 // lane `lane` with light point pi of the lane's pass.  Returns the contribution
 // (before the division by the pixel count); zero when the merge gives nothing.
+template <bool TABLE>
 __device__ __forceinline__ f3 vcm_merge(const SceneDev& S, const CamDev& cam, uint32_t npix, uint32_t maxv,
-                                        const BVert* verts, const BPrefix* prefix, const VcmGrid& G, uint64_t lane,
-                                        int i, uint32_t pi) {
+                                        const BVert* verts, const Prefixes<TABLE>& prefix, const VcmGrid& G,
+                                        uint64_t lane, int i, uint32_t pi) {
     const uint32_t p = (uint32_t)(lane % npix);
     const uint32_t k = G.src[2 * (size_t)pi], j = G.src[2 * (size_t)pi + 1];
     const size_t li = (size_t)k * 2 * maxv + maxv + (j - 1), ei = lane * 2 * maxv;
@@ -824,14 +876,17 @@ __device__ __forceinline__ f3 vcm_merge(const SceneDev& S, const CamDev& cam, ui
     const VcmTerms vm{G.r, (double)npix, true};
     f3 color;
     float prob;
-    const float w = color_prob_weight(S, cam, p, lc, prefix[li], (int)j - 1, ec, prefix[ei + i], i, color, prob, &vm);
+    const float w = color_prob_weight(S, cam, p, lc, prefix.at(S, cam, k, false, (int)j - 1), (int)j - 1, ec,
+                                      prefix.at(S, cam, lane, true, i), i, color, prob, &vm);
     if (len(color) == 0.f || prob == 0.f) return mk(0.f, 0.f, 0.f);
     return divs(muls(color, w), prob);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm(SceneDev S, CamDev cam, uint32_t npix, uint32_t npass, uint32_t maxv,
-                                             const BVert* verts, const BPrefix* prefix, const uint32_t* counts,
-                                             float* pix_all, VisQueue Q, const VcmGrid* grids, MergeQueue M, uint32_t width) {
+template <bool TABLE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm(
+    SceneDev S, CamDev cam, uint32_t npix, uint32_t npass, uint32_t maxv, const BVert* verts, const BPrefix* table,
+    const uint32_t* counts, float* pix_all, VisQueue Q, const VcmGrid* grids, MergeQueue M, uint32_t width) {
+    const Prefixes<TABLE> prefix{table, verts, npix, maxv};
     // every lane of a wave stays to the end (the merge reservations below are
     // wave-wide scans); a lane past the last one stands in for lane 0 and does
     // nothing
@@ -925,9 +980,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // The queued merges of k_vcm, one per lane, each added to its pixel of its pass.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm_merge(SceneDev S, CamDev cam, uint32_t npix, uint32_t maxv,
-                                                   const BVert* verts, const BPrefix* prefix, float* pix_all, MergeQueue M,
-                                                   const VcmGrid* grids) {
+template <bool TABLE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_vcm_merge(
+    SceneDev S, CamDev cam, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* table, float* pix_all,
+    MergeQueue M, const VcmGrid* grids) {
+    const Prefixes<TABLE> prefix{table, verts, npix, maxv};
     const uint32_t n = min(M.ent[2 * (size_t)M.cap], M.cap);
     for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
         const uint32_t w0 = M.ent[2 * (size_t)e], pi = M.ent[2 * (size_t)e + 1];
@@ -1104,7 +1161,6 @@ __global__ __launch_bounds__(256) void k_ppm_density(SceneDev S, CamDev cam, uin
 namespace wr {
 
 size_t bdpt_vertex_bytes() { return sizeof(wrd::BVert); }
-size_t bdpt_prefix_bytes() { return sizeof(wrd::BPrefix); }
 
 float vcm_radius(float base, uint32_t pass) {
     const float alpha = (float)(2.0 / 3);  // vcmTracer.h:39
@@ -1171,8 +1227,9 @@ static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const
         const float r = vcm_radius(base_radius, pass0 + b);
         params[b] = wrd::GridParams{1.f / (r * 2.f), r * r, r};
     }
-    e = build_grids(ctx, mem, vb.pos, vb.src, (uint64_t)lanes + starts[npass], vb.starts, npix, npass, npix,
-                    params.data(), (wrd::GridView*)vb.grids, vb.err, nullptr);
+    const uint64_t total = (uint64_t)lanes + starts[npass];
+    e = build_grids(ctx, mem, vb.pos, vb.src, total, vb.starts, npix, npass, npix, params.data(),
+                    (wrd::GridView*)vb.grids, vb.err, nullptr, vb.cap - total >= total ? vb.pos + 3 * total : nullptr);
     if (e != hipSuccess) return hip_fail(ctx, e, who);
     return WR_OK;
 }
@@ -1212,18 +1269,26 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     int rc = light_point_grids(ctx, mem, S, H, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, q.counts,
                                vb, true, "wr_render_vcm");
     if (rc != WR_OK) return rc;
-    wrd::BPrefix* prefix = (wrd::BPrefix*)q.prefix;
-    wrd::k_bdpt_prefix<<<(2 * lanes + 255) / 256, 256, 0, st>>>(S, cam, npix, lanes, maxv, V, q.counts, prefix);
+    // a merge needs the prefixes of any light path of its pass: without room for
+    // all of them they are formed where they are needed
+    wrd::BPrefix* prefix = nullptr;
+    e = mem.get(&prefix, sizeof(wrd::BPrefix) * 2 * maxv * (size_t)lanes);
+    if (e != hipSuccess && e != hipErrorOutOfMemory) return hip_fail(ctx, e, "wr_render_vcm");
+    if (prefix)
+        wrd::k_bdpt_prefix<<<(uint32_t)((2ull * lanes + 255) / 256), 256, 0, st>>>(S, cam, npix, 0, lanes, maxv, V,
+                                                                                  q.counts, prefix);
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
     const wrd::MergeQueue M{vb.mq, vb.mq_cap};
     e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint32_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     const uint32_t width = connect_width(lanes, kVcmWaves);
-    wrd::k_vcm<<<(lanes + 4 * width - 1) / (4 * width), 256, wrd::kStackLdsBytes, st>>>(
-        S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q, (const wrd::VcmGrid*)vb.grids, M, width);
+    (prefix ? wrd::k_vcm<true> : wrd::k_vcm<false>)<<<(lanes + 4 * width - 1) / (4 * width), 256, wrd::kStackLdsBytes,
+                                                      st>>>(S, cam, npix, npass, maxv, V, prefix, q.counts, pix, Q,
+                                                            (const wrd::VcmGrid*)vb.grids, M, width);
     e = hipGetLastError();
     if (e == hipSuccess) {
-        wrd::k_vcm_merge<<<4096, 256, 0, st>>>(S, cam, npix, maxv, V, prefix, pix, M, (const wrd::VcmGrid*)vb.grids);
+        (prefix ? wrd::k_vcm_merge<true> : wrd::k_vcm_merge<false>)<<<4096, 256, 0, st>>>(
+            S, cam, npix, maxv, V, prefix, pix, M, (const wrd::VcmGrid*)vb.grids);
         e = hipGetLastError();
     }
     uint32_t nq = 0, grid_err = 0;
@@ -1295,11 +1360,23 @@ hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr&
     e = run_subpaths(ctx, S, H, cam, max_depth, seed, pass0, (uint32_t)lanes, npix, maxv, (wrd::BVert*)verts, q.counts,
                      true);
     if (e != hipSuccess) return e;
-    wrd::k_bdpt_prefix<<<(uint32_t)((2 * lanes + 255) / 256), 256, 0, st>>>(
-        S, cam, npix, (uint32_t)lanes, maxv, (const wrd::BVert*)verts, q.counts, (wrd::BPrefix*)q.prefix);
-    const uint32_t width = connect_width(lanes, kBdptWaves);
-    wrd::k_bdpt<<<(uint32_t)((lanes + 4 * width - 1) / (4 * width)), 256, wrd::kStackLdsBytes, st>>>(
-        S, cam, npass, npix, maxv, (const wrd::BVert*)verts, (const wrd::BPrefix*)q.prefix, q.counts, pix, Q, width);
+    // the prefixes of at most 4 GiB of lanes at a time (all of them up to a million
+    // lanes at the longest paths), fewer where the device has no room for them
+    Scratch mem(*ctx->pool);
+    const size_t lane_bytes = sizeof(wrd::BPrefix) * 2 * maxv;
+    uint64_t part = std::min<uint64_t>(lanes, (4ull << 30) / lane_bytes);
+    wrd::BPrefix* prefix = nullptr;
+    while ((e = mem.get(&prefix, lane_bytes * part)) == hipErrorOutOfMemory && part > 1024) part = (part + 3) / 4;
+    if (e != hipSuccess) return e;
+    for (uint64_t a = 0; a < lanes; a += part) {
+        const uint32_t first = (uint32_t)a, end = (uint32_t)std::min<uint64_t>(lanes, a + part), n = end - first;
+        wrd::k_bdpt_prefix<<<(uint32_t)((2ull * n + 255) / 256), 256, 0, st>>>(S, cam, npix, first, end, maxv,
+                                                                              (const wrd::BVert*)verts, q.counts, prefix);
+        const uint32_t width = connect_width(n, kBdptWaves);
+        wrd::k_bdpt<<<(uint32_t)((n + 4ull * width - 1) / (4 * width)), 256, wrd::kStackLdsBytes, st>>>(
+            S, cam, first, end, npix, maxv, (const wrd::BVert*)verts, prefix - (ptrdiff_t)first * 2 * maxv, q.counts, pix,
+            Q, width);
+    }
     uint32_t nq = 0;
     e = hipMemcpyAsync(&nq, q.count, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

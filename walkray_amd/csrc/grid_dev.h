@@ -84,10 +84,13 @@ namespace wr {
 // (nseg device records) describe the grids in buffers taken from mem; *err (a
 // zeroed device word) is set if a grid has too many cells across.  boxes
 // (nullable): the bounding box of every kGridChunk entries of the order.
+// sorted (nullable): where the positions in the grids' order go (3 * total
+// floats; nullptr: into a buffer from mem).
 constexpr uint32_t kGridChunk = 256;
 hipError_t build_grids(wr_ctx* ctx, Scratch& mem, const float* d_pos, const uint32_t* d_src, uint64_t total,
                        const uint32_t* starts, uint32_t lead, uint32_t nseg, uint32_t n_cells,
-                       const wrd::GridParams* params, wrd::GridView* views, uint32_t* err, float** boxes);
+                       const wrd::GridParams* params, wrd::GridView* views, uint32_t* err, float** boxes,
+                       float* sorted = nullptr);
 }  // namespace wr
 
 // A built grid: mCellEnds (inclusive ends per cell), mIndices and the positions

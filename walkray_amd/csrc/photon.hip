@@ -565,7 +565,7 @@ namespace wr {
 
 hipError_t build_grids(wr_ctx* ctx, Scratch& mem, const float* d_pos, const uint32_t* d_src, uint64_t total,
                        const uint32_t* starts, uint32_t lead, uint32_t nseg, uint32_t n_cells,
-                       const GridParams* params, GridView* views, uint32_t* err, float** boxes) {
+                       const GridParams* params, GridView* views, uint32_t* err, float** boxes, float* sorted) {
     hipStream_t st = ctx->stream;
     const uint32_t cells = nseg * n_cells;
     // workgroups of 256 per segment's box: one per 1,024 points, at most 128
@@ -581,10 +581,10 @@ hipError_t build_grids(wr_ctx* ctx, Scratch& mem, const float* d_pos, const uint
     // what the grids keep, and what the build alone needs
     int* ends;
     uint32_t* idx;
-    float* pos;
+    float* pos = sorted;
     if ((e = mem.get(&ends, sizeof(int) * (size_t)cells)) != hipSuccess) return e;
     if ((e = mem.get(&idx, sizeof(uint32_t) * total)) != hipSuccess) return e;
-    if ((e = mem.get(&pos, sizeof(float) * 3 * total)) != hipSuccess) return e;
+    if (!pos && (e = mem.get(&pos, sizeof(float) * 3 * total)) != hipSuccess) return e;
     if (boxes && (e = mem.get(boxes, sizeof(float) * 6 * ((total + kGridChunk - 1) / kGridChunk))) != hipSuccess)
         return e;
     Scratch sc(*ctx->pool);

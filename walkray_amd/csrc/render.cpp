@@ -300,7 +300,8 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     (void)hipSetDevice(ctx->device);
     const CamHost ch = make_cam(*cam);
     const uint32_t maxv = prm->max_depth + 3;  // the longest sub-path: first ray, max_depth scatters, the end
-    // passes per launch: as many as fill the device, within 4 GiB of sub-path records
+    // passes per launch: as many as fill the device, within 4 GiB of sub-path records (their
+    // prefixes, the queue and the walk's lists come to as much again)
     const uint64_t per_pass = bdpt_vertex_bytes() * 2 * maxv * npix;
     uint64_t batch = std::max<uint64_t>(1, (4ull << 30) / per_pass);
     batch = std::min<uint64_t>(std::min<uint64_t>(batch, prm->spp ? prm->spp : 1), std::max<uint64_t>(1, (1ull << 22) / npix));
@@ -316,7 +317,6 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     hipError_t e = mem.get(&verts, per_pass * batch);
     if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * npix * batch);
     if (e == hipSuccess) e = mem.get(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
-    if (e == hipSuccess) e = mem.get(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * npix * batch);
     if (e == hipSuccess) e = mem.get(&q.counts, sizeof(uint32_t) * 2 * npix * batch);
     if (e == hipSuccess) {
         char* b = (char*)qbuf;
@@ -328,11 +328,13 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     }
     if (e == hipSuccess) e = hipEventRecord(ctx->ev0, ctx->stream);
     const FilmBufs fb{film->sum, film->comp, film->sumsq};
-    const bool launched = e == hipSuccess && prm->spp > 0;  // from here on a failure leaves the film part-written
+    bool launched = false;  // a failure leaves the film part-written
     for (uint32_t k = 0; k < prm->spp && e == hipSuccess; k += (uint32_t)batch) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, prm->spp - k);
         e = launch_bdpt_passes(ctx, s->dev, s->hdrs[0], ch, prm->max_depth, prm->seed, film->passes + k, nb, maxv, verts,
                                pix, q, fb);
+        // the first passes allocate before they write
+        launched = launched || e != hipErrorOutOfMemory;
     }
     if (e == hipSuccess) e = hipEventRecord(ctx->ev1, ctx->stream);
     if (e == hipSuccess) e = hipEventSynchronize(ctx->ev1);
@@ -375,7 +377,8 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (film->broken) return film_broken(film, "wr_render_vcm");
     (void)hipSetDevice(ctx->device);
     const CamHost ch = make_cam(*cam);
-    // passes per launch: as many as fill the device, within 4 GiB of sub-path records and 2^31 points
+    // passes per launch: as many as fill the device, within 4 GiB of sub-path records (with their
+    // prefixes, queues and points about 10) and 2^31 points
     const uint64_t per_pass = bdpt_vertex_bytes() * 2 * maxv * npix;
     uint64_t batch = std::max<uint64_t>(1, (4ull << 30) / per_pass);
     batch = std::min<uint64_t>(std::min<uint64_t>(batch, prm->spp ? prm->spp : 1), std::max<uint64_t>(1, (1ull << 22) / npix));
@@ -395,7 +398,6 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * lanes);
     if (e == hipSuccess) e = mem.get(&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 1));
     if (e == hipSuccess) e = mem.get(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
-    if (e == hipSuccess) e = mem.get(&q.prefix, bdpt_prefix_bytes() * 2 * maxv * lanes);
     if (e == hipSuccess) e = mem.get(&q.counts, sizeof(uint32_t) * 2 * lanes);
     if (e == hipSuccess) e = mem.get(&vb.pc, sizeof(uint32_t) * (lanes + 1));
     if (e == hipSuccess) e = mem.get(&vb.offs, sizeof(uint32_t) * (lanes + 1));

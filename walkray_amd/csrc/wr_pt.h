@@ -178,12 +178,10 @@ struct BdptQueue {
     uint32_t* count;
     uint32_t cap;
     uint32_t* counts;  // 2 per pixel and pass: the eye and light sub-path record counts
-    void* prefix;      // one prefix record (bdpt_prefix_bytes() each) per sub-path record
     unsigned long long* work;  // work counters of the batch queries on this stream (wr_ctx::d_work)
 };
 constexpr size_t kBdptQueueEntryBytes = 32 + 16 + 4 + 16;
 size_t bdpt_vertex_bytes();
-size_t bdpt_prefix_bytes();
 hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& cam, uint32_t max_depth,
                               uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
                               const BdptQueue& q, const FilmBufs& film);
