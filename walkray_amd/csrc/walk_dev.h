@@ -81,22 +81,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // Step s: completes every live path's hit and takes the path one vertex on.
 // P::step(sc, path, s, o, d, hit, st, out): the vertex at the hit (hit.rec
 // WR_NONE: the ray escaped); true if the path goes on with out.
-// last: the walk's last launch, which takes any number of paths to their ends.
-template <class P>
+// LAST: the walk's last launch, which takes any number of paths to their ends.
+template <class P, bool LAST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_walk_shade(SceneDev S, P policy,
-                                                                                           WalkLists W, uint32_t s,
-                                                                                           bool last) {
+                                                                                           WalkLists W, uint32_t s) {
     const uint32_t n = W.n[s];
     if (blockIdx.x == 0) UnitQueue::clear(W.work);  // for the next step's trace
     StackSpill spill;
     LaneStack st(&spill);
     const SceneCtx sc = make_scene_ctx(S);
-    if (n <= wr::kWalkFew || last) {  // the rest of every path, the trace included
+    if (LAST || n <= wr::kWalkFew) {  // the rest of every path, the trace included
         uint32_t width = 1;           // lanes of a wave that take a path
         while (width < 64 && (uint64_t)width * gridDim.x * 4 < n) width *= 2;
         const uint32_t lane = threadIdx.x & 63u;
         if (lane >= width) return;
-        for (uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane; i < n; i += gridDim.x * 4 * width) {
+        for (uint32_t i = (blockIdx.x * 4 + (threadIdx.x >> 6)) * width + lane; i < n;
+             i = LAST ? i + gridDim.x * 4 * width : n) {
             const uint32_t path = W.path[s & 1][i];
             const uint32_t* rp = W.rays[s & 1] + 8 * (size_t)i;
             Out out;
@@ -186,9 +186,10 @@ hipError_t run_walk(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const 
         for (uint32_t s = 0; s < list_steps; s++) {
             e = launch_walk_trace(S, H, W.rays[s & 1], W.n + s, n, W.hits, W.work, st);
             if (e != hipSuccess) return e;
-            wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s, false);
+            wrd::k_walk_shade<P, false><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, s);
         }
-        if (list_steps < steps) wrd::k_walk_shade<P><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, list_steps, true);
+        if (list_steps < steps)
+            wrd::k_walk_shade<P, true><<<shade, 256, wrd::kStackLdsBytes, st>>>(S, policy, W, list_steps);
         p += n;
     }
     return hipGetLastError();
