@@ -52,3 +52,21 @@ def test_image_of_more_than_2_24_pixels(ctx):
     before, after = rows[line - 20:line].mean(), rows[line + 1:line + 21].mean()
     assert before > 0
     assert abs(after / before - 1) < 0.1, (before, after)
+
+
+@pytest.mark.gpu
+def test_more_than_2_32_merges(ctx):
+    """Two passes side by side with 6.0e9 merges between them, and one after the other with 3.0e9 each: the
+    same film (a pixel sums up to 250,000 nonnegative contributions, in runs of different lengths)."""
+    from walkray_amd import _lib as W
+    from walkray_amd import scenes as S
+
+    objs, cam = S.cornell(k=1, width=160, height=160)
+    sc, films = W.Scene(ctx, objs), []
+    for calls in ((2,), (1, 1)):
+        film = W.Film(ctx, 160, 160)
+        for spp in calls:
+            W.render_vcm(sc, cam, film, spp, 3, 3, 2.0)
+        films.append(film.read()["sum"])
+    assert (films[0] > 0).mean() > 0.5
+    assert np.allclose(films[0], films[1], rtol=250000 * 2.0 ** -24)

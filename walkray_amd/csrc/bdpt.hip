@@ -854,11 +854,16 @@ __global__ void k_vcm_pass_starts(const uint32_t* offs, uint32_t npix, uint32_t 
 
 // The merges of the VCM lanes, one entry per light point in reach of an eye
 // vertex: word 0 the eye vertex (merge_entry.h), word 1 the light point; count
-// at ent[2 * cap].  A separate kernel takes one merge per lane, so the uneven
-// number of merges per pixel does not leave most lanes of a wave idle.
+// behind them, of all merges, queued or not: in 64 bits, since a pass of a
+// megapixel with a radius of a tenth of the scene has more than 2^32.  A
+// separate kernel takes one merge per lane, so the uneven number of merges per
+// pixel does not leave most lanes of a wave idle.
 struct MergeQueue {
     uint32_t* ent;
     uint32_t cap;
+    __device__ __forceinline__ unsigned long long* count() const {
+        return reinterpret_cast<unsigned long long*>(ent + 2 * (size_t)cap);
+    }
 };
 
 // One merge (throughputByMerging, vcmTracer.cpp:196-213): the eye vertex i of
@@ -913,7 +918,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // nothing.  Each merge is queued for k_vcm_merge: per eye vertex the lane
     // counts its points in reach, the wave reserves their slots with one
     // atomic (an exclusive scan of the counts), and the lane writes them.
-    uint32_t* mcount = M.ent + 2 * (size_t)M.cap;
     bool alive = valid;
     for (int i = 1; i < (int)maxv; i++) {
         bool act = alive && i < max_eye;
@@ -932,17 +936,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const bool q = act && query_corner(G.g, ev.o, pc);
         uint32_t cnt = 0;
         for (int pass2 = 0; pass2 < 2; pass2++) {
-            uint32_t k = 0;
-            if (pass2) {  // the slots of this lane's merges: the wave's scan, one atomic
-                uint32_t v = cnt;
+            uint32_t k = 0;  // cap where the queue is full
+            if (pass2) {     // the slots of this lane's merges: the wave's scan, one atomic
+                unsigned long long v = cnt;
                 for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t t = __shfl_up(v, off, 64);
+                    const unsigned long long t = __shfl_up(v, off, 64);
                     if (wl >= (uint32_t)off) v += t;
                 }
-                const uint32_t total = __shfl(v, 63, 64);
-                uint32_t base = 0;
-                if (wl == 0 && total) base = atomicAdd(mcount, total);
-                k = __shfl(base, 0, 64) + (v - cnt);
+                const unsigned long long total = __shfl(v, 63, 64);
+                unsigned long long base = 0;
+                if (wl == 0 && total) base = atomicAdd(M.count(), total);
+                k = (uint32_t)min(__shfl(base, 0, 64) + (v - cnt), (unsigned long long)M.cap);
                 if (cnt == 0) break;
             }
             f3 contrib = mk(0.f, 0.f, 0.f);
@@ -968,7 +972,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         k++;
                     } else {  // queue full: merge here
                         contrib = add(contrib, vcm_merge(S, cam, npix, maxv, verts, prefix, G, lane, i, pi));
-                        k++;
                     }
                 }
             }
@@ -985,7 +988,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     SceneDev S, CamDev cam, uint32_t npix, uint32_t maxv, const BVert* verts, const BPrefix* table, float* pix_all,
     MergeQueue M, const VcmGrid* grids) {
     const Prefixes<TABLE> prefix{table, verts, npix, maxv};
-    const uint32_t n = min(M.ent[2 * (size_t)M.cap], M.cap);
+    const uint32_t n = (uint32_t)min(*M.count(), (unsigned long long)M.cap);
     for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) {
         const uint32_t w0 = M.ent[2 * (size_t)e], pi = M.ent[2 * (size_t)e + 1];
         const uint32_t lane = wr::merge_lane(w0, maxv);
@@ -1279,7 +1282,7 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
                                                                                   q.counts, prefix);
     const wrd::VisQueue Q{q.rays, q.pay, q.dst, q.count, q.cap};
     const wrd::MergeQueue M{vb.mq, vb.mq_cap};
-    e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint32_t), st);
+    e = hipMemsetAsync(vb.mq + 2 * (size_t)vb.mq_cap, 0, sizeof(uint64_t), st);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_render_vcm");
     const uint32_t width = connect_width(lanes, kVcmWaves);
     (prefix ? wrd::k_vcm<true> : wrd::k_vcm<false>)<<<(lanes + 4 * width - 1) / (4 * width), 256, wrd::kStackLdsBytes,

@@ -396,7 +396,7 @@ extern "C" int wr_render_vcm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     Scratch mem(*ctx->pool);
     hipError_t e = mem.get(&verts, per_pass * batch);
     if (e == hipSuccess) e = mem.get(&pix, sizeof(float) * 3 * lanes);
-    if (e == hipSuccess) e = mem.get(&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 1));
+    if (e == hipSuccess) e = mem.get(&vb.mq, sizeof(uint32_t) * (2 * (size_t)vb.mq_cap + 2));
     if (e == hipSuccess) e = mem.get(&qbuf, kBdptQueueEntryBytes * (size_t)q.cap + 256);
     if (e == hipSuccess) e = mem.get(&q.counts, sizeof(uint32_t) * 2 * lanes);
     if (e == hipSuccess) e = mem.get(&vb.pc, sizeof(uint32_t) * (lanes + 1));

@@ -173,7 +173,7 @@ struct VcmBufs {
     uint64_t cap;
     void* grids;
     uint32_t* err;     // set when a pass's grid cannot be built
-    uint32_t* mq;      // VCM merges queued for k_vcm_merge: 2 words each, then the count
+    uint32_t* mq;      // VCM merges queued for k_vcm_merge: 2 words each, then the count (64 bits)
     uint32_t mq_cap;
 };
 float vcm_radius(float base, uint32_t pass);
