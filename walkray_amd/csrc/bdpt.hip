@@ -626,6 +626,10 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
     __builtin_amdgcn_wave_barrier();  // the table is this wave's own: LDS operations of a wave stay in order
     const uint32_t total = __shfl(upto, 63, 64);
     uint32_t kept = 0, kept_end = 0, used = 0;  // the wave's reserved queue slots, and its entries so far
+    // Once a reservation lies past the queue the wave makes no more, so a wave adds
+    // at most one (512 slots) past it and the 32-bit counter does not come round
+    // below 8M waves, more lanes than the device has memory for.
+    bool full = false;
     for (uint32_t t0 = 0; t0 < total; t0 += 64) {
         BVert ec{};
         f3 contrib{};
@@ -679,13 +683,16 @@ __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc
         const uint32_t n = (uint32_t)__popcll(m), avail = kept_end - kept;
         used += n;
         uint32_t first = kept, fresh = 0;
-        if (n > avail) {
+        if (n > avail && full) {
+            first = fresh = kept = kept_end = Q.cap;
+        } else if (n > avail) {
             const uint32_t seen = min(t0 + 64, total);
             const uint32_t take = n - avail + min((uint32_t)((uint64_t)(total - seen) * used / seen), kReserve);
             if (wl == 0) fresh = atomicAdd(Q.count, take);
             fresh = __shfl(fresh, 0, 64);
             kept = fresh + (n - avail);
             kept_end = fresh + take;
+            full = fresh >= Q.cap;
         } else {
             kept += n;
         }
