@@ -305,9 +305,12 @@ int wr_render(wr_ctx* ctx, const wr_scene* scene, const wr_camera* cam, const wr
               wr_film* film, wr_render_stats* stats);
 
 /* Per-stage statistics of the context's last wr_render with
- * WR_RENDER_STAGE_STATS: device milliseconds summed over the iterations for
- * each of the eight iteration kernels (extend: trace, finish; shade: common
- * case, refraction exits; plan; generate; fold; advance), the path segments
+ * WR_RENDER_STAGE_STATS, which takes every path through the stages to its end
+ * (other renders take the last paths to their ends in one launch, so they make
+ * fewer iterations and are faster than these stages together): device
+ * milliseconds summed over the iterations for each of the eight stage kernels
+ * (extend: trace, finish; shade: common case, refraction exits; plan; generate;
+ * fold; advance), the path segments
  * traced, the refraction exits, the camera paths generated, and the fast-pass
  * records the trace stage fetched (nodes in 32 B units, 48 B triangles). */
 typedef struct {
@@ -523,7 +526,8 @@ int wr_set_render_tuning(wr_ctx* ctx, const wr_render_tuning* tuning);
  * pass and vertex, and passes are folded in order). */
 typedef struct wr_server wr_server;
 typedef struct {
-    uint64_t job_memory_budget; /* device bytes for job state (films + sample windows); 0 = 8 GiB */
+    uint64_t job_memory_budget; /* device bytes that jobs hold (films + sample windows); 0 = 8 GiB.
+                                   The context's unused work buffers are not counted. */
     uint32_t path_slots;        /* shared path pool; 0 = 4,194,304 */
     uint32_t max_jobs;          /* concurrently admitted jobs, <= 64; 0 = 64 */
 } wr_server_config;

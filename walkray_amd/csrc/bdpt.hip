@@ -1,34 +1,32 @@
-// bdpt.hip -- BidirectionalPathTracer (bidirPathTracer.cpp:10-313) on gfx950.
+// bdpt.hip -- BidirectionalPathTracer (bidirPathTracer.cpp:10-313), VCMTracer
+// and PhotonMap on gfx950.
 //
-// One lane per pixel and pass (the reference's per-pixel loop), megakernel
-// style:
-//   1. the eye sub-path: the camera ray (camera.cpp:6-60) and
-//      MCRenderer::samplePath (mcRenderer.cpp:16-57) from it;
-//   2. the light sub-path: Scene::genLightSample as
-//      AbstractObject::genSurfaceSample (abstractObj.cpp:18-52) and samplePath
-//      from it, with the light-path vertex counters;
-//   3. every (light length, eye length) split of every joined length
-//      (bidirPathTracer.cpp:53-140): connectEdge (294-324), the visibility
-//      test (mcRenderer.cpp:59-65), connectingColorProb (266-291) and
-//      connectingMisWeight (142-221) with linkVertex (228-243), from the
-//      connection's two records and their sub-paths' prefixes (BPrefix);
-//   4. contributions with an eye side of two or more vertices go to the
-//      lane's pixel, light-tracing ones (the camera vertex alone on the eye
-//      side) are splatted to the pixel Camera::convToRaster names
-//      (camera.cpp:148-170), scaled by 1 / pixel solid angle / pixel count.
-// The visibility tests of the connections are not traced by the lane that
-// forms them: each connection that passes every other test appends its
-// visibility ray (and its contribution and target pixel) to a queue, traced
-// afterwards one ray per lane by the batch NoSelf query (k_closest_hit:
-// the same traversal, so the same answers) and folded in by k_bdpt_accum; a
-// lane whose queue is full traces in place.
-// The sub-paths live in device memory (one block of records per lane).  A
-// launch runs several passes side by side (lane = pass x pixel: one pass of a
-// 256^2 image is only 1,024 waves of long, serial lanes).  The pixel values
-// of each pass are summed with float atomics in a buffer of their own (the
-// splats of other lanes land on any pixel), then k_bdpt_fold applies
-// isLegalColor and fixVignetting and adds them to the Kahan film in pass
-// order.
+// Several passes run side by side (a lane is a pixel of a pass: one pass of a
+// 256^2 image alone does not fill the chip).  BidirectionalPathTracer:
+//   1. the sub-paths, a path walk (walk_dev.h, SubpathWalk): per lane the eye
+//      sub-path, the camera ray (camera.cpp:6-60) and MCRenderer::samplePath
+//      (mcRenderer.cpp:16-57) from it, and the light sub-path,
+//      Scene::genLightSample as AbstractObject::genSurfaceSample
+//      (abstractObj.cpp:18-52) and samplePath from it, with the light-path
+//      vertex counters, into one block of records per lane;
+//   2. k_bdpt_prefix: what a connection needs of the records before its two
+//      (BPrefix);
+//   3. k_bdpt: every (light length, eye length) split of every joined length
+//      (bidirPathTracer.cpp:53-140), the pairs of a wave's lanes dealt out to its
+//      lanes: connectEdge (294-324), connectingColorProb (266-291) and
+//      connectingMisWeight (142-221) with linkVertex (228-243).  Contributions
+//      with an eye side of two or more vertices go to the lane's pixel,
+//      light-tracing ones (the camera vertex alone on the eye side) are splatted
+//      to the pixel Camera::convToRaster names (camera.cpp:148-170), scaled by
+//      1 / pixel solid angle / pixel count;
+//   4. the visibility tests (mcRenderer.cpp:59-65) of the connections, which
+//      k_bdpt queues with their contribution and target pixel: the batch NoSelf
+//      query (k_closest_hit: the same traversal, so the same answers), then
+//      k_bdpt_accum; with a full queue a connection is traced in place;
+//   5. k_bdpt_fold.  The pixel values of each pass are summed with float atomics
+//      in a buffer of their own (the splats of other lanes land on any pixel);
+//      it applies isLegalColor and fixVignetting and adds them to the Kahan film
+//      in pass order.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -164,9 +162,9 @@ __device__ __forceinline__ BVert link_to(const BVert& v, const BVert& to) {
 // of the probability.  These prefixes, kept per record by k_bdpt_prefix, leave
 // each connection and each merge the two records and the edge between them,
 // instead of a sweep over the joined path with its dozen arrays in scratch
-// (3.5 KB a lane): Cornell 256^2 x 8 passes, maxPathLen 8, 14.7 ms in k_bdpt
-// before, 7.5 and 0.36 in k_bdpt_prefix now; the merges of a 201 x 151 VCM
-// render 0.83 and 0.29 ms.
+// (3.5 KB a lane): Cornell 256^2 x 8 passes, maxPathLen 8, 14.7 ms in k_bdpt with
+// the sweep, 7.5 with the prefixes (0.57 since connect_wave deals the pairs out)
+// and 0.36 in k_bdpt_prefix; the merges of a 201 x 151 VCM render 0.83 and 0.29 ms.
 struct BPrefix {
     double run;     // direct[i] of a light record, reverse of an eye record
     double vc, vm;  // S of the connections and of the merging factors (without K)
@@ -582,8 +580,8 @@ struct PairTable {
 template <bool TABLE>
 __device__ __forceinline__ f3 connect_wave(const SceneDev& S, const SceneCtx& sc, const CamDev& cam, uint32_t npix,
                                            uint32_t maxv, uint64_t lane0, const BVert* verts,
-                                           const Prefixes<TABLE>& prefix, int max_eye, int max_light, float* pix_all, const VisQueue& Q,
-                                           LaneStack& st, const VcmGrid* grids, PairTable& T) {
+                                           const Prefixes<TABLE>& prefix, int max_eye, int max_light,
+                                           float* pix_all, const VisQueue& Q, LaneStack& st, const VcmGrid* grids, PairTable& T) {
     static_assert(wr::kBdptMaxDepth + 3 <= 64, "a record per bit");
     const uint32_t wl = threadIdx.x & 63u;
     f3 own = mk(0.f, 0.f, 0.f);
@@ -1002,7 +1000,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const int i = (int)wr::merge_vertex(w0, maxv);
         const uint32_t kb = lane / npix, p = lane % npix;
         const f3 c = vcm_merge(S, cam, npix, maxv, verts, prefix, grids[kb], lane, i, pi);
-        if (c.x != 0.f || c.y != 0.f || c.z != 0.f) atomic_add3(pix_all + 3 * (size_t)kb * npix, p, divs(c, (float)npix));
+        if (c.x != 0.f || c.y != 0.f || c.z != 0.f)
+            atomic_add3(pix_all + 3 * (size_t)kb * npix, p, divs(c, (float)npix));
     }
 }
 
@@ -1203,8 +1202,8 @@ static hipError_t run_subpaths(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr
 // the grids' buffers come from mem.  vb.err is set on the device if a pass's
 // points spread over too many cells.
 static int light_point_grids(wr_ctx* ctx, Scratch& mem, const SceneDev& S, const wr_tree_hdr& H,
-                             const wrd::CamDev& cam, uint32_t npix, uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius,
-                             uint32_t maxv, wrd::BVert* V, uint32_t* counts, const VcmBufs& vb, bool eye,
+                             const wrd::CamDev& cam, uint32_t npix, uint32_t max_depth, uint64_t seed,
+                             uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, wrd::BVert* V, uint32_t* counts, const VcmBufs& vb, bool eye,
                              const char* who) {
     hipStream_t st = ctx->stream;
     const uint32_t lanes = npass * npix;  // the caller keeps npass * npix below 2^31
@@ -1319,8 +1318,8 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     return WR_OK;
 }
 
-int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth, uint64_t seed,
-                      uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts, uint32_t* counts,
+int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
+                      uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts, uint32_t* counts,
                       float* pix, const VcmBufs& vb, const FilmBufs& film) {
     hipStream_t st = ctx->stream;
     const wrd::CamDev cam = make_cam_dev(ch);
@@ -1329,8 +1328,8 @@ int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
     const uint32_t blocks = (lanes + 255) / 256;
     wrd::BVert* V = (wrd::BVert*)verts;
     Scratch mem(*ctx->pool);  // the grids'
-    int rc = light_point_grids(ctx, mem, S, H, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts, vb,
-                               false, "wr_render_ppm");
+    int rc = light_point_grids(ctx, mem, S, H, cam, npix, max_depth, seed, pass0, npass, base_radius, maxv, V, counts,
+                               vb, false, "wr_render_ppm");
     if (rc != WR_OK) return rc;
     wrd::k_ppm_throughput<<<blocks, 256, 0, st>>>(lanes, maxv, V, counts);
     const wrd::PpmWalk P{cam, pass0, npix, maxv, seed, V};
@@ -1356,8 +1355,8 @@ size_t vcm_scan_bytes(uint32_t lanes) {
     return tb;
 }
 
-hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
-                              uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
+hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch,
+                              uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
                               const BdptQueue& q, const FilmBufs& film) {
     hipStream_t st = ctx->stream;
     const wrd::CamDev cam = make_cam_dev(ch);
@@ -1380,12 +1379,12 @@ hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr&
     if (e != hipSuccess) return e;
     for (uint64_t a = 0; a < lanes; a += part) {
         const uint32_t first = (uint32_t)a, end = (uint32_t)std::min<uint64_t>(lanes, a + part), n = end - first;
-        wrd::k_bdpt_prefix<<<(uint32_t)((2ull * n + 255) / 256), 256, 0, st>>>(S, cam, npix, first, end, maxv,
-                                                                              (const wrd::BVert*)verts, q.counts, prefix);
+        wrd::k_bdpt_prefix<<<(uint32_t)((2ull * n + 255) / 256), 256, 0, st>>>(
+            S, cam, npix, first, end, maxv, (const wrd::BVert*)verts, q.counts, prefix);
         const uint32_t width = connect_width(n, kBdptWaves);
         wrd::k_bdpt<<<(uint32_t)((n + 4ull * width - 1) / (4 * width)), 256, wrd::kStackLdsBytes, st>>>(
-            S, cam, first, end, npix, maxv, (const wrd::BVert*)verts, prefix - (ptrdiff_t)first * 2 * maxv, q.counts, pix,
-            Q, width);
+            S, cam, first, end, npix, maxv, (const wrd::BVert*)verts, prefix - (ptrdiff_t)first * 2 * maxv, q.counts,
+            pix, Q, width);
     }
     uint32_t nq = 0;
     e = hipMemcpyAsync(&nq, q.count, sizeof(uint32_t), hipMemcpyDeviceToHost, st);

@@ -1160,7 +1160,8 @@ int wr_scene_set_closest_hit_tuning(wr_scene* s, const wr_closest_hit_tuning* t)
 int wr_closest_hit_noself(wr_ctx* ctx, const wr_scene* s, const wr_path_ray* d_rays, uint64_t n, wr_hit* d_hits) {
     if (!ctx || !s || (n && (!d_rays || !d_hits))) return fail(ctx, WR_EINVAL, "wr_closest_hit_noself: bad argument");
     if (!s->built) return fail(ctx, WR_ESTATE, "wr_closest_hit_noself: scene not built");
-    hipError_t e = launch_closest_hit_path(s->dev, s->hdrs[0], (const uint32_t*)d_rays, n, d_hits, ctx->d_work, ctx->stream);
+    hipError_t e =
+        launch_closest_hit_path(s->dev, s->hdrs[0], (const uint32_t*)d_rays, n, d_hits, ctx->d_work, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "wr_closest_hit_noself launch");
     return WR_OK;
 }

@@ -750,7 +750,8 @@ int wr_hashgrid_query(wr_hashgrid* g, const float* d_queries, uint64_t nq, uint3
         g->defer_cap = nq + 1;
     }
     PH_CHECK(hipMemsetAsync(g->defer, 0, sizeof(uint32_t), ctx->stream), "wr_hashgrid_query");
-    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts, d_idx, g->defer);
+    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts,
+                                                                         d_idx, g->defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query");
     // the deferred queries: a workgroup each, as many workgroups as fill the device twice
     const unsigned wide_grid = (unsigned)std::min<uint64_t>(nq, 2048);
@@ -775,7 +776,8 @@ int wr_hashgrid_query_noalloc(wr_hashgrid* g, const float* d_queries, uint64_t n
     // the list keeps the previous call's contents: only its counter must start at zero
     k_clear_word<<<1, 1, 0, ctx->stream>>>(defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query_noalloc");
-    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts, d_idx, defer);
+    k_grid_query<<<(unsigned)((nq + 255) / 256), 256, 0, ctx->stream>>>(g->v, d_queries, (uint32_t)nq, cap, d_counts,
+                                                                         d_idx, defer);
     PH_CHECK(hipGetLastError(), "wr_hashgrid_query_noalloc");
     const unsigned wide_grid = (unsigned)std::min<uint64_t>(nq, 2048);
     k_grid_query_wide<<<wide_grid, 256, 0, ctx->stream>>>(g->v, g->boxes, d_queries, cap, d_counts, d_idx, defer);

@@ -331,8 +331,8 @@ extern "C" int wr_render_bdpt(wr_ctx* ctx, const wr_scene* s, const wr_camera* c
     bool launched = false;  // a failure leaves the film part-written
     for (uint32_t k = 0; k < prm->spp && e == hipSuccess; k += (uint32_t)batch) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, prm->spp - k);
-        e = launch_bdpt_passes(ctx, s->dev, s->hdrs[0], ch, prm->max_depth, prm->seed, film->passes + k, nb, maxv, verts,
-                               pix, q, fb);
+        e = launch_bdpt_passes(ctx, s->dev, s->hdrs[0], ch, prm->max_depth, prm->seed, film->passes + k, nb, maxv,
+                               verts, pix, q, fb);
         // the first passes allocate before they write
         launched = launched || e != hipErrorOutOfMemory;
     }
@@ -494,8 +494,8 @@ extern "C" int wr_render_ppm(wr_ctx* ctx, const wr_scene* s, const wr_camera* ca
     const FilmBufs fb{film->sum, film->comp, film->sumsq};
     for (uint32_t k = 0; k < prm->spp; k += (uint32_t)batch) {
         const uint32_t nb = (uint32_t)std::min<uint64_t>(batch, prm->spp - k);
-        const int rc = launch_ppm_passes(ctx, s->dev, s->hdrs[0], ch, prm->max_depth, prm->seed, film->passes + k, nb, base_radius,
-                                         maxv, verts, counts, pix, vb, fb);
+        const int rc = launch_ppm_passes(ctx, s->dev, s->hdrs[0], ch, prm->max_depth, prm->seed, film->passes + k, nb,
+                                         base_radius, maxv, verts, counts, pix, vb, fb);
         if (rc != WR_OK) {  // the film may hold part of this call's passes
             (void)hipStreamSynchronize(ctx->stream);
             film->broken = true;

@@ -90,7 +90,7 @@ struct wr_ctx {
     std::string err;
     float* film_back = nullptr;  // pinned, for small films on their way to the host (read_film)
     std::mutex film_mu;          // held by the read that uses it
-    unsigned long long* d_work = nullptr;  // work counters of the persistent closest-hit kernel (each call leaves them zero)
+    unsigned long long* d_work = nullptr;  // work counters of the persistent kernels (each call leaves them zero)
     wr::Engine engine;  // wavefront engine of wr_render, reused across calls
     uint32_t tuned_slots = 0, tuned_grid = 0;  // wr_autotune_render's choice (0 = defaults)
     uint32_t tuned_lds = 8;                    // wr_autotune_render's traversal stack levels in LDS
@@ -185,8 +185,8 @@ int launch_vcm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, cons
 // PhotonMap (bdpt.hip): passes [pass0, pass0 + npass) side by side [light
 // sub-paths, light points, one hash grid per pass, eye merge paths and density
 // estimates, film]; buffers as for launch_vcm_passes (counts: 2 per lane).
-int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth, uint64_t seed,
-                      uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts, uint32_t* counts,
+int launch_ppm_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& ch, uint32_t max_depth,
+                      uint64_t seed, uint32_t pass0, uint32_t npass, float base_radius, uint32_t maxv, void* verts, uint32_t* counts,
                       float* pix, const VcmBufs& vb, const FilmBufs& film);
 }  // namespace wr
 

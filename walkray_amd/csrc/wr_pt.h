@@ -45,8 +45,8 @@ constexpr uint32_t kDefaultPathSlots = 1u << 22;  // 4M paths in flight: 2 x 416
 constexpr uint32_t kBdptMaxDepth = 32;           // BidirectionalPathTracer: maxPathLen limit of wr_render_bdpt
 
 enum : uint32_t { kJobFree = 0, kJobRunning = 1, kJobDone = 2, kJobCancelled = 3 };
-// A cancelled job's paths still in the pool are dropped by the next extend
-// stage (k_wf_finish reads the job state first), so no kernel touches its
+// A cancelled job's paths still in the pool are dropped by the next iteration
+// (k_wf_finish and k_wf_rest read the job state first), so no kernel touches its
 // sample window or film after the state is written; its slot is reused only
 // after one more replay, once those paths are gone.
 enum : uint32_t { kJobNee = 1 };  // JobDesc::flags: PathTracer's next-event branch
@@ -92,7 +92,9 @@ struct EngineCounters {
     unsigned long long trace_nodes, trace_tris;  // fast-pass records fetched by the counting trace kernel
 };
 
-// The eight kernels of one wavefront iteration, in launch order.
+// The kernels of one wavefront iteration that the statistics time, in launch
+// order.  Between the exits' shade and the plan a render also launches k_wf_rest,
+// which the statistics leave out: they run every path iteration by iteration.
 enum : int { kStTrace = 0, kStFinish, kStShade, kStShadeExits, kStPlan, kStGenerate, kStFold, kStAdvance, kStages };
 
 // How run_wavefront issues its iterations: replays of the captured graphs, the
@@ -150,7 +152,8 @@ struct Engine {
     hipError_t ensure_graphs(hipStream_t st, bool nee);
     uint32_t few() const;  // live paths up to which an iteration takes them to their ends (k_wf_rest)
     hipError_t set_scene(uint32_t slot, const SceneDev& S, hipStream_t st);
-    hipError_t admit(uint32_t slot, const JobDesc& J, hipStream_t st, const SceneDev* scene = nullptr);  // scene: into scene slot 0
+    // scene: also into scene slot 0
+    hipError_t admit(uint32_t slot, const JobDesc& J, hipStream_t st, const SceneDev* scene = nullptr);
     hipError_t release_slot(uint32_t slot, hipStream_t st);
     hipError_t cancel_slot(uint32_t slot, hipStream_t st);
     // One replay: kGraphIters iterations, or kTailIters when `tail` (every
@@ -182,8 +185,8 @@ struct BdptQueue {
 };
 constexpr size_t kBdptQueueEntryBytes = 32 + 16 + 4 + 16;
 size_t bdpt_vertex_bytes();
-hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& cam, uint32_t max_depth,
-                              uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
+hipError_t launch_bdpt_passes(wr_ctx* ctx, const SceneDev& S, const wr_tree_hdr& H, const CamHost& cam,
+                              uint32_t max_depth, uint64_t seed, uint32_t pass0, uint32_t npass, uint32_t maxv, void* verts, float* pix,
                               const BdptQueue& q, const FilmBufs& film);
 
 hipError_t run_wavefront(const SceneDev& S, const CamHost& cam, uint32_t max_depth, uint64_t seed, uint32_t pass0,
