@@ -49,7 +49,7 @@ def test_long_walks(ctx):
 @pytest.mark.parametrize("n", [1000, 70000])
 def test_path_limit_costs_no_launches(ctx, n):
     """The time of a call follows its paths, not the limit on their length: light paths in the open field,
-    where none has 40 scatters, with limits of 40 and 1,000 (two launches a step made that 10 ms of 0.3)."""
+    where none has 40 scatters, with limits of 40 and 1,000 (two launches a step made that 5 ms of 0.3)."""
     sc = W.Scene(ctx, S.random_field(n_objects=30, seed=4)[0])
 
     def best(depth):

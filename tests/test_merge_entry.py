@@ -37,16 +37,16 @@ def test_entries_come_back(tmp_path):
 
 @pytest.mark.gpu
 def test_image_of_more_than_2_24_pixels(ctx):
-    """A pass whose last rows are past lane 2^24.  Rows whose merges went elsewhere would stand out: at this
-    radius merging makes a third of the image or more, and the twenty rows before the line and the twenty
-    after it, 82,000 pixels each, have the same mean within 3% (a row's mean varies by 10%)."""
+    """A pass whose last rows are past lane 2^24, with 25M merges, which the queue holds.  Rows whose merges
+    went elsewhere would stand out: merging makes a quarter of them, and the twenty rows before the line and
+    the twenty after it, 82,000 pixels each, differ by 2%."""
     from walkray_amd import _lib as W
     from walkray_amd import scenes as S
 
     width, height = 4100, 4200
     objs, cam = S.cornell(k=2, width=width, height=height)
     film = W.Film(ctx, width, height)
-    W.render_vcm(W.Scene(ctx, objs), cam, film, 1, 1, 3, 0.001)
+    W.render_vcm(W.Scene(ctx, objs), cam, film, 1, 1, 3, 0.0003)
     rows = film.read()["mean"].reshape(height, width, 3).mean(axis=(1, 2))
     line = (1 << 24) // width
     before, after = rows[line - 20:line].mean(), rows[line + 1:line + 21].mean()
